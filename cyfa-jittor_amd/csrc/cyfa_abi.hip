@@ -83,6 +83,46 @@ int scratch_base(hipStream_t stream, void** out, const char* what) {
     return CYFA_OK;
 }
 
+template <class E>
+int short_conv_as(const CyfaConvArgs* a, const char* what, void* hip_stream) {
+    if (!a) return fail(CYFA_ERR_VALUE, "%s: null args", what);
+    if (a->B < 0 || a->T < 0 || a->D <= 0 || a->split <= 0)
+        return fail(CYFA_ERR_VALUE, "%s: B=%d T=%d D=%d split=%d", what, a->B, a->T, a->D, a->split);
+    if (a->W < 2 || a->W > 4) return fail(CYFA_ERR_UNSUPPORTED, "%s: width %d not in 2..4", what, a->W);
+    if (a->D % 8 != 0 || a->split % 8 != 0 || a->D % a->split != 0 || a->D / a->split > 3)
+        return fail(CYFA_ERR_UNSUPPORTED, "%s: D=%d split=%d (multiples of 8, at most 3 outputs)", what, a->D,
+                    a->split);
+    if (!a->x || !a->weight) return fail(CYFA_ERR_VALUE, "%s: null required pointer", what);
+    for (int i = 0; i < a->D / a->split; i++)
+        if (!a->out[i] || !aligned(a->out[i], 16)) return fail(CYFA_ERR_ALIGN, "%s: output %d null or misaligned", what, i);
+    if (!aligned(a->x, 16) || a->x_row % 8 != 0 || (a->cache && (!aligned(a->cache, 16) || a->cache_row % 8 || a->cache_batch % 8)) ||
+        (a->cache_out && (!aligned(a->cache_out, 16) || a->cache_out_row % 8 || a->cache_out_batch % 8)))
+        return fail(CYFA_ERR_ALIGN, "%s: inputs need 16-byte aligned rows", what);
+    if (a->cache_out && a->cache_out == a->cache && a->T > 32)
+        return fail(CYFA_ERR_VALUE, "%s: in-place cache update needs T <= 32, got %d", what, a->T);
+    if (a->B == 0 || a->T == 0) return CYFA_OK;
+    cyfa::ConvParamsT<E> p;
+    p.B = a->B;
+    p.T = a->T;
+    p.D = a->D;
+    p.W = a->W;
+    p.x = (const E*)a->x;
+    p.x_row = a->x_row;
+    p.cache = (const E*)a->cache;
+    p.cache_row = a->cache_row;
+    p.cache_batch = a->cache_batch;
+    p.weight = (const E*)a->weight;
+    p.bias = (const E*)a->bias;
+    for (int i = 0; i < 3; i++) p.out[i] = (E*)a->out[i];
+    p.split = a->split;
+    p.cache_out = (E*)a->cache_out;
+    p.cache_out_row = a->cache_out_row;
+    p.cache_out_batch = a->cache_out_batch;
+    if (cyfa::launch_short_conv(p, (hipStream_t)hip_stream) != 0)
+        return fail(CYFA_ERR_UNSUPPORTED, "%s: W=%d", what, a->W);
+    return check_launch(what);
+}
+
 }  // namespace
 
 extern "C" {
@@ -552,42 +592,52 @@ int cyfa_rms_norm(const CyfaNormArgs* a, void* hip_stream) {
 }
 
 int cyfa_short_conv(const CyfaConvArgs* a, void* hip_stream) {
-    if (!a) return fail(CYFA_ERR_VALUE, "cyfa_short_conv: null args");
-    if (a->B < 0 || a->T < 0 || a->D <= 0 || a->split <= 0)
-        return fail(CYFA_ERR_VALUE, "cyfa_short_conv: B=%d T=%d D=%d split=%d", a->B, a->T, a->D, a->split);
-    if (a->W < 2 || a->W > 4) return fail(CYFA_ERR_UNSUPPORTED, "cyfa_short_conv: width %d not in 2..4", a->W);
-    if (a->D % 8 != 0 || a->split % 8 != 0 || a->D % a->split != 0 || a->D / a->split > 3)
-        return fail(CYFA_ERR_UNSUPPORTED, "cyfa_short_conv: D=%d split=%d (multiples of 8, at most 3 outputs)", a->D,
-                    a->split);
-    if (!a->x || !a->weight) return fail(CYFA_ERR_VALUE, "cyfa_short_conv: null required pointer");
-    for (int i = 0; i < a->D / a->split; i++)
-        if (!a->out[i] || !aligned(a->out[i], 16)) return fail(CYFA_ERR_ALIGN, "cyfa_short_conv: output %d null or misaligned", i);
-    if (!aligned(a->x, 16) || a->x_row % 8 != 0 || (a->cache && (!aligned(a->cache, 16) || a->cache_row % 8 || a->cache_batch % 8)) ||
-        (a->cache_out && (!aligned(a->cache_out, 16) || a->cache_out_row % 8 || a->cache_out_batch % 8)))
-        return fail(CYFA_ERR_ALIGN, "cyfa_short_conv: inputs need 16-byte aligned rows");
-    if (a->cache_out && a->cache_out == a->cache && a->T > 32)
-        return fail(CYFA_ERR_VALUE, "cyfa_short_conv: in-place cache update needs T <= 32, got %d", a->T);
-    if (a->B == 0 || a->T == 0) return CYFA_OK;
-    cyfa::ConvParams p;
+    return short_conv_as<__bf16>(a, "cyfa_short_conv", hip_stream);
+}
+
+int cyfa_short_conv_f32(const CyfaConvArgs* a, void* hip_stream) {
+    return short_conv_as<float>(a, "cyfa_short_conv_f32", hip_stream);
+}
+
+size_t cyfa_short_conv_grad_workspace_bytes(int B, int T, int D, int W) {
+    if (B <= 0 || T <= 0 || D <= 0 || W < 2 || W > 4) return 0;
+    return cyfa::conv_grad_workspace_bytes(B, T, D, W);
+}
+
+int cyfa_short_conv_grad(const CyfaConvGradArgs* a, int dtype, void* hip_stream) {
+    const char* what = "cyfa_short_conv_grad";
+    if (!a) return fail(CYFA_ERR_VALUE, "%s: null args", what);
+    if (dtype != CYFA_DTYPE_BF16 && dtype != CYFA_DTYPE_F32) return fail(CYFA_ERR_VALUE, "%s: dtype %d", what, dtype);
+    if (a->B <= 0 || a->T <= 0 || a->D <= 0) return fail(CYFA_ERR_VALUE, "%s: B=%d T=%d D=%d", what, a->B, a->T, a->D);
+    if (a->W < 2 || a->W > 4) return fail(CYFA_ERR_UNSUPPORTED, "%s: width %d not in 2..4", what, a->W);
+    if (a->D % 8 != 0) return fail(CYFA_ERR_UNSUPPORTED, "%s: D=%d is not a multiple of 8", what, a->D);
+    if (!a->x || !a->weight || !a->dy || !a->workspace) return fail(CYFA_ERR_VALUE, "%s: null required pointer", what);
+    if (a->workspace_bytes < cyfa::conv_grad_workspace_bytes(a->B, a->T, a->D, a->W))
+        return fail(CYFA_ERR_WORKSPACE, "%s: workspace of %zu bytes", what, a->workspace_bytes);
+    if (!aligned(a->x, 16) || a->x_row < a->D || a->x_row % 8 || !aligned(a->dy, 16) || !aligned(a->workspace, 16) ||
+        (a->dx && !aligned(a->dx, 16)) || (a->dcache && !aligned(a->dcache, 16)) ||
+        (a->cache && (!aligned(a->cache, 16) || a->cache_row % 8 || a->cache_batch % 8)))
+        return fail(CYFA_ERR_ALIGN, "%s: rows need 16-byte alignment", what);
+    cyfa::ConvGradParams p;
     p.B = a->B;
     p.T = a->T;
     p.D = a->D;
     p.W = a->W;
-    p.x = (const __bf16*)a->x;
+    p.x = a->x;
     p.x_row = a->x_row;
-    p.cache = (const __bf16*)a->cache;
+    p.cache = a->cache;
     p.cache_row = a->cache_row;
     p.cache_batch = a->cache_batch;
-    p.weight = (const __bf16*)a->weight;
-    p.bias = (const __bf16*)a->bias;
-    for (int i = 0; i < 3; i++) p.out[i] = (__bf16*)a->out[i];
-    p.split = a->split;
-    p.cache_out = (__bf16*)a->cache_out;
-    p.cache_out_row = a->cache_out_row;
-    p.cache_out_batch = a->cache_out_batch;
-    if (cyfa::launch_short_conv(p, (hipStream_t)hip_stream) != 0)
-        return fail(CYFA_ERR_UNSUPPORTED, "cyfa_short_conv: W=%d", a->W);
-    return check_launch("cyfa_short_conv");
+    p.weight = a->weight;
+    p.dy = a->dy;
+    p.dx = a->dx;
+    p.dcache = a->dcache;
+    p.dweight = a->dweight;
+    p.dbias = a->dbias;
+    p.part = (float*)a->workspace;
+    if (cyfa::launch_conv_grad(p, dtype == CYFA_DTYPE_BF16, (hipStream_t)hip_stream) != 0)
+        return fail(CYFA_ERR_UNSUPPORTED, "%s: B=%d T=%d past the grid's limits", what, a->B, a->T);
+    return check_launch(what);
 }
 
 int cyfa_silu_mul(const void* gu, void* out, int rows, int F, void* hip_stream) {

@@ -143,17 +143,32 @@ struct NormParams {
     __bf16* out;
 };
 
-struct ConvParams {
+template <class E>
+struct ConvParamsT {             // E: __bf16 or float
     int B, T, D, W;
-    const __bf16* x;
+    const E* x;
     long long x_row;             // elements between time rows of x
-    const __bf16* cache;         // nullable: [B, W-1, D] view
+    const E* cache;              // nullable: [B, W-1, D] view
     long long cache_row, cache_batch;
-    const __bf16 *weight, *bias; // [D, W], nullable [D]
-    __bf16* out[3];              // channel c -> out[c / split][(b*T + t)*split + c % split]
+    const E *weight, *bias;      // [D, W], nullable [D]
+    E* out[3];                   // channel c -> out[c / split][(b*T + t)*split + c % split]
     int split;
-    __bf16* cache_out;           // nullable: the last W-1 rows of X, cache addressing
+    E* cache_out;                // nullable: the last W-1 rows of X, cache addressing
     long long cache_out_row, cache_out_batch;
+};
+using ConvParams = ConvParamsT<__bf16>;
+
+// The short convolution's adjoint (cyfa_train.hip); every tensor bf16 or fp32.
+struct ConvGradParams {
+    int B, T, D, W;
+    const void* x;               // element (b, t, c) at x[(b T + t) x_row + c]
+    long long x_row;
+    const void* cache;           // nullable: [B, W-1, D] view
+    long long cache_row, cache_batch;
+    const void *weight, *dy;     // [D, W]; [B, T, D]
+    void *dx, *dcache;           // nullable [B, T, D], [B, W-1, D]
+    void *dweight, *dbias;       // nullable [D, W], [D]
+    float* part;                 // conv_grad_workspace_bytes
 };
 
 struct WorkspaceLayout {
@@ -460,6 +475,9 @@ int launch_general_decode(const GenDecodeParams& p, int bf16, hipStream_t stream
 int launch_rms_norm(const NormParams& p, hipStream_t stream);
 int launch_linear_rows(const LinearParams& p, hipStream_t stream);
 int launch_short_conv(const ConvParams& p, hipStream_t stream);
+int launch_short_conv(const ConvParamsT<float>& p, hipStream_t stream);
+size_t conv_grad_workspace_bytes(int B, int T, int D, int W);
+int launch_conv_grad(const ConvGradParams& p, bool bf16, hipStream_t stream);
 int launch_silu_mul(const __bf16* gu, __bf16* out, int rows, int F, hipStream_t stream);
 int launch_argmax_rows(const __bf16* x, long long ldx, int rows, int n, long long* out, hipStream_t stream);
 int launch_gate_path(const GatePathParams& p, hipStream_t stream);

@@ -883,8 +883,9 @@ __global__ __launch_bounds__(512) void gate_path_kernel(GatePathParams p) {
 // single run it has read its cache rows before, so the update may be in place.
 constexpr int CONV_RUN = 32;
 
-template <int W>
-__global__ __launch_bounds__(256) void short_conv_kernel(ConvParams p) {
+template <class E, int W>
+__global__ __launch_bounds__(256) void short_conv_kernel(ConvParamsT<E> p) {
+    typedef E ex8 __attribute__((ext_vector_type(8), aligned(16)));
     const int c8 = (blockIdx.x * 256 + threadIdx.x) * 8;
     if (c8 >= p.D) return;
     const int b = blockIdx.y, t0 = blockIdx.z * CONV_RUN;
@@ -895,48 +896,48 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ConvParams p) {
         for (int w = 0; w < W; w++) wt[w][i] = (float)p.weight[(size_t)(c8 + i) * W + w];
         bias[i] = p.bias ? (float)p.bias[c8 + i] : 0.f;
     }
-    auto row = [&](int i) -> bf16x8 {
-        if (i >= 0) return *reinterpret_cast<const bf16x8*>(p.x + ((size_t)b * p.T + i) * p.x_row + c8);
+    auto row = [&](int i) -> ex8 {
+        if (i >= 0) return *reinterpret_cast<const ex8*>(p.x + ((size_t)b * p.T + i) * p.x_row + c8);
         if (p.cache)
-            return *reinterpret_cast<const bf16x8*>(p.cache + (size_t)b * p.cache_batch + (size_t)(W - 1 + i) * p.cache_row + c8);
-        bf16x8 z;
+            return *reinterpret_cast<const ex8*>(p.cache + (size_t)b * p.cache_batch + (size_t)(W - 1 + i) * p.cache_row + c8);
+        ex8 z;
 #pragma unroll
-        for (int k = 0; k < 8; k++) z[k] = (bf16_t)0.f;
+        for (int k = 0; k < 8; k++) z[k] = (E)0.f;
         return z;
     };
     float win[W][8];
 #pragma unroll
     for (int w = 0; w < W - 1; w++) {
-        const bf16x8 r = row(t0 + w - (W - 1));
+        const ex8 r = row(t0 + w - (W - 1));
 #pragma unroll
         for (int i = 0; i < 8; i++) win[w][i] = (float)r[i];
     }
     const int out_i = c8 / p.split, col = c8 % p.split;
-    bf16_t* out = p.out[out_i];
+    E* out = p.out[out_i];
     const int t1 = t0 + CONV_RUN < p.T ? t0 + CONV_RUN : p.T;
     // Eight rows at a time: their loads are all in flight before the first is used.
     constexpr int U = 8;
     for (int tb = t0; tb < t1; tb += U) {
-        bf16x8 rows[U];
-        const bf16_t* src = p.x + ((size_t)b * p.T + tb) * p.x_row + c8;  // rows tb.. are never before the start
+        ex8 rows[U];
+        const E* src = p.x + ((size_t)b * p.T + tb) * p.x_row + c8;  // rows tb.. are never before the start
         const int n = t1 - tb;
 #pragma unroll
         for (int u = 0; u < U; u++)
-            rows[u] = *reinterpret_cast<const bf16x8*>(src + (size_t)(u < n ? u : 0) * p.x_row);
+            rows[u] = *reinterpret_cast<const ex8*>(src + (size_t)(u < n ? u : 0) * p.x_row);
 #pragma unroll
         for (int u = 0; u < U; u++) {
             if (tb + u < t1) {
 #pragma unroll
                 for (int i = 0; i < 8; i++) win[W - 1][i] = (float)rows[u][i];
-                bf16x8 y;
+                ex8 y;
 #pragma unroll
                 for (int i = 0; i < 8; i++) {
                     float acc = win[0][i] * wt[0][i];
 #pragma unroll
                     for (int w = 1; w < W; w++) acc = fmaf(win[w][i], wt[w][i], acc);
-                    y[i] = (bf16_t)(acc + bias[i]);
+                    y[i] = (E)(acc + bias[i]);
                 }
-                *reinterpret_cast<bf16x8*>(out + ((size_t)b * p.T + tb + u) * p.split + col) = y;
+                *reinterpret_cast<ex8*>(out + ((size_t)b * p.T + tb + u) * p.split + col) = y;
 #pragma unroll
                 for (int w = 0; w < W - 1; w++)
 #pragma unroll
@@ -947,10 +948,10 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ConvParams p) {
     if (p.cache_out && t1 == p.T) {
 #pragma unroll
         for (int w = 0; w < W - 1; w++) {
-            bf16x8 r;
+            ex8 r;
 #pragma unroll
-            for (int i = 0; i < 8; i++) r[i] = (bf16_t)win[w][i];
-            *reinterpret_cast<bf16x8*>(p.cache_out + (size_t)b * p.cache_out_batch + (size_t)w * p.cache_out_row + c8) = r;
+            for (int i = 0; i < 8; i++) r[i] = (E)win[w][i];
+            *reinterpret_cast<ex8*>(p.cache_out + (size_t)b * p.cache_out_batch + (size_t)w * p.cache_out_row + c8) = r;
         }
     }
 }
@@ -1250,16 +1251,26 @@ int launch_linear_rows(const LinearParams& p_in, hipStream_t stream) {
     return -1;
 }
 
-int launch_short_conv(const ConvParams& p, hipStream_t stream) {
+namespace {
+
+template <class E>
+int launch_short_conv_as(const ConvParamsT<E>& p, hipStream_t stream) {
     const dim3 grid((p.D / 8 + 255) / 256, p.B, (p.T + CONV_RUN - 1) / CONV_RUN), block(256);
     switch (p.W) {
-        case 2: hipLaunchKernelGGL(short_conv_kernel<2>, grid, block, 0, stream, p); break;
-        case 3: hipLaunchKernelGGL(short_conv_kernel<3>, grid, block, 0, stream, p); break;
-        case 4: hipLaunchKernelGGL(short_conv_kernel<4>, grid, block, 0, stream, p); break;
+        case 2: hipLaunchKernelGGL((short_conv_kernel<E, 2>), grid, block, 0, stream, p); break;
+        case 3: hipLaunchKernelGGL((short_conv_kernel<E, 3>), grid, block, 0, stream, p); break;
+        case 4: hipLaunchKernelGGL((short_conv_kernel<E, 4>), grid, block, 0, stream, p); break;
         default: return -1;
     }
     return 0;
 }
+
+}  // namespace
+
+int launch_short_conv(const ConvParams& p, hipStream_t stream) { return launch_short_conv_as(p, stream); }
+
+// fp32 rows (training in fp32): the same kernel.
+int launch_short_conv(const ConvParamsT<float>& p, hipStream_t stream) { return launch_short_conv_as(p, stream); }
 
 int launch_silu_mul(const bf16_t* gu, bf16_t* out, int rows, int F, hipStream_t stream) {
     const size_t n8 = (size_t)rows * F / 8;

@@ -14,7 +14,7 @@ import torch
 import torch.nn.functional as F
 
 LIB_PATH = Path(os.environ.get("CYFA_LIB", Path(__file__).with_name("libcyfa_hip.so")))
-ABI_VERSION = 11
+ABI_VERSION = 12
 
 CYFA_OK = 0
 CYFA_ERR_VALUE = -1
@@ -139,6 +139,17 @@ class CyfaConvArgs(ctypes.Structure):
     ]
 
 
+class CyfaConvGradArgs(ctypes.Structure):
+    _fields_ = [
+        ("B", _c_int), ("T", _c_int), ("D", _c_int), ("W", _c_int),
+        ("x", _c_void_p), ("x_row", ctypes.c_longlong),
+        ("cache", _c_void_p), ("cache_row", ctypes.c_longlong), ("cache_batch", ctypes.c_longlong),
+        ("weight", _c_void_p), ("dy", _c_void_p), ("dx", _c_void_p), ("dcache", _c_void_p),
+        ("dweight", _c_void_p), ("dbias", _c_void_p),
+        ("workspace", _c_void_p), ("workspace_bytes", _c_size_t),
+    ]
+
+
 class CyfaGatePathArgs(ctypes.Structure):
     _fields_ = [
         ("M", _c_int), ("K", _c_int), ("H", _c_int), ("Dv", _c_int),
@@ -162,6 +173,9 @@ SIGNATURES = {
     "cyfa_readout_table": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_int, _c_void_p]),
     "cyfa_rms_norm": (_c_int, [ctypes.POINTER(CyfaNormArgs), _c_void_p]),
     "cyfa_short_conv": (_c_int, [ctypes.POINTER(CyfaConvArgs), _c_void_p]),
+    "cyfa_short_conv_f32": (_c_int, [ctypes.POINTER(CyfaConvArgs), _c_void_p]),
+    "cyfa_short_conv_grad_workspace_bytes": (_c_size_t, [_c_int] * 4),
+    "cyfa_short_conv_grad": (_c_int, [ctypes.POINTER(CyfaConvGradArgs), _c_int, _c_void_p]),
     "cyfa_linear_rows": (_c_int, [ctypes.POINTER(CyfaLinearArgs), _c_void_p]),
     "cyfa_linear_rows_span": (_c_size_t, [_c_int] * 5),
     "cyfa_norm_linear_rows": (_c_int, [ctypes.POINTER(CyfaLinearArgs), ctypes.POINTER(CyfaRowNormArgs), _c_void_p]),
@@ -630,8 +644,8 @@ def linear_swiglu(x, w_interleaved):
 def short_conv(x, weight, bias=None, cache=None, split=None, cache_out=None):
     """Causal depthwise convolution over time of x [B, T, D] (rows may be strided).
 
-    weight [D, W] bf16, cache an optional [B, W-1, D] view. The D channels are
-    written to D // split contiguous [B, T, split] tensors (split defaults to D).
+    x, weight [D, W], bias and cache (an optional [B, W-1, D] view) all bf16, or
+    all fp32. The D channels are written to D // split contiguous [B, T, split] tensors (split defaults to D).
     ``cache_out`` [B, W-1, D] (channel stride 1) receives the last W-1 rows of
     cat(cache, x); it may be ``cache`` itself when T <= 32."""
     dev = require_device(x, weight, bias, cache)
@@ -652,8 +666,34 @@ def short_conv(x, weight, bias=None, cache=None, split=None, cache_out=None):
                         cache_out_batch=0 if cache_out is None else cache_out.stride(0))
     for i, o in enumerate(outs):
         args.out[i] = o.data_ptr()
-    _check(load_library().cyfa_short_conv(ctypes.byref(args), stream_handle(dev)), "cyfa_short_conv")
+    lib = load_library()
+    fn = lib.cyfa_short_conv_f32 if x.dtype == torch.float32 else lib.cyfa_short_conv
+    _check(fn(ctypes.byref(args), stream_handle(dev)), "cyfa_short_conv")
     return outs
+
+
+SHORT_CONV_MAX_GRID = 65535  # batch rows, and blocks of 32 tokens, of a short_conv launch
+
+
+def short_conv_grad(x, weight, cache, dy, needed):
+    """Gradients (dx, dweight, dbias, dcache) of short_conv's y [B, T, D] from
+    its cotangent dy, None where ``needed`` is false. x and cache rows 16-byte
+    aligned, weight [D, W], everything one dtype (bf16 or fp32)."""
+    dev = require_device(x, weight, cache, dy)
+    B, T, D = x.shape
+    W = weight.shape[-1]
+    shapes = ((B, T, D), (D, W), (D,), (B, W - 1, D))
+    dx, dw, db, dc = (torch.empty(s, dtype=x.dtype, device=dev) if n else None for s, n in zip(shapes, needed))
+    lib = load_library()
+    n = int(lib.cyfa_short_conv_grad_workspace_bytes(B, T, D, W))
+    workspace = torch.empty(max(n, 1), dtype=torch.uint8, device=dev)  # alive until the launch
+    args = CyfaConvGradArgs(B=B, T=T, D=D, W=W, x=ptr(x), x_row=x.stride(1), cache=ptr(cache),
+                            cache_row=0 if cache is None else cache.stride(1),
+                            cache_batch=0 if cache is None else cache.stride(0), weight=ptr(weight), dy=ptr(dy),
+                            dx=ptr(dx), dcache=ptr(dc), dweight=ptr(dw), dbias=ptr(db), workspace=ptr(workspace),
+                            workspace_bytes=n)
+    _check(lib.cyfa_short_conv_grad(ctypes.byref(args), general_dtype(x), stream_handle(dev)), "cyfa_short_conv_grad")
+    return dx, dw, db, dc
 
 
 def silu_mul(gu):

@@ -27,6 +27,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from .. import _native
+from .autograd import hip_autograd_ok, short_conv
 from ..ops import chunk_cyfa, fused_recurrent_cyfa
 from ..ops.fused_recurrent import decode_layer_step
 from ..ops.utils import readout_table
@@ -132,15 +133,22 @@ class ShortConvolution(nn.Module):
                                    None if self.bias is None else self.bias.to(x.dtype),
                                    None if cache is None else cache.to(x.dtype))[0]
             return y, conv_cache_tail(x, cache, W)
-        history = x if cache is None else torch.cat([cache.to(x.dtype), x], dim=1)
+        if cache is not None:
+            cache = cache.to(x.dtype)
+        history = x if cache is None else torch.cat([cache, x], dim=1)
         offset = W - 1 if cache is None else 0
-        padded = F.pad(history, (0, 0, offset, 0)) if offset else history
-        y = F.conv1d(
-            padded.transpose(1, 2),
-            self.weight.to(x.dtype),
-            None if self.bias is None else self.bias.to(x.dtype),
-            groups=D,
-        ).transpose(1, 2)
+        weight = self.weight.to(x.dtype)
+        bias = None if self.bias is None else self.bias.to(x.dtype)
+        if (x.dtype in (torch.bfloat16, torch.float32) and 2 <= W <= 4 and D % 8 == 0 and x.numel() > 0
+                and B <= _native.SHORT_CONV_MAX_GRID and T <= 32 * _native.SHORT_CONV_MAX_GRID
+                and (cache is None or tuple(cache.shape) == (B, W - 1, D))
+                and hip_autograd_ok(x, weight, bias, cache)):
+            # training: the convolution and its adjoint as HIP kernels (the
+            # library's depthwise convolution goes through im2col, transposes
+            # and small GEMMs)
+            y = short_conv(x, weight.reshape(D, W), bias, cache, general_short_conv)
+        else:
+            y = general_short_conv(x, weight.reshape(D, W), bias, cache)
         S = history.shape[1]
         if W == 1:
             new_cache = history[:, :0]
@@ -154,6 +162,14 @@ class ShortConvolution(nn.Module):
         return y.contiguous(), new_cache
 
     execute = forward
+
+
+def general_short_conv(x, weight, bias, cache):
+    """The short convolution in torch operations: x [B, T, D], weight [D, W],
+    bias [D] or None, cache [B, W-1, D] or None (W-1 zero rows)."""
+    W = weight.shape[-1]
+    padded = F.pad(x, (0, 0, W - 1, 0)) if cache is None else torch.cat([cache, x], dim=1)
+    return F.conv1d(padded.transpose(1, 2), weight.unsqueeze(1), bias, groups=x.shape[-1]).transpose(1, 2)
 
 
 def shared_conv_cache(conv_state):

@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define CYFA_ABI_VERSION 11
+#define CYFA_ABI_VERSION 12
 
 enum {
     CYFA_OK = 0,
@@ -482,6 +482,31 @@ typedef struct CyfaConvArgs {
 /* Replaces ShortConvolution.execute / _inference (layers/cyfa.py:138-233); the
  * new cache (the last W-1 inputs) stays a view of the input in the caller. */
 int cyfa_short_conv(const CyfaConvArgs *args, void *hip_stream);
+
+/* The same with every tensor f32 (training in fp32). */
+int cyfa_short_conv_f32(const CyfaConvArgs *args, void *hip_stream);
+
+/* The gradients of the convolution above (D a multiple of 8, W in 2..4) from
+ * dy, the cotangent of y with split = D; every tensor of one dtype
+ * (CYFA_DTYPE_BF16 or CYFA_DTYPE_F32), sums over tokens in fp32 and in a fixed
+ * order. Replaces the autograd adjoint behind ShortConvolution.execute
+ * (layers/cyfa.py:138-233). */
+typedef struct CyfaConvGradArgs {
+    int B, T, D, W;
+    const void *x;                /* element (b,t,c) at x[(b*T + t)*x_row + c], 16-byte aligned rows */
+    long long x_row;
+    const void *cache;            /* nullable, (b,i,c) at cache[b*cache_batch + i*cache_row + c] */
+    long long cache_row, cache_batch;
+    const void *weight;           /* [D, W] */
+    const void *dy;               /* [B, T, D], 16-byte aligned */
+    void *dx, *dcache;            /* nullable [B, T, D] and [B, W-1, D], 16-byte aligned */
+    void *dweight, *dbias;        /* nullable [D, W] and [D] */
+    void *workspace;              /* cyfa_short_conv_grad_workspace_bytes(B, T, D, W) bytes, 16-byte aligned */
+    size_t workspace_bytes;
+} CyfaConvGradArgs;
+
+size_t cyfa_short_conv_grad_workspace_bytes(int B, int T, int D, int W);
+int cyfa_short_conv_grad(const CyfaConvGradArgs *args, int dtype, void *hip_stream);
 
 /* out[r, c] = bf16(g sigmoid(g) u), g = gu[r, c], u = gu[r, F + c]; F a
  * multiple of 8. Replaces the activation of GatedMLP.execute
