@@ -98,6 +98,7 @@ int short_conv_as(const CyfaConvArgs* a, const char* what, void* hip_stream) {
     if (!aligned(a->x, 16) || a->x_row % 8 != 0 || (a->cache && (!aligned(a->cache, 16) || a->cache_row % 8 || a->cache_batch % 8)) ||
         (a->cache_out && (!aligned(a->cache_out, 16) || a->cache_out_row % 8 || a->cache_out_batch % 8)))
         return fail(CYFA_ERR_ALIGN, "%s: inputs need 16-byte aligned rows", what);
+    if (a->mask && !a->lengths) return fail(CYFA_ERR_VALUE, "%s: mask without lengths", what);
     if (a->cache_out && a->cache_out == a->cache && a->T > 32)
         return fail(CYFA_ERR_VALUE, "%s: in-place cache update needs T <= 32, got %d", what, a->T);
     if (a->B == 0 || a->T == 0) return CYFA_OK;
@@ -118,6 +119,9 @@ int short_conv_as(const CyfaConvArgs* a, const char* what, void* hip_stream) {
     p.cache_out = (E*)a->cache_out;
     p.cache_out_row = a->cache_out_row;
     p.cache_out_batch = a->cache_out_batch;
+    p.mask = a->mask;
+    p.lengths = a->lengths;
+    p.run = 0;
     if (cyfa::launch_short_conv(p, (hipStream_t)hip_stream) != 0)
         return fail(CYFA_ERR_UNSUPPORTED, "%s: W=%d", what, a->W);
     return check_launch(what);
@@ -640,6 +644,16 @@ int cyfa_short_conv_grad(const CyfaConvGradArgs* a, int dtype, void* hip_stream)
     return check_launch(what);
 }
 
+int cyfa_mask_rows(const long long* mask, int B, int T, float* values, void* valid, int* lengths, void* hip_stream) {
+    const char* what = "cyfa_mask_rows";
+    if (B < 0 || T < 0) return fail(CYFA_ERR_VALUE, "%s: B=%d T=%d", what, B, T);
+    if (!mask || !values || !valid || !lengths) return fail(CYFA_ERR_VALUE, "%s: null pointer", what);
+    if (!aligned(mask, 8) || !aligned(values, 4) || !aligned(lengths, 4)) return fail(CYFA_ERR_ALIGN, "%s", what);
+    if (B == 0) return CYFA_OK;
+    cyfa::launch_mask_rows(mask, B, T, values, (unsigned char*)valid, lengths, (hipStream_t)hip_stream);
+    return check_launch(what);
+}
+
 int cyfa_silu_mul(const void* gu, void* out, int rows, int F, void* hip_stream) {
     if (!gu || !out || rows < 0 || F <= 0) return fail(CYFA_ERR_VALUE, "cyfa_silu_mul: bad arguments");
     if (F % 8 != 0) return fail(CYFA_ERR_UNSUPPORTED, "cyfa_silu_mul: F=%d must be a multiple of 8", F);
@@ -694,6 +708,7 @@ int cyfa_gate_path(const CyfaGatePathArgs* a, void* hip_stream) {
     p.g = a->g;
     p.beta = a->beta;
     p.delta = a->delta;
+    p.valid = (const unsigned char*)a->valid;
     if (cyfa::launch_gate_path(p, (hipStream_t)hip_stream) != 0)
         return fail(CYFA_ERR_UNSUPPORTED, "cyfa_gate_path: shape refused");
     return check_launch("cyfa_gate_path");

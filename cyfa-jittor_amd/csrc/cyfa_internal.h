@@ -155,6 +155,9 @@ struct ConvParamsT {             // E: __bf16 or float
     int split;
     E* cache_out;                // nullable: the last W-1 rows of X, cache addressing
     long long cache_out_row, cache_out_batch;
+    const float* mask;           // nullable [B, T]: row t of x counts as x mask
+    const int* lengths;          // [B], with mask: cache_out gets the W-1 rows of X before lengths[b]
+    int run;                     // tokens per run (set by the launcher)
 };
 using ConvParams = ConvParamsT<__bf16>;
 
@@ -248,6 +251,7 @@ struct GatePathParams {
     __bf16* gate;            // [M, Dv], rows ldg elements apart
     long long ldg;
     float *g, *beta, *delta;  // [M, H]
+    const unsigned char* valid;  // nullable [M]: g, beta and delta of a row are zero where it is zero
 };
 constexpr int GATE_PATH_G0 = 256;       // g_proj[0] width (head_v_dim) the kernel is built for
 constexpr int GATE_PATH_MAX_K = 2048;   // largest hidden size (its k-chunk loop is unrolled to this)
@@ -476,6 +480,8 @@ int launch_rms_norm(const NormParams& p, hipStream_t stream);
 int launch_linear_rows(const LinearParams& p, hipStream_t stream);
 int launch_short_conv(const ConvParams& p, hipStream_t stream);
 int launch_short_conv(const ConvParamsT<float>& p, hipStream_t stream);
+int launch_mask_rows(const long long* mask, int B, int T, float* values, unsigned char* valid, int* lengths,
+                     hipStream_t stream);
 size_t conv_grad_workspace_bytes(int B, int T, int D, int W);
 int launch_conv_grad(const ConvGradParams& p, bool bf16, hipStream_t stream);
 int launch_silu_mul(const __bf16* gu, __bf16* out, int rows, int F, hipStream_t stream);

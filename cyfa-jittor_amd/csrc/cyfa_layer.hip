@@ -805,7 +805,10 @@ __global__ __launch_bounds__(512) void gate_path_kernel(GatePathParams p) {
         for (int i = 0; i < 4; i++) {
             const int row = 16 * ab_rb + 4 * lg + i;
             const float v = (float)(bf16_t)(accab[i] + abias);
-            if (row < mrows) dst[(size_t)(m0 + row) * H + ah] = akind == 0 ? decay_gate(v + adt, aal) : sigmoidf(v);
+            if (row < mrows) {
+                const float out = akind == 0 ? decay_gate(v + adt, aal) : sigmoidf(v);
+                dst[(size_t)(m0 + row) * H + ah] = !p.valid || p.valid[m0 + row] ? out : 0.f;
+            }
         }
     }
     store2(buf[0], r2[0]);
@@ -881,14 +884,18 @@ __global__ __launch_bounds__(512) void gate_path_kernel(GatePathParams p) {
 // c / split, column c % split. The thread of the last run writes its window,
 // the last W - 1 rows of X, to cache_out (layers/cyfa.py:172-182); with a
 // single run it has read its cache rows before, so the update may be in place.
+// MASK (right-padded batches, layers/cyfa.py:309-312): row t of x counts as x
+// mask[b, t], rounded to E, and cache_out gets the W - 1 rows of X before
+// lengths[b] (the first run's thread, which reads all of them before it
+// writes). p.run tokens per run (launch_short_conv).
 constexpr int CONV_RUN = 32;
 
-template <class E, int W>
+template <class E, int W, bool MASK>
 __global__ __launch_bounds__(256) void short_conv_kernel(ConvParamsT<E> p) {
     typedef E ex8 __attribute__((ext_vector_type(8), aligned(16)));
-    const int c8 = (blockIdx.x * 256 + threadIdx.x) * 8;
+    const int c8 = (blockIdx.x * blockDim.x + threadIdx.x) * 8;
     if (c8 >= p.D) return;
-    const int b = blockIdx.y, t0 = blockIdx.z * CONV_RUN;
+    const int b = blockIdx.y, t0 = blockIdx.z * p.run;
     float wt[W][8], bias[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) {
@@ -896,8 +903,16 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ConvParamsT<E> p) {
         for (int w = 0; w < W; w++) wt[w][i] = (float)p.weight[(size_t)(c8 + i) * W + w];
         bias[i] = p.bias ? (float)p.bias[c8 + i] : 0.f;
     }
+    const auto masked = [&](ex8 v, float m) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = (E)((float)v[i] * m);
+        return v;
+    };
     auto row = [&](int i) -> ex8 {
-        if (i >= 0) return *reinterpret_cast<const ex8*>(p.x + ((size_t)b * p.T + i) * p.x_row + c8);
+        if (i >= 0) {
+            const ex8 v = *reinterpret_cast<const ex8*>(p.x + ((size_t)b * p.T + i) * p.x_row + c8);
+            return MASK ? masked(v, p.mask[(size_t)b * p.T + i]) : v;
+        }
         if (p.cache)
             return *reinterpret_cast<const ex8*>(p.cache + (size_t)b * p.cache_batch + (size_t)(W - 1 + i) * p.cache_row + c8);
         ex8 z;
@@ -914,7 +929,7 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ConvParamsT<E> p) {
     }
     const int out_i = c8 / p.split, col = c8 % p.split;
     E* out = p.out[out_i];
-    const int t1 = t0 + CONV_RUN < p.T ? t0 + CONV_RUN : p.T;
+    const int t1 = t0 + p.run < p.T ? t0 + p.run : p.T;
     // Eight rows at a time: their loads are all in flight before the first is used.
     constexpr int U = 8;
     for (int tb = t0; tb < t1; tb += U) {
@@ -924,6 +939,10 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ConvParamsT<E> p) {
 #pragma unroll
         for (int u = 0; u < U; u++)
             rows[u] = *reinterpret_cast<const ex8*>(src + (size_t)(u < n ? u : 0) * p.x_row);
+        if constexpr (MASK) {
+#pragma unroll
+            for (int u = 0; u < U; u++) rows[u] = masked(rows[u], p.mask[(size_t)b * p.T + tb + (u < n ? u : 0)]);
+        }
 #pragma unroll
         for (int u = 0; u < U; u++) {
             if (tb + u < t1) {
@@ -945,6 +964,18 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ConvParamsT<E> p) {
             }
         }
     }
+    if constexpr (MASK) {
+        if (p.cache_out && t0 == 0) {
+            const int end = min(max(p.lengths[b], 0), p.T);
+            ex8 r[W - 1];
+#pragma unroll
+            for (int w = 0; w < W - 1; w++) r[w] = row(end + w - (W - 1));
+#pragma unroll
+            for (int w = 0; w < W - 1; w++)
+                *reinterpret_cast<ex8*>(p.cache_out + (size_t)b * p.cache_out_batch + (size_t)w * p.cache_out_row + c8) = r[w];
+        }
+        return;
+    }
     if (p.cache_out && t1 == p.T) {
 #pragma unroll
         for (int w = 0; w < W - 1; w++) {
@@ -954,6 +985,27 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ConvParamsT<E> p) {
             *reinterpret_cast<ex8*>(p.cache_out + (size_t)b * p.cache_out_batch + (size_t)w * p.cache_out_row + c8) = r;
         }
     }
+}
+
+// An attention mask [B, T] as the kernels read it: its values rounded to bf16
+// (in fp32, which uniform code loads through the scalar cache), whether
+// each is nonzero, and each row's sum (int32), the number of tokens before its
+// right padding. One workgroup per row.
+__global__ __launch_bounds__(256) void mask_rows_kernel(const long long* mask, int T, float* values,
+                                                        unsigned char* valid, int* lengths) {
+    __shared__ int part[4];
+    const size_t base = (size_t)blockIdx.x * T;
+    int n = 0;
+    for (int t = threadIdx.x; t < T; t += 256) {
+        const long long m = mask[base + t];
+        values[base + t] = bf16_round((float)m);
+        valid[base + t] = m != 0;
+        n += (int)m;
+    }
+    for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = n;
+    __syncthreads();
+    if (threadIdx.x == 0) lengths[blockIdx.x] = (part[0] + part[1]) + (part[2] + part[3]);
 }
 
 // SwiGLU product (modeling_cyfa.py:22-27): out = bf16(g sigmoid(g) u) for
@@ -1253,13 +1305,27 @@ int launch_linear_rows(const LinearParams& p_in, hipStream_t stream) {
 
 namespace {
 
-template <class E>
-int launch_short_conv_as(const ConvParamsT<E>& p, hipStream_t stream) {
-    const dim3 grid((p.D / 8 + 255) / 256, p.B, (p.T + CONV_RUN - 1) / CONV_RUN), block(256);
+template <class E, bool MASK>
+int launch_short_conv_as(ConvParamsT<E> p, hipStream_t stream) {
+    // Tokens per run: a long run reads less (the three rows before a run are
+    // read again), a short one leaves no serial chain of load batches. By the
+    // waves that runs of 32 would give, us at 8 / 16 / 32 tokens on MI355X
+    // (bf16, B x T x D): 188 waves (2 x 1500 x 1024) 6.0 / 6.7 / 9.6, 192
+    // (1 x 1024 x 3072) 5.8 / 7.0 / 9.9, 864 (8 x 576 x 3072) 16.8 / 16.2 /
+    // 18.4, 1536 (8 x 1024 x 3072) 25.9 / 23.8 / 22.7, 3072 (8 x 2048 x 3072)
+    // 48 / 45 / 40 (a copy of its bytes: 39). An update in place needs the
+    // single run of 32.
+    const int tpb = p.D / 8 >= 256 ? 256 : (p.D / 8 + 63) / 64 * 64;
+    const long long waves = (long long)((p.D / 8 + 63) / 64) * p.B * ((p.T + CONV_RUN - 1) / CONV_RUN);
+    const int cus = device_cu_count();
+    p.run = (p.cache && p.cache_out == p.cache) || waves >= 5ll * cus || p.T > 8 * 65535 ? CONV_RUN
+            : waves >= 2ll * cus                                                         ? 16
+                                                                                         : 8;
+    const dim3 grid((p.D / 8 + tpb - 1) / tpb, p.B, (p.T + p.run - 1) / p.run), block(tpb);
     switch (p.W) {
-        case 2: hipLaunchKernelGGL((short_conv_kernel<E, 2>), grid, block, 0, stream, p); break;
-        case 3: hipLaunchKernelGGL((short_conv_kernel<E, 3>), grid, block, 0, stream, p); break;
-        case 4: hipLaunchKernelGGL((short_conv_kernel<E, 4>), grid, block, 0, stream, p); break;
+        case 2: hipLaunchKernelGGL((short_conv_kernel<E, 2, MASK>), grid, block, 0, stream, p); break;
+        case 3: hipLaunchKernelGGL((short_conv_kernel<E, 3, MASK>), grid, block, 0, stream, p); break;
+        case 4: hipLaunchKernelGGL((short_conv_kernel<E, 4, MASK>), grid, block, 0, stream, p); break;
         default: return -1;
     }
     return 0;
@@ -1267,10 +1333,20 @@ int launch_short_conv_as(const ConvParamsT<E>& p, hipStream_t stream) {
 
 }  // namespace
 
-int launch_short_conv(const ConvParams& p, hipStream_t stream) { return launch_short_conv_as(p, stream); }
+int launch_short_conv(const ConvParams& p, hipStream_t stream) {
+    return p.mask ? launch_short_conv_as<__bf16, true>(p, stream) : launch_short_conv_as<__bf16, false>(p, stream);
+}
 
 // fp32 rows (training in fp32): the same kernel.
-int launch_short_conv(const ConvParamsT<float>& p, hipStream_t stream) { return launch_short_conv_as(p, stream); }
+int launch_short_conv(const ConvParamsT<float>& p, hipStream_t stream) {
+    return p.mask ? launch_short_conv_as<float, true>(p, stream) : launch_short_conv_as<float, false>(p, stream);
+}
+
+int launch_mask_rows(const long long* mask, int B, int T, float* values, unsigned char* valid, int* lengths,
+                     hipStream_t stream) {
+    hipLaunchKernelGGL(mask_rows_kernel, dim3(B), dim3(256), 0, stream, mask, T, values, valid, lengths);
+    return 0;
+}
 
 int launch_silu_mul(const bf16_t* gu, bf16_t* out, int rows, int F, hipStream_t stream) {
     const size_t n8 = (size_t)rows * F / 8;

@@ -14,7 +14,7 @@ import torch
 import torch.nn.functional as F
 
 LIB_PATH = Path(os.environ.get("CYFA_LIB", Path(__file__).with_name("libcyfa_hip.so")))
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 CYFA_OK = 0
 CYFA_ERR_VALUE = -1
@@ -136,6 +136,7 @@ class CyfaConvArgs(ctypes.Structure):
         ("weight", _c_void_p), ("bias", _c_void_p),
         ("out", _c_void_p * 3), ("split", _c_int),
         ("cache_out", _c_void_p), ("cache_out_row", ctypes.c_longlong), ("cache_out_batch", ctypes.c_longlong),
+        ("mask", _c_void_p), ("lengths", _c_void_p),
     ]
 
 
@@ -156,6 +157,7 @@ class CyfaGatePathArgs(ctypes.Structure):
         ("x", _c_void_p), ("ldx", ctypes.c_longlong), ("w1", _c_void_p), ("abd_bias", _c_void_p),
         ("w2", _c_void_p), ("b2", _c_void_p), ("dt_bias", _c_void_p), ("A_log", _c_void_p),
         ("gate", _c_void_p), ("ldg", ctypes.c_longlong), ("g", _c_void_p), ("beta", _c_void_p), ("delta", _c_void_p),
+        ("valid", _c_void_p),
     ]
 
 
@@ -173,6 +175,7 @@ SIGNATURES = {
     "cyfa_readout_table": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_int, _c_void_p]),
     "cyfa_rms_norm": (_c_int, [ctypes.POINTER(CyfaNormArgs), _c_void_p]),
     "cyfa_short_conv": (_c_int, [ctypes.POINTER(CyfaConvArgs), _c_void_p]),
+    "cyfa_mask_rows": (_c_int, [_c_void_p, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p]),
     "cyfa_short_conv_f32": (_c_int, [ctypes.POINTER(CyfaConvArgs), _c_void_p]),
     "cyfa_short_conv_grad_workspace_bytes": (_c_size_t, [_c_int] * 4),
     "cyfa_short_conv_grad": (_c_int, [ctypes.POINTER(CyfaConvGradArgs), _c_int, _c_void_p]),
@@ -641,14 +644,30 @@ def linear_swiglu(x, w_interleaved):
     return y.view(*x.shape[:-1], N // 2)
 
 
-def short_conv(x, weight, bias=None, cache=None, split=None, cache_out=None):
+def mask_rows(attention_mask):
+    """(values fp32 [B, T], rounded to bf16, valid uint8 [B, T], lengths int32 [B]) of an integer
+    attention mask [B, T], as short_conv and gate_path read them."""
+    dev = require_device(attention_mask)
+    B, T = attention_mask.shape
+    mask = attention_mask.to(torch.int64).contiguous()
+    values = torch.empty(B, T, dtype=torch.float32, device=dev)
+    valid = torch.empty(B, T, dtype=torch.uint8, device=dev)
+    lengths = torch.empty(B, dtype=torch.int32, device=dev)
+    _check(load_library().cyfa_mask_rows(ptr(mask), B, T, ptr(values), ptr(valid), ptr(lengths), stream_handle(dev)),
+           "cyfa_mask_rows")
+    return values, valid, lengths
+
+
+def short_conv(x, weight, bias=None, cache=None, split=None, cache_out=None, mask=None, lengths=None):
     """Causal depthwise convolution over time of x [B, T, D] (rows may be strided).
 
     x, weight [D, W], bias and cache (an optional [B, W-1, D] view) all bf16, or
     all fp32. The D channels are written to D // split contiguous [B, T, split] tensors (split defaults to D).
     ``cache_out`` [B, W-1, D] (channel stride 1) receives the last W-1 rows of
-    cat(cache, x); it may be ``cache`` itself when T <= 32."""
-    dev = require_device(x, weight, bias, cache)
+    cat(cache, x); it may be ``cache`` itself when T <= 32. ``mask`` fp32
+    [B, T] multiplies x's rows, and cache_out then receives the W-1 rows before
+    ``lengths`` (int32 [B]; mask_rows)."""
+    dev = require_device(x, weight, bias, cache, mask, lengths)
     B, T, D = x.shape
     W = weight.shape[-1]
     split = D if split is None else split
@@ -663,7 +682,8 @@ def short_conv(x, weight, bias=None, cache=None, split=None, cache_out=None):
                         cache_batch=0 if cache is None else cache.stride(0),
                         weight=ptr(w), bias=ptr(None if bias is None else bias.contiguous()), split=split,
                         cache_out=ptr(cache_out), cache_out_row=0 if cache_out is None else cache_out.stride(1),
-                        cache_out_batch=0 if cache_out is None else cache_out.stride(0))
+                        cache_out_batch=0 if cache_out is None else cache_out.stride(0), mask=ptr(mask),
+                        lengths=ptr(lengths))
     for i, o in enumerate(outs):
         args.out[i] = o.data_ptr()
     lib = load_library()
@@ -720,15 +740,16 @@ def gate_path_ok(x, w1, w2, b2, H):
             and w2.shape[1] == GATE_PATH_G0 and w2.shape[0] % 256 == 0 and w2.shape[0] <= GATE_PATH_MAX)
 
 
-def gate_path(x, w1, abd_bias, w2, b2, dt_bias, A_log, H):
+def gate_path(x, w1, abd_bias, w2, b2, dt_bias, A_log, H, valid=None):
     """The prefill gate path in one cyfa_gate_path launch: g0 = bf16(x W_g0^T),
     abd = bf16(x [W_a|W_b|W_d]^T + abd_bias), the gate activations of abd and
     gate = bf16(g0 W_g1^T + b2). w1 = [W_g0; W_a; W_b; W_d] [256 + 3H, K].
-    Returns (gate [..., Dv] bf16, g, beta, delta [..., H] fp32)."""
+    Returns (gate [..., Dv] bf16, g, beta, delta [..., H] fp32); g, beta and
+    delta are zero where ``valid`` (uint8 [...], contiguous) is."""
     K = x.shape[-1]
     Dv = w2.shape[0]
     rows = x.numel() // K
-    dev = require_device(x, w1, abd_bias, w2, b2, dt_bias, A_log)
+    dev = require_device(x, w1, abd_bias, w2, b2, dt_bias, A_log, valid)
     x2 = x.reshape(rows, K)
     if x2.stride(-1) != 1 or x2.stride(0) % 8 or x2.data_ptr() % 16:
         x2 = x2.contiguous()
@@ -742,7 +763,7 @@ def gate_path(x, w1, abd_bias, w2, b2, dt_bias, A_log, H):
     args = CyfaGatePathArgs(M=rows, K=K, H=H, Dv=Dv, x=x2.data_ptr(), ldx=x2.stride(0), w1=w1c.data_ptr(),
                             abd_bias=ab.data_ptr(), w2=w2c.data_ptr(), b2=ptr(b2c), dt_bias=db.data_ptr(),
                             A_log=al.data_ptr(), gate=gate.data_ptr(), ldg=Dv, g=g.data_ptr(), beta=beta.data_ptr(),
-                            delta=delta.data_ptr())
+                            delta=delta.data_ptr(), valid=ptr(valid))
     _check(load_library().cyfa_gate_path(ctypes.byref(args), stream_handle(dev)), "cyfa_gate_path")
     lead = tuple(x.shape[:-1])
     return gate.view(lead + (Dv,)), g.view(lead + (H,)), beta.view(lead + (H,)), delta.view(lead + (H,))

@@ -314,9 +314,21 @@ class CyclicFlowAttention(nn.Module):
         return (inference_fast_path(x) and attention_mask is None and self.use_short_conv
                 and 2 <= self.q_conv1d.width <= 4 and self.q_conv1d.bias is None)
 
+    def _fused_mask_ok(self, x, attention_mask):
+        """Whether a masked call takes the fused path: a prefill of more rows
+        than a decode step's at the tuned op's shape, with an integer mask
+        [B, T]. (Other masks, which may broadcast or hold fractions, and other
+        shapes keep the general path.)"""
+        return (attention_mask is not None and self._fused_ok(x, None) and x.dim() == 3 and x.shape[1] > 1
+                and self.head_k_dim == 256 and self.head_v_dim == 256 and self.num_slots == 128
+                and self.chunk_size == 64
+                and x.shape[0] * x.shape[1] > _native.LINEAR_ROWS_MAX
+                and tuple(attention_mask.shape) == tuple(x.shape[:2]) and attention_mask.device == x.device
+                and attention_mask.dtype in (torch.int64, torch.int32, torch.bool, torch.uint8))
+
     def forward(self, x, cache=None, use_cache=False, attention_mask=None):
-        if self._fused_ok(x, attention_mask):
-            return self._forward_fused(x, cache, use_cache)
+        if self._fused_ok(x, attention_mask) or self._fused_mask_ok(x, attention_mask):
+            return self._forward_fused(x, cache, use_cache, attention_mask=attention_mask)
         B, T, _ = x.shape
         H = self.num_heads
         q, k, v = self.q_proj(x), self.k_proj(x), self.v_proj(x)
@@ -408,11 +420,16 @@ class CyclicFlowAttention(nn.Module):
             w = self._in_weight_folded.get(w, norm.weight, build=_native.fold_norm_weight)
         return ((w, _native.linear_rows_span(rows, w.shape[0], w.shape[1], norm=2 if folded else 1), True),)
 
-    def _forward_fused(self, x, cache, use_cache, prenorm=None, prefetch=()):
+    def _forward_fused(self, x, cache, use_cache, prenorm=None, prefetch=(), attention_mask=None):
         """bf16 inference: the same math as forward with fused launches. With
         ``prenorm`` (the block's norm), x is the block input and the result is
-        (x + o, new_cache), as forward_block."""
+        (x + o, new_cache), as forward_block. ``attention_mask``: right-padded
+        prefill (_fused_mask_ok); the convolution multiplies its input rows by
+        the mask and the gate path zeroes the gates of the padding."""
         B, T, _ = x.shape
+        mask = valid = lengths = None
+        if attention_mask is not None:
+            mask, valid, lengths = _native.mask_rows(attention_mask)
         block_in = None
         if prenorm is not None:
             block_in = x
@@ -525,9 +542,10 @@ class CyclicFlowAttention(nn.Module):
             return o, new_cache
         if Dk == Dv:
             q, k, v = _native.short_conv(qkv, wconv.reshape(-1, W).to(x.dtype), None, cat_cache, split=Dk,
-                                         cache_out=tail)
+                                         cache_out=tail, mask=mask, lengths=lengths)
         else:
-            (y,) = _native.short_conv(qkv, wconv.reshape(-1, W).to(x.dtype), None, cat_cache, cache_out=tail)
+            (y,) = _native.short_conv(qkv, wconv.reshape(-1, W).to(x.dtype), None, cat_cache, cache_out=tail,
+                                      mask=mask, lengths=lengths)
             q, k, v = y[..., :Dk].contiguous(), y[..., Dk:2 * Dk].contiguous(), y[..., 2 * Dk:].contiguous()
         cq, ck, cv = tail[..., :Dk], tail[..., Dk:2 * Dk], tail[..., 2 * Dk:]
         gate = None
@@ -536,13 +554,16 @@ class CyclicFlowAttention(nn.Module):
             if _native.gate_path_ok(x, w1, g1.weight, g1.bias, H):
                 # g_proj[0], a|b|d, the gates and g_proj[1] in one launch
                 gate, g, beta, delta = _native.gate_path(x, w1, abd_bias, g1.weight, g1.bias, self.dt_bias,
-                                                         self.A_log, H)
+                                                         self.A_log, H, valid)
                 gate = gate.view(B, T, H, self.head_v_dim)
         if gate is None:
             if abd is None:
                 abd = _native.linear(x, self._abd_weight.get(self.a_proj.weight, self.b_proj.weight,
                                                               self.d_proj.weight), abd_bias)
             g, beta, delta = _native.gates(abd, self.dt_bias, self.A_log)
+            if valid is not None:
+                keep = valid.unsqueeze(-1).bool()
+                g, beta, delta = (torch.where(keep, t, torch.zeros_like(t)) for t in (g, beta, delta))
         kwargs = dict(
             q=q.view(B, T, H, self.head_k_dim),
             k=k.view(B, T, H, self.head_k_dim),

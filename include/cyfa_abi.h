@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define CYFA_ABI_VERSION 12
+#define CYFA_ABI_VERSION 13
 
 enum {
     CYFA_OK = 0,
@@ -453,6 +453,7 @@ typedef struct CyfaGatePathArgs {
     void *gate;                   /* bf16 [M, Dv], rows ldg elements apart, 16-byte aligned */
     long long ldg;                /* a multiple of 8, >= Dv */
     float *g, *beta, *delta;      /* f32 [M, H] */
+    const void *valid;            /* nullable u8 [M]: g, beta and delta of a row are zero where it is zero */
 } CyfaGatePathArgs;
 
 int cyfa_gate_path(const CyfaGatePathArgs *args, void *hip_stream);
@@ -477,7 +478,14 @@ typedef struct CyfaConvArgs {
     int split;
     void *cache_out;              /* nullable bf16, same addressing as cache with cache_out_row / _batch */
     long long cache_out_row, cache_out_batch;
+    const float *mask;            /* nullable f32 [B, T]: X[b, t] is x mask, rounded to x's dtype */
+    const int *lengths;           /* i32 [B], required with mask: cache_out receives X[b, n-(W-1) .. n-1],
+                                   * n = lengths[b] within [0, T] (layers/cyfa.py:175-182) */
 } CyfaConvArgs;
+
+/* An attention mask [B, T] in the forms the prefill kernels read: values
+ * f32 [B, T] (rounded to bf16), valid u8 [B, T] (nonzero or not), lengths i32 [B] (row sums). */
+int cyfa_mask_rows(const long long *mask, int B, int T, float *values, void *valid, int *lengths, void *hip_stream);
 
 /* Replaces ShortConvolution.execute / _inference (layers/cyfa.py:138-233); the
  * new cache (the last W-1 inputs) stays a view of the input in the caller. */

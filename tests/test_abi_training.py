@@ -1,0 +1,42 @@
+"""Host-side checks of the training and masked-prefill entry points: struct
+layouts against the header, and argument errors raised before any launch."""
+
+import ctypes
+
+import pytest
+
+from cyclic_flow_attention import _native
+from test_abi import _c_layout
+
+
+@pytest.mark.parametrize("name", ["CyfaConvGradArgs", "CyfaGatePathArgs"])
+def test_struct_layout_matches_header(tmp_path, name):
+    cls = getattr(_native, name)
+    fields = [f for f, _ in cls._fields_]
+    got = [ctypes.sizeof(cls)] + [getattr(cls, f).offset for f in fields]
+    assert got == _c_layout(tmp_path, name, fields)
+
+
+def test_short_conv_grad_validates_before_launch():
+    lib = _native.load_library()
+    n = lib.cyfa_short_conv_grad_workspace_bytes(2, 100, 64, 4)
+    assert n >= 2 * 2 * 5 * 64 * 4 and lib.cyfa_short_conv_grad_workspace_bytes(2, 100, 64, 5) == 0
+    good = dict(B=2, T=100, D=64, W=4, x=0x10000, x_row=64, weight=0x20000, dy=0x30000, workspace=0x40000,
+                workspace_bytes=n)
+
+    def call(dtype=0, **change):
+        a = _native.CyfaConvGradArgs(**{**good, **change})
+        return lib.cyfa_short_conv_grad(ctypes.byref(a), dtype, None)
+
+    assert call(W=5) == call(D=60) == _native.CYFA_ERR_UNSUPPORTED
+    assert call(dtype=7) == call(x=None) == call(T=0) == _native.CYFA_ERR_VALUE
+    assert call(x=0x10004) == call(x_row=60) == call(dx=0x50002) == _native.CYFA_ERR_ALIGN
+    assert call(workspace_bytes=n - 1) == _native.CYFA_ERR_WORKSPACE
+
+
+def test_mask_entry_points_validate_before_launch():
+    lib = _native.load_library()
+    assert lib.cyfa_mask_rows(None, 1, 4, None, None, None, None) == _native.CYFA_ERR_VALUE
+    c = _native.CyfaConvArgs(B=1, T=4, D=64, W=4, split=64, x=0x10000, x_row=64, weight=0x20000, mask=0x30000)
+    c.out[0] = 0x40000
+    assert lib.cyfa_short_conv(ctypes.byref(c), None) == _native.CYFA_ERR_VALUE  # mask without lengths
