@@ -644,6 +644,46 @@ int cyfa_short_conv_grad(const CyfaConvGradArgs* a, int dtype, void* hip_stream)
     return check_launch(what);
 }
 
+size_t cyfa_norm_grad_workspace_bytes(long long rows, int D) {
+    return rows <= 0 || D <= 0 ? 0 : cyfa::norm_grad_workspace_bytes(rows, D);
+}
+
+int cyfa_norm_train(const CyfaNormTrainArgs* a, int dtype, int grad, void* hip_stream) {
+    const char* what = "cyfa_norm_train";
+    if (!a) return fail(CYFA_ERR_VALUE, "%s: null args", what);
+    if (dtype != CYFA_DTYPE_BF16 && dtype != CYFA_DTYPE_F32) return fail(CYFA_ERR_VALUE, "%s: dtype %d", what, dtype);
+    if (a->rows < 0 || a->D <= 0) return fail(CYFA_ERR_VALUE, "%s: rows=%lld D=%d", what, a->rows, a->D);
+    if (a->D % 4 || a->D > cyfa::NORM_TRAIN_MAX_D)
+        return fail(CYFA_ERR_UNSUPPORTED, "%s: D=%d must be a multiple of 4 up to %d", what, a->D, cyfa::NORM_TRAIN_MAX_D);
+    if (!a->x || !a->weight || (grad ? !a->dy || !a->workspace : !a->out))
+        return fail(CYFA_ERR_VALUE, "%s: null required pointer", what);
+    if (grad && a->dgate && !a->gate) return fail(CYFA_ERR_VALUE, "%s: dgate without a gate", what);
+    const void* rows16[] = {a->x, a->gate, a->weight, a->out, a->dy, a->dx, a->dgate, a->workspace};
+    for (const void* ptr : rows16)
+        if (!aligned(ptr, 16)) return fail(CYFA_ERR_ALIGN, "%s: 16-byte alignment needed", what);
+    if (a->rows == 0 && !grad) return CYFA_OK;
+    if (grad && a->workspace_bytes < cyfa::norm_grad_workspace_bytes(a->rows, a->D))
+        return fail(CYFA_ERR_WORKSPACE, "%s: workspace of %zu bytes", what, a->workspace_bytes);
+    cyfa::NormTrainParams p;
+    p.rows = a->rows;
+    p.D = a->D;
+    p.x = a->x;
+    p.gate = a->gate;
+    p.weight = a->weight;
+    p.eps = a->eps;
+    p.prescale = a->prescale;
+    p.out = a->out;
+    p.dy = a->dy;
+    p.dx = a->dx;
+    p.dgate = a->dgate;
+    p.dweight = a->dweight;
+    p.part = (float*)a->workspace;
+    p.rows_wg = 0;
+    if (cyfa::launch_norm_train(p, dtype == CYFA_DTYPE_BF16, grad != 0, (hipStream_t)hip_stream) != 0)
+        return fail(CYFA_ERR_UNSUPPORTED, "%s: rows=%lld D=%d", what, a->rows, a->D);
+    return check_launch(what);
+}
+
 int cyfa_mask_rows(const long long* mask, int B, int T, float* values, void* valid, int* lengths, void* hip_stream) {
     const char* what = "cyfa_mask_rows";
     if (B < 0 || T < 0) return fail(CYFA_ERR_VALUE, "%s: B=%d T=%d", what, B, T);

@@ -174,6 +174,23 @@ struct ConvGradParams {
     float* part;                 // conv_grad_workspace_bytes
 };
 
+// The gated RMS norm of a training step and its adjoint (cyfa_train.hip): x,
+// gate, out, dy, dx and dgate [rows, D], bf16 or fp32.
+struct NormTrainParams {
+    long long rows;
+    int D;
+    const void *x, *gate;        // gate nullable
+    const float* weight;         // [D]
+    float eps, prescale;
+    void* out;                   // the forward's result
+    const void* dy;              // the adjoint's input
+    void *dx, *dgate;            // nullable
+    float* dweight;              // nullable [D]
+    float* part;                 // norm_grad_workspace_bytes
+    int rows_wg;                 // rows of an adjoint workgroup (set by the launcher)
+};
+constexpr int NORM_TRAIN_MAX_D = 2048;
+
 struct WorkspaceLayout {
     size_t lam, gam, seg, seg_exp, seg_decay, omega, tab_exp, tab16, total;
 };
@@ -484,6 +501,8 @@ int launch_mask_rows(const long long* mask, int B, int T, float* values, unsigne
                      hipStream_t stream);
 size_t conv_grad_workspace_bytes(int B, int T, int D, int W);
 int launch_conv_grad(const ConvGradParams& p, bool bf16, hipStream_t stream);
+size_t norm_grad_workspace_bytes(long long rows, int D);
+int launch_norm_train(const NormTrainParams& p, bool bf16, bool grad, hipStream_t stream);
 int launch_silu_mul(const __bf16* gu, __bf16* out, int rows, int F, hipStream_t stream);
 int launch_argmax_rows(const __bf16* x, long long ldx, int rows, int n, long long* out, hipStream_t stream);
 int launch_gate_path(const GatePathParams& p, hipStream_t stream);

@@ -1,6 +1,7 @@
-// cyfa_train.hip -- the layer-side adjoints of a training step for gfx950: the
-// gradients of the causal depthwise short convolution (ShortConvolution,
-// layers/cyfa.py:138-233). Streaming kernels: each input is read once, sums
+// cyfa_train.hip -- the layer-side operations of a training step for gfx950:
+// the adjoints of the causal depthwise short convolution (ShortConvolution,
+// layers/cyfa.py:138-233) and of the gated RMS norm (RMSNorm,
+// layers/cyfa.py:62-135), with the norm's forward. Streaming kernels: each input is read once, sums
 // over tokens accumulate in fp32 and partial sums are added in a fixed order,
 // so that two backward passes give the same bits.
 #include "cyfa_device.h"
@@ -129,15 +130,13 @@ __global__ __launch_bounds__(256) void conv_grad_kernel(ConvGradParams p) {
     }
 }
 
-// Adds the nparts partials [W + 1][D] of conv_grad_kernel: 32 columns per
-// workgroup, eight threads per column each adding every eighth partial in
-// order (eight loads in flight), then the eight in order. Column w D + c goes
-// to dweight[c][w], column W D + c to dbias[c].
-template <class E>
-__global__ __launch_bounds__(256) void conv_grad_reduce_kernel(const float* part, int nparts, int D, int W, E* dweight,
-                                                               E* dbias) {
+// The sum of column e = blockIdx.x * 32 + threadIdx.x % 32 over the rows of
+// part [nparts][n], for workgroups of 256 threads: eight threads per column
+// each add every eighth row in order (eight loads in flight), then the eight
+// in order. Valid in the first 32 threads.
+__device__ __forceinline__ float column_sum(const float* part, int nparts, int n) {
     __shared__ float red[8][32];
-    const int n = (W + 1) * D, col = threadIdx.x & 31, g = threadIdx.x >> 5, e = blockIdx.x * 32 + col;
+    const int col = threadIdx.x & 31, g = threadIdx.x >> 5, e = blockIdx.x * 32 + col;
     float s = 0.f;
     if (e < n) {
         int i = g;
@@ -152,9 +151,21 @@ __global__ __launch_bounds__(256) void conv_grad_reduce_kernel(const float* part
     }
     red[g][col] = s;
     __syncthreads();
-    if (g != 0 || e >= n) return;
+    if (g == 0) {
 #pragma unroll
-    for (int u = 1; u < 8; u++) s += red[u][col];
+        for (int u = 1; u < 8; u++) s += red[u][col];
+    }
+    return s;
+}
+
+// Adds the nparts partials [W + 1][D] of conv_grad_kernel: column w D + c goes
+// to dweight[c][w], column W D + c to dbias[c].
+template <class E>
+__global__ __launch_bounds__(256) void conv_grad_reduce_kernel(const float* part, int nparts, int D, int W, E* dweight,
+                                                               E* dbias) {
+    const int n = (W + 1) * D, e = blockIdx.x * 32 + (int)threadIdx.x;
+    const float s = column_sum(part, nparts, n);
+    if (threadIdx.x >= 32 || e >= n) return;
     const int w = e / D, c = e % D;
     if (w < W) {
         if (dweight) dweight[(size_t)c * W + w] = (E)s;
@@ -178,7 +189,177 @@ int launch_conv_grad_as(const ConvGradParams& p, hipStream_t stream) {
     return 0;
 }
 
+// out[e] = the column sums of part [nparts][n].
+__global__ __launch_bounds__(256) void column_sum_kernel(const float* part, int nparts, int n, float* out) {
+    const float s = column_sum(part, nparts, n);
+    const int e = blockIdx.x * 32 + (int)threadIdx.x;
+    if (threadIdx.x < 32 && e < n) out[e] = s;
+}
+
+__device__ __forceinline__ float exact_sigmoid(float x) { return 1.f / (1.f + expf(-x)); }
+
+// The gated RMS norm of rows x [rows, D] and its adjoint, one wave per row,
+// lane l holding columns 4 l + 256 j (j < J, columns past D read as zero):
+//   xs  = x prescale (rounded to E; x itself for a prescale of 1), r = (mean xs^2 + eps)^-1/2
+//   out = xs r weight [sigmoid(gate)]
+// and, with u = dy [sigmoid(gate)],
+//   dx      = prescale (r weight u - xs r^3 / D sum_i xs_i weight_i u_i)   (the cotangent of xs rounded to E first)
+//   dgate   = dy xs r weight sigmoid(gate) (1 - sigmoid(gate))
+//   dweight = sum over the rows of u xs r  (a partial per workgroup of p.rows_wg rows, column_sum_kernel adds them)
+// The forward reads x and gate and writes out, the adjoint reads three rows and
+// writes two; as the torch chain of some 25 fp32 elementwise and reduction
+// launches, a gated norm of 12000 x 256 bf16 rows cost about 200 us of a
+// training step. On MI355X the forward takes 6.8 us, the adjoint with its
+// column sum 18 us; at 65536 rows 26 and 52 us (a copy of the bytes: 19, 32).
+// Rows of an adjoint workgroup, a quarter of them per wave: few while that
+// leaves compute units idle, many where the partials would add up.
+int norm_grad_rows(long long rows) { return rows >= 32768 ? 32 : rows >= 8192 ? 16 : 8; }
+
+// xs, sigmoid(gate) (ones without a gate) and r of a row from its loaded values.
+template <class E, int J>
+__device__ __forceinline__ void norm_row(const NormTrainParams& p, f32x4 (&xs)[J], f32x4 (&sg)[J], float& rs) {
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < J; j++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if (p.prescale != 1.f) xs[j][i] = (float)(E)(xs[j][i] * p.prescale);
+            ss = fmaf(xs[j][i], xs[j][i], ss);
+            sg[j][i] = p.gate ? exact_sigmoid(sg[j][i]) : 1.f;
+        }
+    rs = rsqrtf(wave_sum(ss) / (float)p.D + p.eps);
+}
+
+// Row `row`'s columns of this lane, zero past D and past the last row: read
+// from the last row and columns there, and dropped (no branch among the loads,
+// at which the compiler would wait for those in flight).
+template <class E, int J>
+__device__ __forceinline__ void norm_load(const void* x, long long row, const NormTrainParams& p, int lane, f32x4 (&v)[J]) {
+    const E* src = static_cast<const E*>(x) + (size_t)(row < p.rows ? row : p.rows - 1) * p.D;
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        const int d = 4 * lane + 256 * j;
+        v[j] = load4(src + (d < p.D ? d : p.D - 4));
+        if (row >= p.rows || d >= p.D) v[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+}
+
+template <int J>
+__device__ __forceinline__ void norm_weight(const NormTrainParams& p, int lane, f32x4 (&w)[J]) {
+#pragma unroll
+    for (int j = 0; j < J; j++)
+        w[j] = 4 * lane + 256 * j < p.D ? load4(p.weight + 4 * lane + 256 * j) : f32x4{0.f, 0.f, 0.f, 0.f};
+}
+
+template <class E, int J>
+__global__ __launch_bounds__(256) void norm_train_kernel(NormTrainParams p) {
+    const int lane = threadIdx.x & 63;
+    const long long row = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= p.rows) return;
+    f32x4 w[J], xs[J], sg[J];
+    norm_load<E, J>(p.x, row, p, lane, xs);
+    norm_load<E, J>(p.gate ? p.gate : p.x, row, p, lane, sg);
+    norm_weight<J>(p, lane, w);
+    float rs;
+    norm_row<E, J>(p, xs, sg, rs);
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        const int d = 4 * lane + 256 * j;
+        if (d < p.D) store4(static_cast<E*>(p.out) + (size_t)row * p.D + d, xs[j] * rs * w[j] * sg[j]);
+    }
+}
+
+template <class E, int J>
+__global__ __launch_bounds__(256) void norm_grad_kernel(NormTrainParams p) {
+    __shared__ __align__(16) float red[4][J * 256];
+    constexpr int RB = J <= 4 ? 2 : 1;  // rows whose loads are in flight together
+    const int rpw = p.rows_wg / 4;      // rows of a wave, 2, 4 or 8
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    f32x4 w[J], dw[J];
+    norm_weight<J>(p, lane, w);
+#pragma unroll
+    for (int j = 0; j < J; j++) dw[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < rpw; k += RB) {
+        const long long row0 = (long long)blockIdx.x * p.rows_wg + rpw * wv + k;
+        if (row0 >= p.rows) break;
+        f32x4 xs[RB][J], sg[RB][J], dy[RB][J];
+#pragma unroll
+        for (int r = 0; r < RB; r++) {
+            norm_load<E, J>(p.x, row0 + r, p, lane, xs[r]);
+            norm_load<E, J>(p.gate ? p.gate : p.x, row0 + r, p, lane, sg[r]);
+            norm_load<E, J>(p.dy, row0 + r, p, lane, dy[r]);
+        }
+#pragma unroll
+        for (int r = 0; r < RB; r++) {
+            float rs, sum = 0.f;
+            norm_row<E, J>(p, xs[r], sg[r], rs);
+#pragma unroll
+            for (int j = 0; j < J; j++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) sum = fmaf(xs[r][j][i] * w[j][i], dy[r][j][i] * sg[r][j][i], sum);
+            const float cr = rs * rs * rs * wave_sum(sum) / (float)p.D;
+            const size_t base = (size_t)(row0 + r) * p.D;
+#pragma unroll
+            for (int j = 0; j < J; j++) {
+                const int d = 4 * lane + 256 * j;
+                const f32x4 u = dy[r][j] * sg[r][j];
+                dw[j] += u * xs[r][j] * rs;
+                if (row0 + r < p.rows && d < p.D) {
+                    if (p.dx) {
+                        f32x4 dxs = w[j] * u * rs - xs[r][j] * cr;
+                        if (p.prescale != 1.f) {
+#pragma unroll
+                            for (int i = 0; i < 4; i++) dxs[i] = (float)(E)dxs[i] * p.prescale;
+                        }
+                        store4(static_cast<E*>(p.dx) + base + d, dxs);
+                    }
+                    if (p.dgate) store4(static_cast<E*>(p.dgate) + base + d, u * xs[r][j] * rs * w[j] * (1.f - sg[r][j]));
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < J; j++) *reinterpret_cast<f32x4*>(&red[wv][4 * lane + 256 * j]) = dw[j];
+    __syncthreads();
+    for (int d = threadIdx.x; d < p.D; d += 256)
+        p.part[(size_t)blockIdx.x * p.D + d] = (red[0][d] + red[1][d]) + (red[2][d] + red[3][d]);
+}
+
+template <class E, int J>
+int launch_norm_train_as(NormTrainParams p, bool grad, hipStream_t stream) {
+    const dim3 block(256);
+    if (!grad) {
+        hipLaunchKernelGGL((norm_train_kernel<E, J>), dim3((unsigned)((p.rows + 3) / 4)), block, 0, stream, p);
+        return 0;
+    }
+    p.rows_wg = norm_grad_rows(p.rows);
+    const unsigned blocks = (unsigned)((p.rows + p.rows_wg - 1) / p.rows_wg);
+    hipLaunchKernelGGL((norm_grad_kernel<E, J>), dim3(blocks), block, 0, stream, p);
+    if (p.dweight)
+        hipLaunchKernelGGL(column_sum_kernel, dim3((p.D + 31) / 32), block, 0, stream, p.part, (int)blocks, p.D, p.dweight);
+    return 0;
+}
+
+template <class E>
+int launch_norm_train_j(const NormTrainParams& p, bool grad, hipStream_t stream) {
+    const int j = (p.D + 255) / 256;
+    return j <= 1   ? launch_norm_train_as<E, 1>(p, grad, stream)
+           : j <= 2 ? launch_norm_train_as<E, 2>(p, grad, stream)
+           : j <= 4 ? launch_norm_train_as<E, 4>(p, grad, stream)
+                    : launch_norm_train_as<E, 8>(p, grad, stream);
+}
+
 }  // namespace
+
+size_t norm_grad_workspace_bytes(long long rows, int D) {
+    const int n = norm_grad_rows(rows);
+    return (size_t)((rows + n - 1) / n) * D * sizeof(float);
+}
+
+int launch_norm_train(const NormTrainParams& p, bool bf16, bool grad, hipStream_t stream) {
+    if (p.rows < 1 || p.rows > (1ll << 31) - 4 || p.D < 4 || p.D % 4 || p.D > NORM_TRAIN_MAX_D) return -1;
+    return bf16 ? launch_norm_train_j<bf16_t>(p, grad, stream) : launch_norm_train_j<float>(p, grad, stream);
+}
 
 size_t conv_grad_workspace_bytes(int B, int T, int D, int W) {
     return (size_t)B * ((T + CG_TOKENS - 1) / CG_TOKENS) * (W + 1) * D * sizeof(float);

@@ -14,7 +14,7 @@ import torch
 import torch.nn.functional as F
 
 LIB_PATH = Path(os.environ.get("CYFA_LIB", Path(__file__).with_name("libcyfa_hip.so")))
-ABI_VERSION = 13
+ABI_VERSION = 14
 
 CYFA_OK = 0
 CYFA_ERR_VALUE = -1
@@ -151,6 +151,15 @@ class CyfaConvGradArgs(ctypes.Structure):
     ]
 
 
+class CyfaNormTrainArgs(ctypes.Structure):
+    _fields_ = [
+        ("rows", ctypes.c_longlong), ("D", _c_int), ("x", _c_void_p), ("gate", _c_void_p), ("weight", _c_void_p),
+        ("eps", _c_float), ("prescale", _c_float), ("out", _c_void_p), ("dy", _c_void_p),
+        ("dx", _c_void_p), ("dgate", _c_void_p), ("dweight", _c_void_p),
+        ("workspace", _c_void_p), ("workspace_bytes", _c_size_t),
+    ]
+
+
 class CyfaGatePathArgs(ctypes.Structure):
     _fields_ = [
         ("M", _c_int), ("K", _c_int), ("H", _c_int), ("Dv", _c_int),
@@ -175,6 +184,8 @@ SIGNATURES = {
     "cyfa_readout_table": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_int, _c_void_p]),
     "cyfa_rms_norm": (_c_int, [ctypes.POINTER(CyfaNormArgs), _c_void_p]),
     "cyfa_short_conv": (_c_int, [ctypes.POINTER(CyfaConvArgs), _c_void_p]),
+    "cyfa_norm_grad_workspace_bytes": (_c_size_t, [ctypes.c_longlong, _c_int]),
+    "cyfa_norm_train": (_c_int, [ctypes.POINTER(CyfaNormTrainArgs), _c_int, _c_int, _c_void_p]),
     "cyfa_mask_rows": (_c_int, [_c_void_p, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p]),
     "cyfa_short_conv_f32": (_c_int, [ctypes.POINTER(CyfaConvArgs), _c_void_p]),
     "cyfa_short_conv_grad_workspace_bytes": (_c_size_t, [_c_int] * 4),
@@ -690,6 +701,41 @@ def short_conv(x, weight, bias=None, cache=None, split=None, cache_out=None, mas
     fn = lib.cyfa_short_conv_f32 if x.dtype == torch.float32 else lib.cyfa_short_conv
     _check(fn(ctypes.byref(args), stream_handle(dev)), "cyfa_short_conv")
     return outs
+
+
+NORM_TRAIN_MAX_D = 2048
+
+
+def norm_train(x, weight, gate, eps, prescale):
+    """norm(x prescale) [* sigmoid(gate)] over the last dim of contiguous,
+    16-byte aligned bf16 or fp32 rows (weight fp32 [D])."""
+    dev = require_device(x, weight, gate)
+    D = x.shape[-1]
+    out = torch.empty_like(x)
+    args = CyfaNormTrainArgs(rows=x.numel() // D, D=D, x=ptr(x), gate=ptr(gate), weight=ptr(weight), eps=float(eps),
+                             prescale=float(prescale), out=ptr(out))
+    _check(load_library().cyfa_norm_train(ctypes.byref(args), general_dtype(x), 0, stream_handle(dev)),
+           "cyfa_norm_train")
+    return out
+
+
+def norm_grad(x, weight, gate, eps, prescale, dy, needed):
+    """Gradients (dx, dweight fp32, dgate) of norm_train's result from its
+    cotangent dy, None where ``needed`` is false."""
+    dev = require_device(x, weight, gate, dy)
+    D = x.shape[-1]
+    rows = x.numel() // D
+    dx = torch.empty_like(x) if needed[0] else None
+    dw = torch.empty(D, dtype=torch.float32, device=dev) if needed[1] else None
+    dg = torch.empty_like(gate) if needed[2] else None
+    lib = load_library()
+    n = int(lib.cyfa_norm_grad_workspace_bytes(rows, D))
+    workspace = torch.empty(max(n, 1), dtype=torch.uint8, device=dev)  # alive until the launch
+    args = CyfaNormTrainArgs(rows=rows, D=D, x=ptr(x), gate=ptr(gate), weight=ptr(weight), eps=float(eps),
+                             prescale=float(prescale), dy=ptr(dy), dx=ptr(dx), dgate=ptr(dg), dweight=ptr(dw),
+                             workspace=ptr(workspace), workspace_bytes=n)
+    _check(lib.cyfa_norm_train(ctypes.byref(args), general_dtype(x), 1, stream_handle(dev)), "cyfa_norm_train")
+    return dx, dw, dg
 
 
 SHORT_CONV_MAX_GRID = 65535  # batch rows, and blocks of 32 tokens, of a short_conv launch

@@ -68,3 +68,29 @@ class ShortConv(torch.autograd.Function):
             return _recorded_grads(ctx.general, (x, weight, bias, cache), needed, dy) + (None,)
         grads = _native.short_conv_grad(x, weight, cache, rows_16(dy), needed)
         return (*grads, None)
+
+
+def rms_norm(x, weight, gate, eps, prescale, general):
+    """norm(x prescale) [* sigmoid(gate)] (layers/cyfa.py:62-135) with its HIP
+    adjoint: x and gate [..., D] bf16 or fp32 of one dtype, weight fp32 [D].
+    ``general``: the same of (x, weight, gate) in torch operations."""
+    return GatedNorm.apply(rows_16(x), rows_16(weight), None if gate is None else rows_16(gate), eps, prescale, general)
+
+
+class GatedNorm(torch.autograd.Function):
+    """rms_norm's function; every input contiguous."""
+
+    @staticmethod
+    def forward(ctx, x, weight, gate, eps, prescale, general):
+        ctx.save_for_backward(x, weight, gate)
+        ctx.args = (eps, prescale)
+        ctx.general = general
+        return _native.norm_train(x, weight, gate, eps, prescale)
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, weight, gate = ctx.saved_tensors
+        needed = ctx.needs_input_grad[:3]
+        if torch.is_grad_enabled():
+            return _recorded_grads(ctx.general, (x, weight, gate), needed, dy) + (None,) * 3
+        return (*_native.norm_grad(x, weight, gate, *ctx.args, rows_16(dy), needed), None, None, None)

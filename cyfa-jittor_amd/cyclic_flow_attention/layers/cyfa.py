@@ -27,7 +27,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from .. import _native
-from .autograd import hip_autograd_ok, short_conv
+from .autograd import hip_autograd_ok, rms_norm, short_conv
 from ..ops import chunk_cyfa, fused_recurrent_cyfa
 from ..ops.fused_recurrent import decode_layer_step
 from ..ops.utils import readout_table
@@ -99,13 +99,25 @@ class RMSNorm(nn.Module):
         total = None
         if residual is not None:
             x = total = x + residual
-        if prescale != 1.0:
-            x = x * prescale
-        xf = x.float()
-        y = xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + self.eps) * self.weight.float()
-        if gate is not None:
-            y = y * torch.sigmoid(gate.float())
-        y = y.to(x.dtype)
+
+        def general(x, weight, gate):
+            if prescale != 1.0:
+                x = x * prescale
+            xf = x.float()
+            y = xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + self.eps) * weight
+            if gate is not None:
+                y = y * torch.sigmoid(gate.float())
+            return y.to(x.dtype)
+
+        weight = self.weight.float()
+        if (x.dtype in (torch.bfloat16, torch.float32) and D % 4 == 0 and D <= _native.NORM_TRAIN_MAX_D
+                and x.numel() > 0 and tuple(weight.shape) == (D,)
+                and (gate is None or (gate.dtype == x.dtype and gate.shape == x.shape))
+                and hip_autograd_ok(x, weight, gate)):
+            # training: the norm and its adjoint as HIP kernels
+            y = rms_norm(x, weight, gate, self.eps, prescale, general)
+        else:
+            y = general(x, weight, gate)
         return y if residual is None else (total, y)
 
     execute = forward
@@ -378,7 +390,7 @@ class CyclicFlowAttention(nn.Module):
             o, state = chunk_cyfa(**kwargs, chunk_size=self.chunk_size,
                                   table=None if torch.is_grad_enabled() else self.readout_table())
         gate = self.g_proj(x).reshape(B, T, H, self.head_v_dim)
-        o = self.o_norm(o * (self.num_slots - 1), gate).reshape(B, T, self.value_dim)
+        o = self.o_norm(o, gate, prescale=float(self.num_slots - 1)).reshape(B, T, self.value_dim)
         o = self.o_proj(o)
         new_cache = {"recurrent_state": state, "conv_state": (cq, ck, cv)} if use_cache else None
         return o, new_cache

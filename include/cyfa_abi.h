@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define CYFA_ABI_VERSION 13
+#define CYFA_ABI_VERSION 14
 
 enum {
     CYFA_OK = 0,
@@ -515,6 +515,30 @@ typedef struct CyfaConvGradArgs {
 
 size_t cyfa_short_conv_grad_workspace_bytes(int B, int T, int D, int W);
 int cyfa_short_conv_grad(const CyfaConvGradArgs *args, int dtype, void *hip_stream);
+
+/* The gated RMS norm of a training step (RMSNorm.execute, layers/cyfa.py:62-135)
+ * on rows [rows, D], D a multiple of 4 up to 2048, x, gate, out, dy, dx and
+ * dgate of one dtype (CYFA_DTYPE_BF16 or CYFA_DTYPE_F32), every pointer 16-byte
+ * aligned:
+ *   xs = x prescale (rounded to the dtype), r = (mean xs^2 + eps)^-1/2
+ *   out = xs r weight [sigmoid(gate)]                           (grad 0)
+ * and its gradients from dy (grad 1), sums in fp32 and in a fixed order. */
+typedef struct CyfaNormTrainArgs {
+    long long rows;
+    int D;
+    const void *x, *gate;         /* gate nullable */
+    const float *weight;          /* f32 [D] */
+    float eps, prescale;
+    void *out;                    /* grad 0 */
+    const void *dy;               /* grad 1 */
+    void *dx, *dgate;             /* grad 1, nullable */
+    float *dweight;               /* grad 1, nullable f32 [D] */
+    void *workspace;              /* grad 1: cyfa_norm_grad_workspace_bytes(rows, D) bytes */
+    size_t workspace_bytes;
+} CyfaNormTrainArgs;
+
+size_t cyfa_norm_grad_workspace_bytes(long long rows, int D);
+int cyfa_norm_train(const CyfaNormTrainArgs *args, int dtype, int grad, void *hip_stream);
 
 /* out[r, c] = bf16(g sigmoid(g) u), g = gu[r, c], u = gu[r, F + c]; F a
  * multiple of 8. Replaces the activation of GatedMLP.execute

@@ -9,7 +9,7 @@ from cyclic_flow_attention import _native
 from test_abi import _c_layout
 
 
-@pytest.mark.parametrize("name", ["CyfaConvGradArgs", "CyfaGatePathArgs"])
+@pytest.mark.parametrize("name", ["CyfaConvGradArgs", "CyfaGatePathArgs", "CyfaNormTrainArgs"])
 def test_struct_layout_matches_header(tmp_path, name):
     cls = getattr(_native, name)
     fields = [f for f, _ in cls._fields_]
@@ -40,3 +40,19 @@ def test_mask_entry_points_validate_before_launch():
     c = _native.CyfaConvArgs(B=1, T=4, D=64, W=4, split=64, x=0x10000, x_row=64, weight=0x20000, mask=0x30000)
     c.out[0] = 0x40000
     assert lib.cyfa_short_conv(ctypes.byref(c), None) == _native.CYFA_ERR_VALUE  # mask without lengths
+
+
+def test_norm_train_validates_before_launch():
+    lib = _native.load_library()
+    n = lib.cyfa_norm_grad_workspace_bytes(100, 256)
+    assert n >= 256 * 4
+    good = dict(rows=100, D=256, x=0x10000, weight=0x20000, out=0x30000, dy=0x40000, workspace=0x50000, workspace_bytes=n)
+
+    def call(grad, dtype=0, **change):
+        a = _native.CyfaNormTrainArgs(**{**good, **change})
+        return lib.cyfa_norm_train(ctypes.byref(a), dtype, grad, None)
+
+    assert call(0, D=258) == call(1, D=4096) == _native.CYFA_ERR_UNSUPPORTED
+    assert call(0, out=None) == call(1, dy=None) == call(1, dgate=0x60000) == call(0, dtype=3) == _native.CYFA_ERR_VALUE
+    assert call(0, x=0x10008) == _native.CYFA_ERR_ALIGN
+    assert call(1, workspace_bytes=n - 4) == _native.CYFA_ERR_WORKSPACE

@@ -5,7 +5,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from cyclic_flow_attention.layers.cyfa import ShortConvolution
+from cyclic_flow_attention.layers.cyfa import RMSNorm, ShortConvolution
 
 pytestmark = pytest.mark.gpu
 
@@ -86,3 +86,49 @@ def test_short_conv_training_views_second_derivatives_and_transforms():
     assert _rel(out.detach(), torch.stack([_conv64(t.double().cpu(), w64, None, None) for t in xs])) < 1e-6
     _, tangent = torch.func.jvp(lambda t: conv(t)[0], (xs[0],), (xs[1],))
     assert _rel(tangent.detach(), _conv64(xs[1].double().cpu(), w64, None, None)) < 1e-6
+
+
+def _norm64(x, w, gate, prescale):
+    x = x * prescale
+    y = x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + 1e-6) * w
+    return y if gate is None else y * torch.sigmoid(gate)
+
+
+# one row, remainders of a workgroup's 4 and 32 rows, every number of column
+# blocks with remainders, with and without the gate and the prescale
+@pytest.mark.parametrize("rows,D,gate,prescale,dtype", [
+    (1, 4, False, 1.0, torch.float32), (33, 256, True, 127.0, torch.bfloat16), (70, 256, True, 127.0, torch.float32),
+    (37, 300, True, 1.0, torch.bfloat16), (64, 1024, False, 1.0, torch.bfloat16), (5, 1536, False, 1.0, torch.float32),
+    (2000, 256, True, 127.0, torch.bfloat16), (31, 2048, True, 3.0, torch.bfloat16)])
+def test_rms_norm_training_gradients(rows, D, gate, prescale, dtype):
+    """For bf16, x prescale is itself rounded (at most 2^-8 of each value), which
+    moves the result and the gradients by as much again: two roundings. The
+    weight's gradient is an fp32 sum of such terms."""
+    gen = torch.Generator().manual_seed(rows + D)
+    norm = RMSNorm(D, 1e-6)
+    with torch.no_grad():
+        norm.weight.copy_(1 + 0.2 * torch.randn(D, generator=gen))
+    x = torch.randn(rows, D, generator=gen).to(dtype)
+    g = torch.randn(rows, D, generator=gen).to(dtype) if gate else None
+    dy = torch.randn(rows, D, generator=gen).to(dtype)
+    ref = [None if t is None else t.detach().double().requires_grad_(True) for t in (x, norm.weight, g)]
+    ry = _norm64(*ref, prescale)
+    rg = torch.autograd.grad(ry, [t for t in ref if t is not None], dy.double())
+    norm = norm.to(DEV)
+    xg = x.to(DEV).requires_grad_(True)
+    gg = None if g is None else g.to(DEV).requires_grad_(True)
+    leaves = [xg, norm.weight] + ([gg] if gate else [])
+    y = norm(xg, gg, prescale=prescale)
+    assert y.grad_fn.name() == "GatedNormBackward"
+    got = torch.autograd.grad(y, leaves, dy.to(DEV), retain_graph=True)
+    again = torch.autograd.grad(y, leaves, dy.to(DEV))
+    bar = 2 * _bar(dtype)
+    assert _rel(y.detach(), ry.detach()) <= bar
+    for a, b, r, leaf in zip(got, again, rg, leaves):
+        assert a.dtype == leaf.dtype and a.shape == r.shape
+        assert torch.equal(a, b)
+        assert _rel(a, r) <= bar
+    # a recorded backward (second derivatives) gives the same first ones
+    rec = torch.autograd.grad(norm(xg, gg, prescale=prescale), leaves, dy.to(DEV), create_graph=True)
+    for a, r in zip(rec, rg):
+        assert a.requires_grad and _rel(a.detach(), r) <= 2 * bar
