@@ -571,8 +571,8 @@ int cyfa_norm_linear_rows(const CyfaLinearArgs* a, const CyfaRowNormArgs* n, voi
 int cyfa_rms_norm(const CyfaNormArgs* a, void* hip_stream) {
     if (!a) return fail(CYFA_ERR_VALUE, "cyfa_rms_norm: null args");
     if (a->rows < 0 || a->D <= 0) return fail(CYFA_ERR_VALUE, "cyfa_rms_norm: rows=%d D=%d", a->rows, a->D);
-    if (a->D % 256 != 0 || a->D > 2048 || (a->D / 256 & (a->D / 256 - 1)) != 0)
-        return fail(CYFA_ERR_UNSUPPORTED, "cyfa_rms_norm: D=%d must be 256, 512, 1024 or 2048", a->D);
+    if (a->D % 256 != 0 || a->D > 2048)
+        return fail(CYFA_ERR_UNSUPPORTED, "cyfa_rms_norm: D=%d must be a multiple of 256 up to 2048", a->D);
     if (!a->x || !a->weight || !a->out || (a->residual && !a->sum_out))
         return fail(CYFA_ERR_VALUE, "cyfa_rms_norm: null required pointer");
     if (!aligned(a->x, 8) || !aligned(a->out, 8) || !aligned(a->weight, 16) || (a->residual && !aligned(a->residual, 8)) ||
@@ -641,6 +641,66 @@ int cyfa_short_conv_grad(const CyfaConvGradArgs* a, int dtype, void* hip_stream)
     p.part = (float*)a->workspace;
     if (cyfa::launch_conv_grad(p, dtype == CYFA_DTYPE_BF16, (hipStream_t)hip_stream) != 0)
         return fail(CYFA_ERR_UNSUPPORTED, "%s: B=%d T=%d past the grid's limits", what, a->B, a->T);
+    return check_launch(what);
+}
+
+size_t cyfa_gates_grad_workspace_bytes(int rows, int K, int H) {
+    return rows <= 0 || K <= 0 || H <= 0 ? 0 : cyfa::gates_grad_workspace_bytes(rows, K, H);
+}
+
+int cyfa_gates_train(const CyfaGatesTrainArgs* a, int dtype, int grad, void* hip_stream) {
+    const char* what = "cyfa_gates_train";
+    if (!a) return fail(CYFA_ERR_VALUE, "%s: null args", what);
+    if (dtype != CYFA_DTYPE_BF16 && dtype != CYFA_DTYPE_F32) return fail(CYFA_ERR_VALUE, "%s: dtype %d", what, dtype);
+    if (a->rows <= 0 || a->K <= 0 || a->H <= 0)
+        return fail(CYFA_ERR_VALUE, "%s: rows=%d K=%d H=%d", what, a->rows, a->K, a->H);
+    if (a->K % 8 || a->H > cyfa::GATES_MAX_H)
+        return fail(CYFA_ERR_UNSUPPORTED, "%s: K=%d (a multiple of 8), H=%d (at most %d)", what, a->K, a->H, cyfa::GATES_MAX_H);
+    const void* both[] = {a->x, a->wa, a->wb, a->wd, a->dt_bias, a->A_log, a->abd};
+    const void* fwd[] = {a->bb, a->bd, a->g, a->beta, a->delta};
+    const void* bwd[] = {a->dg, a->dbeta, a->ddelta, a->dwa, a->dwb, a->dwd, a->dbb, a->dbd, a->ddt_bias, a->dA_log, a->workspace};
+    for (const void* ptr : both)
+        if (!ptr) return fail(CYFA_ERR_VALUE, "%s: null required pointer", what);
+    if (!grad)
+        for (const void* ptr : fwd)
+            if (!ptr) return fail(CYFA_ERR_VALUE, "%s: null required pointer", what);
+    if (grad)
+        for (const void* ptr : bwd)
+            if (!ptr) return fail(CYFA_ERR_VALUE, "%s: null required pointer", what);
+    const void* rows16[] = {a->x, a->wa, a->wb, a->wd, a->dx, a->workspace};
+    for (const void* ptr : rows16)
+        if (!aligned(ptr, 16)) return fail(CYFA_ERR_ALIGN, "%s: 16-byte alignment needed", what);
+    if (grad && a->workspace_bytes < cyfa::gates_grad_workspace_bytes(a->rows, a->K, a->H))
+        return fail(CYFA_ERR_WORKSPACE, "%s: workspace of %zu bytes", what, a->workspace_bytes);
+    cyfa::GatesTrainParams p{};
+    p.rows = a->rows;
+    p.K = a->K;
+    p.H = a->H;
+    p.x = a->x;
+    p.wa = a->wa;
+    p.wb = a->wb;
+    p.wd = a->wd;
+    p.bb = a->bb;
+    p.bd = a->bd;
+    p.dt_bias = a->dt_bias;
+    p.A_log = a->A_log;
+    p.abd = a->abd;
+    p.g = a->g;
+    p.beta = a->beta;
+    p.delta = a->delta;
+    p.dg = a->dg;
+    p.dbeta = a->dbeta;
+    p.ddelta = a->ddelta;
+    p.dx = a->dx;
+    p.dwa = a->dwa;
+    p.dwb = a->dwb;
+    p.dwd = a->dwd;
+    p.dbb = a->dbb;
+    p.dbd = a->dbd;
+    p.ddt_bias = a->ddt_bias;
+    p.dA_log = a->dA_log;
+    if (cyfa::launch_gates_train(p, dtype == CYFA_DTYPE_BF16, grad != 0, (float*)a->workspace, (hipStream_t)hip_stream) != 0)
+        return fail(CYFA_ERR_UNSUPPORTED, "%s: rows=%d K=%d H=%d", what, a->rows, a->K, a->H);
     return check_launch(what);
 }
 

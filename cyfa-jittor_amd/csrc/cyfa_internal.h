@@ -191,6 +191,22 @@ struct NormTrainParams {
 };
 constexpr int NORM_TRAIN_MAX_D = 2048;
 
+// The gate projections and activations of a training step and their adjoint
+// (cyfa_train.hip): x [rows, K], the weights [H, K], the biases bb, bd [H], abd
+// [rows, 3H] and their gradients bf16 or fp32, the rest fp32.
+struct GatesTrainParams {
+    int rows, K, H;
+    const void *x, *wa, *wb, *wd, *bb, *bd;
+    const float *dt_bias, *A_log;    // [H]
+    void* abd;                       // [rows, 3H]: written forward, read by the adjoint
+    float *g, *beta, *delta;         // [rows, H], the forward's results
+    const float *dg, *dbeta, *ddelta;
+    void *dx, *dwa, *dwb, *dwd, *dbb, *dbd;  // dx nullable
+    float *ddt_bias, *dA_log;
+    float *dabd, *part_sums, *part_w;  // parts of the adjoint's workspace (set by the launcher)
+};
+constexpr int GATES_MAX_H = 8;
+
 struct WorkspaceLayout {
     size_t lam, gam, seg, seg_exp, seg_decay, omega, tab_exp, tab16, total;
 };
@@ -501,6 +517,8 @@ int launch_mask_rows(const long long* mask, int B, int T, float* values, unsigne
                      hipStream_t stream);
 size_t conv_grad_workspace_bytes(int B, int T, int D, int W);
 int launch_conv_grad(const ConvGradParams& p, bool bf16, hipStream_t stream);
+size_t gates_grad_workspace_bytes(int rows, int K, int H);
+int launch_gates_train(const GatesTrainParams& p, bool bf16, bool grad, float* workspace, hipStream_t stream);
 size_t norm_grad_workspace_bytes(long long rows, int D);
 int launch_norm_train(const NormTrainParams& p, bool bf16, bool grad, hipStream_t stream);
 int launch_silu_mul(const __bf16* gu, __bf16* out, int rows, int F, hipStream_t stream);

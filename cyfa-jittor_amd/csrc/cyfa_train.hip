@@ -1,7 +1,8 @@
 // cyfa_train.hip -- the layer-side operations of a training step for gfx950:
 // the adjoints of the causal depthwise short convolution (ShortConvolution,
-// layers/cyfa.py:138-233) and of the gated RMS norm (RMSNorm,
-// layers/cyfa.py:62-135), with the norm's forward. Streaming kernels: each input is read once, sums
+// layers/cyfa.py:138-233), of the gated RMS norm (RMSNorm, layers/cyfa.py:62-135)
+// and of the gate projections and activations (layers/cyfa.py:323-326), with
+// the forwards of the last two. Streaming kernels: each input is read once, sums
 // over tokens accumulate in fp32 and partial sums are added in a fixed order,
 // so that two backward passes give the same bits.
 #include "cyfa_device.h"
@@ -349,7 +350,275 @@ int launch_norm_train_j(const NormTrainParams& p, bool grad, hipStream_t stream)
                     : launch_norm_train_as<E, 8>(p, grad, stream);
 }
 
+
+// ---- the gates of a training step ----
+//
+// a = x W_a^T, b = x W_b^T + c_b, d = x W_d^T + c_d (each rounded to E), and
+//   g = -exp(A_log) softplus(a + dt_bias), beta = sigmoid(b), delta = sigmoid(d)
+// for H <= GATES_MAX_H heads: projections so narrow that a library GEMM per
+// projection and direction spends 7 (forward), 9 (dx) and 39 us (weight
+// gradient) on 3000 x 1024 bf16 tokens, where x is 6 MB, with some 20 small
+// elementwise and reduction launches around them: about 240 us of a training
+// step in all. Here x is read once forward (7.2 us) and once backward (4.9 us
+// for the activations, 13.9 for dx and dW, 4.6 + 4.5 for the sums of their
+// partials).
+
+// softplus as F.softplus forms it (the identity above 20), and its derivative.
+__device__ __forceinline__ float softplus(float x) { return x > 20.f ? x : log1pf(expf(x)); }
+__device__ __forceinline__ float softplus_grad(float x) { return x > 20.f ? 1.f : exact_sigmoid(x); }
+
+// Row n of [W_a; W_b; W_d] (H rows each).
+template <class E>
+__device__ __forceinline__ const E* gates_weight(const GatesTrainParams& p, int n) {
+    const void* w = n < p.H ? p.wa : n < 2 * p.H ? p.wb : p.wd;
+    return static_cast<const E*>(w) + (size_t)(n % p.H) * p.K;
+}
+
+// Forward: a workgroup takes 16 rows of x, its four waves a quarter of the
+// columns each (8 columns per lane and step of 32), on the matrix cores: bf16
+// operands on v_mfma_f32_16x16x32_bf16, fp32 ones as two v_mfma_f32_16x16x4_f32
+// steps per four columns (fp32 products and sums). Lane (lr, lg) loads 8
+// consecutive columns of row lr of x and of weight rows lr, lr + 16; the waves'
+// partial sums meet in LDS, in wave order, where the activations are formed.
+template <class E, int NT>
+__global__ __launch_bounds__(256) void gates_train_kernel(GatesTrainParams p) {
+    typedef E ex8 __attribute__((ext_vector_type(8), aligned(16)));
+    __shared__ float part[4][16][16 * NT + 1];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lr = lane & 15, lg = lane >> 4;
+    const int H = p.H, N = 3 * H, r0 = blockIdx.x * 16;
+    const int steps = (p.K + 31) / 32, per = (steps + 3) / 4, s0 = wv * per, s1 = min(s0 + per, steps);
+    const E* x = static_cast<const E*>(p.x) + (size_t)min(r0 + lr, p.rows - 1) * p.K;
+    const E* w[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) w[t] = gates_weight<E>(p, min(16 * t + lr, N - 1));
+    f32x4 acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    constexpr int U = 4;  // steps whose loads are in flight together
+    for (int s = s0; s < s1; s += U) {
+        ex8 xv[U], wvv[U][NT];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int k = 32 * (s + u) + 8 * lg;
+            const bool live = s + u < s1 && k < p.K;  // K is a multiple of 8
+            const int kk = live ? k : 0;
+            xv[u] = *reinterpret_cast<const ex8*>(x + kk);
+#pragma unroll
+            for (int t = 0; t < NT; t++) wvv[u][t] = *reinterpret_cast<const ex8*>(w[t] + kk);
+            if (!live) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) xv[u][e] = (E)0.f;
+#pragma unroll
+                for (int t = 0; t < NT; t++)
+#pragma unroll
+                    for (int e = 0; e < 8; e++) wvv[u][t][e] = (E)0.f;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                if constexpr (sizeof(E) == 2) {
+                    acc[t] = mfma_bf16(__builtin_bit_cast(bf16x8, xv[u]), __builtin_bit_cast(bf16x8, wvv[u][t]), acc[t]);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+                        acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[u][e], wvv[u][t][e], acc[t], 0, 0, 0);
+                }
+            }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) part[wv][4 * lg + i][16 * t + lr] = acc[t][i];
+    __syncthreads();
+    for (int e = threadIdx.x; e < 16 * N; e += 256) {
+        const int r = e / N, n = e % N, h = n % H, kind = n / H;
+        const long long row = r0 + r;
+        if (row >= p.rows) break;
+        float v = (part[0][r][n] + part[1][r][n]) + (part[2][r][n] + part[3][r][n]);
+        if (kind) v += (float)static_cast<const E*>(kind == 1 ? p.bb : p.bd)[h];
+        const E pre = (E)v;
+        static_cast<E*>(p.abd)[row * N + n] = pre;
+        v = (float)pre;
+        float* dst = kind == 0 ? p.g : kind == 1 ? p.beta : p.delta;
+        dst[row * H + h] = kind == 0 ? -expf(p.A_log[h]) * softplus(v + p.dt_bias[h]) : exact_sigmoid(v);
+    }
+}
+
+// Adjoint of the activations, one row per lane, 64 rows per workgroup: dabd
+// [rows, 3H] rounded to E (the projections' cotangents) as fp32, and per
+// workgroup the sums over its rows of da (dt_bias), of dg g (A_log), and of
+// the rounded db and dd (the biases), each H wide.
+__global__ __launch_bounds__(256) void gates_grad_act_kernel(GatesTrainParams p, int bf16) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, H = p.H, N = 3 * H;
+    const long long row = (long long)blockIdx.x * 64 + lane;
+    const bool live = row < p.rows;
+    const long long rr = live ? row : 0;
+    const auto rnd = [&](float v) { return bf16 ? bf16_round(v) : v; };
+    const auto pre = [&](int n) {
+        return bf16 ? (float)static_cast<const bf16_t*>(p.abd)[rr * N + n] : static_cast<const float*>(p.abd)[rr * N + n];
+    };
+    for (int h = wv; h < H; h += 4) {
+        const float z = pre(h) + p.dt_bias[h], ea = -expf(p.A_log[h]);
+        const float dg = live ? p.dg[rr * H + h] : 0.f;
+        const float be = exact_sigmoid(pre(H + h)), de = exact_sigmoid(pre(2 * H + h));
+        const float da = dg * ea * softplus_grad(z);
+        const float db = rnd(live ? p.dbeta[rr * H + h] * be * (1.f - be) : 0.f);
+        const float dd = rnd(live ? p.ddelta[rr * H + h] * de * (1.f - de) : 0.f);
+        if (live) {
+            p.dabd[rr * N + h] = rnd(da);
+            p.dabd[rr * N + H + h] = db;
+            p.dabd[rr * N + 2 * H + h] = dd;
+        }
+        float* part = p.part_sums + (size_t)blockIdx.x * 4 * H + h;
+        const float sa = wave_sum(da), sl = wave_sum(dg * ea * softplus(z)), sb = wave_sum(db), sd = wave_sum(dd);
+        if (lane == 0) {
+            part[0] = sa;
+            part[H] = sl;
+            part[2 * H] = sb;
+            part[3 * H] = sd;
+        }
+    }
+}
+
+// Adjoint of the projections: dx = da W_a + db W_b (the clock branch passes no
+// gradient into x) and dW[n] = sum over the rows of dabd[n] x. A lane holds
+// four columns, a workgroup 256 columns and GATES_ROWS rows, a wave every
+// fourth of them, the weights and dW in registers (HM: H rounded up to 4 or
+// 8); the waves' parts of dW are added in LDS, in wave order, into one partial
+// per workgroup.
+constexpr int GATES_ROWS = 32;
+
+template <class E, int HM>
+__global__ __launch_bounds__(256) void gates_grad_kernel(GatesTrainParams p) {
+    __shared__ __align__(16) float red[4][4][256];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int H = p.H, N = 3 * H, K = p.K, k = blockIdx.x * 256 + 4 * lane;
+    const bool live = k < K;
+    const int kk = live ? k : 0;
+    f32x4 w[2 * HM], dw[3 * HM];
+#pragma unroll
+    for (int n = 0; n < 2 * HM; n++) {
+        const int h = n % HM, kind = n / HM;
+        w[n] = load4(gates_weight<E>(p, h < H ? kind * H + h : 0) + kk);
+    }
+#pragma unroll
+    for (int n = 0; n < 3 * HM; n++) dw[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int row0 = blockIdx.y * GATES_ROWS;
+    for (int i = 0; i < GATES_ROWS; i += 8) {  // two rows of this wave at a time
+        f32x4 x[2];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int row = min(row0 + i + 4 * u + wv, p.rows - 1);
+            x[u] = load4(static_cast<const E*>(p.x) + (size_t)row * K + kk);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int row = row0 + i + 4 * u + wv;
+            if (row < p.rows) {  // uniform over the wave, as dabd's addresses are
+                const float* da = p.dabd + (size_t)row * N;
+                f32x4 dx = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int n = 0; n < 3 * HM; n++) {
+                    const int h = n % HM, kind = n / HM;
+                    const float c = h < H ? da[kind * H + h] : 0.f;
+                    if (kind < 2) dx += w[n] * c;
+                    dw[n] += x[u] * c;
+                }
+                if (live && p.dx) store4(static_cast<E*>(p.dx) + (size_t)row * K + k, dx);
+            }
+        }
+    }
+    float* part = p.part_w + (size_t)blockIdx.y * N * K;
+    const int col = blockIdx.x * 256 + threadIdx.x;
+#pragma unroll
+    for (int n0 = 0; n0 < 3 * HM; n0 += 4) {
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 4; j++) *reinterpret_cast<f32x4*>(&red[wv][j][4 * lane]) = dw[n0 + j];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int h = (n0 + j) % HM, kind = (n0 + j) / HM, e = threadIdx.x;
+            if (h < H && col < K)
+                part[(size_t)(kind * H + h) * K + col] = (red[0][j][e] + red[1][j][e]) + (red[2][j][e] + red[3][j][e]);
+        }
+    }
+}
+
+// Adds the partials of gates_grad_kernel into dW_a, dW_b and dW_d.
+template <class E>
+__global__ __launch_bounds__(256) void gates_grad_reduce_kernel(GatesTrainParams p, int nparts) {
+    const int n = 3 * p.H * p.K, e = blockIdx.x * 32 + (int)threadIdx.x;
+    const float s = column_sum(p.part_w, nparts, n);
+    if (threadIdx.x >= 32 || e >= n) return;
+    const int hk = p.H * p.K, kind = e / hk;
+    static_cast<E*>(kind == 0 ? p.dwa : kind == 1 ? p.dwb : p.dwd)[e % hk] = (E)s;
+}
+
+// Adds the partial sums of gates_grad_act_kernel: dt_bias, A_log (fp32), then
+// the biases (E).
+template <class E>
+__global__ __launch_bounds__(256) void gates_grad_sums_kernel(GatesTrainParams p, int nparts) {
+    const int n = 4 * p.H, e = blockIdx.x * 32 + (int)threadIdx.x;
+    const float s = column_sum(p.part_sums, nparts, n);
+    if (threadIdx.x >= 32 || e >= n) return;
+    const int kind = e / p.H, h = e % p.H;
+    if (kind < 2)
+        (kind == 0 ? p.ddt_bias : p.dA_log)[h] = s;
+    else
+        static_cast<E*>(kind == 2 ? p.dbb : p.dbd)[h] = (E)s;
+}
+
+template <class E>
+int launch_gates_train_as(const GatesTrainParams& p, hipStream_t stream) {
+    const dim3 grid((unsigned)((p.rows + 15) / 16)), block(256);
+    if (3 * p.H <= 16)
+        hipLaunchKernelGGL((gates_train_kernel<E, 1>), grid, block, 0, stream, p);
+    else
+        hipLaunchKernelGGL((gates_train_kernel<E, 2>), grid, block, 0, stream, p);
+    return 0;
+}
+
+template <class E>
+int launch_gates_grad_as(const GatesTrainParams& p, hipStream_t stream) {
+    const dim3 block(256);
+    const int acts = (p.rows + 63) / 64, parts = (p.rows + GATES_ROWS - 1) / GATES_ROWS;
+    hipLaunchKernelGGL(gates_grad_act_kernel, dim3(acts), block, 0, stream, p, sizeof(E) == 2 ? 1 : 0);
+    const dim3 grid((p.K + 255) / 256, parts);
+    if (p.H <= 4)
+        hipLaunchKernelGGL((gates_grad_kernel<E, 4>), grid, block, 0, stream, p);
+    else
+        hipLaunchKernelGGL((gates_grad_kernel<E, 8>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL(gates_grad_reduce_kernel<E>, dim3((3 * p.H * p.K + 31) / 32), block, 0, stream, p, parts);
+    hipLaunchKernelGGL(gates_grad_sums_kernel<E>, dim3((4 * p.H + 31) / 32), block, 0, stream, p, acts);
+    return 0;
+}
+
 }  // namespace
+
+size_t gates_grad_workspace_bytes(int rows, int K, int H) {
+    return ((size_t)rows * 3 * H + (size_t)((rows + 63) / 64) * 4 * H + (size_t)((rows + GATES_ROWS - 1) / GATES_ROWS) * 3 * H * K) *
+           sizeof(float);
+}
+
+// Splits the adjoint's workspace (gates_grad_workspace_bytes) into its parts.
+static void gates_grad_workspace(GatesTrainParams& p, float* base) {
+    p.dabd = base;
+    p.part_sums = p.dabd + (size_t)p.rows * 3 * p.H;
+    p.part_w = p.part_sums + (size_t)((p.rows + 63) / 64) * 4 * p.H;
+}
+
+int launch_gates_train(const GatesTrainParams& p_in, bool bf16, bool grad, float* workspace, hipStream_t stream) {
+    GatesTrainParams p = p_in;
+    if (p.rows < 1 || p.rows > GATES_ROWS * 65535 || p.K < 8 || p.K % 8 || p.H < 1 || p.H > GATES_MAX_H ||
+        (long long)3 * p.H * p.K >= 1ll << 31)
+        return -1;
+    if (!grad) return bf16 ? launch_gates_train_as<bf16_t>(p, stream) : launch_gates_train_as<float>(p, stream);
+    gates_grad_workspace(p, workspace);
+    return bf16 ? launch_gates_grad_as<bf16_t>(p, stream) : launch_gates_grad_as<float>(p, stream);
+}
 
 size_t norm_grad_workspace_bytes(long long rows, int D) {
     const int n = norm_grad_rows(rows);

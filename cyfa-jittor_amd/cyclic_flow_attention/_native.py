@@ -14,7 +14,7 @@ import torch
 import torch.nn.functional as F
 
 LIB_PATH = Path(os.environ.get("CYFA_LIB", Path(__file__).with_name("libcyfa_hip.so")))
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 CYFA_OK = 0
 CYFA_ERR_VALUE = -1
@@ -160,6 +160,12 @@ class CyfaNormTrainArgs(ctypes.Structure):
     ]
 
 
+class CyfaGatesTrainArgs(ctypes.Structure):
+    _fields_ = [("rows", _c_int), ("K", _c_int), ("H", _c_int)] + [(n, _c_void_p) for n in (
+        "x", "wa", "wb", "wd", "bb", "bd", "dt_bias", "A_log", "abd", "g", "beta", "delta", "dg", "dbeta", "ddelta",
+        "dx", "dwa", "dwb", "dwd", "dbb", "dbd", "ddt_bias", "dA_log", "workspace")] + [("workspace_bytes", _c_size_t)]
+
+
 class CyfaGatePathArgs(ctypes.Structure):
     _fields_ = [
         ("M", _c_int), ("K", _c_int), ("H", _c_int), ("Dv", _c_int),
@@ -184,6 +190,8 @@ SIGNATURES = {
     "cyfa_readout_table": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_int, _c_void_p]),
     "cyfa_rms_norm": (_c_int, [ctypes.POINTER(CyfaNormArgs), _c_void_p]),
     "cyfa_short_conv": (_c_int, [ctypes.POINTER(CyfaConvArgs), _c_void_p]),
+    "cyfa_gates_grad_workspace_bytes": (_c_size_t, [_c_int] * 3),
+    "cyfa_gates_train": (_c_int, [ctypes.POINTER(CyfaGatesTrainArgs), _c_int, _c_int, _c_void_p]),
     "cyfa_norm_grad_workspace_bytes": (_c_size_t, [ctypes.c_longlong, _c_int]),
     "cyfa_norm_train": (_c_int, [ctypes.POINTER(CyfaNormTrainArgs), _c_int, _c_int, _c_void_p]),
     "cyfa_mask_rows": (_c_int, [_c_void_p, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p]),
@@ -434,21 +442,26 @@ def _check(rc, what):
         _raise(rc, what + " failed")
 
 
+def aligned_rows(x):
+    """x itself where it is contiguous and 16-byte aligned, else a copy that is."""
+    x = x.contiguous()
+    return x.clone() if x.data_ptr() % 16 else x
+
+
 def rms_norm(x, weight, eps, gate=None, residual=None, prescale=1.0):
     """Fused (residual add +) RMSNorm (+ sigmoid gate) over the last dim of bf16 x.
 
     Returns out, or (sum, out) when residual is given (sum = bf16(x + residual))."""
     dev = require_device(x, weight, gate, residual)
     D = x.shape[-1]
-    x = x.contiguous()
-    w = weight.detach().to(torch.float32).contiguous()
+    x, w = aligned_rows(x), aligned_rows(weight.detach().to(torch.float32))
     out = torch.empty_like(x)
     total = None
     if residual is not None:
-        residual = residual.contiguous()
+        residual = aligned_rows(residual)
         total = torch.empty_like(x)
     if gate is not None:
-        gate = gate.contiguous()
+        gate = aligned_rows(gate)
     args = CyfaNormArgs(rows=x.numel() // D, D=D, x=ptr(x), residual=ptr(residual), sum_out=ptr(total),
                         weight=ptr(w), gate=ptr(gate), eps=float(eps), prescale=float(prescale), out=ptr(out))
     _check(load_library().cyfa_rms_norm(ctypes.byref(args), stream_handle(dev)), "cyfa_rms_norm")
@@ -701,6 +714,48 @@ def short_conv(x, weight, bias=None, cache=None, split=None, cache_out=None, mas
     fn = lib.cyfa_short_conv_f32 if x.dtype == torch.float32 else lib.cyfa_short_conv
     _check(fn(ctypes.byref(args), stream_handle(dev)), "cyfa_short_conv")
     return outs
+
+
+GATES_TRAIN_MAX_H = 8
+GATES_TRAIN_MAX_ROWS = 32 * 65535
+
+
+def gates_train(x, wa, wb, bb, wd, bd, dt_bias, A_log):
+    """(g, beta, delta fp32 [rows, H], abd [rows, 3H]) of x [rows, K] (bf16 or
+    fp32, as the weights and biases): the gate projections and activations of a
+    training step; contiguous, x and the weights 16-byte aligned."""
+    dev = require_device(x, wa, wb, bb, wd, bd, dt_bias, A_log)
+    rows, K = x.shape
+    H = wa.shape[0]
+    g, beta, delta = (torch.empty(rows, H, dtype=torch.float32, device=dev) for _ in range(3))
+    abd = torch.empty(rows, 3 * H, dtype=x.dtype, device=dev)
+    args = CyfaGatesTrainArgs(rows=rows, K=K, H=H, x=ptr(x), wa=ptr(wa), wb=ptr(wb), wd=ptr(wd), bb=ptr(bb), bd=ptr(bd),
+                              dt_bias=ptr(dt_bias), A_log=ptr(A_log), abd=ptr(abd), g=ptr(g), beta=ptr(beta),
+                              delta=ptr(delta))
+    _check(load_library().cyfa_gates_train(ctypes.byref(args), general_dtype(x), 0, stream_handle(dev)),
+           "cyfa_gates_train")
+    return g, beta, delta, abd
+
+
+def gates_grad(x, wa, wb, wd, dt_bias, A_log, abd, dg, dbeta, ddelta, need_dx):
+    """Gradients (dx or None, dwa, dwb, dbb, dwd, dbd, ddt_bias, dA_log) of
+    gates_train's g, beta and delta from their cotangents (fp32 [rows, H])."""
+    dev = require_device(x, wa, wb, wd, dt_bias, A_log, abd, dg, dbeta, ddelta)
+    rows, K = x.shape
+    H = wa.shape[0]
+    dx = torch.empty_like(x) if need_dx else None
+    dwa, dwb, dwd = (torch.empty_like(w) for w in (wa, wb, wd))
+    dbb, dbd = (torch.empty(H, dtype=x.dtype, device=dev) for _ in range(2))
+    ddt, dal = (torch.empty(H, dtype=torch.float32, device=dev) for _ in range(2))
+    lib = load_library()
+    n = int(lib.cyfa_gates_grad_workspace_bytes(rows, K, H))
+    workspace = torch.empty(max(n, 1), dtype=torch.uint8, device=dev)  # alive until the launch
+    args = CyfaGatesTrainArgs(rows=rows, K=K, H=H, x=ptr(x), wa=ptr(wa), wb=ptr(wb), wd=ptr(wd), dt_bias=ptr(dt_bias),
+                              A_log=ptr(A_log), abd=ptr(abd), dg=ptr(dg), dbeta=ptr(dbeta), ddelta=ptr(ddelta),
+                              dx=ptr(dx), dwa=ptr(dwa), dwb=ptr(dwb), dwd=ptr(dwd), dbb=ptr(dbb), dbd=ptr(dbd),
+                              ddt_bias=ptr(ddt), dA_log=ptr(dal), workspace=ptr(workspace), workspace_bytes=n)
+    _check(lib.cyfa_gates_train(ctypes.byref(args), general_dtype(x), 1, stream_handle(dev)), "cyfa_gates_train")
+    return dx, dwa, dwb, dbb, dwd, dbd, ddt, dal
 
 
 NORM_TRAIN_MAX_D = 2048

@@ -28,18 +28,20 @@ def hip_autograd_ok(*tensors):
             and not torch.compiler.is_compiling() and not torch.jit.is_tracing())
 
 
-def rows_16(x):
-    """x itself where it is contiguous and 16-byte aligned, else a copy that is
-    (made before a function's ``apply``, so that it is part of the graph)."""
-    x = x.contiguous()
-    return x.clone() if x.data_ptr() % 16 else x
+def _through_torch(*cotangents):
+    """Whether a backward pass has to run in torch operations: one that is
+    itself recorded, or batched over several cotangents (vmap)."""
+    return (torch.is_grad_enabled() or torch._C._functorch.peek_interpreter_stack() is not None
+            or any(torch._C._functorch.is_legacy_batchedtensor(t) for t in cotangents))
 
 
-def _recorded_grads(fn, inputs, needed, dy):
-    """Gradients of fn(*inputs), recorded for further derivatives."""
+def _torch_grads(fn, inputs, needed, dy):
+    """Gradients of fn(*inputs) by autograd, themselves recorded when this
+    backward pass is."""
+    recorded = torch.is_grad_enabled()
     with torch.enable_grad():
         wanted = [t for t, n in zip(inputs, needed) if n]
-        grads = iter(torch.autograd.grad(fn(*inputs), wanted, dy, create_graph=True, allow_unused=True))
+        grads = iter(torch.autograd.grad(fn(*inputs), wanted, dy, create_graph=recorded, allow_unused=True))
     return tuple(next(grads) if n else None for n in needed)
 
 
@@ -48,7 +50,8 @@ def short_conv(x, weight, bias, cache, general):
     adjoint: x [B, T, D], weight [D, W], bias [D] or None, cache [B, W-1, D] or
     None, all of one dtype (bf16 or fp32). ``general``: the same in torch
     operations."""
-    return ShortConv.apply(rows_16(x), weight.contiguous(), bias, None if cache is None else rows_16(cache), general)
+    cache = None if cache is None else _native.aligned_rows(cache)
+    return ShortConv.apply(_native.aligned_rows(x), weight.contiguous(), bias, cache, general)
 
 
 class ShortConv(torch.autograd.Function):
@@ -64,9 +67,9 @@ class ShortConv(torch.autograd.Function):
     def backward(ctx, dy):
         x, weight, bias, cache = ctx.saved_tensors
         needed = ctx.needs_input_grad[:4]
-        if torch.is_grad_enabled():
-            return _recorded_grads(ctx.general, (x, weight, bias, cache), needed, dy) + (None,)
-        grads = _native.short_conv_grad(x, weight, cache, rows_16(dy), needed)
+        if _through_torch(dy):
+            return _torch_grads(ctx.general, (x, weight, bias, cache), needed, dy) + (None,)
+        grads = _native.short_conv_grad(x, weight, cache, _native.aligned_rows(dy), needed)
         return (*grads, None)
 
 
@@ -74,7 +77,8 @@ def rms_norm(x, weight, gate, eps, prescale, general):
     """norm(x prescale) [* sigmoid(gate)] (layers/cyfa.py:62-135) with its HIP
     adjoint: x and gate [..., D] bf16 or fp32 of one dtype, weight fp32 [D].
     ``general``: the same of (x, weight, gate) in torch operations."""
-    return GatedNorm.apply(rows_16(x), rows_16(weight), None if gate is None else rows_16(gate), eps, prescale, general)
+    gate = None if gate is None else _native.aligned_rows(gate)
+    return GatedNorm.apply(_native.aligned_rows(x), _native.aligned_rows(weight), gate, eps, prescale, general)
 
 
 class GatedNorm(torch.autograd.Function):
@@ -91,6 +95,40 @@ class GatedNorm(torch.autograd.Function):
     def backward(ctx, dy):
         x, weight, gate = ctx.saved_tensors
         needed = ctx.needs_input_grad[:3]
-        if torch.is_grad_enabled():
-            return _recorded_grads(ctx.general, (x, weight, gate), needed, dy) + (None,) * 3
-        return (*_native.norm_grad(x, weight, gate, *ctx.args, rows_16(dy), needed), None, None, None)
+        if _through_torch(dy):
+            return _torch_grads(ctx.general, (x, weight, gate), needed, dy) + (None,) * 3
+        return (*_native.norm_grad(x, weight, gate, *ctx.args, _native.aligned_rows(dy), needed), None, None, None)
+
+
+def gates(x, wa, wb, bb, wd, bd, dt_bias, A_log, general):
+    """The gates (g, beta, delta) fp32 [..., H] of x [..., K] (layers/cyfa.py:
+    323-326) with their HIP adjoint: the weights [H, K] and biases [H] of x's
+    dtype (bf16 or fp32), dt_bias and A_log fp32 [H]. The clock branch (wd, bd)
+    sends no gradient into x. ``general``: the same in torch operations."""
+    wa, wb, wd = (_native.aligned_rows(w) for w in (wa, wb, wd))
+    flat = _native.aligned_rows(x.reshape(-1, x.shape[-1]))
+    bb, bd, dt_bias, A_log = (t.contiguous() for t in (bb, bd, dt_bias, A_log))
+    out = Gates.apply(flat, wa, wb, bb, wd, bd, dt_bias, A_log, general)
+    return tuple(t.reshape(x.shape[:-1] + t.shape[-1:]) for t in out)
+
+
+class Gates(torch.autograd.Function):
+    """gates' function; every input contiguous, x [rows, K]."""
+
+    @staticmethod
+    def forward(ctx, x, wa, wb, bb, wd, bd, dt_bias, A_log, general):
+        g, beta, delta, abd = _native.gates_train(x, wa, wb, bb, wd, bd, dt_bias, A_log)
+        ctx.save_for_backward(x, wa, wb, bb, wd, bd, dt_bias, A_log, abd)
+        ctx.general = general
+        return g, beta, delta
+
+    @staticmethod
+    def backward(ctx, dg, dbeta, ddelta):
+        *inputs, abd = ctx.saved_tensors
+        x, wa, wb, _, wd, _, dt_bias, A_log = inputs
+        needed = ctx.needs_input_grad[:8]
+        if _through_torch(dg, dbeta, ddelta):
+            return _torch_grads(ctx.general, inputs, needed, (dg, dbeta, ddelta)) + (None,)
+        grads = _native.gates_grad(x, wa, wb, wd, dt_bias, A_log, abd, dg.contiguous(), dbeta.contiguous(),
+                                   ddelta.contiguous(), needed[0])
+        return tuple(t if n else None for t, n in zip(grads, needed)) + (None,)

@@ -27,7 +27,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from .. import _native
-from .autograd import hip_autograd_ok, rms_norm, short_conv
+from .autograd import gates, hip_autograd_ok, rms_norm, short_conv
 from ..ops import chunk_cyfa, fused_recurrent_cyfa
 from ..ops.fused_recurrent import decode_layer_step
 from ..ops.utils import readout_table
@@ -92,7 +92,7 @@ class RMSNorm(nn.Module):
         o * (num_slots - 1)); ``residual`` first forms s = x + residual and
         returns (s, norm(s))."""
         D = x.shape[-1]
-        if (inference_fast_path(x) and D % 256 == 0 and D // 256 in (1, 2, 4, 8)
+        if (inference_fast_path(x) and D % 256 == 0 and 256 <= D <= 2048
                 and (gate is None or gate.dtype == torch.bfloat16)
                 and (residual is None or residual.dtype == torch.bfloat16)):
             return _native.rms_norm(x, self.weight, self.eps, gate, residual, prescale)
@@ -182,6 +182,20 @@ def general_short_conv(x, weight, bias, cache):
     W = weight.shape[-1]
     padded = F.pad(x, (0, 0, W - 1, 0)) if cache is None else torch.cat([cache, x], dim=1)
     return F.conv1d(padded.transpose(1, 2), weight.unsqueeze(1), bias, groups=x.shape[-1]).transpose(1, 2)
+
+
+def plain_linear(m):
+    """Whether calling module m is F.linear on its weight and bias and nothing
+    more (no subclass, wrapper or hook)."""
+    return (type(m) is nn.Linear and not m._forward_hooks and not m._forward_pre_hooks and not m._backward_hooks
+            and not m._backward_pre_hooks and not torch.nn.modules.module._has_any_global_hook())
+
+
+def general_gates(x, wa, wb, bb, wd, bd, dt_bias, A_log):
+    """The gates in torch operations. The clock branch trains d_proj but passes
+    no gradient into x (reference layers/cyfa.py:325: d_proj(x.detach()))."""
+    g = -A_log.exp() * F.softplus(F.linear(x, wa).float() + dt_bias)
+    return g, torch.sigmoid(F.linear(x, wb, bb).float()), torch.sigmoid(F.linear(x.detach(), wd, bd).float())
 
 
 def shared_conv_cache(conv_state):
@@ -360,12 +374,7 @@ class CyclicFlowAttention(nn.Module):
         q = q.reshape(B, T, H, self.head_k_dim)
         k = k.reshape(B, T, H, self.head_k_dim)
         v = v.reshape(B, T, H, self.head_v_dim)
-        a = self.a_proj(x).float() + self.dt_bias.float()
-        g = -self.A_log.float().exp() * F.softplus(a)
-        # the clock branch trains d_proj but passes no gradient into x
-        # (reference layers/cyfa.py:325: d_proj(x.detach()))
-        delta = torch.sigmoid(self.d_proj(x.detach()).float())
-        beta = torch.sigmoid(self.b_proj(x).float())
+        g, beta, delta = self._gates(x)
         if attention_mask is not None:
             valid = attention_mask.unsqueeze(-1).bool()
             g, delta, beta = (torch.where(valid, t, torch.zeros_like(t)) for t in (g, delta, beta))
@@ -394,6 +403,21 @@ class CyclicFlowAttention(nn.Module):
         o = self.o_proj(o)
         new_cache = {"recurrent_state": state, "conv_state": (cq, ck, cv)} if use_cache else None
         return o, new_cache
+
+    def _gates(self, x):
+        """(g, beta, delta) fp32 [B, T, H] of the general path."""
+        H = self.num_heads
+        a, b, d = self.a_proj, self.b_proj, self.d_proj
+        weights = (a.weight, b.weight, b.bias, d.weight, d.bias) if all(plain_linear(m) for m in (a, b, d)) else ()
+        if (weights and a.bias is None and all(w is not None and w.dtype == x.dtype for w in weights)
+                and x.dtype in (torch.bfloat16, torch.float32) and H <= _native.GATES_TRAIN_MAX_H
+                and x.shape[-1] % 8 == 0 and 0 < x.numel() // x.shape[-1] <= _native.GATES_TRAIN_MAX_ROWS
+                and hip_autograd_ok(x, *weights, self.dt_bias, self.A_log)):
+            # training: the projections, the activations and their adjoint as HIP kernels
+            return gates(x, *weights, self.dt_bias.float(), self.A_log.float(), general_gates)
+        delta = torch.sigmoid(d(x.detach()).float())
+        beta = torch.sigmoid(b(x).float())
+        return -self.A_log.float().exp() * F.softplus(a(x).float() + self.dt_bias.float()), beta, delta
 
     def forward_block(self, x, norm, cache=None, use_cache=False, prefetch=()):
         """The attention half of a decoder block, x + self(norm(x), cache,

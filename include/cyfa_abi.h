@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define CYFA_ABI_VERSION 14
+#define CYFA_ABI_VERSION 15
 
 enum {
     CYFA_OK = 0,
@@ -539,6 +539,31 @@ typedef struct CyfaNormTrainArgs {
 
 size_t cyfa_norm_grad_workspace_bytes(long long rows, int D);
 int cyfa_norm_train(const CyfaNormTrainArgs *args, int dtype, int grad, void *hip_stream);
+
+/* The gate projections and activations of a training step (layers/cyfa.py:
+ * 323-326) for rows of x [rows, K], K a multiple of 8, H <= 8 heads; x, the
+ * weights [H, K], the biases [H], abd and their gradients of one dtype
+ * (CYFA_DTYPE_BF16 or CYFA_DTYPE_F32), the rest f32; x, weights, dx and the
+ * workspace 16-byte aligned:
+ *   abd = [x wa^T | x wb^T + bb | x wd^T + bd] (rounded to the dtype)
+ *   g = -exp(A_log) softplus(a + dt_bias), beta = sigmoid(b), delta = sigmoid(d)  (grad 0)
+ * and from dg, dbeta, ddelta the gradients (grad 1; dx without the clock
+ * branch's share, as the layer detaches x there), sums in a fixed order. */
+typedef struct CyfaGatesTrainArgs {
+    int rows, K, H;
+    const void *x, *wa, *wb, *wd, *bb, *bd;
+    const float *dt_bias, *A_log; /* [H] */
+    void *abd;                    /* [rows, 3H]: written by grad 0, read by grad 1 */
+    float *g, *beta, *delta;      /* [rows, H] */
+    const float *dg, *dbeta, *ddelta;
+    void *dx, *dwa, *dwb, *dwd, *dbb, *dbd; /* dx nullable */
+    float *ddt_bias, *dA_log;
+    void *workspace;              /* grad 1: cyfa_gates_grad_workspace_bytes(rows, K, H) bytes */
+    size_t workspace_bytes;
+} CyfaGatesTrainArgs;
+
+size_t cyfa_gates_grad_workspace_bytes(int rows, int K, int H);
+int cyfa_gates_train(const CyfaGatesTrainArgs *args, int dtype, int grad, void *hip_stream);
 
 /* out[r, c] = bf16(g sigmoid(g) u), g = gu[r, c], u = gu[r, F + c]; F a
  * multiple of 8. Replaces the activation of GatedMLP.execute

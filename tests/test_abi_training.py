@@ -9,7 +9,7 @@ from cyclic_flow_attention import _native
 from test_abi import _c_layout
 
 
-@pytest.mark.parametrize("name", ["CyfaConvGradArgs", "CyfaGatePathArgs", "CyfaNormTrainArgs"])
+@pytest.mark.parametrize("name", ["CyfaConvGradArgs", "CyfaGatePathArgs", "CyfaNormTrainArgs", "CyfaGatesTrainArgs"])
 def test_struct_layout_matches_header(tmp_path, name):
     cls = getattr(_native, name)
     fields = [f for f, _ in cls._fields_]
@@ -55,4 +55,21 @@ def test_norm_train_validates_before_launch():
     assert call(0, D=258) == call(1, D=4096) == _native.CYFA_ERR_UNSUPPORTED
     assert call(0, out=None) == call(1, dy=None) == call(1, dgate=0x60000) == call(0, dtype=3) == _native.CYFA_ERR_VALUE
     assert call(0, x=0x10008) == _native.CYFA_ERR_ALIGN
+    assert call(1, workspace_bytes=n - 4) == _native.CYFA_ERR_WORKSPACE
+
+
+def test_gates_train_validates_before_launch():
+    lib = _native.load_library()
+    n = lib.cyfa_gates_grad_workspace_bytes(100, 256, 4)
+    assert n >= (100 * 12 + 12 * 256) * 4
+    names = [f for f, t in _native.CyfaGatesTrainArgs._fields_ if t is ctypes.c_void_p]
+    good = dict(rows=100, K=256, H=4, workspace_bytes=n, **{f: 0x10000 * (i + 1) for i, f in enumerate(names)})
+
+    def call(grad, dtype=0, **change):
+        a = _native.CyfaGatesTrainArgs(**{**good, **change})
+        return lib.cyfa_gates_train(ctypes.byref(a), dtype, grad, None)
+
+    assert call(0, K=60) == call(1, H=9) == _native.CYFA_ERR_UNSUPPORTED
+    assert call(0, rows=0) == call(0, g=None) == call(1, dwa=None) == call(0, dtype=2) == _native.CYFA_ERR_VALUE
+    assert call(0, x=0x10008) == call(1, dx=0x10004) == _native.CYFA_ERR_ALIGN
     assert call(1, workspace_bytes=n - 4) == _native.CYFA_ERR_WORKSPACE

@@ -81,6 +81,11 @@ def test_short_conv_training_views_second_derivatives_and_transforms():
     gg, = torch.autograd.grad(gx.pow(2).sum(), x)
     rr, = torch.autograd.grad(rx.pow(2).sum(), ref)
     assert _rel(gx.detach(), rx.detach()) < 1e-5 and _rel(gg, rr) < 1e-5
+    cots = torch.randn(3, 2, 20, 16, generator=gen).to(DEV)
+    y, _ = conv(x)
+    batched, = torch.autograd.grad(y, x, cots, is_grads_batched=True, retain_graph=True)
+    for c, b in zip(cots, batched):
+        assert _rel(b, torch.autograd.grad(y, x, c, retain_graph=True)[0].double().cpu()) < 1e-5
     xs = torch.randn(3, 2, 20, 16, generator=gen).to(DEV)
     out = torch.func.vmap(lambda t: conv(t)[0])(xs)
     assert _rel(out.detach(), torch.stack([_conv64(t.double().cpu(), w64, None, None) for t in xs])) < 1e-6
@@ -132,3 +137,81 @@ def test_rms_norm_training_gradients(rows, D, gate, prescale, dtype):
     rec = torch.autograd.grad(norm(xg, gg, prescale=prescale), leaves, dy.to(DEV), create_graph=True)
     for a, r in zip(rec, rg):
         assert a.requires_grad and _rel(a.detach(), r) <= 2 * bar
+
+
+@pytest.mark.parametrize("D,gate,residual,prescale", [(768, True, True, 1.0), (1280, True, False, 127.0),
+                                                      (1536, False, True, 1.0), (1792, False, False, 1.0)])
+def test_rms_norm_kernel_every_multiple_of_256(D, gate, residual, prescale):
+    import test_gpu_layer
+
+    test_gpu_layer.test_rms_norm_kernel(D, gate, residual, prescale)
+    norm = RMSNorm(D, 1e-6).to(DEV)
+    x = torch.randn(3 * D + 1, device=DEV).bfloat16()[1:].view(3, D)  # rows off the 16-byte grid
+    with torch.no_grad():
+        assert torch.equal(norm(x), norm(x.clone()))
+
+
+def _gates64(x, wa, wb, bb, wd, bd, dt_bias, A_log, dtype):
+    def rounded(t):  # the projection's rounding, passed straight through by the gradient
+        return t + (t.detach().to(dtype).double() - t.detach())
+
+    a, b, d = rounded(x @ wa.mT), rounded(x @ wb.mT + bb), rounded(x.detach() @ wd.mT + bd)
+    return -A_log.exp() * F.softplus(a + dt_bias), torch.sigmoid(b), torch.sigmoid(d)
+
+
+# one row, remainders of 16, 32 and 64 rows, one and two column tiles of the
+# projection, both register widths, K with remainders of a step and of 256
+@pytest.mark.parametrize("rows,K,H,dtype", [(1, 8, 1, torch.float32), (17, 256, 4, torch.bfloat16),
+                                            (65, 1000, 6, torch.float32), (100, 40, 5, torch.bfloat16),
+                                            (333, 2048, 8, torch.bfloat16), (3000, 1024, 4, torch.bfloat16),
+                                            (70, 264, 3, torch.float32)])
+def test_gates_training_gradients(rows, K, H, dtype):
+    """bf16: the projections' cotangents are rounded (2^-8 of each) before the
+    sums, and the results are rounded again; a projection on a rounding edge may
+    go either way, for few values. fp32: dot products and column sums of up to
+    3000 terms, whose roundings add up as their square root, 64 of them at most."""
+    from cyclic_flow_attention.layers.autograd import gates
+    from cyclic_flow_attention.layers.cyfa import general_gates
+
+    gen = torch.Generator().manual_seed(rows + K)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=gen)
+
+    x = rnd(rows, K).to(dtype)
+    ws = [(rnd(H, K) * K ** -0.5).to(dtype) for _ in range(3)]
+    bb, bd = (0.1 * rnd(H)).to(dtype), (0.1 * rnd(H)).to(dtype)
+    vals = (x, ws[0], ws[1], bb, ws[2], bd, rnd(H) - 2, rnd(H))
+    cots = [rnd(rows, H) for _ in range(3)]
+    ref = [t.double().requires_grad_(True) for t in vals]
+    ro = _gates64(*ref, dtype)
+    rg = torch.autograd.grad(ro, ref, [c.double() for c in cots])
+    got = [t.to(DEV).requires_grad_(True) for t in vals]
+    out = gates(*got, general_gates)
+    cg = [c.to(DEV) for c in cots]
+    g = torch.autograd.grad(out, got, cg, retain_graph=True)
+    again = torch.autograd.grad(out, got, cg)
+    bar = 2 * 2.0 ** -8 if dtype == torch.bfloat16 else 64 * 2.0 ** -24
+    for a, r in zip(out, ro):
+        assert _rel(a.detach(), r.detach()) <= bar
+    for a, b, r, leaf in zip(g, again, rg, vals):
+        assert a.dtype == leaf.dtype and a.shape == r.shape
+        assert torch.equal(a, b)
+        assert _rel(a, r) <= bar
+    rec = torch.autograd.grad(gates(*got, general_gates), got, cg, create_graph=True)
+    assert all(a.requires_grad and _rel(a.detach(), r) <= 2 * bar for a, r in zip(rec, rg))
+
+
+def test_layer_keeps_wrapped_gate_projections():
+    """A hook on a gate projection is called, and a subclass's forward runs."""
+    from cyclic_flow_attention import CyclicFlowAttention
+
+    torch.manual_seed(0)
+    layer = CyclicFlowAttention(hidden_size=256, num_heads=1).to(DEV)
+    x = torch.randn(1, 70, 256, device=DEV, requires_grad=True)
+    y, _ = layer(x)
+    calls = []
+    handle = layer.d_proj.register_forward_hook(lambda *a: calls.append(1))
+    y2, _ = layer(x)
+    handle.remove()
+    assert calls and _rel(y2.detach(), y.detach().double().cpu()) < 1e-5
