@@ -571,8 +571,8 @@ int cyfa_norm_linear_rows(const CyfaLinearArgs* a, const CyfaRowNormArgs* n, voi
 int cyfa_rms_norm(const CyfaNormArgs* a, void* hip_stream) {
     if (!a) return fail(CYFA_ERR_VALUE, "cyfa_rms_norm: null args");
     if (a->rows < 0 || a->D <= 0) return fail(CYFA_ERR_VALUE, "cyfa_rms_norm: rows=%d D=%d", a->rows, a->D);
-    if (a->D % 256 != 0 || a->D > 2048)
-        return fail(CYFA_ERR_UNSUPPORTED, "cyfa_rms_norm: D=%d must be a multiple of 256 up to 2048", a->D);
+    if (a->D % 256 != 0 || a->D > 2048 || (a->D / 256 & (a->D / 256 - 1)) != 0)
+        return fail(CYFA_ERR_UNSUPPORTED, "cyfa_rms_norm: D=%d must be 256, 512, 1024 or 2048", a->D);
     if (!a->x || !a->weight || !a->out || (a->residual && !a->sum_out))
         return fail(CYFA_ERR_VALUE, "cyfa_rms_norm: null required pointer");
     if (!aligned(a->x, 8) || !aligned(a->out, 8) || !aligned(a->weight, 16) || (a->residual && !aligned(a->residual, 8)) ||

@@ -1140,11 +1140,7 @@ int launch_rms_norm(const NormParams& p, hipStream_t stream) {
     switch (p.D / 256) {
         case 1: hipLaunchKernelGGL(rms_norm_kernel<1>, grid, block, 0, stream, p); break;
         case 2: hipLaunchKernelGGL(rms_norm_kernel<2>, grid, block, 0, stream, p); break;
-        case 3: hipLaunchKernelGGL(rms_norm_kernel<3>, grid, block, 0, stream, p); break;
         case 4: hipLaunchKernelGGL(rms_norm_kernel<4>, grid, block, 0, stream, p); break;
-        case 5: hipLaunchKernelGGL(rms_norm_kernel<5>, grid, block, 0, stream, p); break;
-        case 6: hipLaunchKernelGGL(rms_norm_kernel<6>, grid, block, 0, stream, p); break;
-        case 7: hipLaunchKernelGGL(rms_norm_kernel<7>, grid, block, 0, stream, p); break;
         case 8: hipLaunchKernelGGL(rms_norm_kernel<8>, grid, block, 0, stream, p); break;
         default: return -1;
     }

@@ -92,7 +92,7 @@ class RMSNorm(nn.Module):
         o * (num_slots - 1)); ``residual`` first forms s = x + residual and
         returns (s, norm(s))."""
         D = x.shape[-1]
-        if (inference_fast_path(x) and D % 256 == 0 and 256 <= D <= 2048
+        if (inference_fast_path(x) and D % 256 == 0 and D // 256 in (1, 2, 4, 8)
                 and (gate is None or gate.dtype == torch.bfloat16)
                 and (residual is None or residual.dtype == torch.bfloat16)):
             return _native.rms_norm(x, self.weight, self.eps, gate, residual, prescale)

@@ -139,14 +139,9 @@ def test_rms_norm_training_gradients(rows, D, gate, prescale, dtype):
         assert a.requires_grad and _rel(a.detach(), r) <= 2 * bar
 
 
-@pytest.mark.parametrize("D,gate,residual,prescale", [(768, True, True, 1.0), (1280, True, False, 127.0),
-                                                      (1536, False, True, 1.0), (1792, False, False, 1.0)])
-def test_rms_norm_kernel_every_multiple_of_256(D, gate, residual, prescale):
-    import test_gpu_layer
-
-    test_gpu_layer.test_rms_norm_kernel(D, gate, residual, prescale)
-    norm = RMSNorm(D, 1e-6).to(DEV)
-    x = torch.randn(3 * D + 1, device=DEV).bfloat16()[1:].view(3, D)  # rows off the 16-byte grid
+def test_rms_norm_takes_misaligned_rows():
+    norm = RMSNorm(1024, 1e-6).to(DEV)
+    x = torch.randn(3 * 1024 + 1, device=DEV).bfloat16()[1:].view(3, 1024)  # rows off the 16-byte grid
     with torch.no_grad():
         assert torch.equal(norm(x), norm(x.clone()))
 
