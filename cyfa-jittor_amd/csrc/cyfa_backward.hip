@@ -28,10 +28,11 @@
 // table and this workgroup's share of the table cotangent on chip (up to 128
 // slots; above, as tile GEMMs that stream the table); partial sums (table,
 // norm weights, per-tile boundary terms) are added in a fixed order, so the
-// result does not depend on scheduling. With bf16 operands the scans' and
-// chunk kernels' products and the recomputed readout's run on the matrix
-// cores with every fp32 operand split into two bf16 parts (about 16 mantissa
-// bits); with fp32 operands they are fp32 FMA loops, exact to fp32 rounding.
+// result does not depend on scheduling. Every product runs on the matrix
+// cores: with bf16 operands the scans', chunk kernels' and the recomputed
+// readout's with every fp32 operand split into two bf16 parts (about 16
+// mantissa bits); with fp32 operands as fp32 products (v_mfma_f32_16x16x4_f32),
+// exact to fp32 rounding.
 #include <cmath>
 #include <type_traits>
 
@@ -43,6 +44,7 @@ namespace cyfa {
 namespace {
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int BC = 64;           // chunk length of the recompute and the sweeps
 constexpr int BW_MAX_D = 1024;   // largest K and V
@@ -191,10 +193,8 @@ __device__ __forceinline__ f32x4 bf16x4_bits_to_f32x4(uint32_t w0, uint32_t w1) 
                  __builtin_bit_cast(float, w1 << 16), __builtin_bit_cast(float, w1 & 0xffff0000u)};
 }
 
-// The chunk-to-chunk scan of one pass over a [Kq, Vd] matrix X, one
-// SCAN_ROWS x 32 tile per workgroup (grid (ceil(Vd / 32), ceil(Kq /
-// SCAN_ROWS), B*H), 256 threads, each holding SCAN_RPT x 4 elements of X in
-// registers; every element's recurrence is independent of the others):
+// The chunk-to-chunk scan of one pass over a [Kq, Vd] matrix X, one tile per
+// workgroup (every element's recurrence is independent of the others):
 //   X <- e^{G_last} X + sum_t f_t a_t (x) b_t     (a rank-64 update per chunk)
 // Forward (BWD false): the states, n = 0 .. N-1, X_0 = x0 (or zero),
 //   f_t = e^{G_last - G_t}, a = k, b = v; xs[n] = the state before chunk n,
@@ -202,11 +202,8 @@ __device__ __forceinline__ f32x4 bf16x4_bits_to_f32x4(uint32_t w0, uint32_t w1) 
 // Backward (BWD true): the state cotangents, n = N-1 .. 0, X_N = x0 (the
 //   final state's cotangent, or zero), f_t = scale e^{G_t}, a = q, b = dO;
 //   xs[n+1] = the cotangent after chunk n, xs[0] (and x_out) the initial
-//   state's; bnd[tile][n] = the tile's part of <xs[n+1], S[n+1]>.
-// Per chunk the f-scaled rows of a and the columns of b are staged in LDS
-// (two broadcast reads of a and one float4 of b per token feed eight FMAs).
-constexpr int SCAN_ROWS = BWD_SCAN_ROWS;    // rows of a scan tile
-constexpr int SCAN_RPT = SCAN_ROWS / 32;    // rows per thread (8 threads across the 32 columns)
+//   state's; bnd[tile][n] = the 32 x 32 tile's part of <xs[n+1], S[n+1]>.
+constexpr int SCAN_ROWS = BWD_SCAN_ROWS;    // rows of a boundary-term tile
 struct StateScanArgs {
     const float *a, *b;  // head-major [B*H, Tp, Kq] and [B*H, Tp, Vd]
     const float* g;      // [B, T, H]
@@ -221,148 +218,17 @@ struct StateScanArgs {
     int bbf;             // matrix-core form: b holds bf16 (bf16_t) rows
 };
 
-template <bool BWD>
-__global__ __launch_bounds__(256) void bw_state_scan_kernel(StateScanArgs p) {
-    __shared__ float sA[BC][SCAN_ROWS + 4];
-    __shared__ __align__(16) float sB[BC][BW_TILE];
-    __shared__ float sF[BC];
-    __shared__ float sRed[4];
-    __shared__ float sEl;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int c0 = blockIdx.x * BW_TILE, r0 = blockIdx.y * SCAN_ROWS, bhi = blockIdx.z;
-    const int b = bhi / p.H, h = bhi % p.H, tile = blockIdx.y * gridDim.x + blockIdx.x;
-    const int nt = gridDim.x * gridDim.y;
-    const int Kq = p.Kq, Vd = p.Vd, N = p.N;
-    const size_t bh = bhi, ssz = (size_t)Kq * Vd;
-    float* xs = p.xs + bh * (N + 1) * ssz;
-    const float* A = p.a + bh * p.Tp * Kq;
-    const float* Bm = p.b + bh * p.Tp * Vd;
-    // this thread's block: rows r0 + rr .. + SCAN_RPT; columns c0 + cc .. + 3
-    const int rr = SCAN_RPT * (tid >> 3), cc = 4 * (tid & 7);
-    // Every global access below goes through a buffer resource, predicated
-    // through its offset (no branch among the loads); the states per chunk.
-    bool ok[SCAN_RPT][4];
-    uint32_t off[SCAN_RPT][4];  // byte offset of this thread's elements in a [Kq, Vd] state
-    float x[SCAN_RPT][4];
-    const bw_rsrc_t rx0 = bw_rsrc(p.x0 ? p.x0 + bh * ssz : nullptr, p.x0 ? ssz : 0);
-#pragma unroll
-    for (int i = 0; i < SCAN_RPT; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            ok[i][j] = r0 + rr + i < Kq && c0 + cc + j < Vd;
-            off[i][j] = ((uint32_t)(r0 + rr + i) * (uint32_t)Vd + (uint32_t)(c0 + cc + j)) * 4u;
-            x[i][j] = bw_load(rx0, off[i][j], ok[i][j]);  // zero without x0 (empty buffer)
-        }
-    // backward: the forward state S[n] of this thread's block, loaded a chunk
-    // ahead (with the rows and columns below) for the boundary term <X, S[n]>
-    float sv[SCAN_RPT][4] = {};
-    const auto fetch_state = [&](int n) {
-        const bw_rsrc_t rs = bw_rsrc(p.S + (bh * (N + 1) + n) * ssz, ssz);
-#pragma unroll
-        for (int i = 0; i < SCAN_RPT; i++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) sv[i][j] = bw_load(rs, off[i][j], ok[i][j]);
-    };
-    const auto keep = [&](int n) {  // xs[n] = X; returns the block's part of <X, S[n]> (backward)
-        const bw_rsrc_t rs = bw_rsrc(xs + (size_t)n * ssz, ssz);
-        float dot = 0.f;
-#pragma unroll
-        for (int i = 0; i < SCAN_RPT; i++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                bw_store(rs, off[i][j], ok[i][j], x[i][j]);
-                if constexpr (BWD) dot = fmaf(x[i][j], sv[i][j], dot);  // sv is zero where !ok
-            }
-        return dot;
-    };
-    // The next chunk's rows of a, columns of b and gate are loaded into
-    // registers while the current chunk's FMAs run.
-    constexpr int NA = BC * SCAN_ROWS / 256, NB = BC * BW_TILE / 256;
-    float ra[NA], rb[NB], rg = 0.f;
-    // (the host keeps B T H below 2^21: the gate's offsets fit 32 bits)
-    const bw_rsrc_t rgt = bw_rsrc(p.g, (size_t)p.B * p.T * p.H);
-    const auto fetch = [&](int n) {
-        const int t0 = n * BC;
-        const bw_rsrc_t rA = bw_rsrc(A + (size_t)t0 * Kq, (size_t)BC * Kq), rBm = bw_rsrc(Bm + (size_t)t0 * Vd, (size_t)BC * Vd);
-#pragma unroll
-        for (int i = 0; i < NA; i++) {
-            const int e = tid + 256 * i, t = e / SCAN_ROWS, r = e % SCAN_ROWS;
-            ra[i] = bw_load(rA, ((uint32_t)t * (uint32_t)Kq + (uint32_t)(r0 + r)) * 4u, r0 + r < Kq);
-        }
-#pragma unroll
-        for (int i = 0; i < NB; i++) {
-            const int e = tid + 256 * i, t = e / BW_TILE, c = e % BW_TILE;
-            rb[i] = bw_load(rBm, ((uint32_t)t * (uint32_t)Vd + (uint32_t)(c0 + c)) * 4u, c0 + c < Vd);
-        }
-        // (every wave loads the gate; wave 0 uses it)
-        rg = bw_load(rgt, (((uint32_t)b * (uint32_t)p.T + (uint32_t)(t0 + lane)) * (uint32_t)p.H + (uint32_t)h) * 4u,
-                     t0 + lane < p.T);
-    };
-    fetch(BWD ? N - 1 : 0);
-    if constexpr (BWD) fetch_state(N);
-    for (int step = 0; step < N; step++) {
-        const int n = BWD ? N - 1 - step : step;
-        const float dot = keep(BWD ? n + 1 : n);
-        __syncthreads();  // the previous chunk's tiles are done with
-        if constexpr (BWD) {
-            const float wsum = bw_wave_sum(dot);
-            if (lane == 0) sRed[wv] = wsum;
-        }
-        if (wv == 0) {  // G: the in-chunk inclusive cumsum of the prefetched gate
-            const float G = bw_wave_scan(rg);
-            const float Gl = lane_value(G, 63);
-            sF[lane] = BWD ? p.scale * expf(G) : expf(Gl - G);
-            if (lane == 0) sEl = expf(Gl);
-        }
-#pragma unroll
-        for (int i = 0; i < NB; i++) {
-            const int e = tid + 256 * i;
-            sB[e / BW_TILE][e % BW_TILE] = rb[i];
-        }
-        __syncthreads();  // sF is read below
-#pragma unroll
-        for (int i = 0; i < NA; i++) {
-            const int e = tid + 256 * i, t = e / SCAN_ROWS;
-            sA[t][e % SCAN_ROWS] = sF[t] * ra[i];
-        }
-        __syncthreads();
-        if (step + 1 < N) fetch(BWD ? n - 1 : n + 1);
-        if constexpr (BWD) fetch_state(n);  // for the next step's keep(n)
-        if constexpr (BWD) {
-            if (tid == 0) p.bnd[(bh * nt + tile) * N + n] = (sRed[0] + sRed[1]) + (sRed[2] + sRed[3]);
-        }
-        float acc[SCAN_RPT][4] = {};
-        for (int t = 0; t < BC; t++) {
-            const float4 bv = *reinterpret_cast<const float4*>(&sB[t][cc]);
-#pragma unroll
-            for (int i = 0; i < SCAN_RPT; i++) {
-                const float av = sA[t][rr + i];
-                acc[i][0] = fmaf(av, bv.x, acc[i][0]);
-                acc[i][1] = fmaf(av, bv.y, acc[i][1]);
-                acc[i][2] = fmaf(av, bv.z, acc[i][2]);
-                acc[i][3] = fmaf(av, bv.w, acc[i][3]);
-            }
-        }
-        const float el = sEl;
-#pragma unroll
-        for (int i = 0; i < SCAN_RPT; i++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) x[i][j] = fmaf(el, x[i][j], acc[i][j]);
-    }
-    keep(BWD ? 0 : N);
-    const bw_rsrc_t rxo = bw_rsrc(p.x_out ? p.x_out + bh * ssz : nullptr, p.x_out ? ssz : 0);
-#pragma unroll
-    for (int i = 0; i < SCAN_RPT; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) bw_store(rxo, off[i][j], ok[i][j], x[i][j]);  // dropped without x_out
-}
-
-// The same scan for bf16 operands on the matrix cores: the rank-64 update
-// X += A^T B over the chunk's 64 tokens as split-bf16 products on
-// v_mfma_f32_16x16x32_bf16 (each fp32 operand as a bf16 high part and a bf16
-// remainder, lo_a hi_b + hi_a lo_b + hi_a hi_b: about 16 mantissa bits, as in
-// the chunk kernels' tile GEMMs). A workgroup takes a 32 T2 x 32 T2 tile,
-// wave w its 16 T2 x 16 T2 quarter (w >> 1, w & 1) as T2 x T2 accumulator
+// The rank-64 update X += A^T B over the chunk's 64 tokens runs on the matrix
+// cores. bf16 operands: split-bf16 products on v_mfma_f32_16x16x32_bf16 (each
+// fp32 operand as a bf16 high part and a bf16 remainder, lo_a hi_b + hi_a lo_b
+// + hi_a hi_b: about 16 mantissa bits, as in the chunk kernels' tile GEMMs).
+// fp32 operands (F32): fp32 products on v_mfma_f32_16x16x4_f32, lane (lr, lg)
+// holding tokens 8 lg .. + 7 of a 32-token step as its k of eight steps. (As
+// fp32 FMA loops, one 4-byte LDS read of a per row and token, the scan of a
+// 256 x 128 state over 16 chunks of 8 (b, h) took 50 us forward and 35 backward;
+// here 18 and 20.)
+// A workgroup takes a 32 T2 x 32 T2 tile, wave w its 16 T2 x 16 T2 quarter (w
+// >> 1, w & 1) as T2 x T2 accumulator
 // blocks: lane (lr, lg) of block (ib, jb) has rows 16 T2 (w >> 1) + 16 ib +
 // 4 lg + i, column 16 T2 (w & 1) + 16 jb + lr. The larger tile reads each
 // chunk's rows of a and b from fewer workgroups (the scans are bound by those
@@ -370,10 +236,11 @@ __global__ __launch_bounds__(256) void bw_state_scan_kernel(StateScanArgs p) {
 // columns of b). Per chunk, thread (r, q) = (tid % 32 T2, tid / 32 T2) loads
 // tokens 8 T2 q .. + 8 T2 of row r of a and of column r of b and stages them
 // transposed (row = state coordinate, 64 tokens along the row), so that every
-// operand fragment is one 16-byte LDS read. The boundary terms go to bnd per
-// 32 x 32 tile, as the FMA form's: with T2 = 2 one per wave, with T2 = 1 one
+// operand fragment is consecutive in LDS. The boundary terms go to bnd per
+// 32 x 32 tile: with T2 = 2 one per pair of waves, with T2 = 1 one
 // per workgroup.
 constexpr int SCAN_LDT = BC + 8;  // staged row: 64 tokens + 8 of padding (bf16)
+constexpr int SCAN_LDF = BC + 4;  // the same in fp32
 
 __device__ __forceinline__ void split_bf16x8(const float* v, bf16x8& hi, bf16x8& lo) {
 #pragma unroll
@@ -383,8 +250,28 @@ __device__ __forceinline__ void split_bf16x8(const float* v, bf16x8& hi, bf16x8&
     }
 }
 
-template <bool BWD, int T2, bool SB, bool BB>
+// v_mfma_f32_16x16x4_f32 (fp32 operands, fp32 accumulation): lane l holds
+// A[l % 16][l / 16] and B[l / 16][l % 16] of a 16 x 4 by 4 x 16 step and rows
+// 4 (l / 16) .. + 3 of column l % 16 of the 16 x 16 result.
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// c += A B^T over 32 k of fp32 rows: a and b point at this lane's eight
+// consecutive k (k = 8 (lane / 16) ..) of its row of A and of B.
+__device__ __forceinline__ f32x4 mfma_f32x8(const float* a, const float* b, f32x4 c) {
+    const f32x4 a0 = *reinterpret_cast<const f32x4*>(a), a1 = *reinterpret_cast<const f32x4*>(a + 4);
+    const f32x4 b0 = *reinterpret_cast<const f32x4*>(b), b1 = *reinterpret_cast<const f32x4*>(b + 4);
+#pragma unroll
+    for (int e = 0; e < 4; e++) c = mfma4(a0[e], b0[e], c);
+#pragma unroll
+    for (int e = 0; e < 4; e++) c = mfma4(a1[e], b1[e], c);
+    return c;
+}
+
+template <bool BWD, int T2, bool SB, bool BB, bool F32 = false>
 __global__ __launch_bounds__(T2 == 2 ? 512 : 256) void bw_state_scan_mf_kernel(StateScanArgs p) {
+    static_assert(!F32 || (!SB && !BB), "fp32 operands, fp32 states");
     using SE = std::conditional_t<SB, bf16_t, float>;  // the stored states' element
     using BE = std::conditional_t<BB, bf16_t, float>;  // b's element
     static_assert(SCAN_ROWS == 32 && BW_TILE == 32 && (T2 == 1 || T2 == 2), "32 x 32 bnd tiles");
@@ -394,8 +281,9 @@ __global__ __launch_bounds__(T2 == 2 ? 512 : 256) void bw_state_scan_mf_kernel(S
     // the 16 x 16 T2 block of rows 16 (w / 2) and columns 16 T2 (w % 2).
     constexpr int NTH = T2 == 2 ? 512 : 256, NWV = NTH / 64, IB = 1;
     constexpr int TPT = BC / (NTH / TS);  // tokens per staging thread
-    __shared__ __align__(16) bf16_t sAh[TS][SCAN_LDT], sAl[TS][SCAN_LDT];
-    __shared__ __align__(16) bf16_t sBh[TS][SCAN_LDT], sBl[TS][SCAN_LDT];
+    __shared__ __align__(16) bf16_t sAh[F32 ? 1 : TS][SCAN_LDT], sAl[F32 ? 1 : TS][SCAN_LDT];
+    __shared__ __align__(16) bf16_t sBh[F32 ? 1 : TS][SCAN_LDT], sBl[F32 ? 1 : TS][SCAN_LDT];
+    __shared__ __align__(16) float sAf[F32 ? TS : 1][SCAN_LDF], sBf[F32 ? TS : 1][SCAN_LDF];
     __shared__ float sF[BC];
     __shared__ float sRed[NWV];
     __shared__ float sEl;
@@ -497,6 +385,12 @@ __global__ __launch_bounds__(T2 == 2 ? 512 : 256) void bw_state_scan_mf_kernel(S
         }
 #pragma unroll
         for (int u = 0; u < TPT / 8; u++) {
+            if constexpr (F32) {
+                float* d = &sBf[sr][TPT * sq + 8 * u];
+                *reinterpret_cast<f32x4*>(d) = f32x4{rb[8 * u], rb[8 * u + 1], rb[8 * u + 2], rb[8 * u + 3]};
+                *reinterpret_cast<f32x4*>(d + 4) = f32x4{rb[8 * u + 4], rb[8 * u + 5], rb[8 * u + 6], rb[8 * u + 7]};
+                continue;
+            }
             bf16x8 hi, lo;
             split_bf16x8(rb + 8 * u, hi, lo);
             *reinterpret_cast<bf16x8*>(&sBh[sr][TPT * sq + 8 * u]) = hi;
@@ -508,6 +402,12 @@ __global__ __launch_bounds__(T2 == 2 ? 512 : 256) void bw_state_scan_mf_kernel(S
             float fa[8];
 #pragma unroll
             for (int i = 0; i < 8; i++) fa[i] = sF[TPT * sq + 8 * u + i] * ra[8 * u + i];
+            if constexpr (F32) {
+                float* d = &sAf[sr][TPT * sq + 8 * u];
+                *reinterpret_cast<f32x4*>(d) = f32x4{fa[0], fa[1], fa[2], fa[3]};
+                *reinterpret_cast<f32x4*>(d + 4) = f32x4{fa[4], fa[5], fa[6], fa[7]};
+                continue;
+            }
             bf16x8 hi, lo;
             split_bf16x8(fa, hi, lo);
             *reinterpret_cast<bf16x8*>(&sAh[sr][TPT * sq + 8 * u]) = hi;
@@ -531,6 +431,15 @@ __global__ __launch_bounds__(T2 == 2 ? 512 : 256) void bw_state_scan_mf_kernel(S
                 for (int i = 0; i < 4; i++) x[ib][jb][i] *= el;
 #pragma unroll
         for (int s = 0; s < BC / 32; s++) {
+            if constexpr (F32) {
+#pragma unroll
+                for (int ib = 0; ib < IB; ib++)
+#pragma unroll
+                    for (int jb = 0; jb < T2; jb++)
+                        x[ib][jb] = mfma_f32x8(&sAf[wr + 16 * ib + lr][32 * s + 8 * lg], &sBf[wc + 16 * jb + lr][32 * s + 8 * lg],
+                                               x[ib][jb]);
+                continue;
+            }
             bf16x8 ah[IB], al[IB], bh8[T2], bl8[T2];
 #pragma unroll
             for (int ib = 0; ib < IB; ib++) {
@@ -566,13 +475,15 @@ __global__ __launch_bounds__(T2 == 2 ? 512 : 256) void bw_state_scan_mf_kernel(S
             for (int i = 0; i < 4; i++) bw_store(rxo, off[ib][jb][i], ok[ib][jb][i], x[ib][jb][i]);  // dropped without x_out
 }
 
-// Launches the scan over a [Kq, Vd] state (grid: the FMA form's 32 x 32
-// tiles): the matrix-core form for bf16 operands, with 64 x 64 tiles when
-// they still give a workgroup per compute unit.
+// Launches the scan over a [Kq, Vd] state, with split-bf16 products (mfma) or
+// fp32 ones, in 64 x 64 tiles when they still give a workgroup per compute
+// unit, else in 32 x 32 tiles.
 template <bool BWD, int T2>
-void launch_scan_mf(const StateScanArgs& a, dim3 grid, hipStream_t stream) {
+void launch_scan_mf(const StateScanArgs& a, bool mfma, dim3 grid, hipStream_t stream) {
     const dim3 blk(T2 == 2 ? 512 : 256);
-    if (a.sbf && a.bbf)
+    if (!mfma)
+        hipLaunchKernelGGL((bw_state_scan_mf_kernel<BWD, T2, false, false, true>), grid, blk, 0, stream, a);
+    else if (a.sbf && a.bbf)
         hipLaunchKernelGGL((bw_state_scan_mf_kernel<BWD, T2, true, true>), grid, blk, 0, stream, a);
     else if (a.sbf)
         hipLaunchKernelGGL((bw_state_scan_mf_kernel<BWD, T2, true, false>), grid, blk, 0, stream, a);
@@ -585,51 +496,49 @@ void launch_scan_mf(const StateScanArgs& a, dim3 grid, hipStream_t stream) {
 template <bool BWD>
 void launch_state_scan(const StateScanArgs& a, bool mfma, hipStream_t stream) {
     const dim3 g32((a.Vd + 31) / 32, (a.Kq + 31) / 32, a.B * a.H), g64((a.Vd + 63) / 64, (a.Kq + 63) / 64, a.B * a.H);
-    if (!mfma)
-        hipLaunchKernelGGL(bw_state_scan_kernel<BWD>, g32, dim3(256), 0, stream, a);
-    else if ((long long)g64.x * g64.y * g64.z >= device_cu_count())
-        launch_scan_mf<BWD, 2>(a, g64, stream);
+    if ((long long)g64.x * g64.y * g64.z >= device_cu_count())
+        launch_scan_mf<BWD, 2>(a, mfma, g64, stream);
     else
-        launch_scan_mf<BWD, 1>(a, g32, stream);
+        launch_scan_mf<BWD, 1>(a, mfma, g32, stream);
 }
 
-// Tile GEMMs of the chunk kernels: a 64 x 64 output tile (rows = the chunk's
-// tokens, columns = 64 coordinates), acc[a][b] per thread at (TileMap<MF>::row,
-// TileMap<MF>::col), accumulated over a contraction of Kd in k-blocks of 32
-// staged through LDS, the next k-block's operands prefetched into registers
-// while the current one is multiplied. fa(i, kk) and fb(kk, j) read the
-// operands; B_KCONTIG says whether fb is contiguous along kk (else along j).
-//  - MF false (fp32 operands): fp32 FMA, a 4 x 4 block per thread (rows
-//    4 (tid / 16) .., columns 4 (tid % 16) ..), A staged transposed so a
-//    thread's four rows are one float4.
+// Tile GEMMs of the chunk kernels: a 64 x 64 NT output tile (rows = the chunk's
+// tokens, columns = coordinates), accumulated over a contraction of Kd in
+// k-blocks of 32 staged through LDS, the next k-block's operands prefetched
+// into registers while the current one is multiplied. fa(i, kk) and fb(kk, j)
+// read the operands. Wave w forms rows 16 w .. + 16 as 4 NT blocks of 16 x 16:
+// acc[nb][i] = tile[16 w + 4 (lane / 16) + i][16 nb + lane % 16] (TileMap).
 //  - MF true (bf16 operands): matrix cores at near-fp32 accuracy: each fp32
 //    operand is split into hi = bf16(x) and lo = bf16(x - hi), staged in LDS,
 //    and a.b formed as lo_a hi_b + hi_a lo_b + hi_a hi_b on
 //    v_mfma_f32_16x16x32_bf16 with fp32 accumulation (about 16 mantissa
-//    bits; the dropped lo_a lo_b is 2^-16 relative): wave w forms rows 16 w
-//    .. + 16 as four 16 x 16 blocks, acc[nb][i] = tile[16 w + 4 (lane / 16) +
-//    i][16 nb + lane % 16]. The kernels are bound by the staging, not the
-//    matrix cores, so the three products cost about what one does.
-constexpr int GT_K = 32, GT_LD = 68;  // fp32 staging: [32][68] per operand
-constexpr int MT_LD = 40;             // bf16 staging: [64][40] per operand (32 k + 8 pad)
-constexpr int STAGE_BYTES = 4 * BC * MT_LD * 2;  // >= the fp32 staging's 2 * GT_K * GT_LD * 4
-constexpr int STAGE2_BYTES = 6 * BC * MT_LD * 2;  // tile_gemm_mf<2>: A and two B blocks, hi and lo
-static_assert(STAGE_BYTES >= 2 * GT_K * GT_LD * 4, "staging must hold either form");
+//    bits; the dropped lo_a lo_b is 2^-16 relative). The kernels are bound by
+//    the staging, not the matrix cores, so the three products cost about what
+//    one does.
+//  - MF false (fp32 operands): fp32 products and sums on
+//    v_mfma_f32_16x16x4_f32, the operands staged as fp32. (As fp32 FMA loops, a
+//    4 x 4 block per thread with 4-byte operand loads, the chunk kernel took
+//    181 us for 128 chunks of 256 x 128 and the output kernel 88; here, with
+//    the chunk's tiles shared out over three and two workgroups, 48 and 24.)
+// The wide readout's GEMMs (128 < M) keep fp32 FMA in a 4 x 4 block per thread
+// (tile_gemm_fma), whose threads hold neighbouring columns.
+constexpr int GT_K = 32, GT_LD = 68;  // FMA staging: [32][68] per operand
+constexpr int MT_LD = 40;             // bf16 staging: [64][40] per operand part (32 k + 8 pad)
+constexpr int FT_LD = 36;             // fp32 staging: [64][36] per operand
+constexpr int STAGE_BYTES = 4 * BC * MT_LD * 2;   // A and a B block, hi and lo
+constexpr int STAGE2_BYTES = 6 * BC * MT_LD * 2;  // the same with two B blocks
+static_assert(STAGE_BYTES >= 2 * GT_K * GT_LD * 4 && STAGE_BYTES >= 2 * BC * FT_LD * 4 &&
+                  STAGE2_BYTES >= 3 * BC * FT_LD * 4,
+              "staging must hold every form");
 
-template <bool MF>
 struct TileMap {
-    __device__ static int row(int a, int b) {
-        if constexpr (MF)
-            return 16 * (threadIdx.x >> 6) + 4 * ((threadIdx.x & 63) >> 4) + b;
-        else
-            return 4 * (threadIdx.x >> 4) + a;
-    }
-    __device__ static int col(int a, int b) {
-        if constexpr (MF)
-            return 16 * a + (threadIdx.x & 15);
-        else
-            return 4 * (threadIdx.x & 15) + b;
-    }
+    __device__ static int row(int, int b) { return 16 * (threadIdx.x >> 6) + 4 * ((threadIdx.x & 63) >> 4) + b; }
+    __device__ static int col(int a, int) { return 16 * a + (threadIdx.x & 15); }
+};
+
+struct FmaMap {
+    __device__ static int row(int a, int) { return 4 * (threadIdx.x >> 4) + a; }
+    __device__ static int col(int, int b) { return 4 * (threadIdx.x & 15) + b; }
 };
 
 // Global operands of tile_gemm, read through a buffer resource over the
@@ -762,16 +671,17 @@ __device__ __forceinline__ float opB(const FB& fb, int kk, int j, int Kd) {
         return kk < Kd ? fb(kk, j) : 0.f;
 }
 
-// The matrix-core form of tile_gemm (above) for an output of 64 rows by
-// 64 NT columns in one pass over the contraction: A is staged once per
+// tile_gemm (above) for an output of 64 rows by 64 NT columns in one pass over
+// the contraction: A is staged once per
 // k-block and multiplied against NT B tiles, so that a row block feeding
 // several output tiles is read once (NT = 2 halves those reads against two
-// passes). acc[nb][i] = tile[16 w + 4 (lane / 16) + i][16 nb + lane % 16],
-// nb < 4 NT; the staging area holds (2 + 2 NT) 64-row blocks.
-template <int NT, class FA, class FB>
-__device__ __forceinline__ void tile_gemm_mf(FA fa, FB fb, int Kd, unsigned char* stage, float acc[4 * NT][4]) {
+// passes).
+template <bool MF, int NT, class FA, class FB>
+__device__ __forceinline__ void tile_gemm(FA fa, FB fb, int Kd, unsigned char* stage, float acc[4 * NT][4]) {
     const int tid = threadIdx.x;
     {
+        float* saf = reinterpret_cast<float*>(stage);  // fp32: A (64 rows), then B (64 NT rows)
+        float* sbf = saf + BC * FT_LD;
         bf16_t* sah = reinterpret_cast<bf16_t*>(stage);  // hi and lo parts of A (64 rows) and of B (64 NT rows)
         bf16_t* sal = sah + BC * MT_LD;
         bf16_t* sbh = sal + BC * MT_LD;
@@ -818,9 +728,38 @@ __device__ __forceinline__ void tile_gemm_mf(FA fa, FB fb, int Kd, unsigned char
                 *reinterpret_cast<bf16x8*>(base + r * MT_LD + 8 * kg) = v;
             }
         };
+        const auto put_f = [&](float* base, bool split4, const float* v) {
+            const int c0 = split4 ? 4 * kg : 8 * kg, c1 = split4 ? 16 + 4 * kg : 8 * kg + 4;
+            *reinterpret_cast<f32x4*>(base + r * FT_LD + c0) = f32x4{v[0], v[1], v[2], v[3]};
+            *reinterpret_cast<f32x4*>(base + r * FT_LD + c1) = f32x4{v[4], v[5], v[6], v[7]};
+        };
         fetch(0);
         for (int k0 = 0; k0 < Kd; k0 += GT_K) {
             __syncthreads();  // the staging tiles are free
+            if constexpr (!MF) {
+                put_f(saf, VA, ra);
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++) {
+                    float* b0 = sbf + 64 * nt * FT_LD;
+                    if constexpr (JB) {
+#pragma unroll
+                        for (int c = 0; c < 4; c++)
+                            *reinterpret_cast<f32x2*>(b0 + (4 * jq + c) * FT_LD + 2 * kp) = f32x2{rb[nt][c], rb[nt][4 + c]};
+                    } else {
+                        put_f(b0, VB, rb[nt]);
+                    }
+                }
+                __syncthreads();
+                if (k0 + GT_K < Kd) fetch(k0 + GT_K);
+#pragma unroll
+                for (int nb = 0; nb < 4 * NT; nb++) {
+                    f32x4 c = {acc[nb][0], acc[nb][1], acc[nb][2], acc[nb][3]};
+                    c = mfma_f32x8(saf + (16 * w + lr) * FT_LD + 8 * lg, sbf + (16 * nb + lr) * FT_LD + 8 * lg, c);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) acc[nb][i] = c[i];
+                }
+                continue;
+            }
             bf16x8 vah, val;
 #pragma unroll
             for (int x = 0; x < 8; x++) {
@@ -871,12 +810,13 @@ __device__ __forceinline__ void tile_gemm_mf(FA fa, FB fb, int Kd, unsigned char
     }
 }
 
-template <bool MF, bool B_KCONTIG, class FA, class FB>
-__device__ __forceinline__ void tile_gemm(FA fa, FB fb, int Kd, unsigned char* stage, float acc[4][4]) {
-    static_assert(!std::is_base_of_v<RowsK, FB> || B_KCONTIG, "RowsK: B contiguous along kk");
-    static_assert(!std::is_base_of_v<RowsJ, FB> || !B_KCONTIG, "RowsJ: B contiguous along j");
+// The FMA form: B_KCONTIG says whether fb is contiguous along kk (else along
+// j); acc[a][b] at (FmaMap::row, FmaMap::col); A staged transposed so a
+// thread's four rows are one float4.
+template <bool B_KCONTIG, class FA, class FB>
+__device__ __forceinline__ void tile_gemm_fma(FA fa, FB fb, int Kd, unsigned char* stage, float acc[4][4]) {
     const int tid = threadIdx.x;
-    if constexpr (!MF) {
+    {
         float(*sa)[GT_LD] = reinterpret_cast<float(*)[GT_LD]>(stage);
         float(*sb)[GT_LD] = reinterpret_cast<float(*)[GT_LD]>(stage + GT_K * GT_LD * 4);
         constexpr int NE = BC * GT_K / 256;  // staged elements of each operand per thread
@@ -917,43 +857,29 @@ __device__ __forceinline__ void tile_gemm(FA fa, FB fb, int Kd, unsigned char* s
                     for (int j = 0; j < 4; j++) acc[i][j] = fmaf(ar[i], br[j], acc[i][j]);
             }
         }
-    } else {
-        tile_gemm_mf<1>(fa, fb, Kd, stage, acc);
     }
 }
 
-// acc[a][b] *= f(row of (a, b)); NA = 4 NT for a matrix-core tile of 64 NT
-// columns.
-template <bool MF, int NA = 4, class F>
+// acc[a][b] *= f(row of (a, b)); NA = 4 NT for a tile of 64 NT columns.
+template <int NA, class F>
 __device__ __forceinline__ void tile_scale_rows(float acc[NA][4], F f) {
 #pragma unroll
     for (int a = 0; a < NA; a++)
 #pragma unroll
-        for (int b = 0; b < 4; b++) acc[a][b] *= f(TileMap<MF>::row(a, b));
+        for (int b = 0; b < 4; b++) acc[a][b] *= f(TileMap::row(a, b));
 }
 
 // Writes this thread's part of a 64 x 16 NA tile (columns d0 ..) into
 // head-major rows dst [.., D], times a scale.
-template <bool MF, int NA = 4>
+template <int NA>
 __device__ __forceinline__ void tile_store(float acc[NA][4], float* dst, int D, int d0, float scale) {
 #pragma unroll
     for (int a = 0; a < NA; a++)
 #pragma unroll
         for (int b = 0; b < 4; b++) {
-            const int t = TileMap<MF>::row(a, b), c = d0 + TileMap<MF>::col(a, b);
+            const int t = TileMap::row(a, b), c = d0 + TileMap::col(a, b);
             if (c < D) dst[(size_t)t * D + c] = scale * acc[a][b];
         }
-}
-
-// tile_gemm over 64 NT output columns: NT = 2 only on the matrix cores.
-template <bool MF, bool B_KCONTIG, int NT, class FA, class FB>
-__device__ __forceinline__ void tile_gemm_nt(FA fa, FB fb, int Kd, unsigned char* stage, float acc[4 * NT][4]) {
-    if constexpr (NT == 1) {
-        tile_gemm<MF, B_KCONTIG>(fa, fb, Kd, stage, acc);
-    } else {
-        static_assert(MF && NT == 2, "wide tiles on the matrix cores");
-        tile_gemm_mf<NT>(fa, fb, Kd, stage, acc);
-    }
 }
 
 // Masked, decayed scores of one chunk into P: P[t][s] = [s <= t] e^{G_t - G_s}
@@ -963,12 +889,12 @@ __device__ __forceinline__ void chunk_scores(const E* X, const E* Y, int D, cons
                                              float (*P)[BC + 1]) {
     using RK = StateRowsK<std::is_same_v<E, bf16_t>, V4>;  // fp32 or bf16 rows
     float acc[4][4] = {};
-    tile_gemm<MF, true>(RK(X, D, BC, D), RK(Y, D, BC, D), D, stage, acc);
+    tile_gemm<MF, 1>(RK(X, D, BC, D), RK(Y, D, BC, D), D, stage, acc);
 #pragma unroll
     for (int a = 0; a < 4; a++)
 #pragma unroll
         for (int b = 0; b < 4; b++) {
-            const int t = TileMap<MF>::row(a, b), s = TileMap<MF>::col(a, b);
+            const int t = TileMap::row(a, b), s = TileMap::col(a, b);
             P[t][s] = s <= t ? acc[a][b] * expf(sG[t] - sG[s]) : 0.f;
         }
 }
@@ -987,7 +913,8 @@ struct OutArgs {
     int bf16;                // round to bf16
     int B, T, Tp, H, Kq, Vd, N;
     float scale;
-    int sbf;                 // matrix-core form: S holds bf16 states
+    int sbf;                 // S holds bf16 states
+    int parts;               // workgroups per chunk: part i forms output tiles i, i + parts, ..
 };
 
 template <bool MF, bool V4, bool SB>
@@ -1002,7 +929,7 @@ __global__ __launch_bounds__(256) void bw_out_kernel(OutArgs a) {
     constexpr int NT = 1, NA = 4 * NT;
     __shared__ __align__(16) unsigned char sStage[NT == 2 ? STAGE2_BYTES : STAGE_BYTES];
     __shared__ float sG[BC], sEq[BC];
-    const int tid = threadIdx.x, n = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+    const int tid = threadIdx.x, n = blockIdx.x, h = blockIdx.y, b = blockIdx.z / a.parts, part = blockIdx.z % a.parts;
     const int Kq = a.Kq, Vd = a.Vd, t0 = n * BC;
     const size_t bh = (size_t)b * a.H + h, ssz = (size_t)Kq * Vd;
     const float* q = a.q + (bh * a.Tp + t0) * Kq;
@@ -1015,11 +942,11 @@ __global__ __launch_bounds__(256) void bw_out_kernel(OutArgs a) {
     }
     chunk_scores<MF, V4>(q, k, Kq, sG, sStage, sA);
     float* out = a.out + (bh * a.Tp + t0) * Vd;
-    for (int d0 = 0; d0 < Vd; d0 += BC * NT) {
+    for (int d0 = BC * NT * part; d0 < Vd; d0 += BC * NT * a.parts) {
         float acc[NA][4] = {};
-        tile_gemm_nt<MF, false, NT>(RK(q, Kq, BC, Kq), SJ(S + d0, Vd, Kq, Vd - d0), Kq, sStage, acc);
-        tile_scale_rows<MF, NA>(acc, [&](int t) { return sEq[t]; });
-        tile_gemm_nt<MF, false, NT>([&](int i, int kk) { return sA[i][kk]; }, RJ(v + d0, Vd, BC, Vd - d0), BC,
+        tile_gemm<MF, NT>(RK(q, Kq, BC, Kq), SJ(S + d0, Vd, Kq, Vd - d0), Kq, sStage, acc);
+        tile_scale_rows<NA>(acc, [&](int t) { return sEq[t]; });
+        tile_gemm<MF, NT>([&](int i, int kk) { return sA[i][kk]; }, RJ(v + d0, Vd, BC, Vd - d0), BC,
                                     sStage, acc);
         if (!a.out_bthd) {
             if (a.bf16) {
@@ -1027,9 +954,9 @@ __global__ __launch_bounds__(256) void bw_out_kernel(OutArgs a) {
                 for (int i = 0; i < NA; i++)
 #pragma unroll
                     for (int j = 0; j < 4; j++) acc[i][j] = (float)(bf16_t)(a.scale * acc[i][j]);
-                tile_store<MF, NA>(acc, out, Vd, d0, 1.f);
+                tile_store<NA>(acc, out, Vd, d0, 1.f);
             } else {
-                tile_store<MF, NA>(acc, out, Vd, d0, a.scale);
+                tile_store<NA>(acc, out, Vd, d0, a.scale);
             }
             continue;
         }
@@ -1037,7 +964,7 @@ __global__ __launch_bounds__(256) void bw_out_kernel(OutArgs a) {
         for (int i = 0; i < NA; i++)
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const int t = t0 + TileMap<MF>::row(i, j), c = d0 + TileMap<MF>::col(i, j);
+                const int t = t0 + TileMap::row(i, j), c = d0 + TileMap::col(i, j);
                 if (c >= Vd || t >= a.T) continue;
                 const size_t e = (((size_t)b * a.T + t) * a.H + h) * Vd + c;
                 if (a.bf16)
@@ -1059,11 +986,12 @@ struct ChunkGradArgs {
     float *dq, *dk, *dv;          // head-major
     int B, T, Tp, H, Kq, Vd, N;
     float scale;
-    int sbf;                      // matrix-core form: S and D hold bf16 states
-    int rbf;                      // matrix-core form: v and dO hold bf16 rows
+    int sbf;                      // S and D hold bf16 states
+    int rbf;                      // v and dO hold bf16 rows
+    int parts;                    // workgroups per chunk (chunk_parts)
 };
 
-template <bool MF, bool V4, bool SB, bool RB>
+template <bool MF, bool V4, bool SB, bool RB, int NT>
 __global__ __launch_bounds__(256) void bw_chunk_kernel(ChunkGradArgs a) {
     using RK = std::conditional_t<V4, RowsK4, RowsK>;  // 16-byte row loads when aligned
     using RJ = std::conditional_t<V4, RowsJ4, RowsJ>;
@@ -1074,15 +1002,14 @@ __global__ __launch_bounds__(256) void bw_chunk_kernel(ChunkGradArgs a) {
     using VJ = StateRowsJ<RB, V4>;
     using VE = std::conditional_t<RB, bf16_t, float>;
     __shared__ float sA[BC][BC + 1], sB[BC][BC + 1];
-    // Output tiles of 64 NT columns: on the matrix cores two at a time, so that
-    // each row block a product reads (dO, v, k, and the other operands' rows)
-    // is read once per pair of tiles (the kernel reads HBM at its rate: 222 ->
-    // 184 us at configuration 3)
-    constexpr int NT = MF && V4 ? 2 : 1, NA = 4 * NT;
+    // Output tiles of 64 NT columns: with NT = 2 each row block a product reads
+    // (dO, v, k, and the other operands' rows) is read once per pair of tiles
+    // (the kernel reads HBM at its rate: 222 -> 184 us at configuration 3)
+    constexpr int NA = 4 * NT;
     __shared__ __align__(16) unsigned char sStage[NT == 2 ? STAGE2_BYTES : STAGE_BYTES];
     // (the row factors e^{G_t} and e^{G_last - G_t} are formed where used)
     __shared__ float sG[BC];
-    const int tid = threadIdx.x, n = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+    const int tid = threadIdx.x, n = blockIdx.x, h = blockIdx.y, b = blockIdx.z / a.parts, part = blockIdx.z % a.parts;
     const int Kq = a.Kq, Vd = a.Vd, t0 = n * BC;
     const size_t bh = (size_t)b * a.H + h, ssz = (size_t)Kq * Vd;
     const float* q = a.q + (bh * a.Tp + t0) * Kq;
@@ -1095,36 +1022,39 @@ __global__ __launch_bounds__(256) void bw_chunk_kernel(ChunkGradArgs a) {
         const float G = chunk_gam(a.g, b, h, a.T, a.H, n, tid);
         sG[tid] = G;
     }
-    chunk_scores<MF, V4>(q, k, Kq, sG, sStage, sA);
-    chunk_scores<MF, V4>(dO, v, Vd, sG, sStage, sB);
+    // The tiles of dq and dk (nq), then those of dv: this workgroup's are part,
+    // part + parts, ... Each kind needs one of the two score matrices.
+    const int nq = (Kq + BC * NT - 1) / (BC * NT), tiles = nq + (Vd + BC * NT - 1) / (BC * NT);
+    const int last = part + (tiles - 1 - part) / a.parts * a.parts;
+    if (last >= nq) chunk_scores<MF, V4>(q, k, Kq, sG, sStage, sA);
+    if (part < nq) chunk_scores<MF, V4>(dO, v, Vd, sG, sStage, sB);
     const float sc = a.scale;
-    for (int d0 = 0; d0 < Kq; d0 += BC * NT) {
-        // dq = scale (e^{G_t} dO_t S_n^T + B k)
+    for (int u = part; u < tiles; u += a.parts) {
         float acc[NA][4] = {};
-        tile_gemm_nt<MF, true, NT>(VK(dO, Vd, BC, Vd), SK(S + (size_t)d0 * Vd, Vd, Kq - d0, Vd), Vd, sStage, acc);
-        tile_scale_rows<MF, NA>(acc, [&](int t) { return expf(sG[t]); });
-        tile_gemm_nt<MF, false, NT>([&](int i, int kk) { return sB[i][kk]; }, RJ(k + d0, Kq, BC, Kq - d0), BC, sStage,
-                             acc);
-        tile_store<MF, NA>(acc, a.dq + (bh * a.Tp + t0) * Kq, Kq, d0, sc);
-        // dk = e^{G_last - G_s} v_s D_{n+1}^T + scale B^T q
+        if (u < nq) {
+            const int d0 = BC * NT * u;
+            // dq = scale (e^{G_t} dO_t S_n^T + B k)
+            tile_gemm<MF, NT>(VK(dO, Vd, BC, Vd), SK(S + (size_t)d0 * Vd, Vd, Kq - d0, Vd), Vd, sStage, acc);
+            tile_scale_rows<NA>(acc, [&](int t) { return expf(sG[t]); });
+            tile_gemm<MF, NT>([&](int i, int kk) { return sB[i][kk]; }, RJ(k + d0, Kq, BC, Kq - d0), BC, sStage, acc);
+            tile_store<NA>(acc, a.dq + (bh * a.Tp + t0) * Kq, Kq, d0, sc);
+            // dk = e^{G_last - G_s} v_s D_{n+1}^T + scale B^T q
 #pragma unroll
-        for (int x = 0; x < NA; x++)
+            for (int x = 0; x < NA; x++)
 #pragma unroll
-            for (int y = 0; y < 4; y++) acc[x][y] = 0.f;
-        tile_gemm_nt<MF, true, NT>(VK(v, Vd, BC, Vd), SK(D + (size_t)d0 * Vd, Vd, Kq - d0, Vd), Vd, sStage, acc);
-        tile_scale_rows<MF, NA>(acc, [&](int t) { return expf(sG[BC - 1] - sG[t]); });
-        tile_gemm_nt<MF, false, NT>([&](int i, int kk) { return sc * sB[kk][i]; }, RJ(q + d0, Kq, BC, Kq - d0), BC,
-                             sStage, acc);
-        tile_store<MF, NA>(acc, a.dk + (bh * a.Tp + t0) * Kq, Kq, d0, 1.f);
-    }
-    for (int d0 = 0; d0 < Vd; d0 += BC * NT) {
-        // dv = e^{G_last - G_s} k_s D_{n+1} + scale A^T dO
-        float acc[NA][4] = {};
-        tile_gemm_nt<MF, false, NT>(RK(k, Kq, BC, Kq), SJ(D + d0, Vd, Kq, Vd - d0), Kq, sStage, acc);
-        tile_scale_rows<MF, NA>(acc, [&](int t) { return expf(sG[BC - 1] - sG[t]); });
-        tile_gemm_nt<MF, false, NT>([&](int i, int kk) { return sc * sA[kk][i]; }, VJ(dO + d0, Vd, BC, Vd - d0), BC,
-                             sStage, acc);
-        tile_store<MF, NA>(acc, a.dv + (bh * a.Tp + t0) * Vd, Vd, d0, 1.f);
+                for (int y = 0; y < 4; y++) acc[x][y] = 0.f;
+            tile_gemm<MF, NT>(VK(v, Vd, BC, Vd), SK(D + (size_t)d0 * Vd, Vd, Kq - d0, Vd), Vd, sStage, acc);
+            tile_scale_rows<NA>(acc, [&](int t) { return expf(sG[BC - 1] - sG[t]); });
+            tile_gemm<MF, NT>([&](int i, int kk) { return sc * sB[kk][i]; }, RJ(q + d0, Kq, BC, Kq - d0), BC, sStage, acc);
+            tile_store<NA>(acc, a.dk + (bh * a.Tp + t0) * Kq, Kq, d0, 1.f);
+        } else {
+            const int d0 = BC * NT * (u - nq);
+            // dv = e^{G_last - G_s} k_s D_{n+1} + scale A^T dO
+            tile_gemm<MF, NT>(RK(k, Kq, BC, Kq), SJ(D + d0, Vd, Kq, Vd - d0), Kq, sStage, acc);
+            tile_scale_rows<NA>(acc, [&](int t) { return expf(sG[BC - 1] - sG[t]); });
+            tile_gemm<MF, NT>([&](int i, int kk) { return sc * sA[kk][i]; }, VJ(dO + d0, Vd, BC, Vd - d0), BC, sStage, acc);
+            tile_store<NA>(acc, a.dv + (bh * a.Tp + t0) * Vd, Vd, d0, 1.f);
+        }
     }
 }
 
@@ -1147,15 +1077,6 @@ __device__ __forceinline__ float bw_rnd(float x) {
 
 constexpr int RO_LD = BWD_TABLE_M + 4;  // staged table and row rows, 16-byte aligned
 constexpr int RO_FWD_THREADS = 1024;
-
-typedef float f32x4v __attribute__((ext_vector_type(4)));
-
-// v_mfma_f32_16x16x4_f32 (fp32 operands, fp32 accumulation): lane l holds
-// A[l % 16][l / 16] and B[l / 16][l % 16] of a 16 x 4 by 4 x 16 step and rows
-// 4 (l / 16) .. + 3 of column l % 16 of the 16 x 16 result.
-__device__ __forceinline__ f32x4v mfma4(float a, float b, f32x4v c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
 
 template <bool BF>
 __global__ __launch_bounds__(RO_FWD_THREADS) void bw_fwd_readout_kernel(const float* raw, const float* cs, const float* sn,
@@ -1214,9 +1135,9 @@ __global__ __launch_bounds__(RO_FWD_THREADS) void bw_fwd_readout_kernel(const fl
         load_block(b0 + RB);  // the next block (past the end: dead loads)
         __syncthreads();
         {  // logits l[i][r] = sum_m z[i][m] table[r][m]
-            f32x4v acc[CPW];
+            f32x4 acc[CPW];
 #pragma unroll
-            for (int t = 0; t < CPW; t++) acc[t] = f32x4v{0.f, 0.f, 0.f, 0.f};
+            for (int t = 0; t < CPW; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
             for (int k0 = 0; k0 < TM; k0 += 4) {
                 const float az = sZ[16 * it + lr][k0 + lk];
 #pragma unroll
@@ -1240,9 +1161,9 @@ __global__ __launch_bounds__(RO_FWD_THREADS) void bw_fwd_readout_kernel(const fl
         // u[i][m] = sum_r p[i][r] table[r][m] (p and the table zero at r >= R); the
         // weights' pair (2 pr, 2 pr + 1) sits in lanes (lr, lr ^ 1), swapped in by
         // quad_perm [1,0,3,2]
-        f32x4v acc[CPW];
+        f32x4 acc[CPW];
 #pragma unroll
-        for (int t = 0; t < CPW; t++) acc[t] = f32x4v{0.f, 0.f, 0.f, 0.f};
+        for (int t = 0; t < CPW; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
         for (int k0 = 0; k0 < TM; k0 += 4) {
             const float ap = sP[16 * it + lr][k0 + lk];
 #pragma unroll
@@ -1467,9 +1388,9 @@ __global__ __launch_bounds__(RO_ADJ_THREADS) void bw_readout_kernel(ReadoutGradA
     // GEMMs over the block: wave wv takes row tile it = wv & 1 and the column
     // tiles CPW (wv >> 1) .. + CPW - 1 of the logits (r) and of dz, u (m)
     const int it = wv & 1, ct0 = CPW * (wv >> 1), dm = wv & 7, dr0 = DRT * (wv >> 3);
-    f32x4v dacc[DRT];  // dtable tiles (r tile dr0 + rt, m tile dm)
+    f32x4 dacc[DRT];  // dtable tiles (r tile dr0 + rt, m tile dm)
 #pragma unroll
-    for (int rt = 0; rt < DRT; rt++) dacc[rt] = f32x4v{0.f, 0.f, 0.f, 0.f};
+    for (int rt = 0; rt < DRT; rt++) dacc[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int rows = a.B * a.Tp;
     // A block's inputs, element x of this thread = (row i, pair pr) = e / 64,
     // e % 64, e = tid + NT x: loaded one block ahead through buffer
@@ -1515,9 +1436,9 @@ __global__ __launch_bounds__(RO_ADJ_THREADS) void bw_readout_kernel(ReadoutGradA
         __syncthreads();
         // logits l[i][r] = sum_m z[i][m] table[r][m] and dp[i][r] = sum_m du[i][m] table[r][m]
         {
-            f32x4v accl[CPW], accd[CPW];
+            f32x4 accl[CPW], accd[CPW];
 #pragma unroll
-            for (int t = 0; t < CPW; t++) accl[t] = accd[t] = f32x4v{0.f, 0.f, 0.f, 0.f};
+            for (int t = 0; t < CPW; t++) accl[t] = accd[t] = f32x4{0.f, 0.f, 0.f, 0.f};
             for (int k0 = 0; k0 < TM; k0 += 4) {
                 const float az = sZ[16 * it + lr][k0 + lk], ad = sDU[16 * it + lr][k0 + lk];
 #pragma unroll
@@ -1554,9 +1475,9 @@ __global__ __launch_bounds__(RO_ADJ_THREADS) void bw_readout_kernel(ReadoutGradA
         // dz[i][m] = sum_r dl[i][r] table[r][m] and u[i][m] = sum_r p[i][r] table[r][m]
         // (p and dl are zero at r >= R, as is the table); then draw and the clock's share
         {
-            f32x4v accz[CPW], accu[CPW];
+            f32x4 accz[CPW], accu[CPW];
 #pragma unroll
-            for (int t = 0; t < CPW; t++) accz[t] = accu[t] = f32x4v{0.f, 0.f, 0.f, 0.f};
+            for (int t = 0; t < CPW; t++) accz[t] = accu[t] = f32x4{0.f, 0.f, 0.f, 0.f};
             for (int k0 = 0; k0 < TM; k0 += 4) {
                 const float al = sDL[16 * it + lr][k0 + lk], ap = sP[16 * it + lr][k0 + lk];
 #pragma unroll
@@ -1635,7 +1556,7 @@ __global__ __launch_bounds__(RO_ADJ_THREADS) void bw_readout_kernel(ReadoutGradA
 
 // The readout and its adjoint for 128 < M <= 256 slots, where a head's table
 // (up to 255 x 256 fp32) does not fit in LDS beside the row blocks: every
-// product is a 64 x 64 fp32 tile GEMM (tile_gemm<false>) that streams the
+// product is a 64 x 64 fp32 tile GEMM (tile_gemm_fma) that streams the
 // table from memory, and the softmax and its adjoint run per row between
 // them. Token rows rho of head h are the B Tp rows (b, h, t), rho = b Tp + t,
 // at head-major row ((b H + h) Tp + t); X_lam(rho)[m] is U(lam) x (pairs
@@ -1679,7 +1600,7 @@ __global__ __launch_bounds__(256) void bw_wide_logits_kernel(WideArgs a) {
     const float* x = ADJ ? a.dwts : a.raw;
     const float* tb = a.table + (size_t)h * R * M;
     float acc[4][4] = {};
-    tile_gemm<false, true>(
+    tile_gemm_fma<true>(
         [&](int i, int m) {
             return rho0 + i < rows ? wide_rnd(a, wide_rot(a, x, wide_row(a, h, rho0 + i), m)) : 0.f;
         },
@@ -1687,12 +1608,12 @@ __global__ __launch_bounds__(256) void bw_wide_logits_kernel(WideArgs a) {
     float* out = ADJ ? a.dl : a.lg;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        const int rho = rho0 + TileMap<false>::row(i, 0);
+        const int rho = rho0 + FmaMap::row(i, 0);
         if (rho >= rows) continue;
         const size_t row = wide_row(a, h, rho);
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const int r = r0 + TileMap<false>::col(i, j);
+            const int r = r0 + FmaMap::col(i, j);
             if (r < R) out[row * BW_WIDE_MW + r] = acc[i][j];
         }
     }
@@ -1758,23 +1679,23 @@ __global__ __launch_bounds__(256) void bw_wide_u_kernel(WideArgs a) {
     const float* tb = a.table + (size_t)h * R * M;
     const auto tab = [&](int r, int j) { return m0 + j < M ? wide_rnd(a, tb[(size_t)r * M + m0 + j]) : 0.f; };
     float u[4][4] = {}, dz[4][4] = {};
-    tile_gemm<false, false>(
+    tile_gemm_fma<false>(
         [&](int i, int r) { return rho0 + i < rows ? a.lg[wide_row(a, h, rho0 + i) * BW_WIDE_MW + r] : 0.f; }, tab, R,
         sStage, u);
     if (ADJ)
-        tile_gemm<false, false>(
+        tile_gemm_fma<false>(
             [&](int i, int r) { return rho0 + i < rows ? a.dl[wide_row(a, h, rho0 + i) * BW_WIDE_MW + r] : 0.f; },
             tab, R, sStage, dz);
     const int cg = tid & 15;  // this thread's four columns m0 + 4 cg ..: pairs (m0 + 4 cg) / 2 and + 1
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        const int ri = TileMap<false>::row(i, 0), rho = rho0 + ri;
+        const int ri = FmaMap::row(i, 0), rho = rho0 + ri;
         float dls = 0.f;
         if (rho < rows) {
             const size_t row = wide_row(a, h, rho);
 #pragma unroll
             for (int j = 0; j < 4; j += 2) {
-                const int m = m0 + TileMap<false>::col(i, j), pr = m >> 1;
+                const int m = m0 + FmaMap::col(i, j), pr = m >> 1;
                 if (pr >= P) continue;
                 const float c = a.cs[row * P + pr], s = a.sn[row * P + pr];
                 if (!ADJ) {
@@ -1822,11 +1743,11 @@ __global__ __launch_bounds__(256) void bw_wide_dtable_kernel(WideArgs a) {
     const int M = a.M, R = M - 1, rows = a.B * a.Tp, k0 = sp * BW_WIDE_SPLIT;
     const int Kd = min(BW_WIDE_SPLIT, rows - k0);
     float acc[4][4] = {};
-    tile_gemm<false, false>(
+    tile_gemm_fma<false>(
         [&](int i, int k) { return r0 + i < R ? a.lg[wide_row(a, h, k0 + k) * BW_WIDE_MW + r0 + i] : 0.f; },
         [&](int k, int j) { return m0 + j < M ? wide_rot(a, a.dwts, wide_row(a, h, k0 + k), m0 + j) : 0.f; }, Kd,
         sStage, acc);
-    tile_gemm<false, false>(
+    tile_gemm_fma<false>(
         [&](int i, int k) { return r0 + i < R ? a.dl[wide_row(a, h, k0 + k) * BW_WIDE_MW + r0 + i] : 0.f; },
         [&](int k, int j) { return m0 + j < M ? wide_rot(a, a.raw, wide_row(a, h, k0 + k), m0 + j) : 0.f; }, Kd,
         sStage, acc);
@@ -1835,7 +1756,7 @@ __global__ __launch_bounds__(256) void bw_wide_dtable_kernel(WideArgs a) {
     for (int i = 0; i < 4; i++)
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const int r = r0 + TileMap<false>::row(i, j), m = m0 + TileMap<false>::col(i, j);
+            const int r = r0 + FmaMap::row(i, j), m = m0 + FmaMap::col(i, j);
             if (r < R && m < M) dst[(size_t)r * M + m] = acc[i][j];
         }
 }
@@ -2179,23 +2100,60 @@ __global__ __launch_bounds__(256) void bw_pack1_kernel(const float* src, int B, 
     bw_st<BF>(dst, i, src[(((size_t)b * H + h) * Tp + t) * D + j]);
 }
 
-void launch_chunk_grad(const ChunkGradArgs& a, bool mfma, hipStream_t stream) {
+// Workgroups per chunk of the chunk kernels for `chunks` chunks of `tiles`
+// output tiles: one where the chunks give every compute unit two workgroups;
+// below that the tiles are shared out over up to four workgroups per compute
+// unit, each forming its own scores again. One backward on MI355X, us with 1
+// and with 3 (two 64 NT = 128 wide tiles of dq and dk, one of dv): 78 chunks
+// (bf16) 347 / 289, 128 (fp32) 416 / 348, 192 (bf16) 468 / 434, 512 (bf16)
+// 756 / 769, 1024 (bf16) 1266 / 1316.
+int chunk_parts(long long chunks, int tiles) {
+    const long long cus = device_cu_count();
+    if (chunks >= 2 * cus) return 1;
+    const long long parts = (4 * cus + chunks - 1) / chunks;
+    return parts > tiles ? tiles : (int)parts;
+}
+
+template <int NT>
+void launch_chunk_grad_nt(const ChunkGradArgs& a, bool mfma, bool v4, hipStream_t stream) {
+    const dim3 grid(a.N, a.H, a.B * a.parts), blk(256);
+#define CYFA_BW_CHUNK(MF_, V4_, SB_, RB_) \
+    hipLaunchKernelGGL((bw_chunk_kernel<MF_, V4_, SB_, RB_, NT>), grid, blk, 0, stream, a)
+    // (the flags pair as the backward sets them: sbf for bf16 calls, rbf for pass 2's)
+    if (mfma && v4) {
+        if (a.rbf)
+            CYFA_BW_CHUNK(true, true, true, true);
+        else
+            CYFA_BW_CHUNK(true, true, true, false);
+    } else if (mfma) {
+        if (a.rbf)
+            CYFA_BW_CHUNK(true, false, true, true);
+        else
+            CYFA_BW_CHUNK(true, false, true, false);
+    } else if (v4) {
+        CYFA_BW_CHUNK(false, true, false, false);
+    } else {
+        CYFA_BW_CHUNK(false, false, false, false);
+    }
+#undef CYFA_BW_CHUNK
+}
+
+int launch_chunk_grad(ChunkGradArgs a, bool mfma, hipStream_t stream) {
+    if (mfma != (a.sbf != 0)) return -1;  // bf16 calls keep bf16 states, fp32 calls fp32 ones
     // rows and states 16-byte aligned (workspace buffers, rows of Kq and Vd floats)
     const bool v4 = a.Kq % 4 == 0 && a.Vd % 4 == 0;
-    const dim3 grid(a.N, a.H, a.B);
-    // (the flags pair as the backward sets them: sbf for bf16 calls, rbf for pass 2's)
-    if (mfma && v4 && a.rbf)
-        hipLaunchKernelGGL((bw_chunk_kernel<true, true, true, true>), grid, dim3(256), 0, stream, a);
-    else if (mfma && v4)
-        hipLaunchKernelGGL((a.sbf ? bw_chunk_kernel<true, true, true, false> : bw_chunk_kernel<true, true, false, false>),
-                           grid, dim3(256), 0, stream, a);
-    else if (mfma && a.rbf)
-        hipLaunchKernelGGL((bw_chunk_kernel<true, false, true, true>), grid, dim3(256), 0, stream, a);
-    else if (mfma)
-        hipLaunchKernelGGL((a.sbf ? bw_chunk_kernel<true, false, true, false> : bw_chunk_kernel<true, false, false, false>),
-                           grid, dim3(256), 0, stream, a);
-    else
-        hipLaunchKernelGGL((bw_chunk_kernel<false, false, false, false>), grid, dim3(256), 0, stream, a);
+    const long long chunks = (long long)a.N * a.H * a.B;
+    const auto tiles = [&](int w) { return (a.Kq + w - 1) / w + (a.Vd + w - 1) / w; };
+    // 64-wide tiles where even they leave compute units idle (78 chunks: 284 us
+    // against 289 with 128-wide ones, 20 chunks: 217 against 227)
+    if (v4 && chunks * tiles(2 * BC) >= device_cu_count()) {
+        a.parts = chunk_parts(chunks, tiles(2 * BC));
+        launch_chunk_grad_nt<2>(a, mfma, v4, stream);
+    } else {
+        a.parts = chunk_parts(chunks, tiles(BC));
+        launch_chunk_grad_nt<1>(a, mfma, v4, stream);
+    }
+    return 0;
 }
 
 }  // namespace
@@ -2242,13 +2200,16 @@ int launch_chunk_pass(const ChunkPassParams& p, hipStream_t stream) {
     oa.sbf = p.mfma && p.sbf16;
     // rows and states 16-byte aligned (workspace buffers, rows of Kq and Vd floats)
     const bool v4 = p.Kq % 4 == 0 && p.Vd % 4 == 0;
-    const dim3 og(N, p.H, p.B);
+    oa.parts = chunk_parts((long long)N * p.H * p.B, (p.Vd + BC - 1) / BC);
+    const dim3 og(N, p.H, p.B * oa.parts);
     if (p.mfma && v4)
         hipLaunchKernelGGL((oa.sbf ? bw_out_kernel<true, true, true> : bw_out_kernel<true, true, false>), og, dim3(256),
                            0, stream, oa);
     else if (p.mfma)
         hipLaunchKernelGGL((oa.sbf ? bw_out_kernel<true, false, true> : bw_out_kernel<true, false, false>), og,
                            dim3(256), 0, stream, oa);
+    else if (v4)
+        hipLaunchKernelGGL((bw_out_kernel<false, true, false>), og, dim3(256), 0, stream, oa);
     else
         hipLaunchKernelGGL((bw_out_kernel<false, false, false>), og, dim3(256), 0, stream, oa);
     return 0;
@@ -2431,7 +2392,7 @@ int launch_chunk_bwd(const BwdParams& p, hipStream_t stream) {
     c2.Vd = V;
     c2.N = N;
     c2.scale = 1.f;
-    launch_chunk_grad(c2, bf, stream);
+    if (launch_chunk_grad(c2, bf, stream) != 0) return -1;
     // the readout: the pass-1 output's cotangent, the clock's share and the table's
     ReadoutGradArgs ro{};
     ro.raw = ws.raw;
@@ -2482,7 +2443,7 @@ int launch_chunk_bwd(const BwdParams& p, hipStream_t stream) {
     c1.Kq = K;
     c1.Vd = M;
     c1.scale = p.scale;
-    launch_chunk_grad(c1, bf, stream);
+    if (launch_chunk_grad(c1, bf, stream) != 0) return -1;
     // gates, write vector and clock
     TokenGradArgs tg{};
     tg.qh = ws.qh;
