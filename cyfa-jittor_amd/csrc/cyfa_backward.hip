@@ -20,6 +20,11 @@
 //   dk_s = scale sum_{t>=s} e^{G_t-G_s} (dO_t.v_s) q_t + e^{G_last-G_s} D_{n+1} v_s
 //   dv_s = scale sum_{t>=s} e^{G_t-G_s} (q_t.k_s) dO_t + e^{G_last-G_s} D_{n+1}^T k_s
 //   dL/dG_t = q_t.dq_t - k_t.dk_t + [t = last] <D_{n+1}, S_{n+1}>,  dg = in-chunk reverse cumsum
+// where q_t.dq_t = o_t.dO_t (dq_t scale^-1 is what o_t's rows contract with)
+// and k_t.dk_t = v_t.dv_t, so that both passes' terms come from the narrow
+// rows between them: z.dz and u.du in the readout adjoint (a rotation keeps the
+// dot products raw.draw and weights.dweights), and w.(dw_1 + dw_2) = beta
+// dbeta.
 // The states and their cotangents are one sweep per (state tile, b, h) that
 // keeps its tile in registers; outputs and the rows' cotangents are then
 // chunk-parallel, one workgroup per (chunk, h, b), with no reduction across
@@ -1364,7 +1369,7 @@ constexpr int RO_BLK = BWD_RO_BLOCK;
 constexpr int RO_ADJ_THREADS = 1024;
 struct ReadoutGradArgs {
     const float *raw, *cs, *sn, *table, *dwts;  // head-major rows; table [H, M-1, M]
-    float *draw, *dlam, *dtab;                  // dtab: [H, workgroups, (M-1) M]
+    float *draw, *dlam, *dgq, *dtab;            // dgq: z.dz + u.du per row; dtab: [H, workgroups, (M-1) M]
     int B, Tp, H, M;
     int per_wg;                                 // blocks of 32 rows per workgroup
 };
@@ -1377,7 +1382,7 @@ __global__ __launch_bounds__(RO_ADJ_THREADS) void bw_readout_kernel(ReadoutGradA
     __shared__ float sTab[TM * LD];  // rows R .. 127 and columns M .. 127 zero
     __shared__ float sZ[RO_BLK][LD], sDU[RO_BLK][LD], sP[RO_BLK][LD], sDL[RO_BLK][LD];
     __shared__ float sCs[RO_BLK][TM / 2], sSn[RO_BLK][TM / 2];
-    __shared__ float sLam[RO_BLK][NW / 2];
+    __shared__ float sLam[RO_BLK][NW / 2], sGq[RO_BLK][NW / 2];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, blk = blockIdx.x, h = blockIdx.y;
     const int lr = lane & 15, lk = lane >> 4;  // operand row / column and k of this lane
     const int M = a.M, R = M - 1, P = M / 2, RM = R * M;
@@ -1494,7 +1499,8 @@ __global__ __launch_bounds__(RO_ADJ_THREADS) void bw_readout_kernel(ReadoutGradA
             // kappa_p [(z_e dz_o - z_o dz_e) + (du_e u_o - du_o u_e)] (a rotation keeps
             // the 2-d cross product); the even lane of a pair forms it.
             const bool odd = (lr & 1) != 0;
-            float dl[4] = {0.f, 0.f, 0.f, 0.f};
+            // (Every lane adds its column's z dz + u du to the gate's share.)
+            float dl[4] = {0.f, 0.f, 0.f, 0.f}, gq[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int t = 0; t < CPW; t++) {
                 const int m = 16 * (ct0 + t) + lr, pr = m >> 1;
@@ -1502,17 +1508,16 @@ __global__ __launch_bounds__(RO_ADJ_THREADS) void bw_readout_kernel(ReadoutGradA
                 for (int q = 0; q < 4; q++) {
                     const float gz = accz[t][q], gx = dpp_mov<0xB1>(gz);
                     const float gu = accu[t][q], ux = dpp_mov<0xB1>(gu);
+                    const float zm = sZ[16 * it + 4 * lk + q][m], dm = sDU[16 * it + 4 * lk + q][m];
+                    const float zx = dpp_mov<0xB1>(zm), dx = dpp_mov<0xB1>(dm);
+                    gq[q] += zm * gz + dm * gu;  // zero past M and past the last row
                     const float ge = odd ? gx : gz, go = odd ? gz : gx, ue = odd ? ux : gu, uo = odd ? gu : ux;
                     const int i = 16 * it + 4 * lk + q, rho = b0 + i;
                     if (rho < rows && pr < P) {
                         const size_t row = ((size_t)(rho / a.Tp) * a.H + h) * a.Tp + rho % a.Tp;
                         const float c = sCs[i][pr], s = sSn[i][pr];
                         a.draw[row * M + m] = odd ? -s * ge + c * go : c * ge + s * go;
-                        if (!odd) {
-                            const float ze = sZ[i][2 * pr], zo = sZ[i][2 * pr + 1];
-                            const float de = sDU[i][2 * pr], dd = sDU[i][2 * pr + 1];
-                            dl[q] += (float)(kTwoPiBw * pr / R) * ((ze * go - zo * ge) + (de * uo - dd * ue));
-                        }
+                        if (!odd) dl[q] += (float)(kTwoPiBw * pr / R) * ((zm * go - zx * ge) + (dm * uo - dx * ue));
                     }
                 }
             }
@@ -1520,17 +1525,22 @@ __global__ __launch_bounds__(RO_ADJ_THREADS) void bw_readout_kernel(ReadoutGradA
             // in tile order), then the waves of the row tile in wave order
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-                const float v = wave_sum<16>(dl[q]);
-                if (lr == 0) sLam[16 * it + 4 * lk + q][wv >> 1] = v;
+                const float v = wave_sum<16>(dl[q]), g = wave_sum<16>(gq[q]);
+                if (lr == 0) {
+                    sLam[16 * it + 4 * lk + q][wv >> 1] = v;
+                    sGq[16 * it + 4 * lk + q][wv >> 1] = g;
+                }
             }
         }
         __syncthreads();
-        if (tid < RO_BLK && b0 + tid < rows) {  // the clock's share per row
+        if (tid < RO_BLK && b0 + tid < rows) {  // the clock's and the gate's share per row
             const int rho = b0 + tid;
-            float v = sLam[tid][0];
+            float v = sLam[tid][0], g = sGq[tid][0];
 #pragma unroll
-            for (int j = 1; j < NW / 2; j++) v += sLam[tid][j];
-            a.dlam[((size_t)(rho / a.Tp) * a.H + h) * a.Tp + rho % a.Tp] = v;
+            for (int j = 1; j < NW / 2; j++) v += sLam[tid][j], g += sGq[tid][j];
+            const size_t row = ((size_t)(rho / a.Tp) * a.H + h) * a.Tp + rho % a.Tp;
+            a.dlam[row] = v;
+            a.dgq[row] = g;
         }
         // dtable[r][m] += sum_i p[i][r] du[i][m] + dl[i][r] z[i][m] over the block's rows
         for (int k0 = 0; k0 < RO_BLK; k0 += 4) {
@@ -1569,7 +1579,8 @@ constexpr int BW_WIDE_CT = BW_WIDE_MW / BC;    // column tiles of a row (the clo
 struct WideArgs {
     const float *raw, *cs, *sn, *table, *dwts;  // head-major rows; table [H, M-1, M]
     float *lg, *dl;                             // [B H Tp, MW]: logits then p; dp then dl
-    float *wts, *draw, *dlp, *dlam;             // dlp [B H Tp, BW_WIDE_CT]: the clock's partials
+    float *wts, *draw, *dlp, *dlam;             // dlp [B H Tp, 2 BW_WIDE_CT]: the clock's and the gate's partials
+    float* dgq;
     float* dtab;                                // [H, splits, (M-1) M]
     int B, Tp, H, M, splits;
     int bf;                                     // forward: round z, the table, p and the weights to bf16
@@ -1668,12 +1679,13 @@ __global__ __launch_bounds__(256) void bw_wide_softmax_kernel(WideArgs a) {
 //   forward: weights = U(-lam) u into wts;
 //   ADJ: dz = dl table as well; draw = U(-lam) dz, and the clock's share of
 //   the block's pairs, kappa_p [(z_e dz_o - z_o dz_e) + (du_e u_o - du_o u_e)],
-//   summed over the tile's pairs in column order into dlp[row][m0 / 64].
+//   and the gate's, z.dz + u.du, each summed over the tile's pairs in column
+//   order into dlp[row][m0 / 64] and dlp[row][BW_WIDE_CT + m0 / 64].
 // Grid (ceil(B Tp / 64), ceil(M / 64), H).
 template <bool ADJ>
 __global__ __launch_bounds__(256) void bw_wide_u_kernel(WideArgs a) {
     __shared__ __align__(16) unsigned char sStage[STAGE_BYTES];
-    __shared__ float sPart[BC][17];
+    __shared__ float sPart[BC][17], sGate[BC][17];
     const int tid = threadIdx.x, rho0 = blockIdx.x * BC, m0 = blockIdx.y * BC, h = blockIdx.z;
     const int M = a.M, R = M - 1, P = M / 2, rows = a.B * a.Tp;
     const float* tb = a.table + (size_t)h * R * M;
@@ -1690,7 +1702,7 @@ __global__ __launch_bounds__(256) void bw_wide_u_kernel(WideArgs a) {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const int ri = FmaMap::row(i, 0), rho = rho0 + ri;
-        float dls = 0.f;
+        float dls = 0.f, gqs = 0.f;
         if (rho < rows) {
             const size_t row = wide_row(a, h, rho);
 #pragma unroll
@@ -1708,30 +1720,34 @@ __global__ __launch_bounds__(256) void bw_wide_u_kernel(WideArgs a) {
                     const float ze = wide_rot(a, a.raw, row, m), zo = wide_rot(a, a.raw, row, m + 1);
                     const float de = wide_rot(a, a.dwts, row, m), dd = wide_rot(a, a.dwts, row, m + 1);
                     dls += (float)(kTwoPiBw * pr / R) * ((ze * go - zo * ge) + (de * uo - dd * ue));
+                    gqs += (ze * ge + zo * go) + (de * ue + dd * uo);
                 }
             }
         }
-        if (ADJ) sPart[ri][cg] = dls;
+        if (ADJ) sPart[ri][cg] = dls, sGate[ri][cg] = gqs;
     }
     if (ADJ) {
         __syncthreads();
         if (tid < BC && rho0 + tid < rows) {
-            float t = 0.f;
-            for (int g = 0; g < 16; g++) t += sPart[tid][g];
-            a.dlp[wide_row(a, h, rho0 + tid) * BW_WIDE_CT + blockIdx.y] = t;
+            float t = 0.f, u2 = 0.f;
+            for (int g = 0; g < 16; g++) t += sPart[tid][g], u2 += sGate[tid][g];
+            float* dst = a.dlp + wide_row(a, h, rho0 + tid) * 2 * BW_WIDE_CT + blockIdx.y;
+            dst[0] = t;
+            dst[BW_WIDE_CT] = u2;
         }
     }
 }
 
-// The readout's share of the clock cotangent: the column tiles' partials in
-// order. One thread per head-major row.
+// The readout's share of the clock and gate cotangents: the column tiles'
+// partials in order. One thread per head-major row.
 __global__ __launch_bounds__(256) void bw_wide_dlam_kernel(WideArgs a) {
     const size_t row = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (row >= (size_t)a.B * a.H * a.Tp) return;
     const int nt = (a.M + BC - 1) / BC;
-    float t = 0.f;
-    for (int c = 0; c < nt; c++) t += a.dlp[row * BW_WIDE_CT + c];
+    float t = 0.f, g = 0.f;
+    for (int c = 0; c < nt; c++) t += a.dlp[row * 2 * BW_WIDE_CT + c], g += a.dlp[row * 2 * BW_WIDE_CT + BW_WIDE_CT + c];
     a.dlam[row] = t;
+    a.dgq[row] = g;
 }
 
 // dtable[h][r][m] partial over token rows [split BW_WIDE_SPLIT, + BW_WIDE_SPLIT):
@@ -1761,101 +1777,80 @@ __global__ __launch_bounds__(256) void bw_wide_dtable_kernel(WideArgs a) {
         }
 }
 
-// Per chunk of (b, h): the gate cotangent of both passes (dL/dG_t = q.dq -
-// k.dk, plus <D_{n+1}, S_{n+1}> at the chunk's last token, then the in-chunk
-// reverse cumsum), and the write vector's (w = beta a(lam), a[2p] = s_p cos
-// theta_p, a[2p+1] = -s_p sin theta_p, dw = the pass-1 value cotangent + the
-// pass-2 key cotangent): dbeta = dw . a, and dlam = beta dw . da/dlam + the
-// readout's share. Grid (N, B*H), 256 threads: wave w forms tokens w, w + 4,
-// .. (two at a time) with its lanes across the row (coalesced 16- and 8-byte
-// loads), then wave 0 scans.
+// Per chunk of (b, h): the write vector's cotangents (w = beta a(lam), a[2p] =
+// s_p cos theta_p, a[2p+1] = -s_p sin theta_p, dw = the pass-1 value cotangent
+// + the pass-2 key cotangent): dbeta = dw . a and dlam = beta dw . da/dlam +
+// the readout's share; and the gate cotangent of both passes, dL/dG_t = dgq_t -
+// beta_t dbeta_t (the header's identities), plus <D_{n+1}, S_{n+1}> at the
+// chunk's last token, then the in-chunk reverse cumsum. Grid (N, B*H), 256
+// threads: wave w forms rows TG_U at a time with its lanes across the pairs,
+// then wave 0 scans. Bound by HBM: dw_1, dw_2 and the phases, 100 MB at 65536
+// rows of 128 slots, 23 us; reading the rows of q, k and their cotangents for
+// the dot products themselves it took 104 us (470 MB).
 struct TokenGradArgs {
-    const float *qh, *kh, *dqh, *dkh;    // pass 1 rows [.., K]
-    const float *wts, *w, *dwts, *dw2;   // pass 2 query and key rows [.., M]
-    const float* dw1;                    // pass-1 value cotangent [.., M]
+    const float *dw1, *dw2;              // [.., M]
     const float *cs, *sn;                // [.., M/2]
     const float *bnd1, *bnd2;            // [B*H, nt, N]
+    const float* dgq;                    // [B*H, Tp]: q.dq of both passes
     const float* beta;                   // [B, T, H]
     float* dlam;                         // [B*H, Tp]: in, the readout's share; out, the total
     float *dg, *dbeta;                   // [B, T, H]
-    int B, T, Tp, H, K, M, N, nt1, nt2;
+    int B, T, Tp, H, M, N, nt1, nt2;
 };
+constexpr int TG_U = 8;  // rows whose loads a wave has in flight
 
-template <bool V4>
 __global__ __launch_bounds__(256) void bw_token_kernel(TokenGradArgs a) {
-    __shared__ float sdG[BC], sdB[BC], sdL[BC];
+    __shared__ float sdB[BC], sdL[BC], sBnd;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int n = blockIdx.x, bh = blockIdx.y, b = bh / a.H, h = bh % a.H;
-    const int K = a.K, M = a.M, P = M / 2, R = M - 1;
+    const int M = a.M, P = M / 2, R = M - 1;
     // the write vector's per-pair factors: sqrt(1/R) for p = 0, sqrt(2/R) after;
     // the phase derivative's 2 pi p / R for the lane's pairs p = lane, lane + 64
     const float sp0 = (float)sqrt(1.0 / R), sp1 = (float)sqrt(2.0 / R);
     const float kp[2] = {(float)(kTwoPiBw * lane / R), (float)(kTwoPiBw * (lane + 64) / R)};
-    // Wave wv forms the rows wv + 8 u and wv + 8 u + 4 together, so that both
-    // rows' loads are in flight at once. The lane reads four consecutive
-    // elements of the K-rows with V4 (K % 4 == 0), one otherwise, and the
-    // pair (2 p, 2 p + 1) of the M-rows.
-    for (int i0 = wv; i0 < BC; i0 += 8) {
-        size_t row[2];
-        float dG[2], db[2], dl[2];
+    if (wv == 3) {  // the chunk's boundary terms of both passes
+        float x = 0.f;
+        for (int i = lane; i < a.nt1; i += 64) x += a.bnd1[((size_t)bh * a.nt1 + i) * a.N + n];
+        for (int i = lane; i < a.nt2; i += 64) x += a.bnd2[((size_t)bh * a.nt2 + i) * a.N + n];
+        x = bw_wave_sum(x);
+        if (lane == 0) sBnd = x;
+    }
+    for (int i0 = 16 * wv; i0 < 16 * wv + 16; i0 += TG_U) {
+        float db[TG_U], dl[TG_U];
+        const size_t row0 = (size_t)bh * a.Tp + n * BC + i0;
 #pragma unroll
-        for (int u = 0; u < 2; u++) {
-            row[u] = (size_t)bh * a.Tp + n * BC + i0 + 4 * u;
-            dG[u] = db[u] = dl[u] = 0.f;
-        }
-        if constexpr (!V4) {
-            for (int j = lane; j < K; j += 64)
-#pragma unroll
-                for (int u = 0; u < 2; u++)
-                    dG[u] += a.qh[row[u] * K + j] * a.dqh[row[u] * K + j] - a.kh[row[u] * K + j] * a.dkh[row[u] * K + j];
-        }
-        for (int j = 4 * lane; V4 && j < K; j += 256) {
-            float4 q[2], dq[2], k[2], dk[2];
-#pragma unroll
-            for (int u = 0; u < 2; u++) {
-                q[u] = *reinterpret_cast<const float4*>(a.qh + row[u] * K + j);
-                dq[u] = *reinterpret_cast<const float4*>(a.dqh + row[u] * K + j);
-                k[u] = *reinterpret_cast<const float4*>(a.kh + row[u] * K + j);
-                dk[u] = *reinterpret_cast<const float4*>(a.dkh + row[u] * K + j);
-            }
-#pragma unroll
-            for (int u = 0; u < 2; u++)
-                dG[u] += (q[u].x * dq[u].x + q[u].y * dq[u].y + q[u].z * dq[u].z + q[u].w * dq[u].w) -
-                         (k[u].x * dk[u].x + k[u].y * dk[u].y + k[u].z * dk[u].z + k[u].w * dk[u].w);
-        }
+        for (int u = 0; u < TG_U; u++) db[u] = dl[u] = 0.f;
 #pragma unroll
         for (int c = 0; c < 2; c++) {
             const int p = lane + 64 * c;
-            if (p >= P) break;
-            float2 wt[2], dwt[2], w[2], d2[2], d1[2];
-            float cs[2], sn[2];
+            if (64 * c >= P) break;
+            const int pp = p < P ? p : P - 1;  // lanes past the last pair read it and drop it
+            f32x2 d2[TG_U], d1[TG_U];
+            float cs[TG_U], sn[TG_U];
 #pragma unroll
-            for (int u = 0; u < 2; u++) {
-                const size_t e = row[u] * M + 2 * p;
-                wt[u] = *reinterpret_cast<const float2*>(a.wts + e);
-                dwt[u] = *reinterpret_cast<const float2*>(a.dwts + e);
-                w[u] = *reinterpret_cast<const float2*>(a.w + e);
-                d2[u] = *reinterpret_cast<const float2*>(a.dw2 + e);
-                d1[u] = *reinterpret_cast<const float2*>(a.dw1 + e);
-                cs[u] = a.cs[row[u] * P + p];
-                sn[u] = a.sn[row[u] * P + p];
+            for (int u = 0; u < TG_U; u++) {
+                const size_t e = (row0 + u) * M + 2 * pp, f = (row0 + u) * P + pp;
+                d2[u] = *reinterpret_cast<const f32x2*>(a.dw2 + e);
+                d1[u] = *reinterpret_cast<const f32x2*>(a.dw1 + e);
+                cs[u] = a.cs[f];
+                sn[u] = a.sn[f];
             }
-            const float sp = p == 0 ? sp0 : sp1;
+            const float sp = p >= P ? 0.f : p == 0 ? sp0 : sp1;
 #pragma unroll
-            for (int u = 0; u < 2; u++) {
-                dG[u] += (wt[u].x * dwt[u].x + wt[u].y * dwt[u].y) - (w[u].x * d2[u].x + w[u].y * d2[u].y);
-                const float we = d1[u].x + d2[u].x, wo = d1[u].y + d2[u].y;
-                db[u] = fmaf(sp, we * cs[u] - wo * sn[u], db[u]);
-                dl[u] = fmaf(sp * kp[c], -we * sn[u] - wo * cs[u], dl[u]);
+            for (int u = 0; u < TG_U; u++) {
+                const float we = d1[u][0] + d2[u][0], wo = d1[u][1] + d2[u][1];
+                if (p < P) {
+                    db[u] = fmaf(sp, we * cs[u] - wo * sn[u], db[u]);
+                    dl[u] = fmaf(sp * kp[c], -we * sn[u] - wo * cs[u], dl[u]);
+                }
             }
         }
 #pragma unroll
-        for (int u = 0; u < 2; u++) {
-            const float g = bw_wave_sum(dG[u]), bb = bw_wave_sum(db[u]), ll = bw_wave_sum(dl[u]);
+        for (int u = 0; u < TG_U; u++) {
+            const float bb = bw_wave_sum(db[u]), ll = bw_wave_sum(dl[u]);
             if (lane == 0) {
-                sdG[i0 + 4 * u] = g;
-                sdB[i0 + 4 * u] = bb;
-                sdL[i0 + 4 * u] = ll;
+                sdB[i0 + u] = bb;
+                sdL[i0 + u] = ll;
             }
         }
     }
@@ -1863,16 +1858,13 @@ __global__ __launch_bounds__(256) void bw_token_kernel(TokenGradArgs a) {
     if (wv != 0) return;
     const int t = n * BC + lane;
     const size_t row = (size_t)bh * a.Tp + t;
-    float x = sdG[lane];
-    if (lane == BC - 1) {
-        for (int i = 0; i < a.nt1; i++) x += a.bnd1[((size_t)bh * a.nt1 + i) * a.N + n];
-        for (int i = 0; i < a.nt2; i++) x += a.bnd2[((size_t)bh * a.nt2 + i) * a.N + n];
-    }
+    const float bt = t < a.T ? a.beta[((size_t)b * a.T + t) * a.H + h] : 0.f;
+    float x = fmaf(-bt, sdB[lane], a.dgq[row]);
+    if (lane == BC - 1) x += sBnd;
     for (int o = 1; o < 64; o <<= 1) {
         const float y = __shfl_down(x, o);
         if (lane + o < 64) x += y;
     }
-    const float bt = t < a.T ? a.beta[((size_t)b * a.T + t) * a.H + h] : 0.f;
     a.dlam[row] = fmaf(bt, sdL[lane], a.dlam[row]);
     if (t < a.T) {
         a.dg[((size_t)b * a.T + t) * a.H + h] = x;
@@ -2343,6 +2335,7 @@ int launch_chunk_bwd(const BwdParams& p, hipStream_t stream) {
     wa.draw = ws.draw;
     wa.dlp = ws.dlp;
     wa.dlam = ws.dlam;
+    wa.dgq = ws.dgq;
     wa.dtab = ws.dtab;
     wa.B = B;
     wa.Tp = Tp;
@@ -2402,6 +2395,7 @@ int launch_chunk_bwd(const BwdParams& p, hipStream_t stream) {
     ro.dwts = ws.dwts;
     ro.draw = ws.draw;
     ro.dlam = ws.dlam;
+    ro.dgq = ws.dgq;
     ro.dtab = ws.dtab;
     ro.B = B;
     ro.Tp = Tp;
@@ -2446,13 +2440,7 @@ int launch_chunk_bwd(const BwdParams& p, hipStream_t stream) {
     if (launch_chunk_grad(c1, bf, stream) != 0) return -1;
     // gates, write vector and clock
     TokenGradArgs tg{};
-    tg.qh = ws.qh;
-    tg.kh = ws.kh;
-    tg.dqh = ws.dqh;
-    tg.dkh = ws.dkh;
-    tg.wts = ws.wts;
-    tg.w = ws.w;
-    tg.dwts = ws.dwts;
+    tg.dgq = ws.dgq;
     tg.dw2 = ws.dw2;
     tg.dw1 = ws.dw1;
     tg.cs = ws.cs;
@@ -2467,15 +2455,11 @@ int launch_chunk_bwd(const BwdParams& p, hipStream_t stream) {
     tg.T = T;
     tg.Tp = Tp;
     tg.H = H;
-    tg.K = K;
     tg.M = M;
     tg.N = N;
     tg.nt1 = ws.nt1;
     tg.nt2 = ws.nt2;
-    if (K % 4 == 0)
-        hipLaunchKernelGGL(bw_token_kernel<true>, dim3(N, B * H), blk, 0, stream, tg);
-    else
-        hipLaunchKernelGGL(bw_token_kernel<false>, dim3(N, B * H), blk, 0, stream, tg);
+    hipLaunchKernelGGL(bw_token_kernel, dim3(N, B * H), blk, 0, stream, tg);
     hipLaunchKernelGGL(bw_clock_kernel, dim3(B * H), dim3(64), 0, stream, ws.dlam, p.d_clock, B, T, Tp, H, p.ddelta,
                        p.dclock0);
     // the q/k norms, their weights, v's layout

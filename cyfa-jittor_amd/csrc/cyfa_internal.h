@@ -416,8 +416,8 @@ struct BwdParams {
 struct BwdWorkspace {
     double* lam;
     float *qh, *kh, *rq, *rk, *vh, *w, *cs, *sn, *raw, *wts, *sk, *sv;
-    float *dO, *dsk, *dsv, *dwts, *dw2, *dvh, *draw, *dlam, *dqh, *dkh, *dw1, *bnd1, *bnd2, *dtab, *dnq, *dnk;
-    float *lg, *dlw, *dlp;  // the wide readout (M > BWD_TABLE_M): logits / p, dp / dl [rows, 256]; clock partials [rows, 4]
+    float *dO, *dsk, *dsv, *dwts, *dw2, *dvh, *draw, *dlam, *dgq, *dqh, *dkh, *dw1, *bnd1, *bnd2, *dtab, *dnq, *dnk;
+    float *lg, *dlw, *dlp;  // the wide readout (M > BWD_TABLE_M): logits / p, dp / dl [rows, 256]; clock and gate partials [rows, 8]
     int N, nt1, nt2, ro_blocks, norm_blocks;
     size_t bytes;
 };
@@ -477,6 +477,7 @@ inline BwdWorkspace bwd_workspace(int B, int T, int H, int K, int V, int M, void
     w.dvh = f(rows * V);
     w.draw = f(rows * M);
     w.dlam = f(rows);
+    w.dgq = f(rows);
     w.dqh = f(rows * K);
     w.dkh = f(rows * K);
     w.dw1 = f(rows * M);
@@ -487,7 +488,7 @@ inline BwdWorkspace bwd_workspace(int B, int T, int H, int K, int V, int M, void
     w.dnk = f((size_t)w.norm_blocks * K);
     w.lg = f(wide ? rows * BWD_WIDE_MW : 0);
     w.dlw = f(wide ? rows * BWD_WIDE_MW : 0);
-    w.dlp = f(wide ? rows * (BWD_WIDE_MW / 64) : 0);
+    w.dlp = f(wide ? rows * 2 * (BWD_WIDE_MW / 64) : 0);
     w.bytes = off;
     return w;
 }
