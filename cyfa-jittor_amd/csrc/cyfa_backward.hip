@@ -1192,163 +1192,356 @@ __global__ __launch_bounds__(RO_FWD_THREADS) void bw_fwd_readout_kernel(const fl
     }
 }
 
-// The same readout with its two products as split-bf16 products on
-// v_mfma_f32_16x16x32_bf16 (every fp32 operand as a bf16 high part and a bf16
-// remainder, lo_a hi_b + hi_a lo_b + hi_a hi_b: about 16 mantissa bits; with
-// BF the operands are bf16 values and the products exact), for calls whose
-// tile products run on the matrix cores. The table sits in LDS once as its
-// two bf16 parts, row-major [r][m]: the logits read its rows as B fragments,
-// u gathers its columns. Wave w takes row tile w & 1 and the slot tiles
-// CPW (w >> 1) .. + CPW - 1 of both products (CPW = 16 / waves); the softmax
-// reductions on DPP moves.
-constexpr int RO_LDB = BWD_TABLE_M + 8;  // bf16 rows of the split table and row blocks
-// One workgroup per CU fits the LDS; its waves put several on each SIMD, so
-// that one wave's LDS reads and softmax overlap another's products.
-constexpr int RO_MF_THREADS = 1024;
+// The readout and its adjoint for calls with bf16 operands, every product as
+// split-bf16 products on v_mfma_f32_16x16x32_bf16 (each fp32 operand as a bf16
+// high part and a bf16 remainder, lo_a hi_b + hi_a lo_b + hi_a hi_b: about 16
+// mantissa bits; with BF, the general bf16 forward, the operands are bf16
+// values and the products exact). Per block of 32 rows of a head (the formulas
+// are those of bw_fwd_readout_kernel and bw_readout_kernel):
+//   z (and du) as two bf16 parts into LDS; logits (and dp); softmax (and dl);
+//   u (and dz); weights, or draw, the clock's and the gate's shares; dtable.
+// Wave w owns slots and coordinates 16 (w % 8) .. + 15 of every product (and,
+// with 16 waves, row tile w / 8) and holds the table's rows and columns for
+// them as operand registers (64 with both parts), so that the table takes no
+// LDS and no reads per block; its part of dtable stays in accumulators. The
+// products are formed transposed, slots (coordinates) by rows: a lane then
+// holds four neighbouring slots of one row, a row's reductions are three adds
+// and two lane swaps, and a coordinate pair sits in one lane. Row maxima and
+// sums cross the waves through LDS (8 floats per row and step). p and dl are
+// kept twice, by rows (operands of u and dz) and by slots (of dtable), so that
+// each operand is one 16-byte LDS read; du's and z's columns are gathered. Tp
+// is a multiple of 64, so a block's rows are consecutive rows of one batch
+// row, at one scalar base, and none is past the end. Grid (workgroups per
+// head, H); a workgroup takes per_wg blocks (bwd_ro_per_wg).
+// The adjoint's LDS (130 KB) holds one workgroup of eight waves per CU; sixteen
+// waves at 128 registers would spill. 65536 rows of 128 slots on MI355X: the
+// adjoint 76 us and the forward 40 us, where the table staged in LDS, sixteen
+// waves and the adjoint's products on the fp32 matrix cores took 164 and 76;
+// 16384 rows: 25 and 19 us, where they took 53 and 27. Products by rows instead
+// of slots, with a division per row and sums over 16 lanes: 119 and 62, 48 and
+// 30. Bound by the reads of p, dl, z and du from LDS and the vector ALU.
+constexpr int RO_LDB = BWD_TABLE_M + 8;    // bf16 row blocks [32][RO_LDB]
+constexpr int RO_LDP = BWD_RO_BLOCK + 8;   // p and dl by slots [128][RO_LDP]
+constexpr int RO_LDC = BWD_TABLE_M / 2 + 4;  // phases [32][RO_LDC]
+constexpr int RO_MF_FWD_WAVES = 8, RO_MF_ADJ_WAVES = 8;
 
 // lane (lr, lg) gets X[r0 + lr][k0 + 8 lg .. + 7] of a row-major bf16 tile
+template <int LD>
 __device__ __forceinline__ bf16x8 ro_row(const bf16_t* X, int r0, int k0) {
     const int l = threadIdx.x & 63;
-    return *reinterpret_cast<const bf16x8*>(X + (r0 + (l & 15)) * RO_LDB + k0 + 8 * (l >> 4));
+    return *reinterpret_cast<const bf16x8*>(X + (r0 + (l & 15)) * LD + k0 + 8 * (l >> 4));
 }
 
-// lane (lr, lg) gets X[s0 + 8 lg + j][c0 + lr], j = 0..7, of a row-major bf16
-// tile (a B fragment of the transpose), as eight 2-byte LDS reads
-__device__ __forceinline__ bf16x8 ro_col(const bf16_t* X, int s0, int c0) {
+// lane (lr, lg) gets X[8 lg + j][c0 + lr], j = 0..7, of a row-major bf16 tile
+// (an operand of its transpose), as eight 2-byte LDS reads
+__device__ __forceinline__ bf16x8 ro_col(const bf16_t* X, int c0) {
     const int l = threadIdx.x & 63;
-    const bf16_t* p = X + (s0 + 8 * (l >> 4)) * RO_LDB + c0 + (l & 15);
+    const bf16_t* p = X + 8 * (l >> 4) * RO_LDB + c0 + (l & 15);
     bf16x8 r;
 #pragma unroll
     for (int e = 0; e < 8; e++) r[e] = p[e * RO_LDB];
     return r;
 }
 
-__device__ __forceinline__ void split_store(bf16_t* hi, bf16_t* lo, int idx, float v) {
-    const bf16_t h = (bf16_t)v;
-    hi[idx] = h;
-    lo[idx] = (bf16_t)(v - (float)h);
+// c += A B over 32 k with both operands in two bf16 parts (ONE: in one, the
+// remainders zero)
+template <bool ONE>
+__device__ __forceinline__ f32x4 mfma_split(const bf16x8& ah, const bf16x8& al, const bf16x8& bh, const bf16x8& bl,
+                                            f32x4 c) {
+    if constexpr (!ONE) {
+        c = mfma_bf16(al, bh, c);
+        c = mfma_bf16(ah, bl, c);
+    }
+    return mfma_bf16(ah, bh, c);
 }
 
-template <bool BF>
-__global__ __launch_bounds__(RO_MF_THREADS) void bw_fwd_readout_mf_kernel(const float* raw, const float* cs, const float* sn,
-                                                                const float* table, int B, int Tp, int H, int M,
-                                                                int per_wg, float* wts) {
-    constexpr int TM = BWD_TABLE_M, LB = RO_LDB, RB = 32, NT = RO_MF_THREADS, NW = NT / 64, CPW = 16 / NW;
-    static_assert(TM == 128 && RB == 32 && (NW == 8 || NW == 16), "eight 16-wide tiles of slots, two of rows");
-    __shared__ __align__(16) bf16_t sTh[TM * LB], sTl[TM * LB];  // rows R .. 127 and columns M .. 127 zero
-    __shared__ __align__(16) bf16_t sZh[RB * LB], sZl[RB * LB], sPh[RB * LB], sPl[RB * LB];
-    __shared__ float sL[RB][TM + 4];
-    __shared__ float sCs[RB][TM / 2], sSn[RB][TM / 2];
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, h = blockIdx.y;
-    const int lr = lane & 15;
-    const int R = M - 1, P = M / 2, rows = B * Tp;
-    for (int e = tid; e < TM * TM; e += NT) {
-        const int r = e / TM, m = e % TM;
-        split_store(sTh, sTl, r * LB + m, (r < R && m < M) ? bw_rnd<BF>(table[((size_t)h * R + r) * M + m]) : 0.f);
+__device__ __forceinline__ bf16_t bf16_lo(float v) { return (bf16_t)(v - (float)(bf16_t)v); }
+
+// Four floats as bf16 high parts and remainders.
+__device__ __forceinline__ void bf16_split4(const f32x4& v, bf16x4& hi, bf16x4& lo) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        hi[q] = (bf16_t)v[q];
+        lo[q] = bf16_lo(v[q]);
     }
-    const auto row_of = [&](int rho) { return ((size_t)(rho / Tp) * H + h) * Tp + rho % Tp; };
-    const int it = wv & 1, ct0 = CPW * (wv >> 1);
+}
+
+// Sum (max) over the four lanes l, l ^ 16, l ^ 32, l ^ 48, in each of them:
+// permlane16_swap of a register with itself leaves lanes of 16-lane rows 0 and
+// 1 (2 and 3) with both rows' values, permlane32_swap both halves'.
+template <bool MX>
+__device__ __forceinline__ float rows4_reduce(float x) {
+    uint32_t u = __builtin_bit_cast(uint32_t, x);
+    auto w = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    uint32_t a = w[0], b = w[1];
+    float fa = __builtin_bit_cast(float, a), fb = __builtin_bit_cast(float, b);
+    u = __builtin_bit_cast(uint32_t, MX ? fmaxf(fa, fb) : fa + fb);
+    w = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    a = w[0], b = w[1];
+    fa = __builtin_bit_cast(float, a), fb = __builtin_bit_cast(float, b);
+    return MX ? fmaxf(fa, fb) : fa + fb;
+}
+
+struct ReadoutGradArgs {
+    const float *raw, *cs, *sn, *table, *dwts;  // head-major rows; table [H, M-1, M]
+    float* wts;                                 // the forward's slot weights
+    float *draw, *dlam, *dgq, *dtab;            // dgq: z.dz + u.du per row; dtab: [H, workgroups, (M-1) M]
+    int B, Tp, H, M;
+    int per_wg;                                 // blocks of 32 rows per workgroup
+};
+
+template <bool ADJ, bool BF, int NW>
+__global__ __launch_bounds__(64 * NW, ADJ ? NW / 4 : NW / 2) void bw_readout_mf_kernel(ReadoutGradArgs a) {
+    static_assert(!(ADJ && BF), "the adjoint is unrounded");
+    constexpr int TM = BWD_TABLE_M, RB = BWD_RO_BLOCK, LB = RO_LDB, KS = TM / 32, NT = 64 * NW;
+    constexpr int RT = 16 / NW, DT = 64 / NW;  // row tiles and dtable slot tiles of a wave
+    static_assert(TM == 128 && RB == 32 && (NW == 8 || NW == 16), "eight 16-wide tiles of slots, two of rows");
+    __shared__ __align__(16) bf16_t sZ[2][RB * LB], sP[2][RB * LB];                      // [part][row][m | slot]
+    __shared__ __align__(16) bf16_t sDU[ADJ ? 2 : 1][ADJ ? RB * LB : 8], sDL[ADJ ? 2 : 1][ADJ ? RB * LB : 8];
+    __shared__ __align__(16) bf16_t sPt[ADJ ? 2 : 1][ADJ ? TM * RO_LDP : 8], sDt[ADJ ? 2 : 1][ADJ ? TM * RO_LDP : 8];
+    __shared__ __align__(16) float sCs[RB * RO_LDC], sSn[RB * RO_LDC];
+    __shared__ __align__(16) float sMx[RB][8], sSum[RB][8], sSd[RB][8];
+    __shared__ float sLam[RB][8], sGq[RB][8];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), h = blockIdx.y;
+    const int lr = lane & 15, lg = lane >> 4, cw = wv & 7;
+    const int it0 = RT == 2 ? 0 : wv >> 3, dt0 = DT * (wv >> 3);  // DT == 8: wv >> 3 is 0
+    const int M = a.M, R = M - 1, P = M / 2, rows = a.B * a.Tp;
+    const auto load2 = [](bw_rsrc_t r, uint32_t off, bool live) {
+        return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off | (live ? 0u : BW_DEAD), 0, 0));
+    };
+    // the table's operands: rows r = 16 cw + lr (logits, dp) and columns m = 16 cw + lr (u, dz)
+    bf16x8 trh[KS], trl[KS], tch[KS], tcl[KS];
+    {
+        const int mine = 16 * cw + lr;
+        const bw_rsrc_t rt = bw_rsrc(a.table + (size_t)h * R * M, (size_t)R * M);
+        const auto put = [](bf16x8& hi, bf16x8& lo, int e, float v) {
+            v = bw_rnd<BF>(v);
+            hi[e] = (bf16_t)v;
+            lo[e] = bf16_lo(v);
+        };
+#pragma unroll
+        for (int k = 0; k < KS; k++)
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) {
+                const int kk = 32 * k + 8 * lg + e;  // even, as M is
+                const f32x2 vr = load2(rt, (uint32_t)(mine * M + kk) * 4u, mine < R && kk < M);
+                put(trh[k], trl[k], e, vr[0]);
+                put(trh[k], trl[k], e + 1, vr[1]);
+                put(tch[k], tcl[k], e, bw_load(rt, (uint32_t)(kk * M + mine) * 4u, kk < R && mine < M));
+                put(tch[k], tcl[k], e + 1, bw_load(rt, (uint32_t)(kk * M + M + mine) * 4u, kk + 1 < R && mine < M));
+            }
+    }
+    const int s0 = 16 * cw + 4 * lg;  // this lane's slots and coordinates s0 .. s0 + 3: pairs s0 / 2, s0 / 2 + 1
+    float kappa[2];
+#pragma unroll
+    for (int j = 0; j < 2; j++) kappa[j] = s0 / 2 + j < P ? (float)(kTwoPiBw * (s0 / 2 + j) / R) : 0.f;
+    f32x4 dacc[ADJ ? DT : 1];  // dtable rows 16 (dt0 + rt) .. of column 16 cw + lr
+#pragma unroll
+    for (int rt = 0; rt < (ADJ ? DT : 1); rt++) dacc[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // A block's inputs, element x of this thread = (row i, pair pr) = e / 64,
+    // e % 64, e = tid + NT x: loaded one block ahead through buffer resources
+    // (rows < 2^21, M <= 128: offsets below 2^30), predicated through the
+    // offset, so that no block waits for its own loads.
     constexpr int NX = RB * (TM / 2) / NT;
-    const int b_end = min(rows, (int)(blockIdx.x + 1) * per_wg * RB);
-    const bw_rsrc_t rcs = bw_rsrc(cs, (size_t)rows * H * P), rsn = bw_rsrc(sn, (size_t)rows * H * P),
-                    rraw = bw_rsrc(raw, (size_t)rows * H * M);  // every head's rows
-    float nc[NX], ns[NX], nre[NX], nro[NX];
+    const int b_first = blockIdx.x * a.per_wg * RB, b_end = min(rows, b_first + a.per_wg * RB);
+    const auto base_of = [&](int b0) { return ((size_t)(b0 / a.Tp) * a.H + h) * a.Tp + b0 % a.Tp; };
+    const bw_rsrc_t rcs = bw_rsrc(a.cs, (size_t)rows * a.H * P), rsn = bw_rsrc(a.sn, (size_t)rows * a.H * P),
+                    rraw = bw_rsrc(a.raw, (size_t)rows * a.H * M),
+                    rdw = bw_rsrc(a.dwts, ADJ ? (size_t)rows * a.H * M : 0);
+    const int pr_in = tid % (TM / 2), i_in = tid / (TM / 2);
+    float nc[NX], ns[NX];
+    f32x2 nr[NX], nd[NX];
     const auto load_block = [&](int b0) {
+        const bool live = b0 < b_end && pr_in < P;
+        const uint32_t row0 = (b0 < b_end ? (uint32_t)base_of(b0) : 0u) + (uint32_t)i_in;
 #pragma unroll
         for (int x = 0; x < NX; x++) {
-            const int e = tid + NT * x, i = e / (TM / 2), pr = e % (TM / 2), rho = b0 + i;
-            const bool live = rho < b_end && pr < P;
-            const uint32_t row = live ? (uint32_t)row_of(rho) : 0u;
-            nc[x] = bw_load(rcs, (row * (uint32_t)P + (uint32_t)pr) * 4u, live);
-            ns[x] = bw_load(rsn, (row * (uint32_t)P + (uint32_t)pr) * 4u, live);
-            nre[x] = bw_load(rraw, (row * (uint32_t)M + 2u * (uint32_t)pr) * 4u, live);
-            nro[x] = bw_load(rraw, (row * (uint32_t)M + 2u * (uint32_t)pr + 1u) * 4u, live);
+            const uint32_t at = ((row0 + (uint32_t)(NT / (TM / 2) * x)) * (uint32_t)P + (uint32_t)pr_in) * 4u;
+            nc[x] = bw_load(rcs, at, live);
+            ns[x] = bw_load(rsn, at, live);
+            nr[x] = load2(rraw, 2u * at, live);
+            if constexpr (ADJ) nd[x] = load2(rdw, 2u * at, live);
         }
     };
-    const int b_first = blockIdx.x * per_wg * RB;
     load_block(b_first);
     for (int b0 = b_first; b0 < b_end; b0 += RB) {
-        __syncthreads();  // the table is staged; the previous block's tiles are done with
+        __syncthreads();  // the previous block's tiles are done with
 #pragma unroll
         for (int x = 0; x < NX; x++) {
-            const int e = tid + NT * x, i = e / (TM / 2), pr = e % (TM / 2);
-            const bool live = b0 + i < b_end && pr < P;
-            const float c = live ? nc[x] : 1.f, s = ns[x];
-            sCs[i][pr] = c;
-            sSn[i][pr] = s;
-            split_store(sZh, sZl, i * LB + 2 * pr, bw_rnd<BF>(c * nre[x] - s * nro[x]));  // zero where !live
-            split_store(sZh, sZl, i * LB + 2 * pr + 1, bw_rnd<BF>(s * nre[x] + c * nro[x]));
+            const int i = i_in + NT / (TM / 2) * x;
+            const float c = pr_in < P ? nc[x] : 1.f, s = ns[x];  // zero inputs past P
+            sCs[i * RO_LDC + pr_in] = c;
+            sSn[i * RO_LDC + pr_in] = s;
+            const auto put2 = [&](bf16_t* hi, bf16_t* lo, float v0, float v1) {
+                *reinterpret_cast<bf16x2*>(hi + i * LB + 2 * pr_in) = bf16x2{(bf16_t)v0, (bf16_t)v1};
+                if constexpr (!BF) *reinterpret_cast<bf16x2*>(lo + i * LB + 2 * pr_in) = bf16x2{bf16_lo(v0), bf16_lo(v1)};
+            };
+            put2(sZ[0], sZ[1], bw_rnd<BF>(c * nr[x][0] - s * nr[x][1]), bw_rnd<BF>(s * nr[x][0] + c * nr[x][1]));
+            if constexpr (ADJ) put2(sDU[0], sDU[1], c * nd[x][0] - s * nd[x][1], s * nd[x][0] + c * nd[x][1]);
         }
         load_block(b0 + RB);  // the next block (past the end: dead loads)
         __syncthreads();
-        {  // logits l[i][r] = sum_m z[i][m] table[r][m]
-            f32x4 acc[CPW];
+        // logits l[r][i] = table[r] . z[i] and dp[r][i] = table[r] . du[i]: lane holds
+        // slots s0 + q of row 16 (it0 + t) + lr
+        f32x4 l[RT], dp[RT];
 #pragma unroll
-            for (int t = 0; t < CPW; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int t = 0; t < RT; t++) {
+            const int i0 = 16 * (it0 + t);
+            l[t] = dp[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int k0 = 0; k0 < TM; k0 += 32) {
-                const bf16x8 ah = ro_row(sZh, 16 * it, k0), al = ro_row(sZl, 16 * it, k0);
-#pragma unroll
-                for (int t = 0; t < CPW; t++) {
-                    const bf16x8 bh = ro_row(sTh, 16 * (ct0 + t), k0), bl = ro_row(sTl, 16 * (ct0 + t), k0);
-                    acc[t] = mfma_bf16(al, bh, acc[t]);
-                    acc[t] = mfma_bf16(ah, bl, acc[t]);
-                    acc[t] = mfma_bf16(ah, bh, acc[t]);
-                }
+            for (int k = 0; k < KS; k++) {
+                l[t] = mfma_split<BF>(trh[k], trl[k], ro_row<LB>(sZ[0], i0, 32 * k), ro_row<LB>(sZ[1], i0, 32 * k), l[t]);
+                if constexpr (ADJ)
+                    dp[t] = mfma_split<BF>(trh[k], trl[k], ro_row<LB>(sDU[0], i0, 32 * k), ro_row<LB>(sDU[1], i0, 32 * k), dp[t]);
             }
-            const int lg = lane >> 4;
+            // softmax over the slots (this wave's 16, then the eight waves), and dl = p (dp - p . dp)
 #pragma unroll
-            for (int t = 0; t < CPW; t++)
-#pragma unroll
-                for (int q = 0; q < 4; q++) sL[16 * it + 4 * lg + q][16 * (ct0 + t) + lr] = acc[t][q];
+            for (int q = 0; q < 4; q++) l[t][q] = s0 + q < R ? l[t][q] : -INFINITY;
+            const float mx = rows4_reduce<true>(fmaxf(fmaxf(l[t][0], l[t][1]), fmaxf(l[t][2], l[t][3])));
+            if (lg == 0) sMx[i0 + lr][cw] = mx;
         }
         __syncthreads();
-        for (int i = wv; i < RB; i += NW) {
-            const float l0 = lane < R ? sL[i][lane] : -INFINITY, l1 = lane + 64 < R ? sL[i][lane + 64] : -INFINITY;
-            const float mx = bw_wave_max(fmaxf(l0, l1));
-            const float e0 = lane < R ? expf(l0 - mx) : 0.f, e1 = lane + 64 < R ? expf(l1 - mx) : 0.f;
-            const float inv = 1.f / bw_wave_sum(e0 + e1);
-            split_store(sPh, sPl, i * LB + lane, bw_rnd<BF>(e0 * inv));
-            split_store(sPh, sPl, i * LB + lane + 64, bw_rnd<BF>(e1 * inv));
-        }
-        __syncthreads();
-        // u[i][m] = sum_r p[i][r] table[r][m] (p and the table zero at r >= R); the
-        // weights' pair (2 pr, 2 pr + 1) sits in lanes (lr, lr ^ 1), swapped in by
-        // quad_perm [1,0,3,2]
-        f32x4 acc[CPW];
+        const auto across = [&](const float* v, bool mx) {  // over the waves, in wave order
+            const f32x4 v0 = *reinterpret_cast<const f32x4*>(v), v1 = *reinterpret_cast<const f32x4*>(v + 4);
+            if (mx) return fmaxf(fmaxf(fmaxf(v0[0], v0[1]), fmaxf(v0[2], v0[3])), fmaxf(fmaxf(v1[0], v1[1]), fmaxf(v1[2], v1[3])));
+            return ((v0[0] + v0[1]) + (v0[2] + v0[3])) + ((v1[0] + v1[1]) + (v1[2] + v1[3]));
+        };
 #pragma unroll
-        for (int t = 0; t < CPW; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int k0 = 0; k0 < TM; k0 += 32) {
-            const bf16x8 ah = ro_row(sPh, 16 * it, k0), al = ro_row(sPl, 16 * it, k0);
-#pragma unroll
-            for (int t = 0; t < CPW; t++) {
-                const bf16x8 bh = ro_col(sTh, k0, 16 * (ct0 + t)), bl = ro_col(sTl, k0, 16 * (ct0 + t));
-                acc[t] = mfma_bf16(al, bh, acc[t]);
-                acc[t] = mfma_bf16(ah, bl, acc[t]);
-                acc[t] = mfma_bf16(ah, bh, acc[t]);
-            }
-        }
-        const bool odd = (lr & 1) != 0;
-        const int lk = lane >> 4;
-#pragma unroll
-        for (int t = 0; t < CPW; t++) {
-            const int m = 16 * (ct0 + t) + lr, pr = m >> 1;
+        for (int t = 0; t < RT; t++) {
+            const int i = 16 * (it0 + t) + lr;
+            const float mx = across(sMx[i], true);
+            float sum = 0.f, sd = 0.f;
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-                const float un = acc[t][q], ux = dpp_mov<0xB1>(un);
-                const float ue = odd ? ux : un, uo = odd ? un : ux;
-                const int i = 16 * it + 4 * lk + q, rho = b0 + i;
-                if (rho < b_end && pr < P) {
-                    const float c = sCs[i][pr], s = sSn[i][pr];
-                    wts[row_of(rho) * M + m] = bw_rnd<BF>(odd ? -s * ue + c * uo : c * ue + s * uo);
+                l[t][q] = s0 + q < R ? expf(l[t][q] - mx) : 0.f;
+                sum += l[t][q];
+                if constexpr (ADJ) sd += l[t][q] * dp[t][q];
+            }
+            sum = rows4_reduce<false>(sum);
+            if (lg == 0) sSum[i][cw] = sum;
+            if constexpr (ADJ) {
+                sd = rows4_reduce<false>(sd);
+                if (lg == 0) sSd[i][cw] = sd;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < RT; t++) {
+            const int i = 16 * (it0 + t) + lr;
+            const float inv = 1.f / across(sSum[i], false);
+            const float pdp = ADJ ? across(sSd[i], false) * inv : 0.f;
+            f32x4 p, d;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                p[q] = bw_rnd<BF>(l[t][q] * inv);
+                d[q] = ADJ ? p[q] * (dp[t][q] - pdp) : 0.f;
+            }
+            bf16x4 hi, lo;
+            bf16_split4(p, hi, lo);
+            *reinterpret_cast<bf16x4*>(sP[0] + i * LB + s0) = hi;
+            if constexpr (!BF) *reinterpret_cast<bf16x4*>(sP[1] + i * LB + s0) = lo;
+            if constexpr (ADJ) {
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    sPt[0][(s0 + q) * RO_LDP + i] = hi[q];
+                    sPt[1][(s0 + q) * RO_LDP + i] = lo[q];
                 }
+                bf16_split4(d, hi, lo);
+                *reinterpret_cast<bf16x4*>(sDL[0] + i * LB + s0) = hi;
+                *reinterpret_cast<bf16x4*>(sDL[1] + i * LB + s0) = lo;
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    sDt[0][(s0 + q) * RO_LDP + i] = hi[q];
+                    sDt[1][(s0 + q) * RO_LDP + i] = lo[q];
+                }
+            }
+        }
+        __syncthreads();
+        // u[m][i] = sum_r table[r][m] p[i][r] and dz[m][i] = sum_r table[r][m] dl[i][r]
+        // (p, dl and the table are zero at r >= R): lane holds coordinates s0 + q of row
+        // 16 (it0 + t) + lr
+        const size_t row0 = base_of(b0);
+#pragma unroll
+        for (int t = 0; t < RT; t++) {
+            const int i0 = 16 * (it0 + t), i = i0 + lr;
+            f32x4 u = {0.f, 0.f, 0.f, 0.f}, dz = u;
+#pragma unroll
+            for (int k = 0; k < KS; k++) {
+                u = mfma_split<BF>(tch[k], tcl[k], ro_row<LB>(sP[0], i0, 32 * k), ro_row<LB>(sP[1], i0, 32 * k), u);
+                if constexpr (ADJ)
+                    dz = mfma_split<BF>(tch[k], tcl[k], ro_row<LB>(sDL[0], i0, 32 * k), ro_row<LB>(sDL[1], i0, 32 * k), dz);
+            }
+            const f32x2 c2 = *reinterpret_cast<const f32x2*>(sCs + i * RO_LDC + s0 / 2);
+            const f32x2 s2 = *reinterpret_cast<const f32x2*>(sSn + i * RO_LDC + s0 / 2);
+            float* dst = (ADJ ? a.draw : a.wts) + (row0 + i) * M + s0;
+            const f32x4 x = ADJ ? dz : u;
+#pragma unroll
+            for (int j = 0; j < 2; j++) {  // U(-lam) of a pair
+                const float c = c2[j], s = s2[j], e = x[2 * j], o = x[2 * j + 1];
+                if (s0 / 2 + j < P)
+                    *reinterpret_cast<f32x2*>(dst + 2 * j) = f32x2{bw_rnd<BF>(c * e + s * o), bw_rnd<BF>(-s * e + c * o)};
+            }
+            if constexpr (ADJ) {
+                // With z = U(lam) raw and du = U(lam) dweights, the clock's share
+                // kappa_p [dz . dU(lam)/dlam raw + dweights . dU(-lam)/dlam u] is
+                // kappa_p [(z_e dz_o - z_o dz_e) + (du_e u_o - du_o u_e)] (a rotation keeps
+                // the 2-d cross product); the gate's is z . dz + u . du.
+                const auto sum4 = [&](const bf16_t* hi, const bf16_t* lo) {
+                    const bf16x4 vh = *reinterpret_cast<const bf16x4*>(hi + i * LB + s0);
+                    const bf16x4 vl = *reinterpret_cast<const bf16x4*>(lo + i * LB + s0);
+                    return f32x4{(float)vh[0] + (float)vl[0], (float)vh[1] + (float)vl[1], (float)vh[2] + (float)vl[2],
+                                 (float)vh[3] + (float)vl[3]};
+                };
+                const f32x4 z = sum4(sZ[0], sZ[1]), du = sum4(sDU[0], sDU[1]);
+                float v = 0.f, g = 0.f;  // zero past M
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    const int e = 2 * j, o = 2 * j + 1;
+                    v += kappa[j] * ((z[e] * dz[o] - z[o] * dz[e]) + (du[e] * u[o] - du[o] * u[e]));
+                    g += (z[e] * dz[e] + du[e] * u[e]) + (z[o] * dz[o] + du[o] * u[o]);
+                }
+                v = rows4_reduce<false>(v);
+                g = rows4_reduce<false>(g);
+                if (lg == 0) {
+                    sLam[i][cw] = v;
+                    sGq[i][cw] = g;
+                }
+            }
+        }
+        if constexpr (ADJ) {
+            // dtable[r][m] += sum_i p[i][r] du[i][m] + dl[i][r] z[i][m] over the block's rows
+            const bf16x8 uh = ro_col(sDU[0], 16 * cw), ul = ro_col(sDU[1], 16 * cw);
+            const bf16x8 zh = ro_col(sZ[0], 16 * cw), zl = ro_col(sZ[1], 16 * cw);
+#pragma unroll
+            for (int rt = 0; rt < DT; rt++) {
+                const int r0 = 16 * (dt0 + rt);
+                dacc[rt] = mfma_split<BF>(ro_row<RO_LDP>(sPt[0], r0, 0), ro_row<RO_LDP>(sPt[1], r0, 0), uh, ul, dacc[rt]);
+                dacc[rt] = mfma_split<BF>(ro_row<RO_LDP>(sDt[0], r0, 0), ro_row<RO_LDP>(sDt[1], r0, 0), zh, zl, dacc[rt]);
+            }
+            __syncthreads();
+            if (tid < RB) {  // the clock's and the gate's share per row, in wave order
+                float v = sLam[tid][0], g = sGq[tid][0];
+#pragma unroll
+                for (int j = 1; j < 8; j++) v += sLam[tid][j], g += sGq[tid][j];
+                a.dlam[row0 + tid] = v;
+                a.dgq[row0 + tid] = g;
             }
         }
     }
+    if constexpr (ADJ) {  // lane holds dtable rows 16 (dt0 + rt) + 4 lg + q of column 16 cw + lr
+        float* dst = a.dtab + ((size_t)h * gridDim.x + blockIdx.x) * R * M;
+        const int m = 16 * cw + lr;
+#pragma unroll
+        for (int rt = 0; rt < DT; rt++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int r = 16 * (dt0 + rt) + 4 * lg + q;
+                if (r < R && m < M) dst[r * M + m] = dacc[rt][q];
+            }
+    }
 }
 
-// The slot-readout adjoint for blocks of 32 rows of one head (z = U(lam) raw,
+// The slot-readout adjoint of fp32 calls for blocks of 32 rows of one head (z = U(lam) raw,
 // l = table z, p = softmax(l), u = table^T p, weights = U(-lam) u):
 //   du = U(lam) dweights, dp = table du, dl = p (dp - p.dp), dz = table^T dl,
 //   draw = U(-lam) dz, dtable += p du^T + dl z^T, and the clock's share
@@ -1367,12 +1560,6 @@ __global__ __launch_bounds__(RO_MF_THREADS) void bw_fwd_readout_mf_kernel(const 
 // matrix-core steps.
 constexpr int RO_BLK = BWD_RO_BLOCK;
 constexpr int RO_ADJ_THREADS = 1024;
-struct ReadoutGradArgs {
-    const float *raw, *cs, *sn, *table, *dwts;  // head-major rows; table [H, M-1, M]
-    float *draw, *dlam, *dgq, *dtab;            // dgq: z.dz + u.du per row; dtab: [H, workgroups, (M-1) M]
-    int B, Tp, H, M;
-    int per_wg;                                 // blocks of 32 rows per workgroup
-};
 
 __global__ __launch_bounds__(RO_ADJ_THREADS) void bw_readout_kernel(ReadoutGradArgs a) {
     constexpr int TM = BWD_TABLE_M, LD = RO_LD, NT = RO_ADJ_THREADS, NW = NT / 64;
@@ -2234,14 +2421,23 @@ int launch_chunk_readout(const float* raw, const float* cs, const float* sn, con
                            stream, wa);
         return 0;
     }
-    const int per = bwd_ro_per_wg(B, Tp, H), blocks = (B * Tp + BWD_RO_BLOCK - 1) / BWD_RO_BLOCK;
+    const int per = bwd_ro_per_wg(B, Tp, H, split ? 512 : 256), blocks = (B * Tp + BWD_RO_BLOCK - 1) / BWD_RO_BLOCK;
     const dim3 grid((blocks + per - 1) / per, H);
+    ReadoutGradArgs ro{};
+    ro.raw = raw;
+    ro.cs = cs;
+    ro.sn = sn;
+    ro.table = table;
+    ro.wts = wts;
+    ro.B = B;
+    ro.Tp = Tp;
+    ro.H = H;
+    ro.M = M;
+    ro.per_wg = per;
     if (split && bf16)
-        hipLaunchKernelGGL(bw_fwd_readout_mf_kernel<true>, grid, dim3(RO_MF_THREADS), 0, stream, raw, cs, sn, table, B, Tp, H, M, per,
-                           wts);
+        hipLaunchKernelGGL((bw_readout_mf_kernel<false, true, RO_MF_FWD_WAVES>), grid, dim3(64 * RO_MF_FWD_WAVES), 0, stream, ro);
     else if (split)
-        hipLaunchKernelGGL(bw_fwd_readout_mf_kernel<false>, grid, dim3(RO_MF_THREADS), 0, stream, raw, cs, sn, table, B, Tp, H, M, per,
-                           wts);
+        hipLaunchKernelGGL((bw_readout_mf_kernel<false, false, RO_MF_FWD_WAVES>), grid, dim3(64 * RO_MF_FWD_WAVES), 0, stream, ro);
     else if (bf16)
         hipLaunchKernelGGL(bw_fwd_readout_kernel<true>, grid, dim3(RO_FWD_THREADS), 0, stream, raw, cs, sn, table, B, Tp, H, M, per,
                            wts);
@@ -2321,7 +2517,7 @@ int launch_chunk_bwd(const BwdParams& p, hipStream_t stream) {
     if (launch_chunk_pass(p1, stream) != 0 ||
         launch_chunk_readout(ws.raw, ws.cs, ws.sn, p.table, ws.lg, B, Tp, H, M, 0, bf, ws.wts, stream) != 0)
         return -1;
-    const int ro_per_wg = bwd_ro_per_wg(B, Tp, H);
+    const int ro_per_wg = bwd_ro_per_wg(B, Tp, H, 256);
     const bool wide = M > BWD_TABLE_M;
     WideArgs wa{};
     wa.raw = ws.raw;
@@ -2409,6 +2605,8 @@ int launch_chunk_bwd(const BwdParams& p, hipStream_t stream) {
         hipLaunchKernelGGL(bw_wide_dlam_kernel, dim3((unsigned)((rows + 255) / 256)), blk, 0, stream, wa);
         hipLaunchKernelGGL(bw_wide_dtable_kernel, dim3((M - 1 + BC - 1) / BC, (M + BC - 1) / BC, H * ws.ro_blocks), blk, 0,
                            stream, wa);
+    } else if (bf) {
+        hipLaunchKernelGGL((bw_readout_mf_kernel<true, false, RO_MF_ADJ_WAVES>), dim3(ws.ro_blocks, H), dim3(64 * RO_MF_ADJ_WAVES), 0, stream, ro);
     } else {
         hipLaunchKernelGGL(bw_readout_kernel, dim3(ws.ro_blocks, H), dim3(RO_ADJ_THREADS), 0, stream, ro);
     }

@@ -426,11 +426,13 @@ constexpr int BWD_WIDE_SPLIT = 1024;  // token rows per table-cotangent partial 
 constexpr int BWD_SCAN_ROWS = 32;   // rows of a state-scan tile (its columns: 32)
 constexpr int BWD_NORM_ROWS = 64;   // rows per norm-adjoint workgroup
 
-// Blocks of 32 rows per readout workgroup: up to eight (the head's table is
-// staged once per workgroup), as long as 512 or more workgroups remain.
-inline int bwd_ro_per_wg(int B, int Tp, int H) {
-    const int blocks = (B * Tp + BWD_RO_BLOCK - 1) / BWD_RO_BLOCK, per = blocks * H / 512;
-    return per < 1 ? 1 : per > 8 ? 8 : per;
+// Blocks of 32 rows per readout workgroup: rows shared over the wgs workgroups
+// that the chip holds at once (each takes the head's table once), 16 blocks at
+// most.
+inline int bwd_ro_per_wg(int B, int Tp, int H, int wgs) {
+    const int blocks = (B * Tp + BWD_RO_BLOCK - 1) / BWD_RO_BLOCK;
+    const int per = (int)(((long long)blocks * H + wgs - 1) / wgs);
+    return per < 1 ? 1 : per > 16 ? 16 : per;
 }
 
 inline BwdWorkspace bwd_workspace(int B, int T, int H, int K, int V, int M, void* base) {
@@ -451,7 +453,7 @@ inline BwdWorkspace bwd_workspace(int B, int T, int H, int K, int V, int M, void
     if (wide) {  // the table cotangent's partials: one per BWD_WIDE_SPLIT token rows of a head
         w.ro_blocks = (int)((B * Tp + BWD_WIDE_SPLIT - 1) / BWD_WIDE_SPLIT);
     } else {
-        const int blocks = (int)((B * Tp + BWD_RO_BLOCK - 1) / BWD_RO_BLOCK), per = bwd_ro_per_wg(B, (int)Tp, H);
+        const int blocks = (int)((B * Tp + BWD_RO_BLOCK - 1) / BWD_RO_BLOCK), per = bwd_ro_per_wg(B, (int)Tp, H, 256);
         w.ro_blocks = (blocks + per - 1) / per;  // readout workgroups per head
     }
     w.norm_blocks = (int)(((size_t)B * T * H + BWD_NORM_ROWS - 1) / BWD_NORM_ROWS);
