@@ -615,10 +615,16 @@ int cyfa_short_conv_grad(const CyfaConvGradArgs* a, int dtype, void* hip_stream)
     if (a->B <= 0 || a->T <= 0 || a->D <= 0) return fail(CYFA_ERR_VALUE, "%s: B=%d T=%d D=%d", what, a->B, a->T, a->D);
     if (a->W < 2 || a->W > 4) return fail(CYFA_ERR_UNSUPPORTED, "%s: width %d not in 2..4", what, a->W);
     if (a->D % 8 != 0) return fail(CYFA_ERR_UNSUPPORTED, "%s: D=%d is not a multiple of 8", what, a->D);
-    if (!a->x || !a->weight || !a->dy || !a->workspace) return fail(CYFA_ERR_VALUE, "%s: null required pointer", what);
+    const int split = a->split ? a->split : a->D, parts = split > 0 ? a->D / split : 0;
+    if (parts < 1 || parts > 3 || parts * split != a->D || split % 8)
+        return fail(CYFA_ERR_VALUE, "%s: split=%d of D=%d", what, a->split, a->D);
+    if (!a->x || !a->weight || !a->dy || !a->workspace || (parts > 1 && !a->dy1) || (parts > 2 && !a->dy2))
+        return fail(CYFA_ERR_VALUE, "%s: null required pointer", what);
+    const long long dx_row = a->dx_row ? a->dx_row : a->D;
     if (a->workspace_bytes < cyfa::conv_grad_workspace_bytes(a->B, a->T, a->D, a->W))
         return fail(CYFA_ERR_WORKSPACE, "%s: workspace of %zu bytes", what, a->workspace_bytes);
     if (!aligned(a->x, 16) || a->x_row < a->D || a->x_row % 8 || !aligned(a->dy, 16) || !aligned(a->workspace, 16) ||
+        (parts > 1 && !aligned(a->dy1, 16)) || (parts > 2 && !aligned(a->dy2, 16)) || dx_row < a->D || dx_row % 8 ||
         (a->dx && !aligned(a->dx, 16)) || (a->dcache && !aligned(a->dcache, 16)) ||
         (a->cache && (!aligned(a->cache, 16) || a->cache_row % 8 || a->cache_batch % 8)))
         return fail(CYFA_ERR_ALIGN, "%s: rows need 16-byte alignment", what);
@@ -633,8 +639,12 @@ int cyfa_short_conv_grad(const CyfaConvGradArgs* a, int dtype, void* hip_stream)
     p.cache_row = a->cache_row;
     p.cache_batch = a->cache_batch;
     p.weight = a->weight;
-    p.dy = a->dy;
+    p.dy[0] = a->dy;
+    p.dy[1] = a->dy1;
+    p.dy[2] = a->dy2;
+    p.split = split;
     p.dx = a->dx;
+    p.dx_row = dx_row;
     p.dcache = a->dcache;
     p.dweight = a->dweight;
     p.dbias = a->dbias;

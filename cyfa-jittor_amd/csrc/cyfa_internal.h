@@ -168,8 +168,11 @@ struct ConvGradParams {
     long long x_row;
     const void* cache;           // nullable: [B, W-1, D] view
     long long cache_row, cache_batch;
-    const void *weight, *dy;     // [D, W]; [B, T, D]
-    void *dx, *dcache;           // nullable [B, T, D], [B, W-1, D]
+    const void* weight;          // [D, W]
+    const void* dy[3];           // channel c at dy[c / split][(b T + t) split + c % split]
+    int split;
+    void *dx, *dcache;           // nullable: (b, t, c) at dx[(b T + t) dx_row + c]; [B, W-1, D]
+    long long dx_row;
     void *dweight, *dbias;       // nullable [D, W], [D]
     float* part;                 // conv_grad_workspace_bytes
 };

@@ -41,7 +41,8 @@ __device__ __forceinline__ void store4(E* p, f32x4 v) {
 // adds the partials). x and dy are read once, dx written once (the partials
 // are W + 1 floats per channel and 64 tokens), so a large call is bound by HBM;
 // 2 x 1500 tokens of 1024 bf16 channels (18 MB) take 11.2 + 3.9 us on MI355X,
-// latency of a few waves per SIMD. The library's depthwise convolution, as
+// latency of a few waves per SIMD; q's, k's and v's channels in one call (dy in
+// three parts) 16.9 us, where three calls took 32. The library's depthwise convolution, as
 // F.conv1d reaches it, took about 320 us forward and backward for such a
 // tensor: transposes to channel-major, im2col, a GEMM per direction.
 constexpr int CG_RUN = 16, CG_TOKENS = 4 * CG_RUN, CG_CHANNELS = 256;
@@ -53,7 +54,8 @@ __global__ __launch_bounds__(256) void conv_grad_kernel(ConvGradParams p) {
     const int c = blockIdx.x * CG_CHANNELS + 4 * lane, t0 = blockIdx.z * CG_TOKENS + wv * CG_RUN;
     const int T = p.T, D = p.D;
     const E* x = static_cast<const E*>(p.x) + (size_t)b * T * p.x_row;
-    const E* dy = static_cast<const E*>(p.dy) + (size_t)b * T * D;
+    const int part_of = c < D ? c / p.split : 0, S = p.split;  // a lane's four channels are of one part
+    const E* dy = static_cast<const E*>(p.dy[part_of]) + (size_t)b * T * S + (c - part_of * S);
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     f32x4 dw[W + 1];  // dw[W]: the bias
 #pragma unroll
@@ -75,7 +77,7 @@ __global__ __launch_bounds__(256) void conv_grad_kernel(ConvGradParams p) {
 #pragma unroll
         for (int w = 0; w < W - 1; w++) {
             xw[w] = x_at(t0 + w - (W - 1));
-            dyw[w] = t0 + w < T ? load4(dy + (size_t)(t0 + w) * D + c) : zero;
+            dyw[w] = t0 + w < T ? load4(dy + (size_t)(t0 + w) * S) : zero;
         }
         if (t0 == 0 && p.dcache) {  // X[j - (W - 1)] feeds y[0 .. j]
             E* dc = static_cast<E*>(p.dcache) + (size_t)b * (W - 1) * D + c;
@@ -87,7 +89,7 @@ __global__ __launch_bounds__(256) void conv_grad_kernel(ConvGradParams p) {
                 store4(dc + (size_t)j * D, s);
             }
         }
-        E* dx = p.dx ? static_cast<E*>(p.dx) + (size_t)b * T * D + c : nullptr;
+        E* dx = p.dx ? static_cast<E*>(p.dx) + (size_t)b * T * p.dx_row + c : nullptr;
         constexpr int U = 8;
         for (int tb = t0; tb < t0 + CG_RUN && tb < T; tb += U) {
             f32x4 xn[U], dn[U];  // X[tb + u] and dy[tb + u + W - 1], rows past the end read as row T - 1 and dropped
@@ -95,7 +97,7 @@ __global__ __launch_bounds__(256) void conv_grad_kernel(ConvGradParams p) {
             for (int u = 0; u < U; u++) {
                 const int i = tb + u, j = tb + u + W - 1;
                 xn[u] = load4(x + (size_t)(i < T ? i : T - 1) * p.x_row + c);
-                dn[u] = load4(dy + (size_t)(j < T ? j : T - 1) * D + c);
+                dn[u] = load4(dy + (size_t)(j < T ? j : T - 1) * S);
             }
 #pragma unroll
             for (int u = 0; u < U; u++) {
@@ -109,7 +111,7 @@ __global__ __launch_bounds__(256) void conv_grad_kernel(ConvGradParams p) {
                     dw[w] += dyw[0] * xw[w];
                 }
                 dw[W] += dyw[0];
-                if (dx && t < T) store4(dx + (size_t)t * D, s);
+                if (dx && t < T) store4(dx + (size_t)t * p.dx_row, s);
 #pragma unroll
                 for (int w = 0; w < W - 1; w++) {
                     xw[w] = xw[w + 1];

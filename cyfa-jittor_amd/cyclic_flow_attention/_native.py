@@ -14,7 +14,7 @@ import torch
 import torch.nn.functional as F
 
 LIB_PATH = Path(os.environ.get("CYFA_LIB", Path(__file__).with_name("libcyfa_hip.so")))
-ABI_VERSION = 15
+ABI_VERSION = 16
 
 CYFA_OK = 0
 CYFA_ERR_VALUE = -1
@@ -148,6 +148,7 @@ class CyfaConvGradArgs(ctypes.Structure):
         ("weight", _c_void_p), ("dy", _c_void_p), ("dx", _c_void_p), ("dcache", _c_void_p),
         ("dweight", _c_void_p), ("dbias", _c_void_p),
         ("workspace", _c_void_p), ("workspace_bytes", _c_size_t),
+        ("split", _c_int), ("dy1", _c_void_p), ("dy2", _c_void_p), ("dx_row", ctypes.c_longlong),
     ]
 
 
@@ -796,22 +797,28 @@ def norm_grad(x, weight, gate, eps, prescale, dy, needed):
 SHORT_CONV_MAX_GRID = 65535  # batch rows, and blocks of 32 tokens, of a short_conv launch
 
 
-def short_conv_grad(x, weight, cache, dy, needed):
+def short_conv_grad(x, weight, cache, dy, needed, dx=None):
     """Gradients (dx, dweight, dbias, dcache) of short_conv's y [B, T, D] from
     its cotangent dy, None where ``needed`` is false. x and cache rows 16-byte
-    aligned, weight [D, W], everything one dtype (bf16 or fp32)."""
-    dev = require_device(x, weight, cache, dy)
+    aligned, weight [D, W], everything one dtype (bf16 or fp32). dy may be a
+    sequence of up to three tensors [B, T, split], as short_conv's outputs, and
+    dx (with needed[0] false) a [B, T, D] view, 16-byte aligned rows, to write."""
+    dys = [dy] if isinstance(dy, torch.Tensor) else list(dy)
+    dev = require_device(x, weight, cache, dx, *dys)
     B, T, D = x.shape
     W = weight.shape[-1]
     shapes = ((B, T, D), (D, W), (D,), (B, W - 1, D))
-    dx, dw, db, dc = (torch.empty(s, dtype=x.dtype, device=dev) if n else None for s, n in zip(shapes, needed))
+    own_dx, dw, db, dc = (torch.empty(s, dtype=x.dtype, device=dev) if n else None for s, n in zip(shapes, needed))
+    dx = own_dx if dx is None else dx
     lib = load_library()
     n = int(lib.cyfa_short_conv_grad_workspace_bytes(B, T, D, W))
     workspace = torch.empty(max(n, 1), dtype=torch.uint8, device=dev)  # alive until the launch
     args = CyfaConvGradArgs(B=B, T=T, D=D, W=W, x=ptr(x), x_row=x.stride(1), cache=ptr(cache),
                             cache_row=0 if cache is None else cache.stride(1),
-                            cache_batch=0 if cache is None else cache.stride(0), weight=ptr(weight), dy=ptr(dy),
-                            dx=ptr(dx), dcache=ptr(dc), dweight=ptr(dw), dbias=ptr(db), workspace=ptr(workspace),
+                            cache_batch=0 if cache is None else cache.stride(0), weight=ptr(weight),
+                            dy=ptr(dys[0]), dy1=ptr(dys[1] if len(dys) > 1 else None),
+                            dy2=ptr(dys[2] if len(dys) > 2 else None), split=dys[0].shape[-1],
+                            dx_row=0 if dx is None else dx.stride(1), dx=ptr(dx), dcache=ptr(dc), dweight=ptr(dw), dbias=ptr(db), workspace=ptr(workspace),
                             workspace_bytes=n)
     _check(lib.cyfa_short_conv_grad(ctypes.byref(args), general_dtype(x), stream_handle(dev)), "cyfa_short_conv_grad")
     return dx, dw, db, dc

@@ -27,7 +27,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from .. import _native
-from .autograd import gates, hip_autograd_ok, rms_norm, short_conv
+from .autograd import gates, hip_autograd_ok, projections, rms_norm, short_conv
 from ..ops import chunk_cyfa, fused_recurrent_cyfa
 from ..ops.fused_recurrent import decode_layer_step
 from ..ops.utils import readout_table
@@ -184,11 +184,24 @@ def general_short_conv(x, weight, bias, cache):
     return F.conv1d(padded.transpose(1, 2), weight.unsqueeze(1), bias, groups=x.shape[-1]).transpose(1, 2)
 
 
+def plain_module(m, cls):
+    """Whether calling module m is cls.forward and nothing more (no subclass,
+    wrapper or hook)."""
+    return (type(m) is cls and "forward" not in vars(m) and not m._forward_hooks and not m._forward_pre_hooks
+            and not m._backward_hooks and not m._backward_pre_hooks
+            and not torch.nn.modules.module._has_any_global_hook())
+
+
 def plain_linear(m):
     """Whether calling module m is F.linear on its weight and bias and nothing
-    more (no subclass, wrapper or hook)."""
-    return (type(m) is nn.Linear and not m._forward_hooks and not m._forward_pre_hooks and not m._backward_hooks
-            and not m._backward_pre_hooks and not torch.nn.modules.module._has_any_global_hook())
+    more."""
+    return plain_module(m, nn.Linear)
+
+
+def general_projections(x, wq, wk, wv, wg, w2, b2, cq, ck, cv, bq, bk, bv):
+    """projections' q, k, v and gate in torch operations."""
+    q, k, v = (general_short_conv(F.linear(x, w), c, b, None) for w, c, b in ((wq, cq, bq), (wk, ck, bk), (wv, cv, bv)))
+    return q, k, v, F.linear(F.linear(x, wg), w2, b2)
 
 
 def general_gates(x, wa, wb, bb, wd, bd, dt_bias, A_log):
@@ -357,7 +370,8 @@ class CyclicFlowAttention(nn.Module):
             return self._forward_fused(x, cache, use_cache, attention_mask=attention_mask)
         B, T, _ = x.shape
         H = self.num_heads
-        q, k, v = self.q_proj(x), self.k_proj(x), self.v_proj(x)
+        fused = None if use_cache or cache is not None or attention_mask is not None else self._projections(x)
+        q, k, v, gate = (self.q_proj(x), self.k_proj(x), self.v_proj(x), None) if fused is None else fused
         lengths = None
         if attention_mask is not None:
             # Right padding is neutral for both the recurrence and the convolution.
@@ -365,7 +379,9 @@ class CyclicFlowAttention(nn.Module):
             q, k, v = q * mask, k * mask, v * mask
             lengths = attention_mask.to(torch.int32).sum(1)
         conv_cache = (None, None, None) if cache is None else cache.get("conv_state", (None, None, None))
-        if self.use_short_conv:
+        if fused is not None:
+            cq = ck = cv = None
+        elif self.use_short_conv:
             q, cq = self.q_conv1d(q, conv_cache[0], lengths)
             k, ck = self.k_conv1d(k, conv_cache[1], lengths)
             v, cv = self.v_conv1d(v, conv_cache[2], lengths)
@@ -398,11 +414,41 @@ class CyclicFlowAttention(nn.Module):
         else:
             o, state = chunk_cyfa(**kwargs, chunk_size=self.chunk_size,
                                   table=None if torch.is_grad_enabled() else self.readout_table())
-        gate = self.g_proj(x).reshape(B, T, H, self.head_v_dim)
+        gate = (self.g_proj(x) if gate is None else gate).reshape(B, T, H, self.head_v_dim)
         o = self.o_norm(o, gate, prescale=float(self.num_slots - 1)).reshape(B, T, self.value_dim)
         o = self.o_proj(o)
         new_cache = {"recurrent_state": state, "conv_state": (cq, ck, cv)} if use_cache else None
         return o, new_cache
+
+    def _projections(self, x):
+        """(q, k, v, gate) of a training step without a cache or mask, as one
+        function of x (projections), or None where a module among them is not
+        the plain one or the operands are not that function's."""
+        if not self.use_short_conv or x.dim() != 3 or x.dtype not in (torch.bfloat16, torch.float32) or x.numel() == 0:
+            return None
+        linears = (self.q_proj, self.k_proj, self.v_proj)
+        convs = (self.q_conv1d, self.k_conv1d, self.v_conv1d)
+        if not (plain_module(self.g_proj, nn.Sequential) and len(self.g_proj) == 2
+                and all(plain_linear(m) for m in (*linears, *self.g_proj))
+                and all(plain_module(m, ShortConvolution) for m in convs)):
+            return None
+        B, T, D = x.shape
+        W = self.q_conv1d.width
+        proj = [m.weight for m in (*linears, self.g_proj[0])]
+        conv = [m.weight for m in convs]
+        bias = [m.bias for m in convs]
+        last = self.g_proj[1]
+        if any(m.bias is not None for m in (*linears, self.g_proj[0])) or len({b is None for b in bias}) != 1:
+            return None
+        if any(w is not None and w.dtype != x.dtype for w in (*proj, *conv, *bias, last.weight, last.bias)):
+            return None
+        if not (2 <= W <= 4 and all(m.width == W for m in convs) and D % 8 == 0 and all(w.shape[0] % 8 == 0 for w in proj)
+                and all(w.shape[1] == D for w in proj) and last.weight.shape[1] == proj[3].shape[0]
+                and all(tuple(c.shape) == (w.shape[0], 1, W) for c, w in zip(conv, proj))
+                and B <= _native.SHORT_CONV_MAX_GRID and T <= 32 * _native.SHORT_CONV_MAX_GRID
+                and hip_autograd_ok(x, *proj, *conv, *bias, last.weight, last.bias)):
+            return None
+        return projections(x, proj, last.weight, last.bias, [c.reshape(-1, W) for c in conv], bias, general_projections)
 
     def _gates(self, x):
         """(g, beta, delta) fp32 [B, T, H] of the general path."""

@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define CYFA_ABI_VERSION 15
+#define CYFA_ABI_VERSION 16
 
 enum {
     CYFA_OK = 0,
@@ -511,6 +511,9 @@ typedef struct CyfaConvGradArgs {
     void *dweight, *dbias;        /* nullable [D, W] and [D] */
     void *workspace;              /* cyfa_short_conv_grad_workspace_bytes(B, T, D, W) bytes, 16-byte aligned */
     size_t workspace_bytes;
+    int split;                    /* 0, or D / 2 or D / 3 (a multiple of 8): dy holds channels [0, split) as */
+    const void *dy1, *dy2;        /* [B, T, split], dy1 and dy2 the following ones, each 16-byte aligned */
+    long long dx_row;             /* 0 (D), or the elements between rows of dx: at least D, a multiple of 8 */
 } CyfaConvGradArgs;
 
 size_t cyfa_short_conv_grad_workspace_bytes(int B, int T, int D, int W);
