@@ -209,8 +209,20 @@ __device__ __forceinline__ f32x4 bf16x4_bits_to_f32x4(uint32_t w0, uint32_t w1) 
 //   xs[n+1] = the cotangent after chunk n, xs[0] (and x_out) the initial
 //   state's; bnd[tile][n] = the 32 x 32 tile's part of <xs[n+1], S[n+1]>.
 constexpr int SCAN_ROWS = BWD_SCAN_ROWS;    // rows of a boundary-term tile
+// Rows of D elements per (batch row, head) and token: row t of (b, h) is at
+// b * batch + h * head + t * ld, rows t >= T count as zero.
+struct RowsAt {
+    size_t batch, head;
+    int ld, T;
+    __host__ __device__ size_t at(int b, int h, int t) const { return b * batch + h * head + (size_t)t * ld; }
+    __device__ int live(int t0) const { return T - t0 < 0 ? 0 : T - t0 < BC ? T - t0 : BC; }  // of the chunk at t0
+};
+
+RowsAt head_major(int H, int Tp, int D) { return {(size_t)H * Tp * D, (size_t)Tp * D, D, Tp}; }
+
 struct StateScanArgs {
-    const float *a, *b;  // head-major [B*H, Tp, Kq] and [B*H, Tp, Vd]
+    const float *a, *b;  // head-major [B*H, Tp, Kq]; rows of Vd at bl
+    RowsAt bl;
     const float* g;      // [B, T, H]
     const float* x0;     // nullable [B*H, Kq, Vd]
     float* xs;           // [B*H, N+1, Kq, Vd]
@@ -228,10 +240,10 @@ struct StateScanArgs {
 // fp32 operand as a bf16 high part and a bf16 remainder, lo_a hi_b + hi_a lo_b
 // + hi_a hi_b: about 16 mantissa bits, as in the chunk kernels' tile GEMMs).
 // fp32 operands (F32): fp32 products on v_mfma_f32_16x16x4_f32, lane (lr, lg)
-// holding tokens 8 lg .. + 7 of a 32-token step as its k of eight steps. (As
+// holding tokens lg + 4 e as its k of steps e = 0 .. 7. (As
 // fp32 FMA loops, one 4-byte LDS read of a per row and token, the scan of a
 // 256 x 128 state over 16 chunks of 8 (b, h) took 50 us forward and 35 backward;
-// here 18 and 20.)
+// here 19 and 23.)
 // A workgroup takes a 32 T2 x 32 T2 tile, wave w its 16 T2 x 16 T2 quarter (w
 // >> 1, w & 1) as T2 x T2 accumulator
 // blocks: lane (lr, lg) of block (ib, jb) has rows 16 T2 (w >> 1) + 16 ib +
@@ -306,7 +318,8 @@ __global__ __launch_bounds__(T2 == 2 ? 512 : 256) void bw_state_scan_mf_kernel(S
     SE* xs = reinterpret_cast<SE*>(p.xs) + bh * (N + 1) * ssz;
     const SE* Sx = reinterpret_cast<const SE*>(p.S);
     const float* A = p.a + bh * p.Tp * Kq;
-    const BE* Bm = reinterpret_cast<const BE*>(p.b) + bh * p.Tp * Vd;
+    const BE* Bm = reinterpret_cast<const BE*>(p.b) + p.bl.at(b, h, 0);
+    const int ldb = p.bl.ld;
     const int wr = 16 * IB * (wv >> 1), wc = 16 * T2 * (wv & 1);  // the wave's block
     bool ok[IB][T2][4];
     uint32_t off[IB][T2][4];
@@ -357,16 +370,27 @@ __global__ __launch_bounds__(T2 == 2 ? 512 : 256) void bw_state_scan_mf_kernel(S
     // chunk n's rows of a, columns of b and gate into (ra, rb, rg)
     const auto fetch = [&](int n, float* ra, float* rb, float& rg) {
         const int t0 = n * BC;
-        const bw_rsrc_t rA = bw_rsrc(A + (size_t)t0 * Kq, (size_t)BC * Kq), rBm = bw_rsrc(Bm + (size_t)t0 * Vd, (size_t)BC * Vd);
+        const int live = p.bl.live(t0);  // rows past them lie past the resource (ld >= Vd): zero
+        const bw_rsrc_t rA = bw_rsrc(A + (size_t)t0 * Kq, (size_t)BC * Kq),
+                        rBm = bw_rsrc(Bm + (size_t)t0 * ldb, live ? (size_t)(live - 1) * ldb + Vd : 0);
 #pragma unroll
         for (int i = 0; i < TPT; i++) {
             const uint32_t t = TPT * sq + i;
             ra[i] = bw_load(rA, (t * (uint32_t)Kq + (uint32_t)(r0 + sr)) * 4u, r0 + sr < Kq);
-            rb[i] = BB ? bw_load_h(rBm, (t * (uint32_t)Vd + (uint32_t)(c0 + sr)) * 2u, c0 + sr < Vd)
-                       : bw_load(rBm, (t * (uint32_t)Vd + (uint32_t)(c0 + sr)) * 4u, c0 + sr < Vd);
+            rb[i] = BB ? bw_load_h(rBm, (t * (uint32_t)ldb + (uint32_t)(c0 + sr)) * 2u, c0 + sr < Vd)
+                       : bw_load(rBm, (t * (uint32_t)ldb + (uint32_t)(c0 + sr)) * 4u, c0 + sr < Vd);
         }
         rg = bw_load(rgt, (((uint32_t)b * (uint32_t)p.T + (uint32_t)(t0 + lane)) * (uint32_t)p.H + (uint32_t)h) * 4u,
                      t0 + lane < p.T);
+    };
+    // eight tokens t0 .. of an fp32 row: token t at 32 (t / 32) + 8 (t % 4) +
+    // (t % 32) / 4, so that the matrix core adds the tokens in order, four per
+    // step (the decayed ones of a chunk are added smallest first, as a loop
+    // over the tokens adds them)
+    const auto put_f32 = [](float* row, int t0, const float* v) {
+#pragma unroll
+        for (int m = 0; m < 4; m++)
+            *reinterpret_cast<f32x2*>(row + t0 / 32 * 32 + 8 * m + t0 % 32 / 4) = f32x2{v[m], v[m + 4]};
     };
     const auto chunk_of = [&](int step) { return BWD ? N - 1 - step : step; };
     // One chunk step from the registers (ra, rb, rg), which then receive the
@@ -391,9 +415,7 @@ __global__ __launch_bounds__(T2 == 2 ? 512 : 256) void bw_state_scan_mf_kernel(S
 #pragma unroll
         for (int u = 0; u < TPT / 8; u++) {
             if constexpr (F32) {
-                float* d = &sBf[sr][TPT * sq + 8 * u];
-                *reinterpret_cast<f32x4*>(d) = f32x4{rb[8 * u], rb[8 * u + 1], rb[8 * u + 2], rb[8 * u + 3]};
-                *reinterpret_cast<f32x4*>(d + 4) = f32x4{rb[8 * u + 4], rb[8 * u + 5], rb[8 * u + 6], rb[8 * u + 7]};
+                put_f32(sBf[sr], TPT * sq + 8 * u, rb + 8 * u);
                 continue;
             }
             bf16x8 hi, lo;
@@ -408,9 +430,7 @@ __global__ __launch_bounds__(T2 == 2 ? 512 : 256) void bw_state_scan_mf_kernel(S
 #pragma unroll
             for (int i = 0; i < 8; i++) fa[i] = sF[TPT * sq + 8 * u + i] * ra[8 * u + i];
             if constexpr (F32) {
-                float* d = &sAf[sr][TPT * sq + 8 * u];
-                *reinterpret_cast<f32x4*>(d) = f32x4{fa[0], fa[1], fa[2], fa[3]};
-                *reinterpret_cast<f32x4*>(d + 4) = f32x4{fa[4], fa[5], fa[6], fa[7]};
+                put_f32(sAf[sr], TPT * sq + 8 * u, fa);
                 continue;
             }
             bf16x8 hi, lo;
@@ -890,11 +910,11 @@ __device__ __forceinline__ void tile_store(float acc[NA][4], float* dst, int D, 
 // Masked, decayed scores of one chunk into P: P[t][s] = [s <= t] e^{G_t - G_s}
 // sum_j X_t[j] Y_s[j] (X, Y: the chunk's 64 rows, D wide), as one tile GEMM.
 template <bool MF, bool V4, class E>
-__device__ __forceinline__ void chunk_scores(const E* X, const E* Y, int D, const float* sG, unsigned char* stage,
-                                             float (*P)[BC + 1]) {
+__device__ __forceinline__ void chunk_scores(const E* X, int ldx, int nx, const E* Y, int ldy, int ny, int D,
+                                             const float* sG, unsigned char* stage, float (*P)[BC + 1]) {
     using RK = StateRowsK<std::is_same_v<E, bf16_t>, V4>;  // fp32 or bf16 rows
     float acc[4][4] = {};
-    tile_gemm<MF, 1>(RK(X, D, BC, D), RK(Y, D, BC, D), D, stage, acc);
+    tile_gemm<MF, 1>(RK(X, ldx, nx, D), RK(Y, ldy, ny, D), D, stage, acc);
 #pragma unroll
     for (int a = 0; a < 4; a++)
 #pragma unroll
@@ -945,7 +965,7 @@ __global__ __launch_bounds__(256) void bw_out_kernel(OutArgs a) {
         sG[tid] = chunk_gam(a.g, b, h, a.T, a.H, n, tid);
         sEq[tid] = expf(sG[tid]);
     }
-    chunk_scores<MF, V4>(q, k, Kq, sG, sStage, sA);
+    chunk_scores<MF, V4>(q, Kq, BC, k, Kq, BC, Kq, sG, sStage, sA);
     float* out = a.out + (bh * a.Tp + t0) * Vd;
     for (int d0 = BC * NT * part; d0 < Vd; d0 += BC * NT * a.parts) {
         float acc[NA][4] = {};
@@ -985,10 +1005,13 @@ __global__ __launch_bounds__(256) void bw_out_kernel(OutArgs a) {
 // two masked decayed score matrices A (q.k) and B (dO.v), each output tile
 // (64 tokens x 64 coordinates) as two tile GEMMs. Grid (N, H, B), 256 threads.
 struct ChunkGradArgs {
-    const float *q, *k, *v, *dO;  // head-major [B*H, Tp, Kq | Vd]
+    const float *q, *k, *v, *dO;  // head-major [B*H, Tp, Kq]; rows of Vd at vl
+    RowsAt vl;                    // v's, dO's and dv's rows
+    int oT;                       // vl.T of dO
     const float* g;               // [B, T, H]
     const float *S, *D;           // [B*H, N+1, Kq, Vd]: fp32, or bf16_t with sbf
-    float *dq, *dk, *dv;          // head-major
+    float *dq, *dk, *dv;          // head-major; dv at vl
+    int dvbf;                     // dv's rows are bf16 (as v's)
     int B, T, Tp, H, Kq, Vd, N;
     float scale;
     int sbf;                      // S and D hold bf16 states
@@ -1019,8 +1042,10 @@ __global__ __launch_bounds__(256) void bw_chunk_kernel(ChunkGradArgs a) {
     const size_t bh = (size_t)b * a.H + h, ssz = (size_t)Kq * Vd;
     const float* q = a.q + (bh * a.Tp + t0) * Kq;
     const float* k = a.k + (bh * a.Tp + t0) * Kq;
-    const VE* v = reinterpret_cast<const VE*>(a.v) + (bh * a.Tp + t0) * Vd;
-    const VE* dO = reinterpret_cast<const VE*>(a.dO) + (bh * a.Tp + t0) * Vd;
+    const size_t v_at = a.vl.at(b, h, t0);
+    const VE* v = reinterpret_cast<const VE*>(a.v) + v_at;
+    const VE* dO = reinterpret_cast<const VE*>(a.dO) + v_at;
+    const int ldv = a.vl.ld, nv = a.vl.live(t0), no = RowsAt{0, 0, 0, a.oT}.live(t0);
     const SE* S = reinterpret_cast<const SE*>(a.S) + (bh * (a.N + 1) + n) * ssz;
     const SE* D = reinterpret_cast<const SE*>(a.D) + (bh * (a.N + 1) + n + 1) * ssz;
     if (tid < 64) {
@@ -1031,15 +1056,15 @@ __global__ __launch_bounds__(256) void bw_chunk_kernel(ChunkGradArgs a) {
     // part + parts, ... Each kind needs one of the two score matrices.
     const int nq = (Kq + BC * NT - 1) / (BC * NT), tiles = nq + (Vd + BC * NT - 1) / (BC * NT);
     const int last = part + (tiles - 1 - part) / a.parts * a.parts;
-    if (last >= nq) chunk_scores<MF, V4>(q, k, Kq, sG, sStage, sA);
-    if (part < nq) chunk_scores<MF, V4>(dO, v, Vd, sG, sStage, sB);
+    if (last >= nq) chunk_scores<MF, V4>(q, Kq, BC, k, Kq, BC, Kq, sG, sStage, sA);
+    if (part < nq) chunk_scores<MF, V4>(dO, ldv, no, v, ldv, nv, Vd, sG, sStage, sB);
     const float sc = a.scale;
     for (int u = part; u < tiles; u += a.parts) {
         float acc[NA][4] = {};
         if (u < nq) {
             const int d0 = BC * NT * u;
             // dq = scale (e^{G_t} dO_t S_n^T + B k)
-            tile_gemm<MF, NT>(VK(dO, Vd, BC, Vd), SK(S + (size_t)d0 * Vd, Vd, Kq - d0, Vd), Vd, sStage, acc);
+            tile_gemm<MF, NT>(VK(dO, ldv, no, Vd), SK(S + (size_t)d0 * Vd, Vd, Kq - d0, Vd), Vd, sStage, acc);
             tile_scale_rows<NA>(acc, [&](int t) { return expf(sG[t]); });
             tile_gemm<MF, NT>([&](int i, int kk) { return sB[i][kk]; }, RJ(k + d0, Kq, BC, Kq - d0), BC, sStage, acc);
             tile_store<NA>(acc, a.dq + (bh * a.Tp + t0) * Kq, Kq, d0, sc);
@@ -1048,7 +1073,7 @@ __global__ __launch_bounds__(256) void bw_chunk_kernel(ChunkGradArgs a) {
             for (int x = 0; x < NA; x++)
 #pragma unroll
                 for (int y = 0; y < 4; y++) acc[x][y] = 0.f;
-            tile_gemm<MF, NT>(VK(v, Vd, BC, Vd), SK(D + (size_t)d0 * Vd, Vd, Kq - d0, Vd), Vd, sStage, acc);
+            tile_gemm<MF, NT>(VK(v, ldv, nv, Vd), SK(D + (size_t)d0 * Vd, Vd, Kq - d0, Vd), Vd, sStage, acc);
             tile_scale_rows<NA>(acc, [&](int t) { return expf(sG[BC - 1] - sG[t]); });
             tile_gemm<MF, NT>([&](int i, int kk) { return sc * sB[kk][i]; }, RJ(q + d0, Kq, BC, Kq - d0), BC, sStage, acc);
             tile_store<NA>(acc, a.dk + (bh * a.Tp + t0) * Kq, Kq, d0, 1.f);
@@ -1057,21 +1082,34 @@ __global__ __launch_bounds__(256) void bw_chunk_kernel(ChunkGradArgs a) {
             // dv = e^{G_last - G_s} k_s D_{n+1} + scale A^T dO
             tile_gemm<MF, NT>(RK(k, Kq, BC, Kq), SJ(D + d0, Vd, Kq, Vd - d0), Kq, sStage, acc);
             tile_scale_rows<NA>(acc, [&](int t) { return expf(sG[BC - 1] - sG[t]); });
-            tile_gemm<MF, NT>([&](int i, int kk) { return sc * sA[kk][i]; }, VJ(dO + d0, Vd, BC, Vd - d0), BC, sStage, acc);
-            tile_store<NA>(acc, a.dv + (bh * a.Tp + t0) * Vd, Vd, d0, 1.f);
+            tile_gemm<MF, NT>([&](int i, int kk) { return sc * sA[kk][i]; }, VJ(dO + d0, ldv, no, Vd - d0), BC, sStage, acc);
+            const auto store_dv = [&](auto* dst) {
+#pragma unroll
+                for (int x = 0; x < NA; x++)
+#pragma unroll
+                    for (int y = 0; y < 4; y++) {
+                        const int t = TileMap::row(x, y), c = d0 + TileMap::col(x, y);
+                        if (c < Vd && t < nv) dst[(size_t)t * ldv + c] = (std::remove_reference_t<decltype(*dst)>)acc[x][y];
+                    }
+            };
+            if (RB && a.dvbf)
+                store_dv(reinterpret_cast<bf16_t*>(a.dv) + v_at);
+            else
+                store_dv(a.dv + v_at);
         }
     }
 }
 
-// The slot readout for blocks of 32 rows of one head: z = U(lam) raw,
-// l = z table^T, p = softmax(l), u = p table, weights = U(-lam) u; the two
+// The slot readout of fp32 calls for blocks of 32 rows of one head: z = U(lam)
+// raw, l = z table^T, p = softmax(l), u = p table, weights = U(-lam) u; the two
 // products as small GEMMs against the staged table on the fp32 matrix cores
-// (mfma4 below). BF
-// rounds z, the table, p and the weights to bf16 (the general forward's casts
-// to a bf16 input dtype, ops/utils.py:779-882); the backward's recompute is
-// unrounded. Grid (ceil(B Tp / (32 per_wg)), H), RO_FWD_THREADS threads: a
+// (mfma4 below). Grid (ceil(B Tp / (32 per_wg)), H), RO_FWD_THREADS threads: a
 // workgroup stages the table once and takes per_wg blocks; the LDS holds one
 // workgroup per CU, and its waves put several on each SIMD.
+
+// With BF, x rounded to bf16: z, the table, p and the weights of the general
+// forward's bf16 calls (its casts to the input dtype, ops/utils.py:779-882);
+// the backward's recompute is unrounded.
 template <bool BF>
 __device__ __forceinline__ float bw_rnd(float x) {
     if constexpr (BF)
@@ -1083,7 +1121,6 @@ __device__ __forceinline__ float bw_rnd(float x) {
 constexpr int RO_LD = BWD_TABLE_M + 4;  // staged table and row rows, 16-byte aligned
 constexpr int RO_FWD_THREADS = 1024;
 
-template <bool BF>
 __global__ __launch_bounds__(RO_FWD_THREADS) void bw_fwd_readout_kernel(const float* raw, const float* cs, const float* sn,
                                                              const float* table, int B, int Tp, int H, int M,
                                                              int per_wg, float* wts) {
@@ -1097,7 +1134,7 @@ __global__ __launch_bounds__(RO_FWD_THREADS) void bw_fwd_readout_kernel(const fl
     const int R = M - 1, P = M / 2, rows = B * Tp;
     for (int e = tid; e < TM * LD; e += NT) {
         const int r = e / LD, m = e % LD;
-        sTab[e] = (r < R && m < M) ? bw_rnd<BF>(table[((size_t)h * R + r) * M + m]) : 0.f;
+        sTab[e] = (r < R && m < M) ? table[((size_t)h * R + r) * M + m] : 0.f;
     }
     const auto row_of = [&](int rho) { return ((size_t)(rho / Tp) * H + h) * Tp + rho % Tp; };
     // wave wv: row tile it = wv & 1, column tiles CPW (wv >> 1) .. + CPW - 1 (of r, then of m)
@@ -1134,8 +1171,8 @@ __global__ __launch_bounds__(RO_FWD_THREADS) void bw_fwd_readout_kernel(const fl
             const float c = live ? nc[x] : 1.f, s = ns[x];
             sCs[i][pr] = c;
             sSn[i][pr] = s;
-            sZ[i][2 * pr] = bw_rnd<BF>(c * nre[x] - s * nro[x]);  // zero where !live
-            sZ[i][2 * pr + 1] = bw_rnd<BF>(s * nre[x] + c * nro[x]);
+            sZ[i][2 * pr] = c * nre[x] - s * nro[x];  // zero where !live
+            sZ[i][2 * pr + 1] = s * nre[x] + c * nro[x];
         }
         load_block(b0 + RB);  // the next block (past the end: dead loads)
         __syncthreads();
@@ -1159,8 +1196,8 @@ __global__ __launch_bounds__(RO_FWD_THREADS) void bw_fwd_readout_kernel(const fl
             const float mx = bw_wave_max(fmaxf(l0, l1));
             const float e0 = lane < R ? expf(l0 - mx) : 0.f, e1 = lane + 64 < R ? expf(l1 - mx) : 0.f;
             const float inv = 1.f / bw_wave_sum(e0 + e1);
-            sP[i][lane] = bw_rnd<BF>(e0 * inv);
-            sP[i][lane + 64] = bw_rnd<BF>(e1 * inv);
+            sP[i][lane] = e0 * inv;
+            sP[i][lane + 64] = e1 * inv;
         }
         __syncthreads();
         // u[i][m] = sum_r p[i][r] table[r][m] (p and the table zero at r >= R); the
@@ -1185,7 +1222,7 @@ __global__ __launch_bounds__(RO_FWD_THREADS) void bw_fwd_readout_kernel(const fl
                 const int i = 16 * it + 4 * lk + q, rho = b0 + i;
                 if (rho < rows && pr < P) {
                     const float c = sCs[i][pr], s = sSn[i][pr];
-                    wts[row_of(rho) * M + m] = bw_rnd<BF>(odd ? -s * ue + c * uo : c * ue + s * uo);
+                    wts[row_of(rho) * M + m] = odd ? -s * ue + c * uo : c * ue + s * uo;
                 }
             }
         }
@@ -2345,6 +2382,7 @@ int launch_chunk_pass(const ChunkPassParams& p, hipStream_t stream) {
     StateScanArgs sa{};
     sa.a = p.k;
     sa.b = p.v;
+    sa.bl = head_major(p.H, p.Tp, p.Vd);
     sa.g = p.g;
     sa.x0 = p.s0;
     sa.xs = p.states;
@@ -2439,10 +2477,9 @@ int launch_chunk_readout(const float* raw, const float* cs, const float* sn, con
     else if (split)
         hipLaunchKernelGGL((bw_readout_mf_kernel<false, false, RO_MF_FWD_WAVES>), grid, dim3(64 * RO_MF_FWD_WAVES), 0, stream, ro);
     else if (bf16)
-        hipLaunchKernelGGL(bw_fwd_readout_kernel<true>, grid, dim3(RO_FWD_THREADS), 0, stream, raw, cs, sn, table, B, Tp, H, M, per,
-                           wts);
+        return -1;  // bf16 operands come with the split form
     else
-        hipLaunchKernelGGL(bw_fwd_readout_kernel<false>, grid, dim3(RO_FWD_THREADS), 0, stream, raw, cs, sn, table, B, Tp, H, M, per,
+        hipLaunchKernelGGL(bw_fwd_readout_kernel, grid, dim3(RO_FWD_THREADS), 0, stream, raw, cs, sn, table, B, Tp, H, M, per,
                            wts);
     return 0;
 }
@@ -2457,16 +2494,29 @@ int launch_chunk_bwd(const BwdParams& p, hipStream_t stream) {
     const size_t rows = (size_t)B * H * Tp;
     const dim3 blk(256), rb((unsigned)((rows + 3) / 4));
     const bool bf = p.bf16 != 0;
-    // the normalised rows, v and the output cotangent, head-major fp32
+    // v, the output cotangent and v's cotangent are read and written in place,
+    // [B, T, H, V], where their rows take 16-byte accesses and a chunk of them
+    // stays within the kernels' 32-bit offsets; otherwise through head-major
+    // copies (65536 rows of 256 bf16: 33 us for the two copies, 22 us for v's
+    // cotangent, of a training pass of 1178 us in all, 1119 so).
+    const bool direct = V % 4 == 0 && ((uintptr_t)p.v | (uintptr_t)p.d_o | (uintptr_t)p.dv) % 16 == 0 &&
+                        (long long)H * V * BC * 4 < (1ll << 31);
+    const RowsAt vl = direct ? RowsAt{(size_t)T * H * V, (size_t)V, H * V, T} : head_major(H, Tp, V);
+    const float* v_rows = direct ? static_cast<const float*>(p.v) : ws.vh;
+    const float* o_rows = direct ? static_cast<const float*>(p.d_o) : ws.dO;
+    const int oT = direct && !p.d_o ? 0 : vl.T;
+    // the normalised rows, head-major fp32; v and dO
 #define CYFA_BW_ROWS(BFV)                                                                                           \
     hipLaunchKernelGGL(bw_rows_kernel<BFV>, rb, blk, 0, stream, p.q, p.q_w, p.q_eps, B, T, Tp, H, K, ws.qh, ws.rq); \
     hipLaunchKernelGGL(bw_rows_kernel<BFV>, rb, blk, 0, stream, p.k, p.k_w, p.k_eps, B, T, Tp, H, K, ws.kh, ws.rk); \
-    hipLaunchKernelGGL((bw_rows_kernel<BFV, RowT>), rb, blk, 0, stream, p.v, (const float*)nullptr, 0.f, B, T, Tp, H, \
-                       V, reinterpret_cast<RowT*>(ws.vh), (float*)nullptr);                                        \
-    hipLaunchKernelGGL((bw_rows_kernel<BFV, RowT>), rb, blk, 0, stream, p.d_o, (const float*)nullptr, 0.f, B, T, Tp, H, \
-                       V, reinterpret_cast<RowT*>(ws.dO), (float*)nullptr);
-    // v and dO of bf16 calls stay bf16 in the head-major rows (exact): the
-    // pass-2 scans and chunk kernels read half the bytes.
+    if (!direct) {                                                                                                  \
+        hipLaunchKernelGGL((bw_rows_kernel<BFV, RowT>), rb, blk, 0, stream, p.v, (const float*)nullptr, 0.f, B, T, Tp, H, \
+                           V, reinterpret_cast<RowT*>(ws.vh), (float*)nullptr);                                    \
+        hipLaunchKernelGGL((bw_rows_kernel<BFV, RowT>), rb, blk, 0, stream, p.d_o, (const float*)nullptr, 0.f, B, T, Tp, \
+                           H, V, reinterpret_cast<RowT*>(ws.dO), (float*)nullptr);                                 \
+    }
+    // v and dO of bf16 calls stay bf16 in head-major rows (exact): the pass-2
+    // scans and chunk kernels read half the bytes.
     if (bf) {
         using RowT = bf16_t;
         CYFA_BW_ROWS(true)
@@ -2486,6 +2536,7 @@ int launch_chunk_bwd(const BwdParams& p, hipStream_t stream) {
     f1.sbf = bf;
     f1.a = ws.kh;
     f1.b = ws.w;
+    f1.bl = head_major(H, Tp, M);
     f1.g = p.g;
     f1.x0 = p.h0_k;
     f1.xs = ws.sk;
@@ -2543,7 +2594,8 @@ int launch_chunk_bwd(const BwdParams& p, hipStream_t stream) {
     const dim3 g_rows((unsigned)((rows + 3) / 4));
     StateScanArgs f2 = f1;
     f2.a = ws.w;
-    f2.b = ws.vh;
+    f2.b = v_rows;
+    f2.bl = vl;
     f2.x0 = p.h0_v;
     f2.xs = ws.sv;
     f2.bbf = bf;  // v's rows
@@ -2553,7 +2605,8 @@ int launch_chunk_bwd(const BwdParams& p, hipStream_t stream) {
     // pass 2: state cotangents, then the rows' (slot weights, write vector, v)
     StateScanArgs s2 = f2;
     s2.a = ws.wts;
-    s2.b = ws.dO;
+    s2.b = o_rows;
+    s2.bl.T = oT;
     s2.x0 = p.d_hv;
     s2.xs = ws.dsv;
     s2.S = ws.sv;
@@ -2565,14 +2618,17 @@ int launch_chunk_bwd(const BwdParams& p, hipStream_t stream) {
     c2.rbf = bf;  // v's and dO's rows
     c2.q = ws.wts;
     c2.k = ws.w;
-    c2.v = ws.vh;
-    c2.dO = ws.dO;
+    c2.v = v_rows;
+    c2.dO = o_rows;
+    c2.vl = vl;
+    c2.oT = oT;
     c2.g = p.g;
     c2.S = ws.sv;
     c2.D = ws.dsv;
     c2.dq = ws.dwts;
     c2.dk = ws.dw2;
-    c2.dv = ws.dvh;
+    c2.dv = direct ? static_cast<float*>(p.dv) : ws.dvh;
+    c2.dvbf = direct && bf;
     c2.B = B;
     c2.T = T;
     c2.Tp = Tp;
@@ -2625,6 +2681,9 @@ int launch_chunk_bwd(const BwdParams& p, hipStream_t stream) {
     c1.rbf = 0;  // pass 1's rows (the write vector, draw) are fp32
     c1.q = ws.qh;
     c1.k = ws.kh;
+    c1.vl = head_major(H, Tp, M);
+    c1.oT = Tp;
+    c1.dvbf = 0;
     c1.v = ws.w;
     c1.dO = ws.draw;
     c1.S = ws.sk;
@@ -2672,17 +2731,19 @@ int launch_chunk_bwd(const BwdParams& p, hipStream_t stream) {
     const dim3 kb((unsigned)((K + 3) / 4));
     hipLaunchKernelGGL(bw_reduce_kernel, kb, blk, 0, stream, ws.dnq, ws.norm_blocks, (size_t)K, p.dq_w);
     hipLaunchKernelGGL(bw_reduce_kernel, kb, blk, 0, stream, ws.dnk, ws.norm_blocks, (size_t)K, p.dk_w);
-    const size_t nv = (size_t)B * T * H * V;
-    const dim3 vb((unsigned)((nv + 255) / 256)), vb4((unsigned)((nv / 4 + 255) / 256));
-    const bool pack4 = V % 4 == 0 && ((uintptr_t)p.dv & (bf ? 7 : 15)) == 0;
-    if (bf && pack4)
-        hipLaunchKernelGGL(bw_pack_kernel<true>, vb4, blk, 0, stream, ws.dvh, B, T, Tp, H, V, p.dv);
-    else if (pack4)
-        hipLaunchKernelGGL(bw_pack_kernel<false>, vb4, blk, 0, stream, ws.dvh, B, T, Tp, H, V, p.dv);
-    else if (bf)
-        hipLaunchKernelGGL(bw_pack1_kernel<true>, vb, blk, 0, stream, ws.dvh, B, T, Tp, H, V, p.dv);
-    else
-        hipLaunchKernelGGL(bw_pack1_kernel<false>, vb, blk, 0, stream, ws.dvh, B, T, Tp, H, V, p.dv);
+    if (!direct) {
+        const size_t nv = (size_t)B * T * H * V;
+        const dim3 vb((unsigned)((nv + 255) / 256)), vb4((unsigned)((nv / 4 + 255) / 256));
+        const bool pack4 = V % 4 == 0 && ((uintptr_t)p.dv & (bf ? 7 : 15)) == 0;
+        if (bf && pack4)
+            hipLaunchKernelGGL(bw_pack_kernel<true>, vb4, blk, 0, stream, ws.dvh, B, T, Tp, H, V, p.dv);
+        else if (pack4)
+            hipLaunchKernelGGL(bw_pack_kernel<false>, vb4, blk, 0, stream, ws.dvh, B, T, Tp, H, V, p.dv);
+        else if (bf)
+            hipLaunchKernelGGL(bw_pack1_kernel<true>, vb, blk, 0, stream, ws.dvh, B, T, Tp, H, V, p.dv);
+        else
+            hipLaunchKernelGGL(bw_pack1_kernel<false>, vb, blk, 0, stream, ws.dvh, B, T, Tp, H, V, p.dv);
+    }
     const int RM = (M - 1) * M;
     hipLaunchKernelGGL(bw_table_reduce_kernel, dim3((RM + 255) / 256, H), blk, 0, stream, ws.dtab, ws.ro_blocks, RM,
                        p.dtable);

@@ -32,6 +32,8 @@ def test_short_conv_grad_validates_before_launch():
     assert call(dtype=7) == call(x=None) == call(T=0) == _native.CYFA_ERR_VALUE
     assert call(x=0x10004) == call(x_row=60) == call(dx=0x50002) == _native.CYFA_ERR_ALIGN
     assert call(workspace_bytes=n - 1) == _native.CYFA_ERR_WORKSPACE
+    assert call(split=24) == call(split=16) == call(split=32) == call(D=40, split=20) == _native.CYFA_ERR_VALUE  # 32: no dy1
+    assert call(split=32, dy1=0x30004) == call(dx_row=60) == call(dx_row=68) == _native.CYFA_ERR_ALIGN
 
 
 def test_mask_entry_points_validate_before_launch():
