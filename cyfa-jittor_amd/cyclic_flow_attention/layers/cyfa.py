@@ -356,14 +356,25 @@ class CyclicFlowAttention(nn.Module):
     def _fused_mask_ok(self, x, attention_mask):
         """Whether a masked call takes the fused path: a prefill of more rows
         than a decode step's at the tuned op's shape, with an integer mask
-        [B, T]. (Other masks, which may broadcast or hold fractions, and other
-        shapes keep the general path.)"""
+        [B, T]. (Other masks, which may broadcast or hold fractions, other
+        shapes, and layers whose modules have hooks or are replaced by others
+        keep the general path, which calls the modules.)"""
         return (attention_mask is not None and self._fused_ok(x, None) and x.dim() == 3 and x.shape[1] > 1
                 and self.head_k_dim == 256 and self.head_v_dim == 256 and self.num_slots == 128
                 and self.chunk_size == 64
                 and x.shape[0] * x.shape[1] > _native.LINEAR_ROWS_MAX
                 and tuple(attention_mask.shape) == tuple(x.shape[:2]) and attention_mask.device == x.device
-                and attention_mask.dtype in (torch.int64, torch.int32, torch.bool, torch.uint8))
+                and attention_mask.dtype in (torch.int64, torch.int32, torch.bool, torch.uint8)
+                and self._plain())
+
+    def _plain(self):
+        """Whether the modules that the fused path reads the weights of are the
+        plain ones."""
+        return (plain_module(self.g_proj, nn.Sequential) and len(self.g_proj) == 2
+                and all(plain_linear(m) for m in (self.q_proj, self.k_proj, self.v_proj, self.a_proj, self.b_proj,
+                                                  self.d_proj, *self.g_proj, self.o_proj))
+                and all(plain_module(m, ShortConvolution) for m in (self.q_conv1d, self.k_conv1d, self.v_conv1d))
+                and plain_module(self.o_norm, RMSNorm))
 
     def forward(self, x, cache=None, use_cache=False, attention_mask=None):
         if self._fused_ok(x, attention_mask) or self._fused_mask_ok(x, attention_mask):
@@ -415,8 +426,11 @@ class CyclicFlowAttention(nn.Module):
             o, state = chunk_cyfa(**kwargs, chunk_size=self.chunk_size,
                                   table=None if torch.is_grad_enabled() else self.readout_table())
         gate = (self.g_proj(x) if gate is None else gate).reshape(B, T, H, self.head_v_dim)
-        o = self.o_norm(o, gate, prescale=float(self.num_slots - 1)).reshape(B, T, self.value_dim)
-        o = self.o_proj(o)
+        if plain_module(self.o_norm, RMSNorm):
+            o = self.o_norm(o, gate, prescale=float(self.num_slots - 1))
+        else:  # (another norm, or one with hooks, is given the scaled input)
+            o = self.o_norm(o * (self.num_slots - 1), gate)
+        o = self.o_proj(o.reshape(B, T, self.value_dim))
         new_cache = {"recurrent_state": state, "conv_state": (cq, ck, cv)} if use_cache else None
         return o, new_cache
 
@@ -455,7 +469,10 @@ class CyclicFlowAttention(nn.Module):
         H = self.num_heads
         a, b, d = self.a_proj, self.b_proj, self.d_proj
         weights = (a.weight, b.weight, b.bias, d.weight, d.bias) if all(plain_linear(m) for m in (a, b, d)) else ()
-        if (weights and a.bias is None and all(w is not None and w.dtype == x.dtype for w in weights)
+        shapes = ((H, x.shape[-1]), (H, x.shape[-1]), (H,), (H, x.shape[-1]), (H,))
+        if (weights and a.bias is None
+                and all(w is not None and w.dtype == x.dtype and tuple(w.shape) == s for w, s in zip(weights, shapes))
+                and tuple(self.dt_bias.shape) == tuple(self.A_log.shape) == (H,)
                 and x.dtype in (torch.bfloat16, torch.float32) and H <= _native.GATES_TRAIN_MAX_H
                 and x.shape[-1] % 8 == 0 and 0 < x.numel() // x.shape[-1] <= _native.GATES_TRAIN_MAX_ROWS
                 and hip_autograd_ok(x, *weights, self.dt_bias, self.A_log)):

@@ -82,3 +82,21 @@ def test_masked_layer_equals_general_path(B, T, hidden, H, dtype, kind, carried)
     for a, b in pairs:
         assert a.shape == b.shape and a.dtype == b.dtype
         assert ((a.double() - b.double()).norm() <= 2.0 ** -8 * b.double().norm().clamp_min(1e-30)).item()
+
+
+def test_masked_call_of_a_layer_with_hooks_calls_its_modules():
+    torch.manual_seed(0)
+    layer = CyclicFlowAttention(hidden_size=256, num_heads=1).eval().bfloat16().to(DEV)
+    x = torch.randn(2, 40, 256, dtype=torch.bfloat16, device=DEV)
+    mask = torch.ones(2, 40, dtype=torch.long, device=DEV)
+    mask[1, 30:] = 0
+    seen = []
+    with torch.no_grad():
+        for m in (layer.q_proj, layer.g_proj[1], layer.k_conv1d, layer.o_norm, layer.o_proj):
+            assert layer._fused_mask_ok(x, mask)
+            hook = m.register_forward_pre_hook(lambda *_: seen.append(1))
+            layer(x, attention_mask=mask)
+            hook.remove()
+        assert len(seen) == 5
+        layer.v_proj = torch.nn.Sequential(layer.v_proj)
+        assert not layer._fused_mask_ok(x, mask)
