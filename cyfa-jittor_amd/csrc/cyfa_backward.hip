@@ -544,16 +544,26 @@ void launch_state_scan(const StateScanArgs& a, bool mfma, hipStream_t stream) {
 //    v_mfma_f32_16x16x4_f32, the operands staged as fp32. (As fp32 FMA loops, a
 //    4 x 4 block per thread with 4-byte operand loads, the chunk kernel took
 //    181 us for 128 chunks of 256 x 128 and the output kernel 88; here, with
-//    the chunk's tiles shared out over three and two workgroups, 48 and 24.)
+//    the chunk's tiles shared out over three and two workgroups, 47 and 22.)
 // The wide readout's GEMMs (128 < M) keep fp32 FMA in a 4 x 4 block per thread
 // (tile_gemm_fma), whose threads hold neighbouring columns.
 constexpr int GT_K = 32, GT_LD = 68;  // FMA staging: [32][68] per operand
 constexpr int MT_LD = 40;             // bf16 staging: [64][40] per operand part (32 k + 8 pad)
 constexpr int FT_LD = 36;             // fp32 staging: [64][36] per operand
-constexpr int STAGE_BYTES = 4 * BC * MT_LD * 2;   // A and a B block, hi and lo
-constexpr int STAGE2_BYTES = 6 * BC * MT_LD * 2;  // the same with two B blocks
-static_assert(STAGE_BYTES >= 2 * GT_K * GT_LD * 4 && STAGE_BYTES >= 2 * BC * FT_LD * 4 &&
-                  STAGE2_BYTES >= 3 * BC * FT_LD * 4,
+// Row r of a staged 64-row block: every 16 rows start 16 bytes further on. A
+// B operand contiguous along j is staged column by column, lane (jq, kp)
+// writing row 4 jq + c: at an even pitch of 20 dwords (36 in fp32) the sixteen
+// jq of a store fall on four of the 64 banks; with the offset, on sixteen, so
+// that a wave's store touches each bank once (at 1024 chunks of 256 x 128 the
+// chunk kernels 191 -> 174 and 172 -> 157 us, the output kernel 74 -> 66; in
+// fp32 at 128 chunks 50 -> 47 and 24 -> 22). The 16-byte reads of 16
+// neighbouring rows keep their pitch.
+__device__ __forceinline__ constexpr int mt_row(int r) { return r * MT_LD + r / 16 * 8; }
+__device__ __forceinline__ constexpr int ft_row(int r) { return r * FT_LD + r / 16 * 4; }
+constexpr int MT_TILE = BC * MT_LD + BC / 16 * 8, FT_TILE = BC * FT_LD + BC / 16 * 4;
+constexpr int STAGE_BYTES = 4 * MT_TILE * 2;   // A and a B block, hi and lo
+constexpr int STAGE2_BYTES = 6 * MT_TILE * 2;  // the same with two B blocks
+static_assert(STAGE_BYTES >= 2 * GT_K * GT_LD * 4 && STAGE_BYTES >= 2 * FT_TILE * 4 && STAGE2_BYTES >= 3 * FT_TILE * 4,
               "staging must hold every form");
 
 struct TileMap {
@@ -706,11 +716,11 @@ __device__ __forceinline__ void tile_gemm(FA fa, FB fb, int Kd, unsigned char* s
     const int tid = threadIdx.x;
     {
         float* saf = reinterpret_cast<float*>(stage);  // fp32: A (64 rows), then B (64 NT rows)
-        float* sbf = saf + BC * FT_LD;
+        float* sbf = saf + FT_TILE;
         bf16_t* sah = reinterpret_cast<bf16_t*>(stage);  // hi and lo parts of A (64 rows) and of B (64 NT rows)
-        bf16_t* sal = sah + BC * MT_LD;
-        bf16_t* sbh = sal + BC * MT_LD;
-        bf16_t* sbl = sbh + NT * BC * MT_LD;
+        bf16_t* sal = sah + MT_TILE;
+        bf16_t* sbh = sal + MT_TILE;
+        bf16_t* sbl = sbh + NT * MT_TILE;
         const int l = tid & 63, w = tid >> 6, lr = l & 15, lg = l >> 4;
         const int r = tid >> 2, kg = tid & 3;  // staging: row r, k-group kg (8 k)
         // RowsK4 operands: lane (r, kg) holds kk = k0 + 4 kg .. + 3 and
@@ -747,16 +757,16 @@ __device__ __forceinline__ void tile_gemm(FA fa, FB fb, int Kd, unsigned char* s
         // writes the 8 staged values of one operand in its lane order
         const auto put = [&](bf16_t* base, bool split4, const bf16x8& v) {
             if (split4) {
-                *reinterpret_cast<bf16x4*>(base + r * MT_LD + 4 * kg) = bf16x4{v[0], v[1], v[2], v[3]};
-                *reinterpret_cast<bf16x4*>(base + r * MT_LD + 16 + 4 * kg) = bf16x4{v[4], v[5], v[6], v[7]};
+                *reinterpret_cast<bf16x4*>(base + mt_row(r) + 4 * kg) = bf16x4{v[0], v[1], v[2], v[3]};
+                *reinterpret_cast<bf16x4*>(base + mt_row(r) + 16 + 4 * kg) = bf16x4{v[4], v[5], v[6], v[7]};
             } else {
-                *reinterpret_cast<bf16x8*>(base + r * MT_LD + 8 * kg) = v;
+                *reinterpret_cast<bf16x8*>(base + mt_row(r) + 8 * kg) = v;
             }
         };
         const auto put_f = [&](float* base, bool split4, const float* v) {
             const int c0 = split4 ? 4 * kg : 8 * kg, c1 = split4 ? 16 + 4 * kg : 8 * kg + 4;
-            *reinterpret_cast<f32x4*>(base + r * FT_LD + c0) = f32x4{v[0], v[1], v[2], v[3]};
-            *reinterpret_cast<f32x4*>(base + r * FT_LD + c1) = f32x4{v[4], v[5], v[6], v[7]};
+            *reinterpret_cast<f32x4*>(base + ft_row(r) + c0) = f32x4{v[0], v[1], v[2], v[3]};
+            *reinterpret_cast<f32x4*>(base + ft_row(r) + c1) = f32x4{v[4], v[5], v[6], v[7]};
         };
         fetch(0);
         for (int k0 = 0; k0 < Kd; k0 += GT_K) {
@@ -765,11 +775,11 @@ __device__ __forceinline__ void tile_gemm(FA fa, FB fb, int Kd, unsigned char* s
                 put_f(saf, VA, ra);
 #pragma unroll
                 for (int nt = 0; nt < NT; nt++) {
-                    float* b0 = sbf + 64 * nt * FT_LD;
+                    float* b0 = sbf + nt * FT_TILE;
                     if constexpr (JB) {
 #pragma unroll
                         for (int c = 0; c < 4; c++)
-                            *reinterpret_cast<f32x2*>(b0 + (4 * jq + c) * FT_LD + 2 * kp) = f32x2{rb[nt][c], rb[nt][4 + c]};
+                            *reinterpret_cast<f32x2*>(b0 + ft_row(4 * jq + c) + 2 * kp) = f32x2{rb[nt][c], rb[nt][4 + c]};
                     } else {
                         put_f(b0, VB, rb[nt]);
                     }
@@ -779,7 +789,7 @@ __device__ __forceinline__ void tile_gemm(FA fa, FB fb, int Kd, unsigned char* s
 #pragma unroll
                 for (int nb = 0; nb < 4 * NT; nb++) {
                     f32x4 c = {acc[nb][0], acc[nb][1], acc[nb][2], acc[nb][3]};
-                    c = mfma_f32x8(saf + (16 * w + lr) * FT_LD + 8 * lg, sbf + (16 * nb + lr) * FT_LD + 8 * lg, c);
+                    c = mfma_f32x8(saf + ft_row(16 * w + lr) + 8 * lg, sbf + nb / 4 * FT_TILE + ft_row(16 * (nb % 4) + lr) + 8 * lg, c);
 #pragma unroll
                     for (int i = 0; i < 4; i++) acc[nb][i] = c[i];
                 }
@@ -801,13 +811,13 @@ __device__ __forceinline__ void tile_gemm(FA fa, FB fb, int Kd, unsigned char* s
                     vbh[x] = (bf16_t)rb[nt][x];
                     vbl[x] = (bf16_t)(rb[nt][x] - (float)vbh[x]);
                 }
-                bf16_t* bh0 = sbh + 64 * nt * MT_LD;
-                bf16_t* bl0 = sbl + 64 * nt * MT_LD;
+                bf16_t* bh0 = sbh + nt * MT_TILE;
+                bf16_t* bl0 = sbl + nt * MT_TILE;
                 if constexpr (JB) {  // column 4 jq + c: the pair (k0 + 2 kp, + 1) as one 4-byte store
 #pragma unroll
                     for (int c = 0; c < 4; c++) {
-                        *reinterpret_cast<bf16x2*>(bh0 + (4 * jq + c) * MT_LD + 2 * kp) = bf16x2{vbh[c], vbh[4 + c]};
-                        *reinterpret_cast<bf16x2*>(bl0 + (4 * jq + c) * MT_LD + 2 * kp) = bf16x2{vbl[c], vbl[4 + c]};
+                        *reinterpret_cast<bf16x2*>(bh0 + mt_row(4 * jq + c) + 2 * kp) = bf16x2{vbh[c], vbh[4 + c]};
+                        *reinterpret_cast<bf16x2*>(bl0 + mt_row(4 * jq + c) + 2 * kp) = bf16x2{vbl[c], vbl[4 + c]};
                     }
                 } else {
                     put(bh0, VB, vbh);
@@ -816,12 +826,12 @@ __device__ __forceinline__ void tile_gemm(FA fa, FB fb, int Kd, unsigned char* s
             }
             __syncthreads();
             if (k0 + GT_K < Kd) fetch(k0 + GT_K);
-            const int ao = (16 * w + lr) * MT_LD + 8 * lg;
+            const int ao = mt_row(16 * w + lr) + 8 * lg;
             const bf16x8 ah = *reinterpret_cast<const bf16x8*>(sah + ao);
             const bf16x8 al = *reinterpret_cast<const bf16x8*>(sal + ao);
 #pragma unroll
             for (int nb = 0; nb < 4 * NT; nb++) {
-                const int bo = (16 * nb + lr) * MT_LD + 8 * lg;
+                const int bo = nb / 4 * MT_TILE + mt_row(16 * (nb % 4) + lr) + 8 * lg;
                 const bf16x8 bh = *reinterpret_cast<const bf16x8*>(sbh + bo);
                 const bf16x8 bl = *reinterpret_cast<const bf16x8*>(sbl + bo);
                 f32x4 c = {acc[nb][0], acc[nb][1], acc[nb][2], acc[nb][3]};
