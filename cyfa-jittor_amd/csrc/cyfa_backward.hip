@@ -2114,8 +2114,22 @@ __global__ __launch_bounds__(64) void bw_clock_kernel(const float* dlam, const f
                                                       int H, float* ddelta, float* dclock0) {
     const int bh = blockIdx.x, b = bh / H, h = bh % H, lane = threadIdx.x;
     const int per = (Tp + 63) / 64, t0 = lane * per, t1 = min(t0 + per, Tp);
+    // tokens t, t - 1, .. of the run, zero before t0: CLOCK_U loads in flight
+    // for each part of a lane's serial sum
+    constexpr int CLOCK_U = 16;
+    const auto fetch = [&](int t, float* v) {
+#pragma unroll
+        for (int u = 0; u < CLOCK_U; u++) v[u] = dlam[(size_t)bh * Tp + max(min(t, Tp - 1) - u, 0)];
+#pragma unroll
+        for (int u = 0; u < CLOCK_U; u++) v[u] = t - u >= t0 ? v[u] : 0.f;
+    };
+    float v[CLOCK_U];
     double s = 0.0;
-    for (int t = t0; t < t1; t++) s += (double)dlam[(size_t)bh * Tp + t];
+    for (int t = t1 - 1; t >= t0; t -= CLOCK_U) {
+        fetch(t, v);
+#pragma unroll
+        for (int u = 0; u < CLOCK_U; u++) s += (double)v[u];
+    }
     double suf = s;  // sum over this lane's run and every later lane's
     for (int o = 1; o < 64; o <<= 1) {
         const double y = __shfl_down(suf, o);
@@ -2123,9 +2137,13 @@ __global__ __launch_bounds__(64) void bw_clock_kernel(const float* dlam, const f
     }
     const double extra = d_clock ? (double)d_clock[bh] : 0.0;
     double run = suf - s + extra;  // the later lanes' sum
-    for (int t = t1 - 1; t >= t0; t--) {
-        run += (double)dlam[(size_t)bh * Tp + t];
-        if (t < T) ddelta[((size_t)b * T + t) * H + h] = (float)run;
+    for (int t = t1 - 1; t >= t0; t -= CLOCK_U) {
+        fetch(t, v);
+#pragma unroll
+        for (int u = 0; u < CLOCK_U; u++) {
+            run += (double)v[u];
+            if (t - u >= t0 && t - u < T) ddelta[((size_t)b * T + t - u) * H + h] = (float)run;
+        }
     }
     if (dclock0 && lane == 0) dclock0[bh] = (float)(suf + extra);
 }
@@ -2243,12 +2261,24 @@ void launch_norm_adjoint(dim3 nb, const void* x, const float* w, const float* rs
 
 // out[i] = sum over the nb partial rows of part[.][i]: one wave per column,
 // lane l adding rows l, l + 64, .. in order, then the wave's fixed-order sum.
-__global__ __launch_bounds__(256) void bw_reduce_kernel(const float* part, int nb, size_t n, float* out) {
+// blockIdx.y: q's partials or k's.
+__global__ __launch_bounds__(256) void bw_reduce_kernel(const float* part_q, const float* part_k, int nb, size_t n,
+                                                        float* out_q, float* out_k) {
+    const float* part = blockIdx.y ? part_k : part_q;
+    float* out = blockIdx.y ? out_k : out_q;
     const size_t i = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (i >= n) return;
     float s = 0.f;
-    for (int b = lane; b < nb; b += 64) s += part[(size_t)b * n + i];
+    int b = lane;
+    for (; b + 7 * 64 < nb; b += 8 * 64) {  // eight loads in flight
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = part[(size_t)(b + 64 * u) * n + i];
+#pragma unroll
+        for (int u = 0; u < 8; u++) s += v[u];
+    }
+    for (; b < nb; b += 64) s += part[(size_t)b * n + i];
     s = bw_wave_sum(s);
     if (lane == 0) out[i] = s;
 }
@@ -2738,9 +2768,8 @@ int launch_chunk_bwd(const BwdParams& p, hipStream_t stream) {
         launch_norm_adjoint<false>(nb, p.q, p.q_w, ws.rq, ws.dqh, B, T, Tp, H, K, p.dq, ws.dnq, stream);
         launch_norm_adjoint<false>(nb, p.k, p.k_w, ws.rk, ws.dkh, B, T, Tp, H, K, p.dk, ws.dnk, stream);
     }
-    const dim3 kb((unsigned)((K + 3) / 4));
-    hipLaunchKernelGGL(bw_reduce_kernel, kb, blk, 0, stream, ws.dnq, ws.norm_blocks, (size_t)K, p.dq_w);
-    hipLaunchKernelGGL(bw_reduce_kernel, kb, blk, 0, stream, ws.dnk, ws.norm_blocks, (size_t)K, p.dk_w);
+    hipLaunchKernelGGL(bw_reduce_kernel, dim3((unsigned)((K + 3) / 4), 2), blk, 0, stream, ws.dnq, ws.dnk, ws.norm_blocks,
+                       (size_t)K, p.dq_w, p.dk_w);
     if (!direct) {
         const size_t nv = (size_t)B * T * H * V;
         const dim3 vb((unsigned)((nv + 255) / 256)), vb4((unsigned)((nv / 4 + 255) / 256));

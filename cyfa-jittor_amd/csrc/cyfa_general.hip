@@ -135,23 +135,41 @@ __global__ __launch_bounds__(256) void gen_rows_kernel(const void* x, const floa
 // The clock lam_t = clock0 + sum_{s <= t} delta_s (ops/utils.py:229-348), in
 // double, one wave per (b, h): each lane sums a run of tokens, the runs'
 // prefix sums cross the lanes, then each lane writes its run. Padded tokens
-// add nothing; the final clock is lam at the last padded token.
+// add nothing; the final clock is lam at the last padded token. A lane's tokens
+// are a serial chain of sums: CLOCK_U loads of it are in flight at a time.
+constexpr int CLOCK_U = 16;
+
 __global__ __launch_bounds__(64) void gen_clock_kernel(const float* delta, const float* clock0, int B, int T, int Tp,
                                                        int H, double* lam, float* clock_out) {
     const int bh = blockIdx.x, b = bh / H, h = bh % H, lane = threadIdx.x;
     const int per = (Tp + 63) / 64, t0 = lane * per, t1 = min(t0 + per, Tp);
-    const auto dl = [&](int t) { return t < T ? (double)delta[((size_t)b * T + t) * H + h] : 0.0; };
+    // tokens t .. of the run, zero from min(t1, T) on (read from token T - 1 there)
+    const auto fetch = [&](int t, float* v) {
+#pragma unroll
+        for (int u = 0; u < CLOCK_U; u++) v[u] = delta[((size_t)b * T + min(t + u, T - 1)) * H + h];
+#pragma unroll
+        for (int u = 0; u < CLOCK_U; u++) v[u] = t + u < min(t1, T) ? v[u] : 0.f;
+    };
+    float v[CLOCK_U];
     double s = 0.0;
-    for (int t = t0; t < t1; t++) s += dl(t);
+    for (int t = t0; t < t1; t += CLOCK_U) {
+        fetch(t, v);
+#pragma unroll
+        for (int u = 0; u < CLOCK_U; u++) s += (double)v[u];
+    }
     double pre = s;
     for (int o = 1; o < 64; o <<= 1) {
         const double y = __shfl_up(pre, o);
         if (lane >= o) pre += y;
     }
     double run = (clock0 ? (double)clock0[bh] : 0.0) + pre - s;
-    for (int t = t0; t < t1; t++) {
-        run += dl(t);
-        lam[(size_t)bh * Tp + t] = run;
+    for (int t = t0; t < t1; t += CLOCK_U) {
+        fetch(t, v);
+#pragma unroll
+        for (int u = 0; u < CLOCK_U; u++) {
+            run += (double)v[u];
+            if (t + u < t1) lam[(size_t)bh * Tp + t + u] = run;
+        }
     }
     if (clock_out && lane == 63) clock_out[bh] = (float)run;
 }

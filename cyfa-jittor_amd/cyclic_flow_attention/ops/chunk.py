@@ -93,7 +93,7 @@ def chunk_cyfa(
                                             c0, float(q_norm_eps), float(k_norm_eps), scale, int(chunk_size))
         return o, ((hk, hv, clock) if output_final_state else None)
     return _chunk_forward(q, k, v, g, delta, beta, readout, q_norm_weight, k_norm_weight, q_norm_eps, k_norm_eps,
-                          scale, initial_state, output_final_state, chunk_size, table, output_norm, no_alloc)
+                          scale, initial_state, output_final_state, chunk_size, table, output_norm, no_alloc)[:2]
 
 
 # Largest slot count of the backward pass (the reference's decode limit,
@@ -105,7 +105,8 @@ BWD_MAX_SLOTS = 256
 def _chunk_forward(q, k, v, g, delta, beta, readout, q_norm_weight, k_norm_weight, q_norm_eps, k_norm_eps, scale,
                    initial_state, output_final_state, chunk_size, table, output_norm, no_alloc):
     """The forward op: the tuned kernels at K = V = 256, 128 slots and chunk
-    size 64, the general path at every other shape (see chunk_cyfa)."""
+    size 64, the general path at every other shape (see chunk_cyfa). Returns
+    (o, states or None, the readout table it used)."""
     state_in = tuple(initial_state) if initial_state is not None else ()
     B, T, H, K = q.shape
     V = v.shape[-1]
@@ -187,14 +188,15 @@ def _chunk_forward(q, k, v, g, delta, beta, readout, q_norm_weight, k_norm_weigh
             _native.chunk_fwd_normed(args, norm, dev)
     if out_dtype != io_dtype:
         o = o.to(out_dtype)
-    return o, ((hk, hv, clock) if output_final_state else None)
+    return o, ((hk, hv, clock) if output_final_state else None), table
 
 
 class _ChunkCyFA(torch.autograd.Function):
     """chunk_cyfa as an autograd function: the HIP forward, and the
     gradients of every floating input from cyfa_chunk_bwd, which recomputes
-    the forward in fp32 from the saved inputs (so nothing but the inputs is
-    kept between the passes). Replaces the reference's jt.Function adjoints
+    the forward in fp32 from the saved inputs (so nothing but the inputs and
+    the readout table, H (M - 1) M floats whose product takes a launch of 7 us
+    on MI355X, is kept between the passes). Replaces the reference's jt.Function adjoints
     behind chunk_cyfa (ops/chunk.py:51-71; ops/chunk_readout.py:776-786,
     976-988; ops/utils.py:297-299, 589-641, 704-754; ops/qk_norm.py:241-289)."""
 
@@ -202,9 +204,10 @@ class _ChunkCyFA(torch.autograd.Function):
     def forward(ctx, q, k, v, g, delta, beta, readout, q_norm_weight, k_norm_weight, h0k, h0v, c0, q_eps, k_eps,
                 scale, chunk_size):
         init = (h0k, h0v, c0) if h0k is not None else None
-        o, (hk, hv, clock) = _chunk_forward(q, k, v, g, delta, beta, readout, q_norm_weight, k_norm_weight, q_eps,
-                                            k_eps, scale, init, True, chunk_size, None, None, False)
-        ctx.save_for_backward(q, k, v, g, delta, beta, readout, q_norm_weight, k_norm_weight, h0k, h0v, c0)
+        o, (hk, hv, clock), table = _chunk_forward(q, k, v, g, delta, beta, readout, q_norm_weight, k_norm_weight,
+                                                   q_eps, k_eps, scale, init, True, chunk_size, None, None, False)
+        ctx.save_for_backward(q, k, v, g, delta, beta, readout, q_norm_weight, k_norm_weight, h0k, h0v, c0,
+                              table)
         ctx.eps = (q_eps, k_eps)
         ctx.scale = scale
         ctx.set_materialize_grads(False)
@@ -212,7 +215,7 @@ class _ChunkCyFA(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, d_o, d_hk, d_hv, d_clock):
-        q, k, v, g, delta, beta, readout, q_w, k_w, h0k, h0v, c0 = ctx.saved_tensors
+        q, k, v, g, delta, beta, readout, q_w, k_w, h0k, h0v, c0, table = ctx.saved_tensors
         B, T, H, K = q.shape
         V = v.shape[-1]
         M = readout.shape[-1] + 1
@@ -225,7 +228,6 @@ class _ChunkCyFA(torch.autograd.Function):
 
         qc, kc, vc = c(q, io), c(k, io), c(v, io)
         gc, dc, bc, qwc, kwc = c(g), c(delta), c(beta), c(q_w), c(k_w)
-        table = readout_table(readout.detach())
         has_h0 = h0k is not None
         h0kc, h0vc, c0c = c(h0k), c(h0v), c(c0)
         d_oc = c(d_o, io)

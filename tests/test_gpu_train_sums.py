@@ -1,0 +1,26 @@
+"""The training pass's serial sums (the clock and its cotangent, runs of tokens
+per lane in batches of 16; the norm weights' partial rows, eight per lane at a
+time) at runs and counts with remainders, against float64 autograd through the
+CPU oracle (the bars of test_gpu_backward)."""
+
+import pytest
+import torch
+
+import test_gpu_backward as tb
+from tolerance import metrics
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,T,H", [
+    (2, 3, 1),      # runs of one token, most of them padding
+    (1, 1100, 2),   # runs of 18: a batch and two tokens; padding in the last run
+    (1, 2049, 17),  # runs of 33; 545 partial rows: a batch of eight per lane and a remainder
+])
+def test_serial_sums_match_oracle_autograd(B, T, H):
+    x, init, cot = tb._inputs(B, T, H, 16, 16, 8, seed=T, dtype=torch.float32, state=True)
+    ref = tb._oracle_grads(x, init, cot, True, 64)
+    got = tb._gpu_grads(x, init, cot, True, 64)
+    for name, r in ref.items():
+        m = metrics(got[name].float(), r)
+        assert m["rrms"] < tb._bar(name, torch.float32), f"{name}: {m}"
