@@ -306,14 +306,24 @@ __global__ __launch_bounds__(T2 == 2 ? 512 : 256) void bw_state_scan_mf_kernel(S
     __shared__ float sEl;
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lr = lane & 15, lg = lane >> 4;
-    const int c0 = blockIdx.x * TS, r0 = blockIdx.y * TS, bhi = blockIdx.z;
+    // Workgroups go to the eight XCDs in turn; the tiles of one (b, h), which
+    // read the same rows of a and b, are taken eight apart, so that they share
+    // an XCD's L2 (the last B H % 8 in order): at 32 (b, h) of 32 chunks the
+    // four scans 297 -> 290 us. The small tiles, 32 workgroups to a 256 x 128
+    // state, go in order: 8 (b, h) of 16 chunks 75 us, and 81 shared.
+    const int ntile = gridDim.x * gridDim.y, wg = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+    const bool swz = T2 == 2 && wg < (int)(gridDim.z & ~7u) * ntile;
+    const int bhi = swz ? wg / (8 * ntile) * 8 + wg % 8 : wg / ntile;
+    const int tile = swz ? wg % (8 * ntile) / 8 : wg % ntile;
+    const int tcol = tile % (int)gridDim.x, trow = tile / (int)gridDim.x;
+    const int c0 = tcol * TS, r0 = trow * TS;
     const int b = bhi / p.H, h = bhi % p.H;
     const int Kq = p.Kq, Vd = p.Vd, N = p.N;
     // bnd tiles of 32 x 32: nx across Vd, ny down Kq; this workgroup's (T2 = 1)
     // or this wave's and its partner's, wave w ^ 2 (T2 = 2)
     const int nx = (Vd + 31) / 32, ny = (Kq + 31) / 32, nt = nx * ny;
-    const int ty = T2 == 1 ? (int)blockIdx.y : 2 * (int)blockIdx.y + (wv >> 2);
-    const int tx = T2 == 1 ? (int)blockIdx.x : 2 * (int)blockIdx.x + (wv & 1);
+    const int ty = T2 == 1 ? trow : 2 * trow + (wv >> 2);
+    const int tx = T2 == 1 ? tcol : 2 * tcol + (wv & 1);
     const size_t bh = bhi, ssz = (size_t)Kq * Vd;
     SE* xs = reinterpret_cast<SE*>(p.xs) + bh * (N + 1) * ssz;
     const SE* Sx = reinterpret_cast<const SE*>(p.S);
