@@ -683,6 +683,15 @@ def mask_rows(attention_mask):
     return values, valid, lengths
 
 
+def row_strides(x):
+    """(elements between rows, elements between batch rows) of x [B, n, D]; as
+    if packed where a size of one leaves x's own stride without a meaning (a
+    tensor with any stride there is contiguous to torch)."""
+    B, n, D = x.shape
+    row = x.stride(1) if n > 1 else D
+    return row, x.stride(0) if B > 1 else n * row
+
+
 def short_conv(x, weight, bias=None, cache=None, split=None, cache_out=None, mask=None, lengths=None):
     """Causal depthwise convolution over time of x [B, T, D] (rows may be strided).
 
@@ -702,12 +711,14 @@ def short_conv(x, weight, bias=None, cache=None, split=None, cache_out=None, mas
     w = weight.reshape(D, W).contiguous()
     if cache is not None and cache.stride(-1) != 1:
         cache = cache.contiguous()
-    args = CyfaConvArgs(B=B, T=T, D=D, W=W, x=ptr(x), x_row=x.stride(1),
-                        cache=ptr(cache), cache_row=0 if cache is None else cache.stride(1),
-                        cache_batch=0 if cache is None else cache.stride(0),
+    x_row, x_batch = row_strides(x)
+    cache_row, cache_batch = (0, 0) if cache is None else row_strides(cache)
+    out_row, out_batch = (0, 0) if cache_out is None else row_strides(cache_out)
+    # (with one token per batch row, the rows are the batch rows)
+    args = CyfaConvArgs(B=B, T=T, D=D, W=W, x=ptr(x), x_row=x_row if T > 1 else x_batch,
+                        cache=ptr(cache), cache_row=cache_row, cache_batch=cache_batch,
                         weight=ptr(w), bias=ptr(None if bias is None else bias.contiguous()), split=split,
-                        cache_out=ptr(cache_out), cache_out_row=0 if cache_out is None else cache_out.stride(1),
-                        cache_out_batch=0 if cache_out is None else cache_out.stride(0), mask=ptr(mask),
+                        cache_out=ptr(cache_out), cache_out_row=out_row, cache_out_batch=out_batch, mask=ptr(mask),
                         lengths=ptr(lengths))
     for i, o in enumerate(outs):
         args.out[i] = o.data_ptr()
@@ -813,13 +824,13 @@ def short_conv_grad(x, weight, cache, dy, needed, dx=None):
     lib = load_library()
     n = int(lib.cyfa_short_conv_grad_workspace_bytes(B, T, D, W))
     workspace = torch.empty(max(n, 1), dtype=torch.uint8, device=dev)  # alive until the launch
-    args = CyfaConvGradArgs(B=B, T=T, D=D, W=W, x=ptr(x), x_row=x.stride(1), cache=ptr(cache),
-                            cache_row=0 if cache is None else cache.stride(1),
-                            cache_batch=0 if cache is None else cache.stride(0), weight=ptr(weight),
-                            dy=ptr(dys[0]), dy1=ptr(dys[1] if len(dys) > 1 else None),
-                            dy2=ptr(dys[2] if len(dys) > 2 else None), split=dys[0].shape[-1],
-                            dx_row=0 if dx is None else dx.stride(1), dx=ptr(dx), dcache=ptr(dc), dweight=ptr(dw), dbias=ptr(db), workspace=ptr(workspace),
-                            workspace_bytes=n)
+    rows = [(0, 0) if t is None else row_strides(t) for t in (x, dx, cache)]
+    (x_row, dx_row), (cache_row, cache_batch) = (r if T > 1 else b for r, b in rows[:2]), rows[2]
+    args = CyfaConvGradArgs(B=B, T=T, D=D, W=W, x=ptr(x), x_row=x_row, cache=ptr(cache), cache_row=cache_row,
+                            cache_batch=cache_batch, weight=ptr(weight), dy=ptr(dys[0]),
+                            dy1=ptr(dys[1] if len(dys) > 1 else None), dy2=ptr(dys[2] if len(dys) > 2 else None),
+                            split=dys[0].shape[-1], dx_row=dx_row, dx=ptr(dx), dcache=ptr(dc), dweight=ptr(dw),
+                            dbias=ptr(db), workspace=ptr(workspace), workspace_bytes=n)
     _check(lib.cyfa_short_conv_grad(ctypes.byref(args), general_dtype(x), stream_handle(dev)), "cyfa_short_conv_grad")
     return dx, dw, db, dc
 

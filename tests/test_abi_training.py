@@ -4,6 +4,7 @@ layouts against the header, and argument errors raised before any launch."""
 import ctypes
 
 import pytest
+import torch
 
 from cyclic_flow_attention import _native
 from test_abi import _c_layout
@@ -75,3 +76,55 @@ def test_gates_train_validates_before_launch():
     assert call(0, rows=0) == call(0, g=None) == call(1, dwa=None) == call(0, dtype=2) == _native.CYFA_ERR_VALUE
     assert call(0, x=0x10008) == call(1, dx=0x10004) == _native.CYFA_ERR_ALIGN
     assert call(1, workspace_bytes=n - 4) == _native.CYFA_ERR_WORKSPACE
+
+
+class _Recorder:
+    """Stands in for the library: keeps the arguments of the one call made."""
+
+    def __getattr__(self, name):
+        def call(args, *rest):
+            if name.endswith("_workspace_bytes"):
+                return 64
+            self.args = args._obj
+            return _native.CYFA_OK
+
+        return call
+
+
+# [B, T, D] views whose size-1 dimensions carry strides that mean nothing, and
+# ordinary ones: a time-major tensor's single step, one row of a longer batch,
+# channels of a wider buffer, one batch row of a strided buffer
+@pytest.mark.parametrize("make", [
+    lambda: torch.zeros(1, 5, 8).transpose(0, 1), lambda: torch.zeros(5, 1, 24)[..., :8],
+    lambda: torch.zeros(5, 3, 8)[:, 1:2], lambda: torch.zeros(1, 3, 11)[:, 1:2, :8],
+    lambda: torch.zeros(2, 6, 24)[..., 8:16], lambda: torch.zeros(1, 12, 8)[:, ::2], lambda: torch.zeros(3, 6, 8)])
+def test_short_conv_rows_are_where_the_kernels_read_them(monkeypatch, make):
+    """The kernels read row (b, t) of x at (b T + t) x_row elements."""
+    lib = _Recorder()
+    monkeypatch.setattr(_native, "load_library", lambda: lib)
+    monkeypatch.setattr(_native, "require_device", lambda *_: torch.device("cpu"))
+    monkeypatch.setattr(_native, "stream_handle", lambda _: None)
+    x, w = make(), torch.zeros(8, 4)
+    seen = []
+    monkeypatch.setattr(_native, "ptr", lambda t: seen.append(t) or (None if t is None else t.data_ptr()))
+
+    def rows_read_back():
+        xs = next(t for t in seen if t is not None and t.data_ptr() == lib.args.x)  # x, or its copy
+        B, T, _ = xs.shape
+        assert xs.shape == x.shape and xs.stride(2) == 1
+        assert lib.args.x_row % 8 == 0 and lib.args.x_row >= 8
+        for b in range(B):
+            for t in range(T):
+                assert xs[b, t].storage_offset() - xs.storage_offset() == (b * T + t) * lib.args.x_row
+
+    _native.short_conv(x, w, None, torch.zeros(x.shape[0], 5, 11)[:, 1:4, :8].contiguous())
+    rows_read_back()
+    seen.clear()
+    _native.short_conv(x, w[:, :2].contiguous(), None, torch.zeros(x.shape[0], 5, 11)[:, 1:2, :8].contiguous())
+    assert lib.args.cache_row % 8 == lib.args.cache_batch % 8 == 0
+    rows_read_back()
+    seen.clear()
+    if x.stride(2) == 1 and (x.is_contiguous() or x.shape[:2] == (2, 6)):  # rows the gradient's callers give it
+        seen.clear()
+        _native.short_conv_grad(x, w, None, torch.zeros(x.shape), (True, True, False, False))
+        rows_read_back()

@@ -93,6 +93,34 @@ def test_short_conv_training_views_second_derivatives_and_transforms():
     assert _rel(tangent.detach(), _conv64(xs[1].double().cpu(), w64, None, None)) < 1e-6
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_short_conv_of_single_tokens_of_a_time_major_tensor(dtype):
+    """x [B, 1, D], a view of [1, B, D] whose stride over the one token spans
+    the whole tensor, and the same of the cache [B, 1, D]."""
+    gen = torch.Generator().manual_seed(11)
+    for W in (2, 4):
+        conv = ShortConvolution(24, W, True)
+        with torch.no_grad():
+            for p in conv.parameters():
+                p.copy_(0.5 * torch.randn(p.shape, generator=gen))
+        conv = conv.to(dtype)
+        base = torch.randn(1, 5, 24, generator=gen).to(dtype)
+        cbase = torch.randn(W - 1, 5, 24, generator=gen).to(dtype)
+        dy = torch.randn(5, 1, 24, generator=gen).to(dtype)
+        ref = [t.detach().double().requires_grad_(True) for t in (base, conv.weight, conv.bias, cbase)]
+        ry = _conv64(ref[0].transpose(0, 1), *ref[1:3], ref[3].transpose(0, 1))
+        rg = torch.autograd.grad(ry, ref, dy.double())
+        conv = conv.to(DEV)
+        leaves = [base.to(DEV).requires_grad_(True), conv.weight, conv.bias, cbase.to(DEV).requires_grad_(True)]
+        x, cache = leaves[0].transpose(0, 1), leaves[3].transpose(0, 1)
+        y, _ = conv(x, cache)
+        assert y.grad_fn.name() == "ShortConvBackward" and _rel(y.detach(), ry.detach()) <= _bar(dtype)
+        for a, r in zip(torch.autograd.grad(y, leaves, dy.to(DEV)), rg):
+            assert _rel(a, r) <= _bar(dtype)
+        with torch.no_grad():
+            assert _rel(conv(x, cache)[0], ry.detach()) <= _bar(dtype)
+
+
 def _norm64(x, w, gate, prescale):
     x = x * prescale
     y = x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + 1e-6) * w
