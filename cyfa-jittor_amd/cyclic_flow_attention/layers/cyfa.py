@@ -187,8 +187,12 @@ def general_short_conv(x, weight, bias, cache):
 def plain_module(m, cls):
     """Whether calling module m is cls.forward and nothing more (no subclass,
     wrapper or hook)."""
-    return (type(m) is cls and "forward" not in vars(m) and not m._forward_hooks and not m._forward_pre_hooks
-            and not m._backward_hooks and not m._backward_pre_hooks
+    if type(m) is not cls:
+        return False
+    own = m.__dict__
+    return ("forward" not in own
+            and not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"]
+                     or own["_backward_pre_hooks"])
             and not torch.nn.modules.module._has_any_global_hook())
 
 
@@ -357,8 +361,9 @@ class CyclicFlowAttention(nn.Module):
         """Whether a masked call takes the fused path: a prefill of more rows
         than a decode step's at the tuned op's shape, with an integer mask
         [B, T]. (Other masks, which may broadcast or hold fractions, other
-        shapes, and layers whose modules have hooks or are replaced by others
-        keep the general path, which calls the modules.)"""
+        shapes, and layers whose modules have hooks or are replaced by others,
+        also by ones of the same class with other biases or widths, keep the
+        general path, which calls the modules.)"""
         return (attention_mask is not None and self._fused_ok(x, None) and x.dim() == 3 and x.shape[1] > 1
                 and self.head_k_dim == 256 and self.head_v_dim == 256 and self.num_slots == 128
                 and self.chunk_size == 64
@@ -369,11 +374,22 @@ class CyclicFlowAttention(nn.Module):
 
     def _plain(self):
         """Whether the modules that the fused path reads the weights of are the
-        plain ones."""
-        return (plain_module(self.g_proj, nn.Sequential) and len(self.g_proj) == 2
-                and all(plain_linear(m) for m in (self.q_proj, self.k_proj, self.v_proj, self.a_proj, self.b_proj,
-                                                  self.d_proj, *self.g_proj, self.o_proj))
-                and all(plain_module(m, ShortConvolution) for m in (self.q_conv1d, self.k_conv1d, self.v_conv1d))
+        plain ones, of the layer's sizes, with the biases it adds and no others,
+        and convolutions of one width."""
+        if not plain_module(self.g_proj, nn.Sequential) or len(self.g_proj) != 2:
+            return False
+        g0, g1 = self.g_proj
+        H, Dk, Dv = self.num_heads, self.key_dim, self.value_dim
+        W = self.q_conv1d.width
+        linears = ((self.q_proj, Dk, False), (self.k_proj, Dk, False), (self.v_proj, Dv, False), (self.a_proj, H, False),
+                   (self.b_proj, H, True), (self.d_proj, H, True), (g0, self.head_v_dim, False),
+                   (self.o_proj, None, False))
+        convs = ((self.q_conv1d, Dk), (self.k_conv1d, Dk), (self.v_conv1d, Dv))
+        return (all(plain_linear(m) and (n is None or m.weight.shape[0] == n) and (m.bias is not None) == biased
+                    for m, n, biased in linears)
+                and plain_linear(g1) and g1.weight.shape[0] == Dv
+                and all(plain_module(m, ShortConvolution) and m.bias is None and tuple(m.weight.shape) == (n, 1, W)
+                        for m, n in convs)
                 and plain_module(self.o_norm, RMSNorm))
 
     def forward(self, x, cache=None, use_cache=False, attention_mask=None):

@@ -100,3 +100,43 @@ def test_masked_call_of_a_layer_with_hooks_calls_its_modules():
         assert len(seen) == 5
         layer.v_proj = torch.nn.Sequential(layer.v_proj)
         assert not layer._fused_mask_ok(x, mask)
+
+
+def test_masked_call_applies_the_biases_of_replaced_modules():
+    """Against the general path, which a float mask of the same values takes;
+    each replacement changes the result, and what it adds is not lost."""
+    from cyclic_flow_attention.layers.cyfa import ShortConvolution
+
+    def layer():
+        torch.manual_seed(1)
+        return CyclicFlowAttention(hidden_size=256, num_heads=1).eval().bfloat16().to(DEV)
+
+    gen = torch.Generator().manual_seed(2)
+    x = torch.randn(2, 40, 256, generator=gen).bfloat16().to(DEV)
+    mask = _mask(2, 40, gen, "prefix").to(DEV)
+    with torch.no_grad():
+        plain = layer()(x, attention_mask=mask)[0]
+
+        def linear(n, bias=True):
+            m = torch.nn.Linear(256, n, bias=bias)
+            if bias:
+                m.bias.copy_(torch.randn(n, generator=gen))
+            return m
+
+        def conv():
+            m = ShortConvolution(256, 4, True)
+            m.weight.copy_(0.3 * torch.randn(m.weight.shape, generator=gen))
+            m.bias.copy_(torch.randn(256, generator=gen))
+            return m
+
+        for name, module in (("q_proj", linear(256)), ("a_proj", linear(1)), ("o_proj", linear(256)),
+                             ("k_conv1d", conv()), ("b_proj", linear(1, False))):
+            changed = layer()
+            setattr(changed, name, module.bfloat16().to(DEV))
+            y = changed(x, attention_mask=mask)[0]
+            assert torch.equal(y, changed(x, attention_mask=mask.float())[0]), name
+            assert _differs(y, plain), name
+
+
+def _differs(a, b):
+    return ((a.double() - b.double()).norm() > 2.0 ** -6 * b.double().norm()).item()

@@ -33,3 +33,35 @@ def test_replaced_or_hooked_output_norm_gets_the_scaled_input(monkeypatch):
 
     layer.o_norm = Norm(layer.o_norm)
     assert torch.equal(layer(x)[0], plain)
+
+
+def _replacements():
+    """Modules of a layer's own classes that the fused masked path does not
+    compute: (name, module of a layer of 32 columns, 2 heads)."""
+    from torch import nn
+
+    for name in ("q_proj", "k_proj", "v_proj", "o_proj"):
+        yield name, nn.Linear(32, 32)
+    yield "a_proj", nn.Linear(32, 2)
+    for name in ("b_proj", "d_proj"):
+        yield name, nn.Linear(32, 2, bias=False)
+    yield "g_proj", nn.Sequential(nn.Linear(32, 16), nn.Linear(16, 32))
+    for name in ("q_conv1d", "k_conv1d", "v_conv1d"):
+        yield name, cyfa.ShortConvolution(32, 4, True)
+        yield name, cyfa.ShortConvolution(32, 3)
+        yield name, cyfa.ShortConvolution(16, 4)
+    yield "k_proj", nn.Linear(32, 16, bias=False)
+
+
+def test_only_layers_with_the_biases_and_sizes_of_the_fused_path_are_plain():
+    def layer():
+        return CyclicFlowAttention(hidden_size=32, num_heads=2, head_dim=16, num_slots=8)
+
+    assert layer()._plain()
+    for name, module in _replacements():
+        changed = layer()
+        setattr(changed, name, module)
+        assert not changed._plain(), (name, module)
+    unbiased = layer()  # g_proj[1]'s bias may be missing: the fused path takes that
+    unbiased.g_proj[1].bias = None
+    assert unbiased._plain()
