@@ -24,3 +24,21 @@ def test_serial_sums_match_oracle_autograd(B, T, H):
     for name, r in ref.items():
         m = metrics(got[name].float(), r)
         assert m["rrms"] < tb._bar(name, torch.float32), f"{name}: {m}"
+
+
+@pytest.fixture(scope="module")
+def long_fp32_errors():
+    """Relative errors against float64 of the fp32 gradients of 131072 token
+    rows (16 blocks of 32 rows per readout workgroup, 2048 chunks): one pass, so
+    the kernels' rounding alone, the same on every run."""
+    x, init, cot = tb._inputs(4, 4096, 8, 16, 16, 8, seed=4, dtype=torch.float32, state=False)
+    ref = tb._oracle_grads(x, init, cot, False, 64)
+    got = tb._gpu_grads(x, init, cot, False, 64)
+    return {name: metrics(got[name], r)["rrms"] for name, r in ref.items()}
+
+
+# what fp32 FMA loops over the tokens and rows, in order, left on these inputs
+# (measured), and half a percent
+@pytest.mark.parametrize("name,loops", [("q", 3.796e-7), ("k", 4.013e-7), ("v", 3.034e-7)])
+def test_fp32_gradients_are_no_further_off_than_loops(long_fp32_errors, name, loops):
+    assert long_fp32_errors[name] <= 1.005 * loops
