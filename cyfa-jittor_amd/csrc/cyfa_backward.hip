@@ -1820,16 +1820,23 @@ __global__ __launch_bounds__(RO_ADJ_THREADS) void bw_readout_kernel(ReadoutGradA
             a.dlam[row] = v;
             a.dgq[row] = g;
         }
-        // dtable[r][m] += sum_i p[i][r] du[i][m] + dl[i][r] z[i][m] over the block's rows
+        // dtable[r][m] += sum_i p[i][r] du[i][m] + dl[i][r] z[i][m] over the block's rows,
+        // each block's sum added to the workgroup's (one chain over all of its rows
+        // left the readout's gradient 2 to 3% further off at two blocks)
+        f32x4 dblk[DRT];
+#pragma unroll
+        for (int rt = 0; rt < DRT; rt++) dblk[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
         for (int k0 = 0; k0 < RO_BLK; k0 += 4) {
             const float bu = sDU[k0 + lk][16 * dm + lr], bz = sZ[k0 + lk][16 * dm + lr];
 #pragma unroll
             for (int rt = 0; rt < DRT; rt++) {
                 const float ap = sP[k0 + lk][16 * (dr0 + rt) + lr], al = sDL[k0 + lk][16 * (dr0 + rt) + lr];
-                dacc[rt] = mfma4(ap, bu, dacc[rt]);
-                dacc[rt] = mfma4(al, bz, dacc[rt]);
+                dblk[rt] = mfma4(ap, bu, dblk[rt]);
+                dblk[rt] = mfma4(al, bz, dblk[rt]);
             }
         }
+#pragma unroll
+        for (int rt = 0; rt < DRT; rt++) dacc[rt] += dblk[rt];
     }
     // lane holds dtable rows 16 (dr0 + rt) + 4 lk + q of column 16 dm + lr
     float* dst = a.dtab + ((size_t)h * gridDim.x + blk) * RM;
