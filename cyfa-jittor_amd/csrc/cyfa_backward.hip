@@ -1376,7 +1376,8 @@ __device__ __forceinline__ float rows4_reduce(float x) {
 struct ReadoutGradArgs {
     const float *raw, *cs, *sn, *table, *dwts;  // head-major rows; table [H, M-1, M]
     float* wts;                                 // the forward's slot weights
-    float *draw, *dlam, *dgq, *dtab;            // dgq: z.dz + u.du per row; dtab: [H, workgroups, (M-1) M]
+    float *draw, *dtab;                         // dtab: [H, workgroups, (M-1) M]
+    double *dlam, *dgq;                         // per row: the clock's share; z.dz + u.du
     int B, Tp, H, M;
     int per_wg;                                 // blocks of 32 rows per workgroup
 };
@@ -1660,7 +1661,7 @@ __global__ __launch_bounds__(RO_ADJ_THREADS) void bw_readout_kernel(ReadoutGradA
     __shared__ float sTab[TM * LD];  // rows R .. 127 and columns M .. 127 zero
     __shared__ float sZ[RO_BLK][LD], sDU[RO_BLK][LD], sP[RO_BLK][LD], sDL[RO_BLK][LD];
     __shared__ float sCs[RO_BLK][TM / 2], sSn[RO_BLK][TM / 2];
-    __shared__ float sLam[RO_BLK][NW / 2], sGq[RO_BLK][NW / 2];
+    __shared__ double sLam[RO_BLK][NW / 2], sGq[RO_BLK][NW / 2];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, blk = blockIdx.x, h = blockIdx.y;
     const int lr = lane & 15, lk = lane >> 4;  // operand row / column and k of this lane
     const int M = a.M, R = M - 1, P = M / 2, RM = R * M;
@@ -1777,25 +1778,28 @@ __global__ __launch_bounds__(RO_ADJ_THREADS) void bw_readout_kernel(ReadoutGradA
             // kappa_p [(z_e dz_o - z_o dz_e) + (du_e u_o - du_o u_e)] (a rotation keeps
             // the 2-d cross product); the even lane of a pair forms it.
             const bool odd = (lr & 1) != 0;
-            // (Every lane adds its column's z dz + u du to the gate's share.)
-            float dl[4] = {0.f, 0.f, 0.f, 0.f}, gq[4] = {0.f, 0.f, 0.f, 0.f};
+            // (Every lane adds its column's z dz + u du to the gate's share.) Both in
+            // double: bw_token_kernel's terms cancel most of them.
+            double dl[4] = {0.0, 0.0, 0.0, 0.0}, gq[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
             for (int t = 0; t < CPW; t++) {
                 const int m = 16 * (ct0 + t) + lr, pr = m >> 1;
+                const double kappa = kTwoPiBw * pr / R;
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     const float gz = accz[t][q], gx = dpp_mov<0xB1>(gz);
                     const float gu = accu[t][q], ux = dpp_mov<0xB1>(gu);
                     const float zm = sZ[16 * it + 4 * lk + q][m], dm = sDU[16 * it + 4 * lk + q][m];
                     const float zx = dpp_mov<0xB1>(zm), dx = dpp_mov<0xB1>(dm);
-                    gq[q] += zm * gz + dm * gu;  // zero past M and past the last row
+                    gq[q] += (double)zm * gz + (double)dm * gu;  // zero past M and past the last row
                     const float ge = odd ? gx : gz, go = odd ? gz : gx, ue = odd ? ux : gu, uo = odd ? gu : ux;
                     const int i = 16 * it + 4 * lk + q, rho = b0 + i;
                     if (rho < rows && pr < P) {
                         const size_t row = ((size_t)(rho / a.Tp) * a.H + h) * a.Tp + rho % a.Tp;
                         const float c = sCs[i][pr], s = sSn[i][pr];
                         a.draw[row * M + m] = odd ? -s * ge + c * go : c * ge + s * go;
-                        if (!odd) dl[q] += (float)(kTwoPiBw * pr / R) * ((zm * go - zx * ge) + (dm * uo - dx * ue));
+                        if (!odd)
+                            dl[q] += kappa * (((double)zm * go - (double)zx * ge) + ((double)dm * uo - (double)dx * ue));
                     }
                 }
             }
@@ -1803,17 +1807,20 @@ __global__ __launch_bounds__(RO_ADJ_THREADS) void bw_readout_kernel(ReadoutGradA
             // in tile order), then the waves of the row tile in wave order
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-                const float v = wave_sum<16>(dl[q]), g = wave_sum<16>(gq[q]);
+                for (int o = 8; o > 0; o >>= 1) {
+                    dl[q] += __shfl_xor(dl[q], o);
+                    gq[q] += __shfl_xor(gq[q], o);
+                }
                 if (lr == 0) {
-                    sLam[16 * it + 4 * lk + q][wv >> 1] = v;
-                    sGq[16 * it + 4 * lk + q][wv >> 1] = g;
+                    sLam[16 * it + 4 * lk + q][wv >> 1] = dl[q];
+                    sGq[16 * it + 4 * lk + q][wv >> 1] = gq[q];
                 }
             }
         }
         __syncthreads();
         if (tid < RO_BLK && b0 + tid < rows) {  // the clock's and the gate's share per row
             const int rho = b0 + tid;
-            float v = sLam[tid][0], g = sGq[tid][0];
+            double v = sLam[tid][0], g = sGq[tid][0];
 #pragma unroll
             for (int j = 1; j < NW / 2; j++) v += sLam[tid][j], g += sGq[tid][j];
             const size_t row = ((size_t)(rho / a.Tp) * a.H + h) * a.Tp + rho % a.Tp;
@@ -1864,8 +1871,8 @@ constexpr int BW_WIDE_CT = BW_WIDE_MW / BC;    // column tiles of a row (the clo
 struct WideArgs {
     const float *raw, *cs, *sn, *table, *dwts;  // head-major rows; table [H, M-1, M]
     float *lg, *dl;                             // [B H Tp, MW]: logits then p; dp then dl
-    float *wts, *draw, *dlp, *dlam;             // dlp [B H Tp, 2 BW_WIDE_CT]: the clock's and the gate's partials
-    float* dgq;
+    float *wts, *draw, *dlp;                    // dlp [B H Tp, 2 BW_WIDE_CT]: the clock's and the gate's partials
+    double *dlam, *dgq;
     float* dtab;                                // [H, splits, (M-1) M]
     int B, Tp, H, M, splits;
     int bf;                                     // forward: round z, the table, p and the weights to bf16
@@ -2072,39 +2079,52 @@ __global__ __launch_bounds__(256) void bw_wide_dtable_kernel(WideArgs a) {
 // then wave 0 scans. Bound by HBM: dw_1, dw_2 and the phases, 100 MB at 65536
 // rows of 128 slots, 23 us; reading the rows of q, k and their cotangents for
 // the dot products themselves it took 104 us (470 MB).
+// A: the accumulator of the gate's and the clock's terms, which cancel those of
+// the readout in part: float for bf16 calls, double for fp32 ones. Against 64
+// bits, over 30 inputs each of seven fp32 shapes, dg's error is 0.89 to 0.96 of
+// what the rows' dot products left (in float 0.98 to 1.04 of it), ddelta's 0.84
+// to 0.99 of that in float.
 struct TokenGradArgs {
     const float *dw1, *dw2;              // [.., M]
     const float *cs, *sn;                // [.., M/2]
     const float *bnd1, *bnd2;            // [B*H, nt, N]
-    const float* dgq;                    // [B*H, Tp]: q.dq of both passes
+    const double* dgq;                   // [B*H, Tp]: q.dq of both passes
     const float* beta;                   // [B, T, H]
-    float* dlam;                         // [B*H, Tp]: in, the readout's share; out, the total
+    double* dlam;                        // [B*H, Tp]: in, the readout's share; out, the total
     float *dg, *dbeta;                   // [B, T, H]
     int B, T, Tp, H, M, N, nt1, nt2;
 };
 constexpr int TG_U = 8;  // rows whose loads a wave has in flight
 
+// The wave's sum in every lane.
+__device__ __forceinline__ float bw_wave_sum_of(float x) { return bw_wave_sum(x); }
+__device__ __forceinline__ double bw_wave_sum_of(double x) {
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+    return x;
+}
+
+template <class A>
 __global__ __launch_bounds__(256) void bw_token_kernel(TokenGradArgs a) {
-    __shared__ float sdB[BC], sdL[BC], sBnd;
+    __shared__ A sdB[BC], sdL[BC], sBnd;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int n = blockIdx.x, bh = blockIdx.y, b = bh / a.H, h = bh % a.H;
     const int M = a.M, P = M / 2, R = M - 1;
     // the write vector's per-pair factors: sqrt(1/R) for p = 0, sqrt(2/R) after;
     // the phase derivative's 2 pi p / R for the lane's pairs p = lane, lane + 64
-    const float sp0 = (float)sqrt(1.0 / R), sp1 = (float)sqrt(2.0 / R);
-    const float kp[2] = {(float)(kTwoPiBw * lane / R), (float)(kTwoPiBw * (lane + 64) / R)};
+    const A sp0 = (A)sqrt(1.0 / R), sp1 = (A)sqrt(2.0 / R);
+    const A kp[2] = {(A)(kTwoPiBw * lane / R), (A)(kTwoPiBw * (lane + 64) / R)};
     if (wv == 3) {  // the chunk's boundary terms of both passes
-        float x = 0.f;
+        A x = 0;
         for (int i = lane; i < a.nt1; i += 64) x += a.bnd1[((size_t)bh * a.nt1 + i) * a.N + n];
         for (int i = lane; i < a.nt2; i += 64) x += a.bnd2[((size_t)bh * a.nt2 + i) * a.N + n];
-        x = bw_wave_sum(x);
+        x = bw_wave_sum_of(x);
         if (lane == 0) sBnd = x;
     }
     for (int i0 = 16 * wv; i0 < 16 * wv + 16; i0 += TG_U) {
-        float db[TG_U], dl[TG_U];
+        A db[TG_U], dl[TG_U];
         const size_t row0 = (size_t)bh * a.Tp + n * BC + i0;
 #pragma unroll
-        for (int u = 0; u < TG_U; u++) db[u] = dl[u] = 0.f;
+        for (int u = 0; u < TG_U; u++) db[u] = dl[u] = 0;
 #pragma unroll
         for (int c = 0; c < 2; c++) {
             const int p = lane + 64 * c;
@@ -2120,19 +2140,19 @@ __global__ __launch_bounds__(256) void bw_token_kernel(TokenGradArgs a) {
                 cs[u] = a.cs[f];
                 sn[u] = a.sn[f];
             }
-            const float sp = p >= P ? 0.f : p == 0 ? sp0 : sp1;
+            const A sp = p >= P ? (A)0 : p == 0 ? sp0 : sp1;
 #pragma unroll
             for (int u = 0; u < TG_U; u++) {
-                const float we = d1[u][0] + d2[u][0], wo = d1[u][1] + d2[u][1];
+                const A we = (A)d1[u][0] + d2[u][0], wo = (A)d1[u][1] + d2[u][1];
                 if (p < P) {
-                    db[u] = fmaf(sp, we * cs[u] - wo * sn[u], db[u]);
-                    dl[u] = fmaf(sp * kp[c], -we * sn[u] - wo * cs[u], dl[u]);
+                    db[u] = fma(sp, we * cs[u] - wo * sn[u], db[u]);
+                    dl[u] = fma(sp * kp[c], -we * sn[u] - wo * cs[u], dl[u]);
                 }
             }
         }
 #pragma unroll
         for (int u = 0; u < TG_U; u++) {
-            const float bb = bw_wave_sum(db[u]), ll = bw_wave_sum(dl[u]);
+            const A bb = bw_wave_sum_of(db[u]), ll = bw_wave_sum_of(dl[u]);
             if (lane == 0) {
                 sdB[i0 + u] = bb;
                 sdL[i0 + u] = ll;
@@ -2144,16 +2164,16 @@ __global__ __launch_bounds__(256) void bw_token_kernel(TokenGradArgs a) {
     const int t = n * BC + lane;
     const size_t row = (size_t)bh * a.Tp + t;
     const float bt = t < a.T ? a.beta[((size_t)b * a.T + t) * a.H + h] : 0.f;
-    float x = fmaf(-bt, sdB[lane], a.dgq[row]);
+    A x = fma((A)-bt, sdB[lane], (A)a.dgq[row]);
     if (lane == BC - 1) x += sBnd;
     for (int o = 1; o < 64; o <<= 1) {
-        const float y = __shfl_down(x, o);
+        const A y = __shfl_down(x, o);
         if (lane + o < 64) x += y;
     }
-    a.dlam[row] = fmaf(bt, sdL[lane], a.dlam[row]);
+    a.dlam[row] = fma((A)bt, sdL[lane], (A)a.dlam[row]);
     if (t < a.T) {
-        a.dg[((size_t)b * a.T + t) * a.H + h] = x;
-        a.dbeta[((size_t)b * a.T + t) * a.H + h] = sdB[lane];
+        a.dg[((size_t)b * a.T + t) * a.H + h] = (float)x;
+        a.dbeta[((size_t)b * a.T + t) * a.H + h] = (float)sdB[lane];
     }
 }
 
@@ -2161,25 +2181,25 @@ __global__ __launch_bounds__(256) void bw_token_kernel(TokenGradArgs a) {
 // delta_s; the final clock is clock0 + sum delta), dclock0 = sum_t dlam_t +
 // dclock, in double. One wave per (b, h): each lane sums a run of tokens, the
 // runs' suffix sums cross the lanes.
-__global__ __launch_bounds__(64) void bw_clock_kernel(const float* dlam, const float* d_clock, int B, int T, int Tp,
+__global__ __launch_bounds__(64) void bw_clock_kernel(const double* dlam, const float* d_clock, int B, int T, int Tp,
                                                       int H, float* ddelta, float* dclock0) {
     const int bh = blockIdx.x, b = bh / H, h = bh % H, lane = threadIdx.x;
     const int per = (Tp + 63) / 64, t0 = lane * per, t1 = min(t0 + per, Tp);
     // tokens t, t - 1, .. of the run, zero before t0: CLOCK_U loads in flight
     // for each part of a lane's serial sum
     constexpr int CLOCK_U = 16;
-    const auto fetch = [&](int t, float* v) {
+    const auto fetch = [&](int t, double* v) {
 #pragma unroll
         for (int u = 0; u < CLOCK_U; u++) v[u] = dlam[(size_t)bh * Tp + max(min(t, Tp - 1) - u, 0)];
 #pragma unroll
-        for (int u = 0; u < CLOCK_U; u++) v[u] = t - u >= t0 ? v[u] : 0.f;
+        for (int u = 0; u < CLOCK_U; u++) v[u] = t - u >= t0 ? v[u] : 0.0;
     };
-    float v[CLOCK_U];
+    double v[CLOCK_U];
     double s = 0.0;
     for (int t = t1 - 1; t >= t0; t -= CLOCK_U) {
         fetch(t, v);
 #pragma unroll
-        for (int u = 0; u < CLOCK_U; u++) s += (double)v[u];
+        for (int u = 0; u < CLOCK_U; u++) s += v[u];
     }
     double suf = s;  // sum over this lane's run and every later lane's
     for (int o = 1; o < 64; o <<= 1) {
@@ -2192,7 +2212,7 @@ __global__ __launch_bounds__(64) void bw_clock_kernel(const float* dlam, const f
         fetch(t, v);
 #pragma unroll
         for (int u = 0; u < CLOCK_U; u++) {
-            run += (double)v[u];
+            run += v[u];
             if (t - u >= t0 && t - u < T) ddelta[((size_t)b * T + t - u) * H + h] = (float)run;
         }
     }
@@ -2807,7 +2827,10 @@ int launch_chunk_bwd(const BwdParams& p, hipStream_t stream) {
     tg.N = N;
     tg.nt1 = ws.nt1;
     tg.nt2 = ws.nt2;
-    hipLaunchKernelGGL(bw_token_kernel, dim3(N, B * H), blk, 0, stream, tg);
+    if (bf)
+        hipLaunchKernelGGL(bw_token_kernel<float>, dim3(N, B * H), blk, 0, stream, tg);
+    else
+        hipLaunchKernelGGL(bw_token_kernel<double>, dim3(N, B * H), blk, 0, stream, tg);
     hipLaunchKernelGGL(bw_clock_kernel, dim3(B * H), dim3(64), 0, stream, ws.dlam, p.d_clock, B, T, Tp, H, p.ddelta,
                        p.dclock0);
     // the q/k norms, their weights, v's layout

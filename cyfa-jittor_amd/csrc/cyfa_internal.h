@@ -417,9 +417,9 @@ struct BwdParams {
 // per-chunk boundary terms of the gate cotangent, per-block partial sums of
 // the table and norm-weight cotangents).
 struct BwdWorkspace {
-    double* lam;
+    double *lam, *dlam, *dgq;
     float *qh, *kh, *rq, *rk, *vh, *w, *cs, *sn, *raw, *wts, *sk, *sv;
-    float *dO, *dsk, *dsv, *dwts, *dw2, *dvh, *draw, *dlam, *dgq, *dqh, *dkh, *dw1, *bnd1, *bnd2, *dtab, *dnq, *dnk;
+    float *dO, *dsk, *dsv, *dwts, *dw2, *dvh, *draw, *dqh, *dkh, *dw1, *bnd1, *bnd2, *dtab, *dnq, *dnk;
     float *lg, *dlw, *dlp;  // the wide readout (M > BWD_TABLE_M): logits / p, dp / dl [rows, 256]; clock and gate partials [rows, 8]
     int N, nt1, nt2, ro_blocks, norm_blocks;
     size_t bytes;
@@ -481,8 +481,8 @@ inline BwdWorkspace bwd_workspace(int B, int T, int H, int K, int V, int M, void
     w.dw2 = f(rows * M);
     w.dvh = f(rows * V);
     w.draw = f(rows * M);
-    w.dlam = f(rows);
-    w.dgq = f(rows);
+    w.dlam = reinterpret_cast<double*>(take(rows * 8));
+    w.dgq = reinterpret_cast<double*>(take(rows * 8));
     w.dqh = f(rows * K);
     w.dkh = f(rows * K);
     w.dw1 = f(rows * M);

@@ -40,6 +40,7 @@ def long_fp32_errors():
 # what fp32 FMA loops over the tokens and rows, in order, left on these inputs
 # (measured), and half a percent
 @pytest.mark.parametrize("name,loops", [("q", 3.796e-7), ("k", 4.013e-7), ("v", 3.034e-7),
-                                        ("readout", 5.572e-7)])
+                                        ("readout", 5.572e-7), ("g", 4.79e-7), ("beta", 3.254e-7),
+                                        ("delta", 5.014e-6)])
 def test_fp32_gradients_are_no_further_off_than_loops(long_fp32_errors, name, loops):
     assert long_fp32_errors[name] <= 1.005 * loops
