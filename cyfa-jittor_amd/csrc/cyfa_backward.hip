@@ -1807,13 +1807,10 @@ __global__ __launch_bounds__(RO_ADJ_THREADS) void bw_readout_kernel(ReadoutGradA
             // in tile order), then the waves of the row tile in wave order
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-                for (int o = 8; o > 0; o >>= 1) {
-                    dl[q] += __shfl_xor(dl[q], o);
-                    gq[q] += __shfl_xor(gq[q], o);
-                }
+                const double v = wave_sum<16>(dl[q]), g = wave_sum<16>(gq[q]);
                 if (lr == 0) {
-                    sLam[16 * it + 4 * lk + q][wv >> 1] = dl[q];
-                    sGq[16 * it + 4 * lk + q][wv >> 1] = gq[q];
+                    sLam[16 * it + 4 * lk + q][wv >> 1] = v;
+                    sGq[16 * it + 4 * lk + q][wv >> 1] = g;
                 }
             }
         }
@@ -2096,13 +2093,6 @@ struct TokenGradArgs {
 };
 constexpr int TG_U = 8;  // rows whose loads a wave has in flight
 
-// The wave's sum in every lane.
-__device__ __forceinline__ float bw_wave_sum_of(float x) { return bw_wave_sum(x); }
-__device__ __forceinline__ double bw_wave_sum_of(double x) {
-    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
-    return x;
-}
-
 template <class A>
 __global__ __launch_bounds__(256) void bw_token_kernel(TokenGradArgs a) {
     __shared__ A sdB[BC], sdL[BC], sBnd;
@@ -2117,7 +2107,7 @@ __global__ __launch_bounds__(256) void bw_token_kernel(TokenGradArgs a) {
         A x = 0;
         for (int i = lane; i < a.nt1; i += 64) x += a.bnd1[((size_t)bh * a.nt1 + i) * a.N + n];
         for (int i = lane; i < a.nt2; i += 64) x += a.bnd2[((size_t)bh * a.nt2 + i) * a.N + n];
-        x = bw_wave_sum_of(x);
+        x = wave_sum(x);
         if (lane == 0) sBnd = x;
     }
     for (int i0 = 16 * wv; i0 < 16 * wv + 16; i0 += TG_U) {
@@ -2152,7 +2142,7 @@ __global__ __launch_bounds__(256) void bw_token_kernel(TokenGradArgs a) {
         }
 #pragma unroll
         for (int u = 0; u < TG_U; u++) {
-            const A bb = bw_wave_sum_of(db[u]), ll = bw_wave_sum_of(dl[u]);
+            const A bb = wave_sum(db[u]), ll = wave_sum(dl[u]);
             if (lane == 0) {
                 sdB[i0 + u] = bb;
                 sdL[i0 + u] = ll;

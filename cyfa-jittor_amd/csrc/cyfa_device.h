@@ -150,21 +150,36 @@ __device__ __forceinline__ float lane_value(float x, int lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
 }
 
+// The same of a double, half by half.
+typedef int i32x2 __attribute__((ext_vector_type(2)));
+
+template <int CTRL>
+__device__ __forceinline__ double dpp_mov(double x) {
+    const i32x2 v = __builtin_bit_cast(i32x2, x);
+    return __builtin_bit_cast(double, i32x2{__builtin_amdgcn_mov_dpp(v[0], CTRL, 0xF, 0xF, true),
+                                            __builtin_amdgcn_mov_dpp(v[1], CTRL, 0xF, 0xF, true)});
+}
+
+__device__ __forceinline__ double lane_value(double x, int lane) {
+    const i32x2 v = __builtin_bit_cast(i32x2, x);
+    return __builtin_bit_cast(double, i32x2{__builtin_amdgcn_readlane(v[0], lane), __builtin_amdgcn_readlane(v[1], lane)});
+}
+
 // Sum (max) over aligned groups of W lanes, in every lane of the group; every
 // lane of the wave must be active. Fixed order: pairs (quad_perm [1,0,3,2]),
 // quads ([2,3,0,1]), octets (row_half_mirror), rows of 16 (row_mirror) - after
 // each step every lane of a group holds the same value, so a mirror reads the
 // value the matching xor lane holds - then rows (0 + 1) and (2 + 3), then
 // their sum.
-template <int W = 64>
-__device__ __forceinline__ float wave_sum(float x) {
+template <int W = 64, class X = float>
+__device__ __forceinline__ X wave_sum(X x) {
     static_assert(W == 16 || W == 32 || W == 64, "group of 16, 32 or 64 lanes");
     x += dpp_mov<0xB1>(x);
     x += dpp_mov<0x4E>(x);
     x += dpp_mov<0x141>(x);
     x += dpp_mov<0x140>(x);
     if (W == 16) return x;
-    const float lo = lane_value(x, 0) + lane_value(x, 16), hi = lane_value(x, 32) + lane_value(x, 48);
+    const X lo = lane_value(x, 0) + lane_value(x, 16), hi = lane_value(x, 32) + lane_value(x, 48);
     if (W == 32) return (threadIdx.x & 32) ? hi : lo;
     return lo + hi;
 }
