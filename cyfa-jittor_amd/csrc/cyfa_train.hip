@@ -302,12 +302,13 @@ __global__ __launch_bounds__(256) void norm_grad_kernel(NormTrainParams p) {
                 for (int i = 0; i < 4; i++) sum = fmaf(xs[r][j][i] * w[j][i], dy[r][j][i] * sg[r][j][i], sum);
             const float cr = rs * rs * rs * wave_sum(sum) / (float)p.D;
             const size_t base = (size_t)(row0 + r) * p.D;
+            if (row0 + r >= p.rows) break;  // (a zero row's r is infinite where eps is zero)
 #pragma unroll
             for (int j = 0; j < J; j++) {
                 const int d = 4 * lane + 256 * j;
                 const f32x4 u = dy[r][j] * sg[r][j];
                 dw[j] += u * xs[r][j] * rs;
-                if (row0 + r < p.rows && d < p.D) {
+                if (d < p.D) {
                     if (p.dx) {
                         f32x4 dxs = w[j] * u * rs - xs[r][j] * cr;
                         if (p.prescale != 1.f) {

@@ -167,6 +167,23 @@ def test_rms_norm_training_gradients(rows, D, gate, prescale, dtype):
         assert a.requires_grad and _rel(a.detach(), r) <= 2 * bar
 
 
+# rows that leave a place of the last pair of rows empty, and eps that adds nothing
+@pytest.mark.parametrize("rows,D", [(1, 256), (3, 1024), (33, 256), (33, 1024), (7, 2048)])
+@pytest.mark.parametrize("eps", [0.0, 1e-46])
+def test_rms_norm_gradients_without_eps(rows, D, eps):
+    gen = torch.Generator().manual_seed(rows + D)
+    norm = RMSNorm(D, eps).to(DEV)
+    x, g, dy = (torch.randn(rows, D, generator=gen) for _ in range(3))
+    ref = [t.detach().double().cpu().requires_grad_(True) for t in (x, norm.weight, g)]
+    r = ref[0] * torch.rsqrt(ref[0].pow(2).mean(-1, keepdim=True)) * ref[1] * torch.sigmoid(ref[2])
+    rg = torch.autograd.grad(r, ref, dy.double())
+    xg, gg = x.to(DEV).requires_grad_(True), g.to(DEV).requires_grad_(True)
+    y = norm(xg, gg)
+    assert y.grad_fn.name() == "GatedNormBackward"
+    for a, b in zip(torch.autograd.grad(y, [xg, norm.weight, gg], dy.to(DEV)), rg):
+        assert _rel(a, b) <= 2 * _bar(torch.float32)
+
+
 def test_rms_norm_takes_misaligned_rows():
     norm = RMSNorm(1024, 1e-6).to(DEV)
     x = torch.randn(3 * 1024 + 1, device=DEV).bfloat16()[1:].view(3, 1024)  # rows off the 16-byte grid
