@@ -102,7 +102,8 @@ __global__ __launch_bounds__(256) void conv_grad_kernel(ConvGradParams p) {
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 const int t = tb + u;
-                xw[W - 1] = t < T ? xn[u] : zero;
+                if (t >= T) break;  // (zero times a row of X before the end may be a NaN)
+                xw[W - 1] = xn[u];
                 dyw[W - 1] = t + W - 1 < T ? dn[u] : zero;
                 f32x4 s = zero;
 #pragma unroll
@@ -111,7 +112,7 @@ __global__ __launch_bounds__(256) void conv_grad_kernel(ConvGradParams p) {
                     dw[w] += dyw[0] * xw[w];
                 }
                 dw[W] += dyw[0];
-                if (dx && t < T) store4(dx + (size_t)t * p.dx_row, s);
+                if (dx) store4(dx + (size_t)t * p.dx_row, s);
 #pragma unroll
                 for (int w = 0; w < W - 1; w++) {
                     xw[w] = xw[w + 1];

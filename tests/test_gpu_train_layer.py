@@ -121,6 +121,21 @@ def test_short_conv_of_single_tokens_of_a_time_major_tensor(dtype):
             assert _rel(conv(x, cache)[0], ry.detach()) <= _bar(dtype)
 
 
+@pytest.mark.parametrize("T,dtype", [(1, torch.float32), (13, torch.bfloat16), (21, torch.float32), (66, torch.bfloat16)])
+def test_short_conv_gradients_with_an_infinite_last_token(T, dtype):
+    """The last row of x meets one tap only: the others' gradients are finite."""
+    gen = torch.Generator().manual_seed(T)
+    conv = ShortConvolution(16, 4, True).to(dtype).to(DEV)
+    x, dy = torch.randn(2, T, 16, generator=gen).to(dtype), torch.randn(2, T, 16, generator=gen).to(dtype)
+    x[:, -1] = float("inf")
+    h = F.pad(x.double(), (0, 0, 3, 0))
+    ref = torch.stack([(dy.double() * h[:, w:w + T]).sum((0, 1)) for w in range(4)], -1)
+    y, _ = conv(x.to(DEV).requires_grad_(True))
+    gw, gb = torch.autograd.grad(y, [conv.weight, conv.bias], dy.to(DEV))
+    assert _rel(gw[:, 0, :3], ref[:, :3]) <= _bar(dtype) and _rel(gb, dy.double().sum((0, 1))) <= _bar(dtype)
+    assert torch.equal(gw[:, 0, 3].double().cpu().isfinite(), ref[:, 3].isfinite())
+
+
 def _norm64(x, w, gate, prescale):
     x = x * prescale
     y = x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + 1e-6) * w
