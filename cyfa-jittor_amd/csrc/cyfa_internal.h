@@ -193,6 +193,7 @@ struct NormTrainParams {
     int rows_wg;                 // rows of an adjoint workgroup (set by the launcher)
 };
 constexpr int NORM_TRAIN_MAX_D = 2048;
+constexpr long long NORM_TRAIN_MAX_ROWS = 4ll * ((1 << 24) - 1);  // four rows per workgroup of 256, fewer than 2^32 threads
 
 // The gate projections and activations of a training step and their adjoint
 // (cyfa_train.hip): x [rows, K], the weights [H, K], the biases bb, bd [H], abd

@@ -630,7 +630,7 @@ size_t norm_grad_workspace_bytes(long long rows, int D) {
 }
 
 int launch_norm_train(const NormTrainParams& p, bool bf16, bool grad, hipStream_t stream) {
-    if (p.rows < 1 || p.rows > (1ll << 31) - 4 || p.D < 4 || p.D % 4 || p.D > NORM_TRAIN_MAX_D) return -1;
+    if (p.rows < 1 || p.rows > NORM_TRAIN_MAX_ROWS || p.D < 4 || p.D % 4 || p.D > NORM_TRAIN_MAX_D) return -1;
     return bf16 ? launch_norm_train_j<bf16_t>(p, grad, stream) : launch_norm_train_j<float>(p, grad, stream);
 }
 

@@ -771,6 +771,7 @@ def gates_grad(x, wa, wb, wd, dt_bias, A_log, abd, dg, dbeta, ddelta, need_dx):
 
 
 NORM_TRAIN_MAX_D = 2048
+NORM_TRAIN_MAX_ROWS = 4 * ((1 << 24) - 1)  # a launch has fewer than 2^32 threads, a wave per row
 
 
 def norm_train(x, weight, gate, eps, prescale):

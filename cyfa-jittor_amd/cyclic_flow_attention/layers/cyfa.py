@@ -111,7 +111,7 @@ class RMSNorm(nn.Module):
 
         weight = self.weight.float()
         if (x.dtype in (torch.bfloat16, torch.float32) and D % 4 == 0 and D <= _native.NORM_TRAIN_MAX_D
-                and x.numel() > 0 and tuple(weight.shape) == (D,)
+                and 0 < x.numel() <= D * _native.NORM_TRAIN_MAX_ROWS and tuple(weight.shape) == (D,)
                 and (gate is None or (gate.dtype == x.dtype and gate.shape == x.shape))
                 and hip_autograd_ok(x, weight, gate)):
             # training: the norm and its adjoint as HIP kernels

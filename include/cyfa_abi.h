@@ -520,7 +520,7 @@ size_t cyfa_short_conv_grad_workspace_bytes(int B, int T, int D, int W);
 int cyfa_short_conv_grad(const CyfaConvGradArgs *args, int dtype, void *hip_stream);
 
 /* The gated RMS norm of a training step (RMSNorm.execute, layers/cyfa.py:62-135)
- * on rows [rows, D], D a multiple of 4 up to 2048, x, gate, out, dy, dx and
+ * on up to 2^26 - 4 rows [rows, D], D a multiple of 4 up to 2048, x, gate, out, dy, dx and
  * dgate of one dtype (CYFA_DTYPE_BF16 or CYFA_DTYPE_F32), every pointer 16-byte
  * aligned:
  *   xs = x prescale (rounded to the dtype), r = (mean xs^2 + eps)^-1/2

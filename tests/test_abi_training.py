@@ -56,6 +56,9 @@ def test_norm_train_validates_before_launch():
         return lib.cyfa_norm_train(ctypes.byref(a), dtype, grad, None)
 
     assert call(0, D=258) == call(1, D=4096) == _native.CYFA_ERR_UNSUPPORTED
+    past = _native.NORM_TRAIN_MAX_ROWS + 1  # past a grid of 2^32 threads
+    size = lib.cyfa_norm_grad_workspace_bytes(past, 4)
+    assert call(0, rows=past, D=4) == call(1, rows=past, D=4, workspace_bytes=size) == _native.CYFA_ERR_UNSUPPORTED
     assert call(0, out=None) == call(1, dy=None) == call(1, dgate=0x60000) == call(0, dtype=3) == _native.CYFA_ERR_VALUE
     assert call(0, x=0x10008) == _native.CYFA_ERR_ALIGN
     assert call(1, workspace_bytes=n - 4) == _native.CYFA_ERR_WORKSPACE

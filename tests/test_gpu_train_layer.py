@@ -5,6 +5,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
+from cyclic_flow_attention import _native
 from cyclic_flow_attention.layers.cyfa import RMSNorm, ShortConvolution
 
 pytestmark = pytest.mark.gpu
@@ -197,6 +198,16 @@ def test_rms_norm_gradients_without_eps(rows, D, eps):
     assert y.grad_fn.name() == "GatedNormBackward"
     for a, b in zip(torch.autograd.grad(y, [xg, norm.weight, gg], dy.to(DEV)), rg):
         assert _rel(a, b) <= 2 * _bar(torch.float32)
+
+
+def test_rms_norm_of_more_rows_than_a_launch_takes(monkeypatch):
+    norm = RMSNorm(64, 1e-6).to(DEV)
+    x = torch.randn(5, 7, 64, device=DEV, requires_grad=True)
+    y = norm(x)
+    monkeypatch.setattr(_native, "NORM_TRAIN_MAX_ROWS", 34)
+    z = norm(x)
+    assert y.grad_fn.name() == "GatedNormBackward" != z.grad_fn.name()
+    assert _rel(z.detach(), y.detach().double().cpu()) <= 1e-6
 
 
 def test_rms_norm_takes_misaligned_rows():
