@@ -368,6 +368,7 @@ class CyclicFlowAttention(nn.Module):
                 and self.head_k_dim == 256 and self.head_v_dim == 256 and self.num_slots == 128
                 and self.chunk_size == 64
                 and x.shape[0] * x.shape[1] > _native.LINEAR_ROWS_MAX
+                and x.shape[0] <= _native.SHORT_CONV_MAX_GRID and x.shape[1] <= 32 * _native.SHORT_CONV_MAX_GRID
                 and tuple(attention_mask.shape) == tuple(x.shape[:2]) and attention_mask.device == x.device
                 and attention_mask.dtype in (torch.int64, torch.int32, torch.bool, torch.uint8)
                 and self._plain())

@@ -102,6 +102,19 @@ def test_masked_call_of_a_layer_with_hooks_calls_its_modules():
         assert not layer._fused_mask_ok(x, mask)
 
 
+def test_masked_call_past_the_convolution_launch_keeps_the_general_path(monkeypatch):
+    """More tokens, or batch rows, than a launch of the convolution takes."""
+    torch.manual_seed(0)
+    layer = CyclicFlowAttention(hidden_size=256, num_heads=1).eval().bfloat16().to(DEV)
+    x = torch.randn(3, 96, 256, dtype=torch.bfloat16, device=DEV)
+    mask = torch.ones(3, 96, dtype=torch.long, device=DEV)
+    with torch.no_grad():
+        assert layer._fused_mask_ok(x, mask)
+        monkeypatch.setattr(_native, "SHORT_CONV_MAX_GRID", 3)
+        assert layer._fused_mask_ok(x, mask) and not layer._fused_mask_ok(x.repeat(2, 1, 1), mask.repeat(2, 1))
+        assert not layer._fused_mask_ok(x.repeat(1, 2, 1), mask.repeat(1, 2))
+
+
 def test_masked_call_applies_the_biases_of_replaced_modules():
     """Against the general path, which a float mask of the same values takes;
     each replacement changes the result, and what it adds is not lost."""
