@@ -17,7 +17,7 @@ def hip_autograd_ok(*tensors):
     """Whether a call that records gradients may take these functions: plain
     tensors of one GPU, and nothing that has to see the torch operations
     themselves (torch.func transforms, forward-mode derivatives, tracing or
-    compiling, autocast)."""
+    compiling, dispatch modes, which make_fx and operation counters are, autocast)."""
     given = [t for t in tensors if t is not None]
     if not all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda for t in given):
         return False
@@ -25,7 +25,8 @@ def hip_autograd_ok(*tensors):
         return False
     return (torch.is_grad_enabled() and not torch.is_autocast_enabled("cuda")
             and torch._C._functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0
-            and not torch.compiler.is_compiling() and not torch.jit.is_tracing())
+            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+            and torch._C._len_torch_dispatch_stack() == 0)
 
 
 def _through_torch(*cotangents):

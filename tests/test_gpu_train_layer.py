@@ -137,6 +137,21 @@ def test_short_conv_gradients_with_an_infinite_last_token(T, dtype):
     assert torch.equal(gw[:, 0, 3].double().cpu().isfinite(), ref[:, 3].isfinite())
 
 
+def test_traced_training_calls_record_the_torch_operations():
+    """A graph traced from one input gives another input's result."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    torch.manual_seed(0)
+    conv, norm = ShortConvolution(16, 4).to(DEV), RMSNorm(16, 1e-6).to(DEV)
+    x, x2 = torch.randn(2, 20, 16, device=DEV), torch.randn(2, 20, 16, device=DEV)
+
+    def call(t):
+        return norm(conv(t)[0])
+
+    graph = make_fx(call)(x)
+    assert _rel(graph(x2).detach(), call(x2).detach().double().cpu()) <= 1e-5
+
+
 def _norm64(x, w, gate, prescale):
     x = x * prescale
     y = x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + 1e-6) * w
