@@ -184,16 +184,21 @@ def general_short_conv(x, weight, bias, cache):
     return F.conv1d(padded.transpose(1, 2), weight.unsqueeze(1), bias, groups=x.shape[-1]).transpose(1, 2)
 
 
-def plain_module(m, cls):
-    """Whether calling module m is cls.forward and nothing more (no subclass,
-    wrapper or hook)."""
+def plain_parameters(m, cls):
+    """Module m's own parameters by name where calling m is cls.forward and
+    nothing more (no subclass, wrapper or hook of its own), else None."""
     if type(m) is not cls:
-        return False
+        return None
     own = m.__dict__
-    return ("forward" not in own
-            and not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"]
-                     or own["_backward_pre_hooks"])
-            and not torch.nn.modules.module._has_any_global_hook())
+    if ("forward" in own or own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"]
+            or own["_backward_pre_hooks"]):
+        return None
+    return own["_parameters"]
+
+
+def plain_module(m, cls):
+    """Whether calling module m is cls.forward and nothing more."""
+    return plain_parameters(m, cls) is not None and not torch.nn.modules.module._has_any_global_hook()
 
 
 def plain_linear(m):
@@ -358,7 +363,8 @@ class CyclicFlowAttention(nn.Module):
                 and 2 <= self.q_conv1d.width <= 4 and self.q_conv1d.bias is None)
 
     def _fused_mask_ok(self, x, attention_mask):
-        """Whether a masked call takes the fused path: a prefill of more rows
+        """Whether a masked call takes the fused path (the parameters it
+        concatenates, _plain, or a false value): a prefill of more rows
         than a decode step's at the tuned op's shape, with an integer mask
         [B, T]. (Other masks, which may broadcast or hold fractions, other
         shapes, and layers whose modules have hooks or are replaced by others,
@@ -374,28 +380,46 @@ class CyclicFlowAttention(nn.Module):
                 and self._plain())
 
     def _plain(self):
-        """Whether the modules that the fused path reads the weights of are the
-        plain ones, of the layer's sizes, with the biases it adds and no others,
-        and convolutions of one width."""
-        if not plain_module(self.g_proj, nn.Sequential) or len(self.g_proj) != 2:
-            return False
-        g0, g1 = self.g_proj
-        H, Dk, Dv = self.num_heads, self.key_dim, self.value_dim
-        W = self.q_conv1d.width
-        linears = ((self.q_proj, Dk, False), (self.k_proj, Dk, False), (self.v_proj, Dv, False), (self.a_proj, H, False),
-                   (self.b_proj, H, True), (self.d_proj, H, True), (g0, self.head_v_dim, False),
-                   (self.o_proj, None, False))
-        convs = ((self.q_conv1d, Dk), (self.k_conv1d, Dk), (self.v_conv1d, Dv))
-        return (all(plain_linear(m) and (n is None or m.weight.shape[0] == n) and (m.bias is not None) == biased
-                    for m, n, biased in linears)
-                and plain_linear(g1) and g1.weight.shape[0] == Dv
-                and all(plain_module(m, ShortConvolution) and m.bias is None and tuple(m.weight.shape) == (n, 1, W)
-                        for m, n in convs)
-                and plain_module(self.o_norm, RMSNorm))
+        """The parameters that a masked prefill concatenates, ([q|k|v|g_proj[0]|
+        a|b|d weights], [convolution weights], [b|d biases]), where every module
+        that the fused path computes is the plain one, of the layer's sizes, with
+        the biases it adds and no others, and the convolutions are of one width;
+        else None. (Read from the modules' own dictionaries: 8 us of a call that
+        is bound by the host's work, 17 by attribute.)"""
+        if torch.nn.modules.module._has_any_global_hook():
+            return None
+        mods = self._modules
+        g = mods.get("g_proj")
+        if plain_parameters(g, nn.Sequential) is None or len(g._modules) != 2:
+            return None
+        g0, g1 = g._modules.values()
+        H, Dk, Dv, W = self.num_heads, self.key_dim, self.value_dim, self.q_conv1d.width
+        weights, biases, convs = [], [], []
+        for m, n, biased in ((mods.get("q_proj"), Dk, False), (mods.get("k_proj"), Dk, False), (mods.get("v_proj"), Dv, False),
+                             (g0, self.head_v_dim, False), (mods.get("a_proj"), H, False), (mods.get("b_proj"), H, True),
+                             (mods.get("d_proj"), H, True), (mods.get("o_proj"), None, False), (g1, Dv, None)):
+            p = plain_parameters(m, nn.Linear)
+            if p is None or p.get("weight") is None or "bias" not in p:
+                return None
+            w, b = p["weight"], p["bias"]
+            if (n is not None and w.shape[0] != n) or (biased is not None and (b is not None) != biased):
+                return None
+            weights.append(w)
+            if biased:
+                biases.append(b)
+        for name, n in (("q_conv1d", Dk), ("k_conv1d", Dk), ("v_conv1d", Dv)):
+            m = mods.get(name)
+            p = plain_parameters(m, ShortConvolution)
+            if p is None or p.get("weight") is None or m.bias is not None or m.width != W \
+                    or tuple(p["weight"].shape) != (n, 1, W):
+                return None
+            convs.append(p["weight"])
+        return None if plain_parameters(mods.get("o_norm"), RMSNorm) is None else (weights[:7], convs, biases)
 
     def forward(self, x, cache=None, use_cache=False, attention_mask=None):
-        if self._fused_ok(x, attention_mask) or self._fused_mask_ok(x, attention_mask):
-            return self._forward_fused(x, cache, use_cache, attention_mask=attention_mask)
+        masked = self._fused_mask_ok(x, attention_mask)
+        if masked or self._fused_ok(x, attention_mask):
+            return self._forward_fused(x, cache, use_cache, masked=masked and (attention_mask, *masked))
         B, T, _ = x.shape
         H = self.num_heads
         fused = None if use_cache or cache is not None or attention_mask is not None else self._projections(x)
@@ -536,16 +560,19 @@ class CyclicFlowAttention(nn.Module):
             w = self._in_weight_folded.get(w, norm.weight, build=_native.fold_norm_weight)
         return ((w, _native.linear_rows_span(rows, w.shape[0], w.shape[1], norm=2 if folded else 1), True),)
 
-    def _forward_fused(self, x, cache, use_cache, prenorm=None, prefetch=(), attention_mask=None):
+    def _forward_fused(self, x, cache, use_cache, prenorm=None, prefetch=(), masked=None):
         """bf16 inference: the same math as forward with fused launches. With
         ``prenorm`` (the block's norm), x is the block input and the result is
-        (x + o, new_cache), as forward_block. ``attention_mask``: right-padded
-        prefill (_fused_mask_ok); the convolution multiplies its input rows by
-        the mask and the gate path zeroes the gates of the padding."""
+        (x + o, new_cache), as forward_block. ``masked``: (mask, *_plain()) of a
+        right-padded prefill (_fused_mask_ok); the convolution multiplies its
+        input rows by the mask and the gate path zeroes the gates of the padding.
+        Such a call concatenates the weights as they are, as the general path
+        reads them (the kept concatenations follow the parameters' version
+        counters, which writes through ``.data`` do not move). 8 x 576 tokens at
+        1024 wide, bound by the host's work, take 218 us with kept ones and 233
+        so; the general path took 910."""
         B, T, _ = x.shape
-        mask = valid = lengths = None
-        if attention_mask is not None:
-            mask, valid, lengths = _native.mask_rows(attention_mask)
+        mask = valid = lengths = now = None
         block_in = None
         if prenorm is not None:
             block_in = x
@@ -557,7 +584,13 @@ class CyclicFlowAttention(nn.Module):
         if self._a_bias_zero is None or self._a_bias_zero.dtype != self.b_proj.bias.dtype \
                 or self._a_bias_zero.device != self.b_proj.bias.device:
             self._a_bias_zero = torch.zeros_like(self.b_proj.bias.detach())
-        abd_bias = self._abd_bias.get(self._a_bias_zero, self.b_proj.bias, self.d_proj.bias)
+        if masked:
+            mask, valid, lengths = _native.mask_rows(masked[0])
+            w = torch.cat(masked[1])
+            now = dict(qkv=w[:2 * Dk + Dv], g0_abd=w[2 * Dk + Dv:], conv=torch.cat(masked[2]),
+                       abd_bias=torch.cat((self._a_bias_zero, *masked[3])))
+        abd_bias = (self._abd_bias.get(self._a_bias_zero, self.b_proj.bias, self.d_proj.bias) if now is None
+                    else now["abd_bias"])
         if B * T <= _native.LINEAR_ROWS_MAX:
             # one launch for the q|k|v, g_proj[0] and a|b|d projections; the
             # outputs are column slices of one buffer with 16-byte aligned rows
@@ -579,7 +612,8 @@ class CyclicFlowAttention(nn.Module):
                 y_in = _native.linear(x, w_in, b_in, out_cols=(D3 + Dg + 3 * H + 7) // 8 * 8)
             qkv, g0_out, abd = y_in[..., :D3], y_in[..., D3:D3 + Dg], y_in[..., D3 + Dg:]
         else:
-            qkv = _native.linear(x, self._qkv_weight.get(self.q_proj.weight, self.k_proj.weight, self.v_proj.weight))
+            qkv = _native.linear(x, now["qkv"] if now is not None else self._qkv_weight.get(
+                self.q_proj.weight, self.k_proj.weight, self.v_proj.weight))
             g0_out = abd = None
         conv_cache = None if cache is None else cache.get("conv_state")
         cat_cache = None
@@ -600,7 +634,8 @@ class CyclicFlowAttention(nn.Module):
             tail = nxt_conv
         else:
             tail = torch.empty(B, W - 1, qkv.shape[-1], dtype=x.dtype, device=x.device)
-        wconv = self._conv_weight.get(self.q_conv1d.weight, self.k_conv1d.weight, self.v_conv1d.weight)
+        wconv = (self._conv_weight.get(self.q_conv1d.weight, self.k_conv1d.weight, self.v_conv1d.weight) if now is None
+                 else now["conv"])
         if (not self.training and T == 1 and W == 4 and self.head_k_dim == 256 and self.head_v_dim == 256
                 and all(c.bias is None for c in (self.q_conv1d, self.k_conv1d, self.v_conv1d))
                 and (cat_cache is None or cat_cache.stride() == tail.stride())):
@@ -666,7 +701,8 @@ class CyclicFlowAttention(nn.Module):
         cq, ck, cv = tail[..., :Dk], tail[..., Dk:2 * Dk], tail[..., 2 * Dk:]
         gate = None
         if abd is None and g0_out is None:
-            w1 = self._gp_weight.get(g0.weight, self.a_proj.weight, self.b_proj.weight, self.d_proj.weight)
+            w1 = now["g0_abd"] if now is not None else self._gp_weight.get(
+                g0.weight, self.a_proj.weight, self.b_proj.weight, self.d_proj.weight)
             if _native.gate_path_ok(x, w1, g1.weight, g1.bias, H):
                 # g_proj[0], a|b|d, the gates and g_proj[1] in one launch
                 gate, g, beta, delta = _native.gate_path(x, w1, abd_bias, g1.weight, g1.bias, self.dt_bias,
@@ -674,8 +710,8 @@ class CyclicFlowAttention(nn.Module):
                 gate = gate.view(B, T, H, self.head_v_dim)
         if gate is None:
             if abd is None:
-                abd = _native.linear(x, self._abd_weight.get(self.a_proj.weight, self.b_proj.weight,
-                                                              self.d_proj.weight), abd_bias)
+                abd = _native.linear(x, now["g0_abd"][g0.weight.shape[0]:] if now is not None else self._abd_weight.get(
+                    self.a_proj.weight, self.b_proj.weight, self.d_proj.weight), abd_bias)
             g, beta, delta = _native.gates(abd, self.dt_bias, self.A_log)
             if valid is not None:
                 keep = valid.unsqueeze(-1).bool()

@@ -102,6 +102,24 @@ def test_masked_call_of_a_layer_with_hooks_calls_its_modules():
         assert not layer._fused_mask_ok(x, mask)
 
 
+def test_masked_call_sees_weights_written_through_data():
+    """An average of the weights copied in through ``.data``, and weights that
+    come back at an address used before: no version counter tells of either."""
+    torch.manual_seed(0)
+    layer = CyclicFlowAttention(hidden_size=256, num_heads=1).eval().bfloat16().to(DEV)
+    x = torch.randn(2, 40, 256, dtype=torch.bfloat16, device=DEV)
+    mask = torch.ones(2, 40, dtype=torch.long, device=DEV)
+    mask[1, 30:] = 0
+    with torch.no_grad():
+        layer(x, attention_mask=mask)
+        for p in (layer.q_proj.weight, layer.v_proj.weight, layer.k_conv1d.weight, layer.g_proj[0].weight,
+                  layer.b_proj.weight, layer.d_proj.bias):
+            p.data.copy_(0.1 * torch.randn(p.shape, device=DEV))
+            y, ref = layer(x, attention_mask=mask)[0], layer(x, attention_mask=mask.float())[0]
+            # (the paths' own difference, as in test_masked_layer_equals_general_path)
+            assert ((y.double() - ref.double()).norm() <= 2.0 ** -8 * ref.double().norm()).item()
+
+
 def test_masked_call_past_the_convolution_launch_keeps_the_general_path(monkeypatch):
     """More tokens, or batch rows, than a launch of the convolution takes."""
     torch.manual_seed(0)
