@@ -872,8 +872,8 @@ def gate_path(x, w1, abd_bias, w2, b2, dt_bias, A_log, H, valid=None):
     dev = require_device(x, w1, abd_bias, w2, b2, dt_bias, A_log, valid)
     x2 = x.reshape(rows, K)
     if x2.stride(-1) != 1 or x2.stride(0) % 8 or x2.data_ptr() % 16:
-        x2 = x2.contiguous()
-    w1c, w2c = w1.detach().contiguous(), w2.detach().contiguous()
+        x2 = aligned_rows(x2)
+    w1c, w2c = aligned_rows(w1.detach()), aligned_rows(w2.detach())
     ab = abd_bias.detach().to(torch.bfloat16).contiguous()
     b2c = None if b2 is None else b2.detach().contiguous()
     db = dt_bias.detach().to(torch.float32).contiguous()

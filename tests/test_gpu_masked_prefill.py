@@ -120,6 +120,24 @@ def test_masked_call_sees_weights_written_through_data():
             assert ((y.double() - ref.double()).norm() <= 2.0 ** -8 * ref.double().norm()).item()
 
 
+def test_masked_call_takes_operands_off_the_16_byte_grid():
+    """x, and g_proj[1]'s weight, as views into larger buffers."""
+    torch.manual_seed(0)
+    layer = CyclicFlowAttention(hidden_size=256, num_heads=1).eval().bfloat16().to(DEV)
+    x = torch.randn(2, 40, 256, dtype=torch.bfloat16, device=DEV)
+    mask = torch.ones(2, 40, dtype=torch.long, device=DEV)
+    mask[1, 30:] = 0
+
+    def off(t):
+        return torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)[1:].view(t.shape).copy_(t)
+
+    with torch.no_grad():
+        y = layer(x, attention_mask=mask)[0]
+        assert torch.equal(layer(off(x), attention_mask=mask)[0], y)
+        layer.g_proj[1].weight.data = off(layer.g_proj[1].weight)
+        assert torch.equal(layer(x, attention_mask=mask)[0], y)
+
+
 def test_masked_call_past_the_convolution_launch_keeps_the_general_path(monkeypatch):
     """More tokens, or batch rows, than a launch of the convolution takes."""
     torch.manual_seed(0)
