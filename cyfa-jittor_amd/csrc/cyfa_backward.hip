@@ -1172,6 +1172,20 @@ __device__ __forceinline__ float bw_rnd(float x) {
         return x;
 }
 
+// The readouts' block inputs, read from the buffers of all rows: fewer than 2^23
+// of them (the general forward; 2^21 in the backward) of at most 128 floats, so
+// regions of at most 2^32 - 2^15 bytes, past which a dead load's offset lies (in
+// one with the top bit set it would reach into another row's values from 2^31
+// bytes on).
+constexpr uint32_t RO_DEAD = 0xfffff000u;
+
+__device__ __forceinline__ float ro_load(bw_rsrc_t r, uint32_t off, bool live) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, live ? off : RO_DEAD, 0, 0));
+}
+__device__ __forceinline__ f32x2 ro_load2(bw_rsrc_t r, uint32_t off, bool live) {
+    return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(r, live ? off : RO_DEAD, 0, 0));
+}
+
 constexpr int RO_LD = BWD_TABLE_M + 4;  // staged table and row rows, 16-byte aligned
 constexpr int RO_FWD_THREADS = 1024;
 
@@ -1195,8 +1209,8 @@ __global__ __launch_bounds__(RO_FWD_THREADS) void bw_fwd_readout_kernel(const fl
     const int it = wv & 1, ct0 = CPW * (wv >> 1);
     // A block's inputs, element x of this thread = (row i, pair pr) = e / 64,
     // e % 64, e = tid + NT x: loaded one block ahead through buffer
-    // resources (rows < 2^21, M <= 128: offsets below 2^30), predicated
-    // through the offset, so that no block waits for its own loads.
+    // resources, predicated through the offset (ro_load), so that no block
+    // waits for its own loads.
     constexpr int NX = RB * (TM / 2) / NT;
     const int b_end = min(rows, (int)(blockIdx.x + 1) * per_wg * RB);
     const bw_rsrc_t rcs = bw_rsrc(cs, (size_t)rows * H * P), rsn = bw_rsrc(sn, (size_t)rows * H * P),
@@ -1208,10 +1222,10 @@ __global__ __launch_bounds__(RO_FWD_THREADS) void bw_fwd_readout_kernel(const fl
             const int e = tid + NT * x, i = e / (TM / 2), pr = e % (TM / 2), rho = b0 + i;
             const bool live = rho < b_end && pr < P;
             const uint32_t row = live ? (uint32_t)row_of(rho) : 0u;
-            nc[x] = bw_load(rcs, (row * (uint32_t)P + (uint32_t)pr) * 4u, live);
-            ns[x] = bw_load(rsn, (row * (uint32_t)P + (uint32_t)pr) * 4u, live);
-            nre[x] = bw_load(rraw, (row * (uint32_t)M + 2u * (uint32_t)pr) * 4u, live);
-            nro[x] = bw_load(rraw, (row * (uint32_t)M + 2u * (uint32_t)pr + 1u) * 4u, live);
+            nc[x] = ro_load(rcs, (row * (uint32_t)P + (uint32_t)pr) * 4u, live);
+            ns[x] = ro_load(rsn, (row * (uint32_t)P + (uint32_t)pr) * 4u, live);
+            nre[x] = ro_load(rraw, (row * (uint32_t)M + 2u * (uint32_t)pr) * 4u, live);
+            nro[x] = ro_load(rraw, (row * (uint32_t)M + 2u * (uint32_t)pr + 1u) * 4u, live);
         }
     };
     const int b_first = blockIdx.x * per_wg * RB;
@@ -1431,9 +1445,9 @@ __global__ __launch_bounds__(64 * NW, ADJ ? NW / 4 : NW / 2) void bw_readout_mf_
 #pragma unroll
     for (int rt = 0; rt < (ADJ ? DT : 1); rt++) dacc[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
     // A block's inputs, element x of this thread = (row i, pair pr) = e / 64,
-    // e % 64, e = tid + NT x: loaded one block ahead through buffer resources
-    // (rows < 2^21, M <= 128: offsets below 2^30), predicated through the
-    // offset, so that no block waits for its own loads.
+    // e % 64, e = tid + NT x: loaded one block ahead through buffer resources,
+    // predicated through the offset (ro_load), so that no block waits for its
+    // own loads.
     constexpr int NX = RB * (TM / 2) / NT;
     const int b_first = blockIdx.x * a.per_wg * RB, b_end = min(rows, b_first + a.per_wg * RB);
     const auto base_of = [&](int b0) { return ((size_t)(b0 / a.Tp) * a.H + h) * a.Tp + b0 % a.Tp; };
@@ -1449,10 +1463,10 @@ __global__ __launch_bounds__(64 * NW, ADJ ? NW / 4 : NW / 2) void bw_readout_mf_
 #pragma unroll
         for (int x = 0; x < NX; x++) {
             const uint32_t at = ((row0 + (uint32_t)(NT / (TM / 2) * x)) * (uint32_t)P + (uint32_t)pr_in) * 4u;
-            nc[x] = bw_load(rcs, at, live);
-            ns[x] = bw_load(rsn, at, live);
-            nr[x] = load2(rraw, 2u * at, live);
-            if constexpr (ADJ) nd[x] = load2(rdw, 2u * at, live);
+            nc[x] = ro_load(rcs, at, live);
+            ns[x] = ro_load(rsn, at, live);
+            nr[x] = ro_load2(rraw, 2u * at, live);
+            if constexpr (ADJ) nd[x] = ro_load2(rdw, 2u * at, live);
         }
     };
     load_block(b_first);
@@ -1678,8 +1692,8 @@ __global__ __launch_bounds__(RO_ADJ_THREADS) void bw_readout_kernel(ReadoutGradA
     const int rows = a.B * a.Tp;
     // A block's inputs, element x of this thread = (row i, pair pr) = e / 64,
     // e % 64, e = tid + NT x: loaded one block ahead through buffer
-    // resources (rows < 2^21, M <= 128: offsets below 2^30), predicated
-    // through the offset, so that no block waits for its own loads.
+    // resources, predicated through the offset (ro_load), so that no block
+    // waits for its own loads.
     constexpr int NX = RO_BLK * (TM / 2) / NT;
     const int b_end = min(rows, (blk + 1) * a.per_wg * RO_BLK);
     const bw_rsrc_t rcs = bw_rsrc(a.cs, (size_t)rows * a.H * P), rsn = bw_rsrc(a.sn, (size_t)rows * a.H * P),
@@ -1691,12 +1705,12 @@ __global__ __launch_bounds__(RO_ADJ_THREADS) void bw_readout_kernel(ReadoutGradA
             const int e = tid + NT * x, i = e / (TM / 2), pr = e % (TM / 2), rho = b0 + i;
             const bool live = rho < b_end && pr < P;
             const uint32_t row = live ? (uint32_t)(((rho / a.Tp) * a.H + h) * a.Tp + rho % a.Tp) : 0u;
-            nc[x] = bw_load(rcs, (row * (uint32_t)P + (uint32_t)pr) * 4u, live);
-            ns[x] = bw_load(rsn, (row * (uint32_t)P + (uint32_t)pr) * 4u, live);
-            nre[x] = bw_load(rraw, (row * (uint32_t)M + 2u * (uint32_t)pr) * 4u, live);
-            nro[x] = bw_load(rraw, (row * (uint32_t)M + 2u * (uint32_t)pr + 1u) * 4u, live);
-            nde[x] = bw_load(rdw, (row * (uint32_t)M + 2u * (uint32_t)pr) * 4u, live);
-            ndd[x] = bw_load(rdw, (row * (uint32_t)M + 2u * (uint32_t)pr + 1u) * 4u, live);
+            nc[x] = ro_load(rcs, (row * (uint32_t)P + (uint32_t)pr) * 4u, live);
+            ns[x] = ro_load(rsn, (row * (uint32_t)P + (uint32_t)pr) * 4u, live);
+            nre[x] = ro_load(rraw, (row * (uint32_t)M + 2u * (uint32_t)pr) * 4u, live);
+            nro[x] = ro_load(rraw, (row * (uint32_t)M + 2u * (uint32_t)pr + 1u) * 4u, live);
+            nde[x] = ro_load(rdw, (row * (uint32_t)M + 2u * (uint32_t)pr) * 4u, live);
+            ndd[x] = ro_load(rdw, (row * (uint32_t)M + 2u * (uint32_t)pr + 1u) * 4u, live);
         }
     };
     const int b_first = blk * a.per_wg * RO_BLK;
