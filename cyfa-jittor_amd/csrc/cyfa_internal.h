@@ -208,6 +208,7 @@ struct GatesTrainParams {
     void *dx, *dwa, *dwb, *dwd, *dbb, *dbd;  // dx nullable
     float *ddt_bias, *dA_log;
     float *dabd, *part_sums, *part_w;  // parts of the adjoint's workspace (set by the launcher)
+    int rows_wg;                     // rows of an adjoint workgroup (set by the launcher)
 };
 constexpr int GATES_MAX_H = 8;
 

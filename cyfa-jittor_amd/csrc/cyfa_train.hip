@@ -488,11 +488,16 @@ __global__ __launch_bounds__(256) void gates_grad_act_kernel(GatesTrainParams p,
 
 // Adjoint of the projections: dx = da W_a + db W_b (the clock branch passes no
 // gradient into x) and dW[n] = sum over the rows of dabd[n] x. A lane holds
-// four columns, a workgroup 256 columns and GATES_ROWS rows, a wave every
+// four columns, a workgroup 256 columns and p.rows_wg rows, a wave every
 // fourth of them, the weights and dW in registers (HM: H rounded up to 4 or
 // 8); the waves' parts of dW are added in LDS, in wave order, into one partial
 // per workgroup.
-constexpr int GATES_ROWS = 32;
+// Rows of a workgroup: 32, and 128 where that still leaves 256 workgroups per
+// 256 columns, so that the partials, 3 H floats per column and workgroup, stay
+// below x itself (65536 rows of 2048 bf16 columns, 8 heads: 101 MB, where 32
+// rows made 403 MB and a step of the gates held 687 MB, 544 as torch
+// operations; with 128 it holds 385 and takes 558 us, 798 before).
+int gates_rows(int rows) { return rows >= 32768 ? 128 : 32; }
 
 template <class E, int HM>
 __global__ __launch_bounds__(256) void gates_grad_kernel(GatesTrainParams p) {
@@ -509,8 +514,8 @@ __global__ __launch_bounds__(256) void gates_grad_kernel(GatesTrainParams p) {
     }
 #pragma unroll
     for (int n = 0; n < 3 * HM; n++) dw[n] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int row0 = blockIdx.y * GATES_ROWS;
-    for (int i = 0; i < GATES_ROWS; i += 8) {  // two rows of this wave at a time
+    const int row0 = blockIdx.y * p.rows_wg;
+    for (int i = 0; i < p.rows_wg && row0 + i < p.rows; i += 8) {  // two rows of this wave at a time
         f32x4 x[2];
 #pragma unroll
         for (int u = 0; u < 2; u++) {
@@ -586,9 +591,10 @@ int launch_gates_train_as(const GatesTrainParams& p, hipStream_t stream) {
 }
 
 template <class E>
-int launch_gates_grad_as(const GatesTrainParams& p, hipStream_t stream) {
+int launch_gates_grad_as(GatesTrainParams p, hipStream_t stream) {
     const dim3 block(256);
-    const int acts = (p.rows + 63) / 64, parts = (p.rows + GATES_ROWS - 1) / GATES_ROWS;
+    p.rows_wg = gates_rows(p.rows);
+    const int acts = (p.rows + 63) / 64, parts = (p.rows + p.rows_wg - 1) / p.rows_wg;
     hipLaunchKernelGGL(gates_grad_act_kernel, dim3(acts), block, 0, stream, p, sizeof(E) == 2 ? 1 : 0);
     const dim3 grid((p.K + 255) / 256, parts);
     if (p.H <= 4)
@@ -603,7 +609,8 @@ int launch_gates_grad_as(const GatesTrainParams& p, hipStream_t stream) {
 }  // namespace
 
 size_t gates_grad_workspace_bytes(int rows, int K, int H) {
-    return ((size_t)rows * 3 * H + (size_t)((rows + 63) / 64) * 4 * H + (size_t)((rows + GATES_ROWS - 1) / GATES_ROWS) * 3 * H * K) *
+    const int n = gates_rows(rows);
+    return ((size_t)rows * 3 * H + (size_t)((rows + 63) / 64) * 4 * H + (size_t)((rows + n - 1) / n) * 3 * H * K) *
            sizeof(float);
 }
 
@@ -616,7 +623,7 @@ static void gates_grad_workspace(GatesTrainParams& p, float* base) {
 
 int launch_gates_train(const GatesTrainParams& p_in, bool bf16, bool grad, float* workspace, hipStream_t stream) {
     GatesTrainParams p = p_in;
-    if (p.rows < 1 || p.rows > GATES_ROWS * 65535 || p.K < 8 || p.K % 8 || p.H < 1 || p.H > GATES_MAX_H ||
+    if (p.rows < 1 || p.rows > 32 * 65535 || p.K < 8 || p.K % 8 || p.H < 1 || p.H > GATES_MAX_H ||
         (long long)3 * p.H * p.K >= 1ll << 31)
         return -1;
     if (!grad) return bf16 ? launch_gates_train_as<bf16_t>(p, stream) : launch_gates_train_as<float>(p, stream);

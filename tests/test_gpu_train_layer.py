@@ -245,7 +245,8 @@ def _gates64(x, wa, wb, bb, wd, bd, dt_bias, A_log, dtype):
 @pytest.mark.parametrize("rows,K,H,dtype", [(1, 8, 1, torch.float32), (17, 256, 4, torch.bfloat16),
                                             (65, 1000, 6, torch.float32), (100, 40, 5, torch.bfloat16),
                                             (333, 2048, 8, torch.bfloat16), (3000, 1024, 4, torch.bfloat16),
-                                            (70, 264, 3, torch.float32)])
+                                            (70, 264, 3, torch.float32),
+                                            (32768 + 41, 264, 2, torch.bfloat16)])  # 128 rows per workgroup
 def test_gates_training_gradients(rows, K, H, dtype):
     """bf16: the projections' cotangents are rounded (2^-8 of each) before the
     sums, and the results are rounded again; a projection on a rounding edge may
