@@ -227,7 +227,7 @@ struct StateScanArgs {
     const float* x0;     // nullable [B*H, Kq, Vd]
     float* xs;           // [B*H, N+1, Kq, Vd]
     const float* S;      // backward: the forward states [B*H, N+1, Kq, Vd]
-    float* bnd;          // backward: [B*H, ntiles, N], ntiles = ceil(Vd / 32) ceil(Kq / 64)
+    float* bnd;          // backward: [B*H, ntiles, N], ntiles = ceil(Vd / 32) ceil(Kq / 32)
     float* x_out;        // nullable [B*H, Kq, Vd]
     int B, T, Tp, H, Kq, Vd, N;
     float scale;
@@ -244,14 +244,14 @@ struct StateScanArgs {
 // fp32 FMA loops, one 4-byte LDS read of a per row and token, the scan of a
 // 256 x 128 state over 16 chunks of 8 (b, h) took 50 us forward and 35 backward;
 // here 19 and 23.)
-// A workgroup takes a 32 T2 x 32 T2 tile, wave w its 16 T2 x 16 T2 quarter (w
-// >> 1, w & 1) as T2 x T2 accumulator
-// blocks: lane (lr, lg) of block (ib, jb) has rows 16 T2 (w >> 1) + 16 ib +
-// 4 lg + i, column 16 T2 (w & 1) + 16 jb + lr. The larger tile reads each
+// A workgroup takes a 32 T2 x 32 T2 tile, wave w of its 4 (T2 = 1) or 8 the
+// 16 x 16 T2 block of rows 16 (w >> 1) and columns 16 T2 (w & 1) as T2
+// accumulators: lane (lr, lg) of accumulator jb has rows 16 (w >> 1) + 4 lg + i,
+// column 16 T2 (w & 1) + 16 jb + lr. The larger tile reads each
 // chunk's rows of a and b from fewer workgroups (the scans are bound by those
 // reads: every column tile reads the rows of a again, every row tile the
 // columns of b). Per chunk, thread (r, q) = (tid % 32 T2, tid / 32 T2) loads
-// tokens 8 T2 q .. + 8 T2 of row r of a and of column r of b and stages them
+// tokens 8 q .. + 8 of row r of a and of column r of b and stages them
 // transposed (row = state coordinate, 64 tokens along the row), so that every
 // operand fragment is consecutive in LDS. The boundary terms go to bnd per
 // 32 x 32 tile: with T2 = 2 one per pair of waves, with T2 = 1 one
@@ -522,9 +522,7 @@ void launch_scan_mf(const StateScanArgs& a, bool mfma, dim3 grid, hipStream_t st
         hipLaunchKernelGGL((bw_state_scan_mf_kernel<BWD, T2, true, true>), grid, blk, 0, stream, a);
     else if (a.sbf)
         hipLaunchKernelGGL((bw_state_scan_mf_kernel<BWD, T2, true, false>), grid, blk, 0, stream, a);
-    else if (a.bbf)
-        hipLaunchKernelGGL((bw_state_scan_mf_kernel<BWD, T2, false, true>), grid, blk, 0, stream, a);
-    else
+    else  // (bf16 rows come with bf16 states)
         hipLaunchKernelGGL((bw_state_scan_mf_kernel<BWD, T2, false, false>), grid, blk, 0, stream, a);
 }
 
@@ -1006,8 +1004,8 @@ __global__ __launch_bounds__(256) void bw_out_kernel(OutArgs a) {
     __shared__ float sA[BC][BC + 1];
     // (output tiles of 64 columns: two at a time read q once instead of twice
     // but measured slower here, 80 -> 84 us at configuration 3)
-    constexpr int NT = 1, NA = 4 * NT;
-    __shared__ __align__(16) unsigned char sStage[NT == 2 ? STAGE2_BYTES : STAGE_BYTES];
+    constexpr int NA = 4;
+    __shared__ __align__(16) unsigned char sStage[STAGE_BYTES];
     __shared__ float sG[BC], sEq[BC];
     const int tid = threadIdx.x, n = blockIdx.x, h = blockIdx.y, b = blockIdx.z / a.parts, part = blockIdx.z % a.parts;
     const int Kq = a.Kq, Vd = a.Vd, t0 = n * BC;
@@ -1022,11 +1020,11 @@ __global__ __launch_bounds__(256) void bw_out_kernel(OutArgs a) {
     }
     chunk_scores<MF, V4>(q, Kq, BC, k, Kq, BC, Kq, sG, sStage, sA);
     float* out = a.out + (bh * a.Tp + t0) * Vd;
-    for (int d0 = BC * NT * part; d0 < Vd; d0 += BC * NT * a.parts) {
+    for (int d0 = BC * part; d0 < Vd; d0 += BC * a.parts) {
         float acc[NA][4] = {};
-        tile_gemm<MF, NT>(RK(q, Kq, BC, Kq), SJ(S + d0, Vd, Kq, Vd - d0), Kq, sStage, acc);
+        tile_gemm<MF, 1>(RK(q, Kq, BC, Kq), SJ(S + d0, Vd, Kq, Vd - d0), Kq, sStage, acc);
         tile_scale_rows<NA>(acc, [&](int t) { return sEq[t]; });
-        tile_gemm<MF, NT>(in_order([&](int i, int kk) { return sA[i][kk]; }), RJ(v + d0, Vd, BC, Vd - d0), BC, sStage, acc);
+        tile_gemm<MF, 1>(in_order([&](int i, int kk) { return sA[i][kk]; }), RJ(v + d0, Vd, BC, Vd - d0), BC, sStage, acc);
         if (!a.out_bthd) {
             if (a.bf16) {
 #pragma unroll
@@ -1305,9 +1303,8 @@ __global__ __launch_bounds__(RO_FWD_THREADS) void bw_fwd_readout_kernel(const fl
 // are those of bw_fwd_readout_kernel and bw_readout_kernel):
 //   z (and du) as two bf16 parts into LDS; logits (and dp); softmax (and dl);
 //   u (and dz); weights, or draw, the clock's and the gate's shares; dtable.
-// Wave w owns slots and coordinates 16 (w % 8) .. + 15 of every product (and,
-// with 16 waves, row tile w / 8) and holds the table's rows and columns for
-// them as operand registers (64 with both parts), so that the table takes no
+// Wave w of eight owns slots and coordinates 16 w .. + 15 of every product and
+// holds the table's rows and columns for them as operand registers (64 with both parts), so that the table takes no
 // LDS and no reads per block; its part of dtable stays in accumulators. The
 // products are formed transposed, slots (coordinates) by rows: a lane then
 // holds four neighbouring slots of one row, a row's reductions are three adds
@@ -1328,7 +1325,7 @@ __global__ __launch_bounds__(RO_FWD_THREADS) void bw_fwd_readout_kernel(const fl
 constexpr int RO_LDB = BWD_TABLE_M + 8;    // bf16 row blocks [32][RO_LDB]
 constexpr int RO_LDP = BWD_RO_BLOCK + 8;   // p and dl by slots [128][RO_LDP]
 constexpr int RO_LDC = BWD_TABLE_M / 2 + 4;  // phases [32][RO_LDC]
-constexpr int RO_MF_FWD_WAVES = 8, RO_MF_ADJ_WAVES = 8;
+constexpr int RO_MF_WAVES = 8;
 
 // lane (lr, lg) gets X[r0 + lr][k0 + 8 lg .. + 7] of a row-major bf16 tile
 template <int LD>
@@ -1396,12 +1393,12 @@ struct ReadoutGradArgs {
     int per_wg;                                 // blocks of 32 rows per workgroup
 };
 
-template <bool ADJ, bool BF, int NW>
-__global__ __launch_bounds__(64 * NW, ADJ ? NW / 4 : NW / 2) void bw_readout_mf_kernel(ReadoutGradArgs a) {
+template <bool ADJ, bool BF>
+__global__ __launch_bounds__(64 * RO_MF_WAVES, ADJ ? 2 : 4) void bw_readout_mf_kernel(ReadoutGradArgs a) {
     static_assert(!(ADJ && BF), "the adjoint is unrounded");
-    constexpr int TM = BWD_TABLE_M, RB = BWD_RO_BLOCK, LB = RO_LDB, KS = TM / 32, NT = 64 * NW;
-    constexpr int RT = 16 / NW, DT = 64 / NW;  // row tiles and dtable slot tiles of a wave
-    static_assert(TM == 128 && RB == 32 && (NW == 8 || NW == 16), "eight 16-wide tiles of slots, two of rows");
+    constexpr int TM = BWD_TABLE_M, RB = BWD_RO_BLOCK, LB = RO_LDB, KS = TM / 32, NT = 64 * RO_MF_WAVES;
+    constexpr int RT = RB / 16, DT = TM / 16;  // row tiles and dtable slot tiles of a wave
+    static_assert(TM == 16 * RO_MF_WAVES && RB == 32, "a 16-wide tile of slots per wave, two of rows");
     __shared__ __align__(16) bf16_t sZ[2][RB * LB], sP[2][RB * LB];                      // [part][row][m | slot]
     __shared__ __align__(16) bf16_t sDU[ADJ ? 2 : 1][ADJ ? RB * LB : 8], sDL[ADJ ? 2 : 1][ADJ ? RB * LB : 8];
     __shared__ __align__(16) bf16_t sPt[ADJ ? 2 : 1][ADJ ? TM * RO_LDP : 8], sDt[ADJ ? 2 : 1][ADJ ? TM * RO_LDP : 8];
@@ -1409,8 +1406,7 @@ __global__ __launch_bounds__(64 * NW, ADJ ? NW / 4 : NW / 2) void bw_readout_mf_
     __shared__ __align__(16) float sMx[RB][8], sSum[RB][8], sSd[RB][8];
     __shared__ float sLam[RB][8], sGq[RB][8];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), h = blockIdx.y;
-    const int lr = lane & 15, lg = lane >> 4, cw = wv & 7;
-    const int it0 = RT == 2 ? 0 : wv >> 3, dt0 = DT * (wv >> 3);  // DT == 8: wv >> 3 is 0
+    const int lr = lane & 15, lg = lane >> 4, cw = wv;
     const int M = a.M, R = M - 1, P = M / 2, rows = a.B * a.Tp;
     const auto load2 = [](bw_rsrc_t r, uint32_t off, bool live) {
         return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off | (live ? 0u : BW_DEAD), 0, 0));
@@ -1441,7 +1437,7 @@ __global__ __launch_bounds__(64 * NW, ADJ ? NW / 4 : NW / 2) void bw_readout_mf_
     float kappa[2];
 #pragma unroll
     for (int j = 0; j < 2; j++) kappa[j] = s0 / 2 + j < P ? (float)(kTwoPiBw * (s0 / 2 + j) / R) : 0.f;
-    f32x4 dacc[ADJ ? DT : 1];  // dtable rows 16 (dt0 + rt) .. of column 16 cw + lr
+    f32x4 dacc[ADJ ? DT : 1];  // dtable rows 16 rt .. of column 16 cw + lr
 #pragma unroll
     for (int rt = 0; rt < (ADJ ? DT : 1); rt++) dacc[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
     // A block's inputs, element x of this thread = (row i, pair pr) = e / 64,
@@ -1488,11 +1484,11 @@ __global__ __launch_bounds__(64 * NW, ADJ ? NW / 4 : NW / 2) void bw_readout_mf_
         load_block(b0 + RB);  // the next block (past the end: dead loads)
         __syncthreads();
         // logits l[r][i] = table[r] . z[i] and dp[r][i] = table[r] . du[i]: lane holds
-        // slots s0 + q of row 16 (it0 + t) + lr
+        // slots s0 + q of row 16 t + lr
         f32x4 l[RT], dp[RT];
 #pragma unroll
         for (int t = 0; t < RT; t++) {
-            const int i0 = 16 * (it0 + t);
+            const int i0 = 16 * t;
             l[t] = dp[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int k = 0; k < KS; k++) {
@@ -1514,7 +1510,7 @@ __global__ __launch_bounds__(64 * NW, ADJ ? NW / 4 : NW / 2) void bw_readout_mf_
         };
 #pragma unroll
         for (int t = 0; t < RT; t++) {
-            const int i = 16 * (it0 + t) + lr;
+            const int i = 16 * t + lr;
             const float mx = across(sMx[i], true);
             float sum = 0.f, sd = 0.f;
 #pragma unroll
@@ -1533,7 +1529,7 @@ __global__ __launch_bounds__(64 * NW, ADJ ? NW / 4 : NW / 2) void bw_readout_mf_
         __syncthreads();
 #pragma unroll
         for (int t = 0; t < RT; t++) {
-            const int i = 16 * (it0 + t) + lr;
+            const int i = 16 * t + lr;
             const float inv = 1.f / across(sSum[i], false);
             const float pdp = ADJ ? across(sSd[i], false) * inv : 0.f;
             f32x4 p, d;
@@ -1565,11 +1561,11 @@ __global__ __launch_bounds__(64 * NW, ADJ ? NW / 4 : NW / 2) void bw_readout_mf_
         __syncthreads();
         // u[m][i] = sum_r table[r][m] p[i][r] and dz[m][i] = sum_r table[r][m] dl[i][r]
         // (p, dl and the table are zero at r >= R): lane holds coordinates s0 + q of row
-        // 16 (it0 + t) + lr
+        // 16 t + lr
         const size_t row0 = base_of(b0);
 #pragma unroll
         for (int t = 0; t < RT; t++) {
-            const int i0 = 16 * (it0 + t), i = i0 + lr;
+            const int i0 = 16 * t, i = i0 + lr;
             f32x4 u = {0.f, 0.f, 0.f, 0.f}, dz = u;
 #pragma unroll
             for (int k = 0; k < KS; k++) {
@@ -1620,7 +1616,7 @@ __global__ __launch_bounds__(64 * NW, ADJ ? NW / 4 : NW / 2) void bw_readout_mf_
             const bf16x8 zh = ro_col(sZ[0], 16 * cw), zl = ro_col(sZ[1], 16 * cw);
 #pragma unroll
             for (int rt = 0; rt < DT; rt++) {
-                const int r0 = 16 * (dt0 + rt);
+                const int r0 = 16 * rt;
                 dacc[rt] = mfma_split<BF>(ro_row<RO_LDP>(sPt[0], r0, 0), ro_row<RO_LDP>(sPt[1], r0, 0), uh, ul, dacc[rt]);
                 dacc[rt] = mfma_split<BF>(ro_row<RO_LDP>(sDt[0], r0, 0), ro_row<RO_LDP>(sDt[1], r0, 0), zh, zl, dacc[rt]);
             }
@@ -1634,14 +1630,14 @@ __global__ __launch_bounds__(64 * NW, ADJ ? NW / 4 : NW / 2) void bw_readout_mf_
             }
         }
     }
-    if constexpr (ADJ) {  // lane holds dtable rows 16 (dt0 + rt) + 4 lg + q of column 16 cw + lr
+    if constexpr (ADJ) {  // lane holds dtable rows 16 rt + 4 lg + q of column 16 cw + lr
         float* dst = a.dtab + ((size_t)h * gridDim.x + blockIdx.x) * R * M;
         const int m = 16 * cw + lr;
 #pragma unroll
         for (int rt = 0; rt < DT; rt++)
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-                const int r = 16 * (dt0 + rt) + 4 * lg + q;
+                const int r = 16 * rt + 4 * lg + q;
                 if (r < R && m < M) dst[r * M + m] = dacc[rt][q];
             }
     }
@@ -2588,9 +2584,9 @@ int launch_chunk_readout(const float* raw, const float* cs, const float* sn, con
     ro.M = M;
     ro.per_wg = per;
     if (split && bf16)
-        hipLaunchKernelGGL((bw_readout_mf_kernel<false, true, RO_MF_FWD_WAVES>), grid, dim3(64 * RO_MF_FWD_WAVES), 0, stream, ro);
+        hipLaunchKernelGGL((bw_readout_mf_kernel<false, true>), grid, dim3(64 * RO_MF_WAVES), 0, stream, ro);
     else if (split)
-        hipLaunchKernelGGL((bw_readout_mf_kernel<false, false, RO_MF_FWD_WAVES>), grid, dim3(64 * RO_MF_FWD_WAVES), 0, stream, ro);
+        hipLaunchKernelGGL((bw_readout_mf_kernel<false, false>), grid, dim3(64 * RO_MF_WAVES), 0, stream, ro);
     else if (bf16)
         return -1;  // bf16 operands come with the split form
     else
@@ -2777,7 +2773,7 @@ int launch_chunk_bwd(const BwdParams& p, hipStream_t stream) {
         hipLaunchKernelGGL(bw_wide_dtable_kernel, dim3((M - 1 + BC - 1) / BC, (M + BC - 1) / BC, H * ws.ro_blocks), blk, 0,
                            stream, wa);
     } else if (bf) {
-        hipLaunchKernelGGL((bw_readout_mf_kernel<true, false, RO_MF_ADJ_WAVES>), dim3(ws.ro_blocks, H), dim3(64 * RO_MF_ADJ_WAVES), 0, stream, ro);
+        hipLaunchKernelGGL((bw_readout_mf_kernel<true, false>), dim3(ws.ro_blocks, H), dim3(64 * RO_MF_WAVES), 0, stream, ro);
     } else {
         hipLaunchKernelGGL(bw_readout_kernel, dim3(ws.ro_blocks, H), dim3(RO_ADJ_THREADS), 0, stream, ro);
     }
