@@ -433,7 +433,9 @@ constexpr int BWD_NORM_ROWS = 64;   // rows per norm-adjoint workgroup
 
 // Blocks of 32 rows per readout workgroup: rows shared over the wgs workgroups
 // that the chip holds at once (each takes the head's table once), 16 blocks at
-// most.
+// most. wgs is 256 for the kernels whose LDS or registers hold one workgroup
+// per compute unit, 512 for the bf16 forward: written in, not asked of the
+// device, since the workspace's size depends on it and is asked without one.
 inline int bwd_ro_per_wg(int B, int Tp, int H, int wgs) {
     const int blocks = (B * Tp + BWD_RO_BLOCK - 1) / BWD_RO_BLOCK;
     const int per = (int)(((long long)blocks * H + wgs - 1) / wgs);
