@@ -569,7 +569,7 @@ class CyclicFlowAttention(nn.Module):
         Such a call concatenates the weights as they are, as the general path
         reads them (the kept concatenations follow the parameters' version
         counters, which writes through ``.data`` do not move). 8 x 576 tokens at
-        1024 wide, bound by the host's work, take 218 us with kept ones and 233
+        1024 wide, bound by the host's work, take 214 us with kept ones and 226
         so; the general path took 910."""
         B, T, _ = x.shape
         mask = valid = lengths = now = None
