@@ -384,7 +384,7 @@ class CyclicFlowAttention(nn.Module):
         a|b|d weights], [convolution weights], [b|d biases]), where every module
         that the fused path computes is the plain one, of the layer's sizes, with
         the biases it adds and no others, and the convolutions are of one width;
-        else None. (Read from the modules' own dictionaries: 8 us of a call that
+        else None. (Read from the modules' own dictionaries: 6 us of a call that
         is bound by the host's work, 17 by attribute.)"""
         if torch.nn.modules.module._has_any_global_hook():
             return None
